@@ -364,8 +364,8 @@ int ccgpu_mlp_features(int mlp, int handle, float *feat, float *target);
  * counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under hipGraph capture, serving loops).  It allocates nothing:
  * its block partials live in a static per-device array of 4096 complex values,
- * one per span of 65536 amplitudes, so n is limited to 268 435 456; larger n
- * is rejected with an error.  Calls that overlap on one GPU share that array
+ * one per span of 2048 to 65536 amplitudes, so n is limited to 268 435 456;
+ * larger n is rejected with an error.  Calls that overlap on one GPU share that array
  * and race. */
 int ccgpu_energy_noalloc(long long n, const double *t, const double *r0, double *ecorr, void *stream);
 
