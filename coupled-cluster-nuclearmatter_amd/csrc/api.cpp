@@ -2840,6 +2840,11 @@ void build_triples(Solve &S) {
     td.chiral = 1;
     td.ch = S.chiral_dev;
     td.tnf = S.tnf >= 2 ? 1 : 0;
+    // without the constants the generator leaves behind, the <cb||kd> fill
+    // would read through null tables
+    if (td.tnf && !S.chiral3.kx)
+      throw Error("the three-nucleon force was set after the interaction was generated: call "
+                  "ccgpu_generate_interaction again");
     td.c3 = S.chiral3;
   } else if (S.native_v) {
     // radial Minnesota factors over the integer momentum transfer (the

@@ -208,3 +208,17 @@ T, 2
     assert abs(got - cc) < 1e-7 * abs(cc) + 20 * TOL / 14, (got, cc)
     rows = [l.split() for l in res.stdout.splitlines() if l.startswith("twist")]
     assert [int(r[-1]) for r in rows] == [len(p["e3"]) - 1 for p in ps]
+
+
+def test_three_body_force_set_after_generation_is_an_error(ccnm):
+    """The constants of a 3NF given after the interaction was generated without
+    one: the element tables of the triples cannot be filled, and say so."""
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1)
+    s.set_chiral(ccnm.NNLO, 450.0)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    s.setup_t_amplitudes()
+    s.set_3nf(2)
+    with pytest.raises(RuntimeError, match="after the interaction was generated"):
+        s.setup_t3()
+    with pytest.raises(RuntimeError, match="after the interaction was generated"):
+        s.pert_triples2()
