@@ -78,11 +78,13 @@ void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, do
 void launch_t3_td(const SolveDesc &d, const TriplesDesc &td, double2 *tdt, hipStream_t st);
 // mlp.hip
 void launch_mlp_forward(const float *params, const uint16_t *feat, int64_t n, float *y, hipStream_t st);
-void launch_mlp_loss_grad(const float *params, const uint16_t *feat, const float *target, const int64_t *idx,
-                          int64_t n, int64_t npad, const MlpTrainBufs &tb, float *part, int max_split, float *grad,
-                          double *loss_sum, hipStream_t st);
-void launch_mlp_adam(float *th, const float *g, float *m, float *v, float lr, int step, hipStream_t st);
-void launch_mlp_sample(int64_t *idx, int64_t B, int64_t ntot, uint64_t seed, hipStream_t st);
+void launch_mlp_loss_grad(const float *params, const uint16_t *feat, const float *target, int64_t n, int64_t npad,
+                          const MlpTrainBufs &tb, float *part, int max_split, float *grad, double *loss_sum,
+                          hipStream_t st);
+void launch_mlp_step(float *th, float *m, float *v, const uint16_t *feat, const float *target, int64_t ntot,
+                     uint64_t seed, int64_t B, const MlpTrainBufs &tb, float *part, int max_split, float lr, int step,
+                     hipStream_t st);
+void launch_mlp_loss(const MlpTrainBufs &tb, int64_t npad, double *loss_sum, hipStream_t st);
 void launch_mlp_features(const SolveDesc &d, float kf, float ef, const float tw[3], float scale, uint16_t *feat,
                          float *target, hipStream_t st);
 void launch_mlp_apply(const SolveDesc &d, const float *y, float scale, float ef, hipStream_t st);
@@ -2095,7 +2097,6 @@ struct Mlp {
   // minibatch buffers
   int64_t bcap = 0;
   MlpTrainBufs tb{};
-  int64_t *idx = nullptr;
   float *part = nullptr;
   static constexpr int kMaxSplit = 256;
   std::vector<void *> batch_owned;
@@ -2126,7 +2127,6 @@ struct Mlp {
     tb.dz3t = dalloc<uint16_t>((size_t)64 * B, batch_owned);
     tb.g = dalloc<float>((size_t)B, batch_owned);
     tb.loss_part = dalloc<float>(2048, batch_owned);
-    idx = dalloc<int64_t>((size_t)B, batch_owned);
     part = dalloc<float>((size_t)kMaxSplit * kMlpParamCount, batch_owned);
     bcap = B;
   }
@@ -3141,8 +3141,7 @@ int ccgpu_mlp_loss_grad(int mlp, int n, const float *x, const float *t, double *
     HIPCHK(hipMemcpyAsync(M.st, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice, M.stream));
     const int64_t npad = ((int64_t)n + 63) / 64 * 64;
     M.ensure_batch(npad);
-    launch_mlp_loss_grad(M.params, M.sfeat, M.st, nullptr, n, npad, M.tb, M.part, Mlp::kMaxSplit, M.grad, M.loss,
-                         M.stream);
+    launch_mlp_loss_grad(M.params, M.sfeat, M.st, n, npad, M.tb, M.part, Mlp::kMaxSplit, M.grad, M.loss, M.stream);
     check_launch();
     double l = 0;
     HIPCHK(hipMemcpyAsync(&l, M.loss, sizeof(double), hipMemcpyDeviceToHost, M.stream));
@@ -3203,12 +3202,12 @@ int ccgpu_mlp_train(int mlp, int steps, int batch, double lr, unsigned long long
     if (steps <= 0) throw Error("steps must be positive");
     M.ensure_batch(batch);
     for (int k = 0; k < steps; ++k) {
-      launch_mlp_sample(M.idx, batch, M.n, seed + 0x51ED27ull * (uint64_t)(M.step + 1), M.stream);
-      launch_mlp_loss_grad(M.params, M.feat, M.target, M.idx, batch, batch, M.tb, M.part, Mlp::kMaxSplit, M.grad,
-                           M.loss, M.stream);
+      const uint64_t draw = seed + 0x51ED27ull * (uint64_t)(M.step + 1);
       ++M.step;
-      launch_mlp_adam(M.params, M.grad, M.m, M.v, (float)lr, M.step, M.stream);
+      launch_mlp_step(M.params, M.m, M.v, M.feat, M.target, M.n, draw, batch, M.tb, M.part, Mlp::kMaxSplit, (float)lr,
+                      M.step, M.stream);
     }
+    launch_mlp_loss(M.tb, batch, M.loss, M.stream);   // the loss of the last minibatch is what returns
     check_launch();
     double l = 0;
     HIPCHK(hipMemcpyAsync(&l, M.loss, sizeof(double), hipMemcpyDeviceToHost, M.stream));

@@ -112,16 +112,39 @@ struct MlpLds {
   float red[4];
 };
 
+// 36 KB of parameters per block: 16-byte loads, all of a thread's in flight
+// before the first is converted.
 __device__ void mlp_load_lds(const float *__restrict__ p, MlpLds &L) {
-  for (int e = threadIdx.x; e < kMlpIn * kMlpH; e += blockDim.x) {
-    int k = e / kMlpH, o = e % kMlpH;
-    L.wt1[o * kLdW1 + k] = f2bf(p[kOffW1 + e]);
+  const float4 *p4 = reinterpret_cast<const float4 *>(p);   // the blocks start at multiples of 64 floats
+  float4 v1 = p4[kOffW1 / 4 + threadIdx.x], v2[4], v3[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    v2[t] = p4[kOffW2 / 4 + 256 * t + threadIdx.x];
+    v3[t] = p4[kOffW3 / 4 + 256 * t + threadIdx.x];
   }
-  for (int e = threadIdx.x; e < kMlpH * kMlpH; e += blockDim.x) {
-    int k = e / kMlpH, o = e % kMlpH;
-    uint16_t v2 = f2bf(p[kOffW2 + e]), v3 = f2bf(p[kOffW3 + e]);
-    L.wt2[o * kLdW + k] = v2; L.w2[k * kLdW + o] = v2;
-    L.wt3[o * kLdW + k] = v3; L.w3[k * kLdW + o] = v3;
+  auto bits = [](const float4 &v, uint16_t (&o)[4]) {
+    o[0] = f2bf(v.x); o[1] = f2bf(v.y); o[2] = f2bf(v.z); o[3] = f2bf(v.w);
+  };
+  const int k0 = threadIdx.x >> 4, o0 = (threadIdx.x & 15) * 4;   // 64 outputs per input row
+  uint16_t h[4];
+  bits(v1, h);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) L.wt1[(o0 + i) * kLdW1 + k0] = h[i];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int k = 16 * t + k0;
+    bits(v2[t], h);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      L.wt2[(o0 + i) * kLdW + k] = h[i];
+      L.w2[k * kLdW + o0 + i] = h[i];
+    }
+    bits(v3[t], h);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      L.wt3[(o0 + i) * kLdW + k] = h[i];
+      L.w3[k * kLdW + o0 + i] = h[i];
+    }
   }
   for (int e = threadIdx.x; e < kMlpH; e += blockDim.x) {
     L.b1[e] = p[kOffB1 + e]; L.b2[e] = p[kOffB2 + e]; L.b3[e] = p[kOffB3 + e]; L.w4[e] = p[kOffW4 + e];
@@ -130,16 +153,42 @@ __device__ void mlp_load_lds(const float *__restrict__ p, MlpLds &L) {
   __syncthreads();
 }
 
-// Stores one lane's 16 BF16 values (features 16mt+4q+i of its sample, packed
-// in pairs) into a feature-major [64][B] array.
-__device__ __forceinline__ void store_t(uint16_t *dst, const uint32_t (&v)[4][2], int q, int64_t B, int64_t pos) {
+// Activations and gradients of a minibatch: blocks of 64 samples, feature-major
+// within a block, so a 16x16 tile of one MFMA step sits in 2 KB (rows of all B
+// samples put the 16 rows a load touches B * 2 bytes apart: at power-of-two
+// batches on one L2 channel).  Within a row of 64 the order is that of the
+// weight-gradient MFMA's lanes: lane quarter q takes samples 4q..4q+3 of each
+// of the four steps, 32 bytes in a row.  Position of sample s of feature f, F
+// features:
+__device__ __forceinline__ int mlp_in_row(int s) { return ((s >> 2) & 3) * 16 + ((s >> 4) & 3) * 4 + (s & 3); }
+__device__ __forceinline__ int64_t mlp_at(int F, int f, int64_t s) {
+  return ((s >> 6) * F + f) * 64 + mlp_in_row((int)(s & 63));
+}
+
+// Stores a block's 64 samples x 64 BF16 features (lane (r, q) of wave w holds
+// features 16mt+4q+i of sample 16w+r, packed in pairs) as the row block at
+// dst.  The tile is turned in LDS, so that a thread stores 32 bytes and a row
+// of 64 samples one 128-byte line, instead of 2 bytes sixteen times.  Arrays
+// alternate between the two tiles: the barrier of one also says that every
+// thread has read the tile before it.
+constexpr int kLdT = 72;   // padded LDS row: 64 samples
+__device__ __forceinline__ void store_t(uint16_t *dst, const uint32_t (&v)[4][2], uint16_t *tile) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int col = mlp_in_row(16 * (threadIdx.x >> 6) + r);
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t w = v[mt][i >> 1];
-      dst[(int64_t)(16 * mt + 4 * q + i) * B + pos] = (uint16_t)((i & 1) ? (w >> 16) : (w & 0xFFFF));
+      tile[(16 * mt + 4 * q + i) * kLdT + col] = (uint16_t)((i & 1) ? (w >> 16) : (w & 0xFFFF));
     }
+  __syncthreads();
+  const int f = threadIdx.x >> 2, c = (threadIdx.x & 3) * 16;
+  const uint4 *src = reinterpret_cast<const uint4 *>(tile + f * kLdT + c);
+  uint4 *out = reinterpret_cast<uint4 *>(dst + f * 64 + c);
+  const uint4 x = src[0], y = src[1];
+  out[0] = x;
+  out[1] = y;
 }
 
 // One hidden 64 -> 64 layer, transposed: outputs 16mt+4q+i of this lane's
@@ -221,27 +270,54 @@ __device__ __forceinline__ float mlp_forward16(const uint16_t *wt1, const float 
   return part + b4;
 }
 
+// minibatch position -> training-set sample (with replacement, splitmix64)
+__device__ __forceinline__ int64_t mlp_draw(int64_t pos, int64_t ntot, uint64_t seed) {
+  uint64_t z = seed + 0x9E3779B97F4A7C15ull * (uint64_t)(pos + 1);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  return (int64_t)(z % (uint64_t)ntot);
+}
+
+// A training step is three launches (this pass, k_mlp_wgrad, k_mlp_reduce with
+// Adam in it): at batch 16384 15.3 + 14.7 + 4.7 us, where drawing the samples,
+// the sums of the loss and the gradient and Adam as launches of their own,
+// 2-byte stores and serial weight gradients took 123 us.  What is left is
+// latency: 256 blocks of four waves, one round each.
+//
 // Forward (TRAIN: and backward) over samples at positions [0, npad), npad a
-// multiple of 64; position p reads sample idx[p] (or p), positions >= n are
-// padding (zero input, no loss, no gradient).  Inference writes y[p].
+// multiple of 64; position p reads sample p, or with ntot > 0 the sample drawn
+// for it from the ntot of the training set; positions >= n are padding (zero
+// input, no loss, no gradient).  Inference writes y[p].
 template <bool TRAIN>
 __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ params, const uint16_t *__restrict__ feat,
-                                                  const float *__restrict__ target, const int64_t *__restrict__ idx,
+                                                  const float *__restrict__ target, int64_t ntot, uint64_t seed,
                                                   int64_t n, int64_t npad, float inv_n, float *__restrict__ yout,
                                                   MlpTrainBufs tb) {
   __shared__ MlpLds L;
-  mlp_load_lds(params, L);
+  __shared__ __align__(16) uint16_t tiles[2][TRAIN ? kMlpH * kLdT : 8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, q = lane >> 4;
-  const int64_t B = npad;
+  uint16_t *tile0 = tiles[0], *tile1 = tiles[1];
   float loss = 0.f;
+  // inputs: lane holds features 4q..4q+3 of its sample (fetched before the
+  // weights, whose staging covers the latency of the random sample)
+  uint2 xin = make_uint2(0u, 0u);
+  float tgt = 0.f;
+  auto fetch = [&](int64_t pos) {
+    xin = make_uint2(0u, 0u);
+    if (pos < n) {
+      const int64_t smp = ntot > 0 ? mlp_draw(pos, ntot, seed) : pos;
+      xin = *reinterpret_cast<const uint2 *>(feat + smp * kMlpIn + 4 * q);
+      if constexpr (TRAIN) tgt = target[smp];
+    }
+  };
+  fetch((int64_t)blockIdx.x * 64 + 16 * wave + r);
+  mlp_load_lds(params, L);
   for (int64_t base = (int64_t)blockIdx.x * 64; base < npad; base += (int64_t)gridDim.x * 64) {
-    const int64_t pos = base + 16 * wave + r;
+    const int64_t pos = base + 16 * wave + r, blk = base * kMlpH;   // row block of the 64-wide arrays
     const bool valid = pos < n;
-    const int64_t smp = valid ? (idx ? idx[pos] : pos) : 0;
-    // inputs: lane holds features 4q..4q+3 of its sample
-    uint2 xin = make_uint2(0u, 0u);
-    if (valid) xin = *reinterpret_cast<const uint2 *>(feat + smp * kMlpIn + 4 * q);
+    if (base != (int64_t)blockIdx.x * 64) fetch(pos);
     if constexpr (!TRAIN) {
       const float y = mlp_forward16(L.wt1, L.b1, L.wt2, L.b2, L.wt3, L.b3, L.w4, L.b4, xin, lane);
       if (q == 0 && valid) yout[pos] = y;
@@ -265,16 +341,16 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
       h1[mt][1] = o[2] | (o[3] << 16);
     }
     if constexpr (TRAIN) {
-      tb.x1t[(int64_t)(4 * q + 0) * B + pos] = (uint16_t)(xin.x & 0xFFFF);
-      tb.x1t[(int64_t)(4 * q + 1) * B + pos] = (uint16_t)(xin.x >> 16);
-      tb.x1t[(int64_t)(4 * q + 2) * B + pos] = (uint16_t)(xin.y & 0xFFFF);
-      tb.x1t[(int64_t)(4 * q + 3) * B + pos] = (uint16_t)(xin.y >> 16);
-      store_t(tb.h1t, h1, q, B, pos);
+      tb.x1t[mlp_at(kMlpIn, 4 * q + 0, pos)] = (uint16_t)(xin.x & 0xFFFF);
+      tb.x1t[mlp_at(kMlpIn, 4 * q + 1, pos)] = (uint16_t)(xin.x >> 16);
+      tb.x1t[mlp_at(kMlpIn, 4 * q + 2, pos)] = (uint16_t)(xin.y & 0xFFFF);
+      tb.x1t[mlp_at(kMlpIn, 4 * q + 3, pos)] = (uint16_t)(xin.y >> 16);
+      store_t(tb.h1t + blk, h1, tile0);
     }
     mlp_layer64<TRAIN>(L.wt2, L.b2, h1, h2, gd2, lane);
-    if constexpr (TRAIN) store_t(tb.h2t, h2, q, B, pos);
+    if constexpr (TRAIN) store_t(tb.h2t + blk, h2, tile1);
     mlp_layer64<TRAIN>(L.wt3, L.b3, h2, h3, gd3, lane);
-    if constexpr (TRAIN) store_t(tb.h3t, h3, q, B, pos);
+    if constexpr (TRAIN) store_t(tb.h3t + blk, h3, tile0);
     float part = 0.f;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
@@ -287,7 +363,7 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
     part += __shfl_xor(part, 32);
     const float y = part + L.b4;
     {
-      const float d = valid ? y - target[smp] : 0.f;
+      const float d = valid ? y - tgt : 0.f;
       if (q == 0) loss += d * d;
       const float g = 2.f * d * inv_n;
       uint32_t dz3[4][2], dz2[4][2], dz1[4][2];
@@ -299,11 +375,11 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
         dz3[mt][0] = o[0] | (o[1] << 16);
         dz3[mt][1] = o[2] | (o[3] << 16);
       }
-      store_t(tb.dz3t, dz3, q, B, pos);
+      store_t(tb.dz3t + blk, dz3, tile1);
       mlp_back64(L.w3, dz3, gd2, dz2, lane);
-      store_t(tb.dz2t, dz2, q, B, pos);
+      store_t(tb.dz2t + blk, dz2, tile0);
       mlp_back64(L.w2, dz2, gd1, dz1, lane);
-      store_t(tb.dz1t, dz1, q, B, pos);
+      store_t(tb.dz1t + blk, dz1, tile1);
       if (q == 0) tb.g[pos] = g;
     }
   }
@@ -317,97 +393,192 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
   }
 }
 
-// Weight gradients of one sample chunk: grid (nsplit, 4 layers).  Layer 0..2:
-// gW[k][o] = sum_s X[k][s] dZ[o][s] on MFMA (contraction over samples) and
-// gb[o] = sum_s dZ[o][s]; layer 3: gw4[f] = sum_s h3[f][s] g[s], gb4 = sum_s g[s].
-// Partials part[split][param] are summed in fixed order by k_mlp_reduce.
-__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpTrainBufs tb, int64_t B, int chunk, float *__restrict__ part) {
-  const int split = blockIdx.x, layer = blockIdx.y;
-  const int64_t s_begin = (int64_t)split * chunk;
-  const int64_t s_end = s_begin + chunk < B ? s_begin + chunk : B;
-  float *P = part + (int64_t)split * kMlpParams;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  if (layer == 3) {
-    const int t = threadIdx.x;
-    if (t < kMlpH) {
-      float acc = 0.f;
-      for (int64_t s = s_begin; s < s_end; ++s) acc += bf2f(tb.h3t[(int64_t)t * B + s]) * tb.g[s];
-      P[kOffW4 + t] = acc;
-    } else if (t == kMlpH) {
-      float acc = 0.f;
-      for (int64_t s = s_begin; s < s_end; ++s) acc += tb.g[s];
-      P[kOffB4] = acc;
-    }
-    return;
-  }
-  const uint16_t *X = layer == 0 ? tb.x1t : layer == 1 ? tb.h1t : tb.h2t;
-  const uint16_t *DZ = layer == 0 ? tb.dz1t : layer == 1 ? tb.dz2t : tb.dz3t;
-  const int K = layer == 0 ? kMlpIn : kMlpH;
-  const int offW = layer == 0 ? kOffW1 : layer == 1 ? kOffW2 : kOffW3;
-  const int offB = layer == 0 ? kOffB1 : layer == 1 ? kOffB2 : kOffB3;
-  // K=64: wave w owns input rows 16w..16w+15 and all 4 output tiles;
-  // K=16: every wave owns the single input tile and output tile w
-  const int mt = K == kMlpH ? wave : 0;
-  const int nt0 = K == kMlpH ? 0 : wave, nt1 = K == kMlpH ? 4 : wave + 1;
-  mf4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = mf4{0.f, 0.f, 0.f, 0.f};
-  for (int64_t s0 = s_begin; s0 < s_end; s0 += 16) {
-    const mbf4 a = lds4(X + (int64_t)(16 * mt + r) * B + s0 + 4 * q);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (t >= nt0 && t < nt1) acc[t] = mfma_bf16(a, lds4(DZ + (int64_t)(16 * t + r) * B + s0 + 4 * q), acc[t]);
-  }
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-    if (t >= nt0 && t < nt1)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) P[offW + (16 * mt + 4 * q + i) * kMlpH + 16 * t + r] = acc[t][i];
-  if (threadIdx.x < kMlpH) {
-    const int o = threadIdx.x;
-    float sb = 0.f;
-    for (int64_t s = s_begin; s < s_end; ++s) sb += bf2f(DZ[(int64_t)o * B + s]);
-    P[offB + o] = sb;
-  }
+// Weight gradients of one sample chunk, one task per wave: grid (nsplit,
+// kWgradBlocks).  Tasks 0..15 and 16..31 are the 16x16 tiles of gW2 and gW3,
+// 32..35 those of gW1: gW[k][o] = sum_s X[k][s] dZ[o][s] on MFMA (contraction
+// over samples); 36..38 the bias sums gb[o] = sum_s dZ[o][s], 39 gw4[f] = sum_s
+// h3[f][s] g[s], 40 gb4 = sum_s g[s].  Partials part[split][param] are summed in
+// fixed order by k_mlp_reduce.
+//
+// The work is small (4.7 MMAC per chunk of 512); what bounds it is the chain of
+// loads, so every wave has one tile, the 32 loads of a chunk of 512 are in
+// flight together, and the sums fetch the next 64 samples while they add.  At
+// batch 16384: 71 us per step with four blocks per chunk that load step by
+// step and sum sample by sample, 14.7 us like this, in the same order of
+// additions.
+constexpr int kWgradTasks = 41, kWgradBlocks = (kWgradTasks + 3) / 4;
+
+// a lane's value, the same in every lane of the wave
+__device__ __forceinline__ float lane_of(float x, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
-__global__ void k_mlp_reduce(const float *__restrict__ part, int nsplit, float *__restrict__ grad) {
+// the 64 values of a row block in sample order; FN(value, sample)
+template <class FN>
+__device__ __forceinline__ void each64(const uint4 (&v)[8], FN fn) {
+#pragma unroll
+  for (int s = 0; s < 64; s += 2) {
+    const int e = ((s >> 2) & 3) * 16 + ((s >> 4) & 3) * 4 + (s & 3), u = e >> 1;   // mlp_in_row, an even element
+    const uint4 x = v[u >> 2];
+    const uint32_t w = (u & 3) == 0 ? x.x : (u & 3) == 1 ? x.y : (u & 3) == 2 ? x.z : x.w;
+    fn(bf2f((uint16_t)(w & 0xFFFF)), s);
+    fn(bf2f((uint16_t)(w >> 16)), s + 1);
+  }
+}
+__device__ __forceinline__ void load64(uint4 (&v)[8], const uint16_t *row) {
+#pragma unroll
+  for (int t = 0; t < 8; ++t) v[t] = reinterpret_cast<const uint4 *>(row)[t];
+}
+
+__global__ __launch_bounds__(256, 2) void k_mlp_wgrad(MlpTrainBufs tb, int64_t B, int chunk, float *__restrict__ part) {
+  const int split = blockIdx.x, task = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int64_t s_begin = (int64_t)split * chunk;
+  const int64_t s_end = s_begin + chunk < B ? s_begin + chunk : B;   // a multiple of 16 samples
+  float *P = part + (int64_t)split * kMlpParams;
+  const int lane = threadIdx.x & 63;
+  if (task < 36) {
+    const int layer = task >> 4;   // 0 W2, 1 W3, 2 W1
+    const uint16_t *X = layer == 2 ? tb.x1t : layer == 0 ? tb.h1t : tb.h2t;
+    const uint16_t *DZ = layer == 2 ? tb.dz1t : layer == 0 ? tb.dz2t : tb.dz3t;
+    const int offW = layer == 2 ? kOffW1 : layer == 0 ? kOffW2 : kOffW3;
+    const int mt = layer == 2 ? 0 : (task & 15) >> 2, nt = task & 3;
+    const int r = lane & 15, q = lane >> 4;
+    const int F = layer == 2 ? kMlpIn : kMlpH;
+    const uint16_t *pa = X + (16 * mt + r) * 64 + 16 * q, *pb = DZ + (16 * nt + r) * 64 + 16 * q;
+    mf4 acc = mf4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](const uint4 &a, const uint4 &b) {
+      acc = mfma_bf16(pack4(a.x, a.y), pack4(b.x, b.y), acc);
+      acc = mfma_bf16(pack4(a.z, a.w), pack4(b.z, b.w), acc);
+    };
+    int64_t s0 = s_begin;
+    auto one = [&]() {   // 16 samples
+      const int st = (int)(s0 >> 4) & 3;
+      const uint2 a = reinterpret_cast<const uint2 *>(pa + (s0 >> 6) * F * 64)[st];
+      const uint2 b = reinterpret_cast<const uint2 *>(pb + (s0 >> 6) * kMlpH * 64)[st];
+      acc = mfma_bf16(pack4(a.x, a.y), pack4(b.x, b.y), acc);
+      s0 += 16;
+    };
+    while ((s0 & 63) && s0 < s_end) one();
+    for (; s0 + 512 <= s_end; s0 += 512) {
+      const uint4 *xa = reinterpret_cast<const uint4 *>(pa + (s0 >> 6) * F * 64);
+      const uint4 *xb = reinterpret_cast<const uint4 *>(pb + (s0 >> 6) * kMlpH * 64);
+      uint4 a[16], b[16];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        a[2 * t] = xa[0];
+        a[2 * t + 1] = xa[1];
+        b[2 * t] = xb[0];
+        b[2 * t + 1] = xb[1];
+        xa += F * 8;
+        xb += kMlpH * 8;
+      }
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the products
+#pragma unroll
+      for (int t = 0; t < 16; ++t) step(a[t], b[t]);
+    }
+    for (; s0 + 64 <= s_end; s0 += 64) {
+      const uint4 *xa = reinterpret_cast<const uint4 *>(pa + (s0 >> 6) * F * 64);
+      const uint4 *xb = reinterpret_cast<const uint4 *>(pb + (s0 >> 6) * kMlpH * 64);
+      const uint4 a0 = xa[0], a1 = xa[1], b0 = xb[0], b1 = xb[1];
+      step(a0, b0);
+      step(a1, b1);
+    }
+    while (s0 < s_end) one();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) P[offW + (16 * mt + 4 * q + i) * kMlpH + 16 * nt + r] = acc[i];
+    return;
+  }
+  if (task >= kWgradTasks) return;
+  // sums over the samples in order: task 36..38 biases, 39 w4, 40 b4 (lane 0)
+  const uint16_t *z = (task == 36 ? tb.dz1t : task == 37 ? tb.dz2t : task == 38 ? tb.dz3t : tb.h3t) + lane * 64;
+  const bool ones = task == 40, plain = task < 39;
+  float acc = 0.f;
+  int64_t s = s_begin;
+  auto single = [&](int64_t end) {
+    for (; s < end; ++s) {
+      const float x = ones ? 1.f : bf2f(z[(s >> 6) * kMlpH * 64 + mlp_in_row((int)(s & 63))]);
+      if (plain) acc += x;
+      else acc += x * tb.g[s];
+    }
+  };
+  const int64_t s1 = (s_begin + 63) / 64 * 64;
+  single(s1 < s_end ? s1 : s_end);
+  if (s + 64 <= s_end) {
+    uint4 v[8];
+    float g = 0.f;   // of sample s + lane, read back lane by lane
+    load64(v, z + (s >> 6) * kMlpH * 64);
+    if (!plain) g = tb.g[s + lane];
+#pragma unroll 1
+    for (; s + 64 <= s_end; s += 64) {
+      uint4 w[8];
+      float gn = 0.f;
+      const int64_t n = s + 128 <= s_end ? s + 64 : s;   // the next block, in flight meanwhile
+      load64(w, z + (n >> 6) * kMlpH * 64);
+      if (!plain) gn = tb.g[n + lane];
+      __builtin_amdgcn_sched_barrier(0);
+      if (plain) {
+        each64(v, [&](float x, int) { acc += x; });
+      } else if (ones) {
+#pragma unroll
+        for (int k = 0; k < 64; ++k) acc += lane_of(g, k);
+      } else {
+        each64(v, [&](float x, int k) { acc += x * lane_of(g, k); });
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) v[t] = w[t];
+      g = gn;
+    }
+  }
+  single(s_end);
+  if (plain) P[(task == 36 ? kOffB1 : task == 37 ? kOffB2 : kOffB3) + lane] = acc;
+  else if (!ones) P[kOffW4 + lane] = acc;
+  else if (lane == 0) P[kOffB4] = acc;
+}
+
+// Gradient of one parameter per thread: the splits' partials in order, 16 loads
+// in flight.  ADAM: the Adam step on it (one launch per step less, and the
+// gradient never leaves the registers), else the gradient to grad.  One wave
+// per block, so that the 149 waves spread over as many CUs.
+template <bool ADAM>
+__global__ __launch_bounds__(64) void k_mlp_reduce(const float *__restrict__ part, int nsplit, float *__restrict__ grad,
+                                                   float *__restrict__ th, float *__restrict__ m,
+                                                   float *__restrict__ v, float lr, float b1, float b2, float eps,
+                                                   float c1, float c2) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= kMlpParams) return;
   float s = 0.f;
-  for (int k = 0; k < nsplit; ++k) s += part[(int64_t)k * kMlpParams + p];
-  grad[p] = s;
-}
-
-__global__ void k_mlp_loss_reduce(const float *__restrict__ part, int n, double *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double s = 0.0;
-  for (int k = 0; k < n; ++k) s += part[k];
-  out[0] = s;
-}
-
-__global__ void k_mlp_adam(float *__restrict__ th, const float *__restrict__ g, float *__restrict__ m,
-                           float *__restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kMlpParams) return;
-  const float gp = g[p];
-  const float mp = b1 * m[p] + (1.f - b1) * gp;
-  const float vp = b2 * v[p] + (1.f - b2) * gp * gp;
-  m[p] = mp;
-  v[p] = vp;
-  th[p] -= lr * (mp / c1) / (sqrtf(vp / c2) + eps);
-}
-
-// minibatch positions -> training-set samples (with replacement, splitmix64)
-__global__ void k_mlp_sample(int64_t *__restrict__ idx, int64_t B, int64_t ntot, uint64_t seed) {
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < B; p += (int64_t)gridDim.x * blockDim.x) {
-    uint64_t z = seed + 0x9E3779B97F4A7C15ull * (uint64_t)(p + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    idx[p] = (int64_t)(z % (uint64_t)ntot);
+  int k = 0;
+  for (; k + 16 <= nsplit; k += 16) {
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) x[t] = part[(int64_t)(k + t) * kMlpParams + p];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) s += x[t];
   }
+  for (; k < nsplit; ++k) s += part[(int64_t)k * kMlpParams + p];
+  if constexpr (ADAM) {
+    const float gp = s;
+    const float mp = b1 * m[p] + (1.f - b1) * gp;
+    const float vp = b2 * v[p] + (1.f - b2) * gp * gp;
+    m[p] = mp;
+    v[p] = vp;
+    th[p] -= lr * (mp / c1) / (sqrtf(vp / c2) + eps);
+  } else {
+    grad[p] = s;
+  }
+}
+
+// Sum of the blocks' losses (at most 2048): loaded by the whole block, added
+// in order by one thread.
+__global__ __launch_bounds__(256) void k_mlp_loss_reduce(const float *__restrict__ part, int n,
+                                                         double *__restrict__ out) {
+  __shared__ float x[2048];
+  for (int k = threadIdx.x; k < n; k += 256) x[k] = part[k];
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double s = 0.0;
+  for (int k = 0; k < n; ++k) s += x[k];
+  out[0] = s;
 }
 
 // MBPT2 amplitude of unique element u (the formula of k_mbpt2)
@@ -562,6 +733,8 @@ __global__ void k_mlp_apply(SolveDesc d, const float *__restrict__ y, float scal
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+void launch_mlp_loss(const MlpTrainBufs &tb, int64_t npad, double *loss_sum, hipStream_t st);
+
 static unsigned mlp_grid(int64_t npad) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(npad / 64, 2048));
 }
@@ -569,39 +742,53 @@ static unsigned mlp_grid(int64_t npad) {
 void launch_mlp_forward(const float *params, const uint16_t *feat, int64_t n, float *y, hipStream_t st) {
   const int64_t npad = (n + 63) / 64 * 64;
   MlpTrainBufs none{};
-  hipLaunchKernelGGL(k_mlp_pass<false>, dim3(mlp_grid(npad)), dim3(256), 0, st, params, feat, nullptr, nullptr, n,
-                     npad, 0.f, y, none);
+  hipLaunchKernelGGL(k_mlp_pass<false>, dim3(mlp_grid(npad)), dim3(256), 0, st, params, feat, nullptr, (int64_t)0,
+                     (uint64_t)0, n, npad, 0.f, y, none);
 }
 
-// One loss+gradient evaluation over positions [0, npad) (npad multiple of 64):
-// grad (kMlpParams floats) and the summed squared error in *loss_sum (device).
-void launch_mlp_loss_grad(const float *params, const uint16_t *feat, const float *target, const int64_t *idx,
-                          int64_t n, int64_t npad, const MlpTrainBufs &tb, float *part, int max_split, float *grad,
-                          double *loss_sum, hipStream_t st) {
-  const unsigned grid = mlp_grid(npad);
-  hipLaunchKernelGGL(k_mlp_pass<true>, dim3(grid), dim3(256), 0, st, params, feat, target, idx, n, npad,
-                     1.0f / (float)n, nullptr, tb);
+// Forward, backward and the partial weight gradients over positions [0, npad)
+// (npad a multiple of 64); returns the number of partials.
+static int mlp_gradient_parts(const float *params, const uint16_t *feat, const float *target, int64_t ntot,
+                              uint64_t seed, int64_t n, int64_t npad, const MlpTrainBufs &tb, float *part,
+                              int max_split, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_pass<true>, dim3(mlp_grid(npad)), dim3(256), 0, st, params, feat, target, ntot, seed, n,
+                     npad, 1.0f / (float)n, nullptr, tb);
   int chunk = 512;
   int nsplit = (int)((npad + chunk - 1) / chunk);
   if (nsplit > max_split) {
     chunk = (int)(((npad + max_split - 1) / max_split + 15) / 16 * 16);
     nsplit = (int)((npad + chunk - 1) / chunk);
   }
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(nsplit, 4), dim3(256), 0, st, tb, npad, chunk, part);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, part, nsplit, grad);
-  hipLaunchKernelGGL(k_mlp_loss_reduce, dim3(1), dim3(64), 0, st, tb.loss_part, (int)grid, loss_sum);
+  hipLaunchKernelGGL(k_mlp_wgrad, dim3(nsplit, kWgradBlocks), dim3(256), 0, st, tb, npad, chunk, part);
+  return nsplit;
 }
 
-void launch_mlp_adam(float *th, const float *g, float *m, float *v, float lr, int step, hipStream_t st) {
+// One loss+gradient evaluation: grad (kMlpParams floats) and the summed
+// squared error in *loss_sum (device).
+void launch_mlp_loss_grad(const float *params, const uint16_t *feat, const float *target, int64_t n, int64_t npad,
+                          const MlpTrainBufs &tb, float *part, int max_split, float *grad, double *loss_sum,
+                          hipStream_t st) {
+  const int nsplit = mlp_gradient_parts(params, feat, target, 0, 0, n, npad, tb, part, max_split, st);
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 63) / 64), dim3(64), 0, st, part, nsplit, grad, nullptr,
+                     nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
+  launch_mlp_loss(tb, npad, loss_sum, st);
+}
+
+// One Adam step (the step-th, from 1) on a minibatch of B samples drawn from
+// the ntot of the training set: three launches.
+void launch_mlp_step(float *th, float *m, float *v, const uint16_t *feat, const float *target, int64_t ntot,
+                     uint64_t seed, int64_t B, const MlpTrainBufs &tb, float *part, int max_split, float lr, int step,
+                     hipStream_t st) {
+  const int nsplit = mlp_gradient_parts(th, feat, target, ntot, seed, B, B, tb, part, max_split, st);
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, th, g, m, v, lr, b1, b2, 1e-8f,
-                     c1, c2);
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 63) / 64), dim3(64), 0, st, part, nsplit, nullptr, th, m,
+                     v, lr, b1, b2, 1e-8f, c1, c2);
 }
 
-void launch_mlp_sample(int64_t *idx, int64_t B, int64_t ntot, uint64_t seed, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_sample, dim3((unsigned)std::min<int64_t>((B + 255) / 256, 4096)), dim3(256), 0, st, idx, B,
-                     ntot, seed);
+// Summed squared error of the last pass over npad positions
+void launch_mlp_loss(const MlpTrainBufs &tb, int64_t npad, double *loss_sum, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_loss_reduce, dim3(1), dim3(256), 0, st, tb.loss_part, (int)mlp_grid(npad), loss_sum);
 }
 
 void launch_mlp_features(const SolveDesc &d, float kf, float ef, const float tw[3], float scale, uint16_t *feat,

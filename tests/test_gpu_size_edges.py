@@ -6,6 +6,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import mlp_oracle as mo
+
 pytestmark = pytest.mark.gpu
 
 
@@ -47,3 +49,56 @@ def test_energy_noalloc_sum_at_span_edges(ccnm, hip, n):
     prod = t * np.conj(r0)
     want = complex(np.sum(prod.real.astype(np.longdouble)), np.sum(prod.imag.astype(np.longdouble)))
     assert abs(out[0] - want) <= 64 * 2.0 ** -53 * np.sum(np.abs(t) * np.abs(r0))
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 255, 257, 513, 576, 131136])
+def test_mlp_gradient_at_chunk_edges(ccnm, n):
+    """Minibatches whose last chunk leaves remainders of the unrolled loads
+    (chunks of 512; 131136 samples make chunks of 528), against the oracle with
+    the same BF16 rounding points, at the tolerance of
+    test_mlp_gradient_matches_oracle: a dropped MFMA step of 16 samples would
+    be 3% of its chunk and show in the small cases as a whole."""
+    from test_mlp import random_problem
+    theta, x, t = random_problem(n, n)
+    net = ccnm.WarmStart(seed=1)
+    net.params = theta.astype(np.float32)
+    loss, g = net.loss_grad(x, t)
+    lo, go = mo.loss_grad(theta, x.astype(np.float64), t.astype(np.float64), bf=True)
+    assert abs(loss - lo) < 1e-4 * lo
+    o = 0
+    for name, shp in mo.SHAPES:
+        m = int(np.prod(shp))
+        a, b = g[o:o + m], go[o:o + m]
+        assert np.linalg.norm(a - b) < 1e-2 * np.linalg.norm(b) + 1e-7, (name, np.linalg.norm(a - b))
+        o += m
+
+
+@pytest.mark.parametrize("batch", [64, 192, 576])
+def test_mlp_training_step_takes_the_gradient_of_its_minibatch(ccnm, batch):
+    """The first Adam step of train() restated on loss_grad of the same
+    minibatch (the splitmix64 draw over the training set) at the same
+    parameters.  (From the second step on the parameters differ in their last
+    bits and single BF16 weights may round the other way.)"""
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1)
+    s.generate_interaction()
+    s.setup_t_amplitudes()
+    s.ccd_iter()
+    net, ref = ccnm.WarmStart(seed=5), ccnm.WarmStart(seed=5)
+    n = net.add_solve(s)
+    f, tgt = net.features(s)
+    lr, seed, M64 = 1e-3, 77, (1 << 64) - 1
+    loss = net.train(1, batch=batch, lr=lr, seed=seed)
+    idx = []
+    for pos in range(batch):
+        z = (seed + 0x51ED27 + 0x9E3779B97F4A7C15 * (pos + 1)) & M64
+        z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & M64
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & M64
+        idx.append((z ^ (z >> 31)) % n)
+    th = ref.params
+    want, g = ref.loss_grad(f[idx], tgt[idx])
+    g = g.astype(np.float64)
+    step = lr * g / (np.abs(g) + 1e-8)   # m / (1 - b1) over the root of v / (1 - b2)
+    assert abs(loss - want) <= 1e-6 * want
+    # float32 powers of beta (1 - beta2 keeps 2^-24 / 1e-3 = 6e-5 relative,
+    # half of it after the root) and the roundings of m, v and the step
+    assert np.max(np.abs(net.params - (th - step))) <= 1e-4 * lr + 2.0 ** -23 * np.max(np.abs(th))
