@@ -2269,6 +2269,13 @@ int ccgpu_get_orbitals(int handle, int *nx, int *ny, int *nz, int *sz, int *tz, 
 
 }  // extern "C"
 namespace {
+// every orbital of one isospin projection (neutron matter)
+int one_species(const Orbitals &o) {
+  for (int x = 1; x < o.nsp; ++x)
+    if (o.tz[x] != o.tz[0]) return 0;
+  return 1;
+}
+
 // Device tables of the chiral NN for this lattice: radial functions over
 // m = |dn|^2 <= 3 (4 nmax)^2 and the per-side factors over j <= 3 (2 nmax)^2.
 void make_chiral_tables(Solve &S) {
@@ -2335,6 +2342,7 @@ int ccgpu_generate_interaction(int handle, int kind) {
         c = chiral3_constants(S.chiral, S.tnf_ce, S.tnf_cd, S.tnf_cutoff, S.tnf_nexp);
         c.kx = S.desc.kx; c.ky = S.desc.ky; c.kz = S.desc.kz;
         c.nx = S.desc.nx; c.ny = S.desc.ny; c.nz = S.desc.nz; c.sz = S.desc.sz; c.tz = S.desc.tz;
+        c.one_species = one_species(P.orb);
         c.scale = std::pow(197.326968, 6) / (P.orb.volume * P.orb.volume);
         // parity images for the V_pppp fill: with no twist n -> -n maps the
         // lattice onto itself with k -> -k bit for bit and the closed Fermi
@@ -2936,6 +2944,7 @@ double2 triples_sum(Solve &S, int mode) {
     Chiral3Dev c = chiral3_constants(S.chiral, S.tnf_ce, S.tnf_cd, S.tnf_cutoff, S.tnf_nexp);
     c.kx = S.desc.kx; c.ky = S.desc.ky; c.kz = S.desc.kz;
     c.nx = S.desc.nx; c.ny = S.desc.ny; c.nz = S.desc.nz; c.sz = S.desc.sz; c.tz = S.desc.tz;
+    c.one_species = one_species(P.orb);
     c.scale = std::pow(197.326968, 6) / (P.orb.volume * P.orb.volume);
     S.t3.c3w = c;
     S.have_w3 = true;

@@ -200,6 +200,7 @@ struct Chiral3Dev {
   double two_thirds;         // float32(2/3)
   double scale;              // hbarc^6 / volume^2
   int nexp;                  // regulator power
+  int one_species;           // every orbital has the same tz (neutron matter)
   const double *kx, *ky, *kz;   // single-particle momenta, fm^-1
   const int *nx, *ny, *nz, *sz, *tz;
 };
@@ -221,127 +222,207 @@ static __device__ __forceinline__ double freg3(const Chiral3Dev &c, const double
   return exp(-e);
 }
 
-// <t1|tau|t4> . (<t2|tau|t5> x <t3|tau|t6>)  (chp_tau1_dot_tauXtau, :3544-3602)
-static __device__ __forceinline__ double2 tau_triple(int t1, int t2, int t3, int t4, int t5, int t6) {
-  // Cartesian components of <a|tau|b>: x, y (complex), z
-  auto comp = [](int a, int b, int axis) -> double2 {
-    if (axis == 0) return make_double2(a != b ? 1.0 : 0.0, 0.0);
-    if (axis == 1) return a != b ? make_double2(0.0, a > 0 ? -1.0 : 1.0) : make_double2(0.0, 0.0);
-    return make_double2(a == b ? (double)a : 0.0, 0.0);
-  };
-  double2 s2[3], s3[3], s1[3];
-  for (int a = 0; a < 3; ++a) {
-    s2[a] = comp(t2, t5, a);
-    s3[a] = comp(t3, t6, a);
-    s1[a] = comp(t1, t4, a);
-  }
-  auto sub = [](double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); };
-  const double2 fx = sub(cmul_i(s2[1], s3[2]), cmul_i(s2[2], s3[1]));
-  const double2 fy = sub(cmul_i(s2[2], s3[0]), cmul_i(s2[0], s3[2]));
-  const double2 fz = sub(cmul_i(s2[0], s3[1]), cmul_i(s2[1], s3[0]));
-  const double2 a = cmul_i(fx, s1[0]), b = cmul_i(fy, s1[1]), e = cmul_i(fz, s1[2]);
-  return make_double2(a.x + b.x + e.x, a.y + b.y + e.y);
+// ---------------------------------------------------------------------------
+// The antisymmetrized element <abc||def> = sum over the six ket permutations
+// (chiral_3nf_with_delta_asym, :6904-6917) of the direct element
+// (chiral_3nf_with_delta, :6670-6902), in two parts.
+//
+// Geo3, what the momenta decide: the nine transfers q[x][y] from bra nucleon x
+// to ket nucleon y, their pion propagators, and per choice z of the third
+// nucleon's ket the regulators of both sides (the regulator is symmetric in
+// its first two nucleons, so the six permutations need three).  asym3 then
+// runs the spin-isospin algebra of the 18 (permutation, pair) terms.  Every
+// quantity of the direct element thus is evaluated once per element instead of
+// once per permutation, and the holes of one momentum share the geometry.
+//
+// Isospin: <ta|tau|td>.(<tb|tau|te> x <tc|tau|tf>) (chp_tau1_dot_tauXtau,
+// :3544-3602) is imaginary and antisymmetric in its nucleons, so the difference
+// that multiplies c4 is twice one of them; it vanishes unless exactly two
+// nucleons exchange charge, and with one species (N1) always.
+//
+// FP64 issue bounds every kernel that sums these.  Against the six direct
+// elements each evaluated in full (six regulators, 18 divisions, 36 general
+// isospin products), SNM A=28 |n_i|<=2: V_pppp 10.2 to 1.54 ms, W0 4.75 to 0.63
+// ms, V_hhpp 1.02 to 0.27 ms, the <cb||kd> table of (T) 15.2 to 4.7 ms.
+// ---------------------------------------------------------------------------
+struct Nucleon {
+  double k[3];   // MeV
+  int sz, tz;
+};
+static __device__ __forceinline__ Nucleon nucleon_of(const Chiral3Dev &c, int p) {
+  const double hbarc = 197.326968;
+  Nucleon o;
+  o.k[0] = c.kx[p] * hbarc;
+  o.k[1] = c.ky[p] * hbarc;
+  o.k[2] = c.kz[p] * hbarc;
+  o.sz = c.sz[p];
+  o.tz = c.tz[p];
+  return o;
+}
+// total momentum and isospin conserved
+static __device__ __forceinline__ bool conserves3(const Chiral3Dev &c, int p, int q, int r, int s, int t, int u) {
+  return c.tz[p] + c.tz[q] + c.tz[r] == c.tz[s] + c.tz[t] + c.tz[u] &&
+         c.nx[p] + c.nx[q] + c.nx[r] == c.nx[s] + c.nx[t] + c.nx[u] &&
+         c.ny[p] + c.ny[q] + c.ny[r] == c.ny[s] + c.ny[t] + c.ny[u] &&
+         c.nz[p] + c.nz[q] + c.nz[r] == c.nz[s] + c.nz[t] + c.nz[u];
 }
 
-// v3(p,q,r,s,t,u) in MeV; the bra regulator is passed in (it is the same for
-// every ket permutation of the antisymmetrized element)
-static __device__ __forceinline__ double2 chiral3_direct(const Chiral3Dev &c, double freg_bra, int p, int q, int r,
-                                                         int s, int t, int u) {
-  const int id[6] = {p, q, r, s, t, u};
-  if (c.tz[p] + c.tz[q] + c.tz[r] != c.tz[s] + c.tz[t] + c.tz[u] ||
-      c.nx[p] + c.nx[q] + c.nx[r] != c.nx[s] + c.nx[t] + c.nx[u] ||
-      c.ny[p] + c.ny[q] + c.ny[r] != c.ny[s] + c.ny[t] + c.ny[u] ||
-      c.nz[p] + c.nz[q] + c.nz[r] != c.nz[s] + c.nz[t] + c.nz[u])
-    return make_double2(0.0, 0.0);
-  const double hbarc = 197.326968;
-  double k[6][3];
-  for (int a = 0; a < 6; ++a) {
-    k[a][0] = c.kx[id[a]] * hbarc;
-    k[a][1] = c.ky[id[a]] * hbarc;
-    k[a][2] = c.kz[id[a]] * hbarc;
-  }
-  double q1[3], q2[3], q3[3];
+struct Geo3 {
+  double q[3][3][3];
+  double w[3][3];
+  double f[3];   // bra regulator x ket regulator x scale; the caller multiplies the bra's in
+};
+template <int X, int Y>
+static __device__ __forceinline__ void geo3_transfer(const Chiral3Dev &c, Geo3 &g, const Nucleon &bra,
+                                                     const Nucleon &ket) {
+  double q2 = 0.0;
+#pragma unroll
   for (int x = 0; x < 3; ++x) {
-    q1[x] = k[3][x] - k[0][x];
-    q2[x] = k[4][x] - k[1][x];
-    q3[x] = k[5][x] - k[2][x];
+    const double v = ket.k[x] - bra.k[x];
+    g.q[X][Y][x] = v;
+    q2 += v * v;
   }
-  auto cross = [](const double *a, const double *b, double *o) {
-    o[0] = a[1] * b[2] - a[2] * b[1];
-    o[1] = a[2] * b[0] - a[0] * b[2];
-    o[2] = a[0] * b[1] - a[1] * b[0];
-  };
-  double q1xq2[3], q1xq3[3], q2xq3[3];
-  cross(q1, q2, q1xq2);
-  cross(q1, q3, q1xq3);
-  cross(q2, q3, q2xq3);
-  const double Q1 = q1[0] * q1[0] + q1[1] * q1[1] + q1[2] * q1[2];
-  const double Q2 = q2[0] * q2[0] + q2[1] * q2[1] + q2[2] * q2[2];
-  const double Q3 = q3[0] * q3[0] + q3[1] * q3[1] + q3[2] * q3[2];
-  const int m1 = c.sz[p], m2 = c.sz[q], m3 = c.sz[r], m4 = c.sz[s], m5 = c.sz[t], m6 = c.sz[u];
-  const int t1 = c.tz[p], t2 = c.tz[q], t3 = c.tz[r], t4 = c.tz[s], t5 = c.tz[t], t6 = c.tz[u];
-  auto sdq = [](int a, int b, const double *v) { return pauli_dot(a, b, v[0], v[1], v[2]); };
-  const double2 q252 = sdq(m2, m5, q2), q142 = sdq(m1, m4, q2), q362 = sdq(m3, m6, q2);
-  const double2 q251 = sdq(m2, m5, q1), q141 = sdq(m1, m4, q1), q361 = sdq(m3, m6, q1);
-  const double2 q363 = sdq(m3, m6, q3), q143 = sdq(m1, m4, q3), q253 = sdq(m2, m5, q3);
-  const double w1 = 1.0 / (Q1 + c.mpi2), w2 = 1.0 / (Q2 + c.mpi2), w3 = 1.0 / (Q3 + c.mpi2);
-  auto scl = [](double a, double2 b) { return make_double2(a * b.x, a * b.y); };
-  auto add = [](double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); };
-  auto dl = [](int a, int b) { return a == b ? 1.0 : 0.0; };
-  const double2 ope141 = scl(w1, q141), ope252 = scl(w2, q252), ope363 = scl(w3, q363);
-  // one "middle nucleon" term; (x,y) the two pion-coupled nucleons
-  auto term = [&](double ttf, double dspec, double e_d, double2 qa_b, double2 qc_d, double wab, double2 qe_f,
-                  double2 qg_h, double wef, double2 opex, double2 opey, double qdot, double2 sig_qxq, double2 tau_a,
-                  double2 tau_b) {
-    double2 in = make_double2(c.econst * e_d, 0.0);
-    const double2 dterm = add(scl(wab, cmul_i(qa_b, qc_d)), scl(wef, cmul_i(qe_f, qg_h)));
-    in = make_double2(in.x - c.dconst * c.k21 * dterm.x, in.y - c.dconst * c.k21 * dterm.y);
-    const double2 oo = cmul_i(opex, opey);
-    in = add(in, scl(c.c1t + c.c3f * qdot, oo));
-    double2 r = scl(ttf * dspec, in);
-    const double2 tdiff = make_double2(tau_a.x - tau_b.x, tau_a.y - tau_b.y);
-    r = add(r, scl(c.c4f, cmul_i(oo, cmul_i(sig_qxq, tdiff))));
+  g.w[X][Y] = 1.0 / (q2 + c.mpi2);
+}
+
+// <mo| sigma.v |mi>, v in an array
+static __device__ __forceinline__ double2 pauli_of(int mo, int mi, const double *v) {
+  return pauli_dot(mo, mi, v[0], v[1], v[2]);
+}
+
+// ONE: one species; HH: the third nucleons of bra and ket are the same state
+// (q[2][2] = 0, the normal-ordering sum), so terms in its one-pion exchange drop
+template <bool ONE, bool HH>
+static __device__ __forceinline__ double2 asym3(const Chiral3Dev &c, const Geo3 &g, const int (&mb)[3],
+                                                const int (&mk)[3], const int (&tb)[3], const int (&tk)[3]) {
+  double2 ope[3][3];
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      if (HH && x == 2 && y == 2) continue;
+      const double2 s = pauli_of(mb[x], mk[y], g.q[x][y]);
+      ope[x][y] = make_double2(g.w[x][y] * s.x, g.w[x][y] * s.y);
+    }
+  // the term of nucleons A -> a and B -> b with C -> cc as the spectator (or
+  // the middle nucleon of the c4 part)
+  auto pair = [&](int A, int a, int B, int b, int C, int cc) -> double2 {
+    const bool za = HH && A == 2 && a == 2, zb = HH && B == 2 && b == 2;   // no pion at A (B)
+    double2 r = make_double2(0.0, 0.0);
+    double wt;
+    if (ONE) wt = mb[C] == mk[cc] ? 1.0 : 0.0;
+    else wt = mb[C] == mk[cc] && tb[C] == tk[cc] ? sig_dot_sig(tb[A], tb[B], tk[a], tk[b]) : 0.0;
+    // 4 t_Z t_X: Z the nucleon that keeps its charge, X the next one
+    int td = 0;
+    if (!ONE && !za && !zb) {
+      const bool fa = tb[A] != tk[a], fb = tb[B] != tk[b], fc = tb[C] != tk[cc];
+      if (fa && fb && !fc) td = 4 * tb[C] * tb[A];
+      else if (fb && fc && !fa) td = 4 * tb[A] * tb[B];
+      else if (fa && fc && !fb) td = 4 * tb[B] * tb[C];
+    }
+    double2 oo = make_double2(0.0, 0.0);
+    if (!za && !zb) oo = cmul_i(ope[A][a], ope[B][b]);
+    if (wt != 0.0) {
+      double2 in = make_double2(mb[A] == mk[a] && mb[B] == mk[b] ? c.econst : 0.0, 0.0);
+      const double dk = c.dconst * c.k21;
+      if (!zb) {
+        const double2 d = cmul_i(ope[B][b], pauli_of(mb[A], mk[a], g.q[B][b]));
+        in.x -= dk * d.x;
+        in.y -= dk * d.y;
+      }
+      if (!za) {
+        const double2 d = cmul_i(ope[A][a], pauli_of(mb[B], mk[b], g.q[A][a]));
+        in.x -= dk * d.x;
+        in.y -= dk * d.y;
+      }
+      if (!za && !zb) {
+        const double *p = g.q[A][a], *q = g.q[B][b];
+        const double cc3 = c.c1t + c.c3f * (p[0] * q[0] + p[1] * q[1] + p[2] * q[2]);
+        in.x += cc3 * oo.x;
+        in.y += cc3 * oo.y;
+      }
+      r.x += wt * in.x;
+      r.y += wt * in.y;
+    }
+    if (!ONE && !za && !zb && td != 0) {
+      const double *p = g.q[A][a], *q = g.q[B][b];
+      const double x[3] = {p[1] * q[2] - p[2] * q[1], p[2] * q[0] - p[0] * q[2], p[0] * q[1] - p[1] * q[0]};
+      const double2 s = cmul_i(oo, pauli_of(mb[C], mk[cc], x));
+      const double f = c.c4f * (double)td;
+      r.x -= f * s.y;
+      r.y += f * s.x;
+    }
     return r;
   };
-  const double2 s1 = term(sig_dot_sig(t1, t2, t4, t5), dl(m3, m6) * dl(t3, t6), dl(m1, m4) * dl(m2, m5), q252, q142,
-                          w2, q141, q251, w1, ope141, ope252, q1[0] * q2[0] + q1[1] * q2[1] + q1[2] * q2[2],
-                          sdq(m3, m6, q1xq2), tau_triple(t3, t1, t2, t6, t4, t5), tau_triple(t3, t2, t1, t6, t5, t4));
-  const double2 s2 = term(sig_dot_sig(t1, t3, t4, t6), dl(m2, m5) * dl(t2, t5), dl(m1, m4) * dl(m3, m6), q363, q143,
-                          w3, q141, q361, w1, ope141, ope363, q1[0] * q3[0] + q1[1] * q3[1] + q1[2] * q3[2],
-                          sdq(m2, m5, q1xq3), tau_triple(t2, t1, t3, t5, t4, t6), tau_triple(t2, t3, t1, t5, t6, t4));
-  const double2 s3 = term(sig_dot_sig(t2, t3, t5, t6), dl(m1, m4) * dl(t1, t4), dl(m2, m5) * dl(m3, m6), q363, q253,
-                          w3, q252, q362, w2, ope252, ope363, q2[0] * q3[0] + q2[1] * q3[1] + q2[2] * q3[2],
-                          sdq(m1, m4, q2xq3), tau_triple(t1, t2, t3, t4, t5, t6), tau_triple(t1, t3, t2, t4, t6, t5));
-  const double2 v = add(add(s1, s2), s3);
-  const double f = freg_bra * freg3(c, k[3], k[4], k[5]) * c.scale;
-  return make_double2(f * v.x, f * v.y);
-}
-
-static __device__ __forceinline__ double freg3_of(const Chiral3Dev &c, int p, int q, int r) {
-  const double hbarc = 197.326968;
-  const double k1[3] = {c.kx[p] * hbarc, c.ky[p] * hbarc, c.kz[p] * hbarc};
-  const double k2[3] = {c.kx[q] * hbarc, c.ky[q] * hbarc, c.kz[q] * hbarc};
-  const double k3[3] = {c.kx[r] * hbarc, c.ky[r] * hbarc, c.kz[r] * hbarc};
-  return freg3(c, k1, k2, k3);
-}
-
-// chiral_3nf_with_delta_asym(i,j,p,k,l,q) (:6904-6917): the ket antisymmetrized
-static __device__ double2 chiral3_asym(const Chiral3Dev &c, int i, int j, int p, int k, int l, int q) {
-  const double fb = freg3_of(c, i, j, p);
-  double2 r = chiral3_direct(c, fb, i, j, p, k, l, q);
-  const double2 a = chiral3_direct(c, fb, i, j, p, l, k, q), b = chiral3_direct(c, fb, i, j, p, q, l, k);
-  const double2 d = chiral3_direct(c, fb, i, j, p, k, q, l), e = chiral3_direct(c, fb, i, j, p, l, q, k);
-  const double2 f = chiral3_direct(c, fb, i, j, p, q, k, l);
-  r.x = r.x - a.x - b.x - d.x + e.x + f.x;
-  r.y = r.y - a.y - b.y - d.y + e.y + f.y;
+  auto direct = [&](int x, int y, int z) -> double2 {   // nucleons 0, 1, 2 to kets x, y, z
+    const double2 u = pair(0, x, 1, y, 2, z), v = pair(0, x, 2, z, 1, y), t = pair(1, y, 2, z, 0, x);
+    return make_double2(u.x + v.x + t.x, u.y + v.y + t.y);
+  };
+  double2 r = make_double2(0.0, 0.0);
+  auto both = [&](int x, int y, int z, double f) {   // + (x, y, z) - (y, x, z)
+    const double2 u = direct(x, y, z), v = direct(y, x, z);
+    r.x += f * (u.x - v.x);
+    r.y += f * (u.y - v.y);
+  };
+  both(0, 1, 2, g.f[2]);
+  both(1, 2, 0, g.f[0]);
+  both(2, 0, 1, g.f[1]);
   return r;
 }
 
-// sum over the holes h of <pqh||rsh> (the normal-ordered two-body part)
-static __device__ double2 no2b_sum(const Chiral3Dev &c, int A, int p, int q, int r, int s) {
+// <abc||def> of three bra and three ket nucleons (momentum and isospin
+// conserved); fb the bra regulator
+template <bool ONE>
+static __device__ __forceinline__ double2 chiral3_asym(const Chiral3Dev &c, double fb, const Nucleon &a,
+                                                       const Nucleon &b, const Nucleon &e, const Nucleon &k,
+                                                       const Nucleon &l, const Nucleon &m) {
+  Geo3 g;
+  geo3_transfer<0, 0>(c, g, a, k);
+  geo3_transfer<0, 1>(c, g, a, l);
+  geo3_transfer<0, 2>(c, g, a, m);
+  geo3_transfer<1, 0>(c, g, b, k);
+  geo3_transfer<1, 1>(c, g, b, l);
+  geo3_transfer<1, 2>(c, g, b, m);
+  geo3_transfer<2, 0>(c, g, e, k);
+  geo3_transfer<2, 1>(c, g, e, l);
+  geo3_transfer<2, 2>(c, g, e, m);
+  const double f = fb * c.scale;
+  g.f[0] = f * freg3(c, l.k, m.k, k.k);
+  g.f[1] = f * freg3(c, k.k, m.k, l.k);
+  g.f[2] = f * freg3(c, k.k, l.k, m.k);
+  const int mb[3] = {a.sz, b.sz, e.sz}, mk[3] = {k.sz, l.sz, m.sz};
+  const int tb[3] = {a.tz, b.tz, e.tz}, tk[3] = {k.tz, l.tz, m.tz};
+  return asym3<ONE, false>(c, g, mb, mk, tb, tk);
+}
+
+// sum over the holes h of <pqh||rsh> (the normal-ordered two-body part); the
+// geometry is that of h's momentum, kept over its spin and isospin states
+template <bool ONE>
+static __device__ __forceinline__ double2 no2b_sum(const Chiral3Dev &c, int A, int p, int q, int r, int s) {
   double2 acc = make_double2(0.0, 0.0);
+  if (!conserves3(c, p, q, 0, r, s, 0)) return acc;
+  const Nucleon a = nucleon_of(c, p), b = nucleon_of(c, q), k = nucleon_of(c, r), l = nucleon_of(c, s);
+  Geo3 g;
+  geo3_transfer<0, 0>(c, g, a, k);
+  geo3_transfer<0, 1>(c, g, a, l);
+  geo3_transfer<1, 0>(c, g, b, k);
+  geo3_transfer<1, 1>(c, g, b, l);
+#pragma unroll 1
   for (int h = 0; h < A; ++h) {
-    const double2 v = chiral3_asym(c, p, q, h, r, s, h);
+    const Nucleon n = nucleon_of(c, h);
+    if (h == 0 || c.nx[h] != c.nx[h - 1] || c.ny[h] != c.ny[h - 1] || c.nz[h] != c.nz[h - 1]) {
+      geo3_transfer<0, 2>(c, g, a, n);
+      geo3_transfer<1, 2>(c, g, b, n);
+      geo3_transfer<2, 0>(c, g, n, k);
+      geo3_transfer<2, 1>(c, g, n, l);
+      const double f = freg3(c, a.k, b.k, n.k) * c.scale;
+      g.f[0] = f * freg3(c, l.k, n.k, k.k);
+      g.f[1] = f * freg3(c, k.k, n.k, l.k);
+      g.f[2] = f * freg3(c, k.k, l.k, n.k);
+    }
+    const int mb[3] = {a.sz, b.sz, n.sz}, mk[3] = {k.sz, l.sz, n.sz};
+    const int tb[3] = {a.tz, b.tz, n.tz}, tk[3] = {k.tz, l.tz, n.tz};
+    const double2 v = asym3<ONE, true>(c, g, mb, mk, tb, tk);
     acc.x += v.x;
     acc.y += v.y;
   }

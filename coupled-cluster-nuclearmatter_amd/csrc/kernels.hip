@@ -155,10 +155,11 @@ __global__ void k_e0(SolveDesc d, V vas) {
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bool pair_le(int a, int b, int c, int d) { return a < c || (a == c && b <= d); }
 
+template <bool ONE>
 __device__ __forceinline__ double2 herm_no2b(const Chiral3Dev &c, int A, int p, int q, int r, int s) {
-  if (pair_le(p, q, r, s)) return no2b_sum(c, A, p, q, r, s);
-  const double2 v = no2b_sum(c, A, r, s, p, q);
-  return make_double2(v.x, -v.y);
+  const bool le = pair_le(p, q, r, s);
+  const double2 v = no2b_sum<ONE>(c, A, le ? p : r, le ? q : s, le ? r : p, le ? s : q);
+  return make_double2(v.x, le ? v.y : -v.y);
 }
 
 // The Hermitian blocks (V_pppp, V_hhhh, W0) take herm_no2b, which evaluates
@@ -189,6 +190,7 @@ __device__ __forceinline__ void tri_rs(int64_t t, int &r, int &s) {
 // is even); the image of the stored pair r is sr times pair ri of channel
 // chi, so V(chi)[ri][si] = sr ss v.  Of the two, the element with the
 // smaller (channel, upper-triangle position) evaluates and writes both.
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_no2b_vpppp(SolveDesc d, Chiral3Dev c) {
   const int ch = blockIdx.y;
   const int n = d.npp[ch];
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(256) void k_no2b_vpppp(SolveDesc d, Chiral3Dev c) {
         sg = ((pr.v ^ ps.v) & 1) ? -1.0 : 1.0;
       }
     }
-    const double2 v = herm_no2b(c, d.A, pb[r], pa[r], pb[s], pa[s]);   // descending orientation
+    const double2 v = herm_no2b<ONE>(c, d.A, pb[r], pa[r], pb[s], pa[s]);   // descending orientation
     add_herm_pair(d.Vpppp + d.off_vpp[ch], n, r, s, v, 1.0);
     if (chi >= 0) {
       const double2 w = make_double2(sg * v.x, sg * v.y);
@@ -222,6 +224,7 @@ __global__ __launch_bounds__(256) void k_no2b_vpppp(SolveDesc d, Chiral3Dev c) {
   }
 }
 
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_no2b_vhhhh(SolveDesc d, Chiral3Dev c) {
   const int ch = blockIdx.y;
   const int nh = d.nhh[ch];
@@ -230,11 +233,12 @@ __global__ __launch_bounds__(256) void k_no2b_vhhhh(SolveDesc d, Chiral3Dev c) {
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x) {
     int s, t;
     tri_rs(e, s, t);
-    const double2 v = herm_no2b(c, d.A, hj[s], hi[s], hj[t], hi[t]);
+    const double2 v = herm_no2b<ONE>(c, d.A, hj[s], hi[s], hj[t], hi[t]);
     add_herm_pair(d.Vhhhh + d.off_vhh[ch], nh, s, t, v, 1.0);
   }
 }
 
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_no2b_vhhpp(SolveDesc d, Chiral3Dev c) {
   const int ch = blockIdx.y;
   const int np_ = d.npp[ch], nh = d.nhh[ch];
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(256) void k_no2b_vhhpp(SolveDesc d, Chiral3Dev c) {
   const int *hi = d.hh_i + d.off_hh[ch], *hj = d.hh_j + d.off_hh[ch];
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x) {
     const int s = (int)(e / np_), r = (int)(e % np_);
-    const double2 v = no2b_sum(c, d.A, pa[r], pb[r], hi[s], hj[s]);
+    const double2 v = no2b_sum<ONE>(c, d.A, pa[r], pb[r], hi[s], hj[s]);
     double2 &o = d.Vhhpp[d.off_t[ch] + e];
     o.x += v.x;
     o.y += v.y;
@@ -251,6 +255,7 @@ __global__ __launch_bounds__(256) void k_no2b_vhhpp(SolveDesc d, Chiral3Dev c) {
 }
 
 // W0((i,a),(j,b)) = -<ib||ja>
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_no2b_w0(SolveDesc d, Chiral3Dev c) {
   const int K = blockIdx.y;
   const int n = d.nhp[K];
@@ -260,44 +265,14 @@ __global__ __launch_bounds__(256) void k_no2b_w0(SolveDesc d, Chiral3Dev c) {
     int r, s;
     tri_rs(e, r, s);
     const int i = hj[r], a = hb[r], j = hj[s], b = hb[s];
-    const double2 v = herm_no2b(c, d.A, i, b, j, a);
+    const double2 v = herm_no2b<ONE>(c, d.A, i, b, j, a);
     add_herm_pair(d.W0 + d.off_i4[K], n, r, s, v, -1.0);
   }
 }
 
-// f_pq += sum_{i<=j} <ijp||ijq> for q in {p, partner(p)} (ccm_main.f90:1826-1995)
-__global__ __launch_bounds__(256) void k_3nf_fock(SolveDesc d, Chiral3Dev c) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= d.nsp) return;
-  const int pp = d.partner[p];
-  double2 fd = make_double2(0.0, 0.0), fp = make_double2(0.0, 0.0);
-  for (int i = 0; i < d.A; ++i)
-    for (int j = i; j < d.A; ++j) {
-      const double2 v = chiral3_asym(c, i, j, p, i, j, p);
-      fd.x += v.x;
-      fd.y += v.y;
-      if (pp >= 0) {
-        const double2 w = chiral3_asym(c, i, j, p, i, j, pp);
-        fp.x += w.x;
-        fp.y += w.y;
-      }
-    }
-  d.fdiag[p] = make_double2(d.fdiag[p].x + fd.x, d.fdiag[p].y + fd.y);
-  d.fpart[p] = make_double2(d.fpart[p].x + fp.x, d.fpart[p].y + fp.y);
-}
-
-// E0 += sum_{i<j<k} <ijk||ijk> (ccm_main.f90:1687-1800).  One block.
-__global__ __launch_bounds__(256) void k_3nf_e0(SolveDesc d, Chiral3Dev c) {
+// Sum of one complex value per thread over a block of 256, fixed order.
+__device__ __forceinline__ double2 block_sum256(double re, double im) {
   __shared__ double sre[256], sim[256];
-  double re = 0.0, im = 0.0;
-  const int64_t A = d.A, n = A * A * A;
-  for (int64_t e = threadIdx.x; e < n; e += blockDim.x) {
-    const int i = (int)(e / (A * A)), j = (int)((e / A) % A), k = (int)(e % A);
-    if (!(i < j && j < k)) continue;
-    const double2 v = chiral3_asym(c, i, j, k, i, j, k);
-    re += v.x;
-    im += v.y;
-  }
   sre[threadIdx.x] = re;
   sim[threadIdx.x] = im;
   __syncthreads();
@@ -308,7 +283,67 @@ __global__ __launch_bounds__(256) void k_3nf_e0(SolveDesc d, Chiral3Dev c) {
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) d.e0[0] = make_double2(d.e0[0].x + sre[0], d.e0[0].y + sim[0]);
+  const double2 r = make_double2(sre[0], sim[0]);
+  __syncthreads();
+  return r;
+}
+
+// f_pq += sum_{i<j} <ijp||ijq> for q = p (blockIdx.y 0) and q = partner(p)
+// (1) (ccm_main.f90:1826-1995; the terms i = j vanish).  One block per target,
+// its threads over the hole pairs: one thread per orbital left most of the
+// chip idle (SNM A=28 |n_i|<=2: 9.4 ms, now under 0.06 ms).
+template <bool ONE>
+__global__ __launch_bounds__(256) void k_3nf_fock(SolveDesc d, Chiral3Dev c) {
+  const int p = blockIdx.x, q = blockIdx.y == 0 ? p : d.partner[p];
+  if (q < 0) return;
+  const Nucleon np_ = nucleon_of(c, p), nq = nucleon_of(c, q);
+  double re = 0.0, im = 0.0;
+  const int npair = d.A * (d.A - 1) / 2;
+  if (conserves3(c, 0, 0, p, 0, 0, q))
+    for (int e = threadIdx.x; e < npair; e += 256) {
+      int i, j;   // i < j
+      tri_rs(e, i, j);
+      const Nucleon a = nucleon_of(c, i), b = nucleon_of(c, j + 1);
+      const double2 v = chiral3_asym<ONE>(c, freg3(c, a.k, b.k, np_.k), a, b, np_, a, b, nq);
+      re += v.x;
+      im += v.y;
+    }
+  const double2 s = block_sum256(re, im);
+  if (threadIdx.x != 0) return;
+  double2 &o = blockIdx.y == 0 ? d.fdiag[p] : d.fpart[p];
+  o = make_double2(o.x + s.x, o.y + s.y);
+}
+
+// E0 += sum_{i<j<k} <ijk||ijk> (ccm_main.f90:1687-1800): one block per hole
+// pair (i, j) and stride, its threads over k; the partials (d.red) in order.
+constexpr int kE0Blocks = 1024;
+template <bool ONE>
+__global__ __launch_bounds__(256) void k_3nf_e0(SolveDesc d, Chiral3Dev c) {
+  double re = 0.0, im = 0.0;
+  const int npair = d.A * (d.A - 1) / 2;
+  for (int e = blockIdx.x; e < npair; e += gridDim.x) {
+    int i, j;
+    tri_rs(e, i, j);
+    ++j;
+    const Nucleon a = nucleon_of(c, i), b = nucleon_of(c, j);
+    for (int k = j + 1 + threadIdx.x; k < d.A; k += 256) {
+      const Nucleon n = nucleon_of(c, k);
+      const double2 v = chiral3_asym<ONE>(c, freg3(c, a.k, b.k, n.k), a, b, n, a, b, n);
+      re += v.x;
+      im += v.y;
+    }
+  }
+  const double2 s = block_sum256(re, im);
+  if (threadIdx.x == 0) d.red[blockIdx.x] = s;
+}
+__global__ __launch_bounds__(256) void k_3nf_e0_final(SolveDesc d, int nparts) {
+  double re = 0.0, im = 0.0;
+  for (int k = threadIdx.x; k < nparts; k += 256) {
+    re += d.red[k].x;
+    im += d.red[k].y;
+  }
+  const double2 s = block_sum256(re, im);
+  if (threadIdx.x == 0) d.e0[0] = make_double2(d.e0[0].x + s.x, d.e0[0].y + s.y);
 }
 
 // <pq||rs> for a list of orbital quadruples; zero where momentum or isospin
@@ -1832,17 +1867,26 @@ void launch_elements(const SolveDesc &d, double volume, const ChiralDev *c, cons
 }
 
 // approx 0: E0 only; 1: and the Fock matrix; 2: and the two-body blocks
+template <bool ONE>
+static void launch_3nf_t(const SolveDesc &d, const Chiral3Dev &c, int approx, int nch, int nphc, int max_npp,
+                         int max_nhh, int max_nhp, hipStream_t st) {
+  auto gx = [](int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 8192)); };
+  const int nb = std::max(1, std::min(kE0Blocks, d.A * (d.A - 1) / 2));
+  hipLaunchKernelGGL(k_3nf_e0<ONE>, dim3(nb), dim3(256), 0, st, d, c);
+  hipLaunchKernelGGL(k_3nf_e0_final, dim3(1), dim3(256), 0, st, d, nb);
+  if (approx < 1) return;
+  hipLaunchKernelGGL(k_3nf_fock<ONE>, dim3(d.nsp, 2), dim3(256), 0, st, d, c);
+  if (approx < 2) return;
+  hipLaunchKernelGGL(k_no2b_vpppp<ONE>, dim3(gx((int64_t)max_npp * (max_npp + 1) / 2), nch), dim3(256), 0, st, d, c);
+  hipLaunchKernelGGL(k_no2b_vhhpp<ONE>, dim3(gx((int64_t)max_npp * max_nhh), nch), dim3(256), 0, st, d, c);
+  hipLaunchKernelGGL(k_no2b_vhhhh<ONE>, dim3(gx((int64_t)max_nhh * (max_nhh + 1) / 2), nch), dim3(256), 0, st, d, c);
+  hipLaunchKernelGGL(k_no2b_w0<ONE>, dim3(gx((int64_t)max_nhp * (max_nhp + 1) / 2), nphc), dim3(256), 0, st, d, c);
+}
+
 void launch_3nf(const SolveDesc &d, const Chiral3Dev &c, int approx, int nch, int nphc, int max_npp, int max_nhh,
                 int max_nhp, hipStream_t st) {
-  auto gx = [](int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 8192)); };
-  hipLaunchKernelGGL(k_3nf_e0, dim3(1), dim3(256), 0, st, d, c);
-  if (approx < 1) return;
-  hipLaunchKernelGGL(k_3nf_fock, dim3((d.nsp + 255) / 256), dim3(256), 0, st, d, c);
-  if (approx < 2) return;
-  hipLaunchKernelGGL(k_no2b_vpppp, dim3(gx((int64_t)max_npp * (max_npp + 1) / 2), nch), dim3(256), 0, st, d, c);
-  hipLaunchKernelGGL(k_no2b_vhhpp, dim3(gx((int64_t)max_npp * max_nhh), nch), dim3(256), 0, st, d, c);
-  hipLaunchKernelGGL(k_no2b_vhhhh, dim3(gx((int64_t)max_nhh * (max_nhh + 1) / 2), nch), dim3(256), 0, st, d, c);
-  hipLaunchKernelGGL(k_no2b_w0, dim3(gx((int64_t)max_nhp * (max_nhp + 1) / 2), nphc), dim3(256), 0, st, d, c);
+  if (c.one_species) launch_3nf_t<true>(d, c, approx, nch, nphc, max_npp, max_nhh, max_nhp, st);
+  else launch_3nf_t<false>(d, c, approx, nch, nphc, max_npp, max_nhh, max_nhp, st);
 }
 
 void launch_derive(const SolveDesc &d, int nch, int nphc, int max_npp, int max_nhh, int max_nph,

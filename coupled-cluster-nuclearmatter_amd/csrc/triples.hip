@@ -144,6 +144,7 @@ __device__ double2 h_term(const SolveDesc &d, const TriplesDesc &td, double vol,
 // <cb||kd> = -<bc||kd> (the NN element and the normal-ordered 3NF sum are
 // both antisymmetric in the bra): the fill evaluates c < b and writes both
 // entries, c = b is zero.  Grid stride over the half (c < b) only.
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_t3_fill_hppp(SolveDesc d, TriplesDesc td, double vol, double2 *out) {
   const int np = d.np;
   const int64_t npair = (int64_t)np * (np - 1) / 2;   // c < b, in the order of pairs (b, c) with c < b
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(256) void k_t3_fill_hppp(SolveDesc d, TriplesDesc t
     if (dd >= d.A) {
       v = vas_t(d, td, vol, c, b, k, dd);
       if (td.tnf) {
-        const double2 w = no2b_sum(td.c3, d.A, c, b, k, dd);
+        const double2 w = no2b_sum<ONE>(td.c3, d.A, c, b, k, dd);
         v.x += w.x;
         v.y += w.y;
       }
@@ -313,31 +314,6 @@ __global__ __launch_bounds__(256) void k_triples(SolveDesc d, TriplesDesc td, do
   }
 }
 
-// chiral3_asym with the six ket permutations in a loop over one inlined copy
-// of the direct element (fewer registers); the same terms summed in the same
-// order, so the value is identical.
-__device__ __forceinline__ double2 w3_element(const Chiral3Dev &c, int a, int b, int cc, int i, int j, int k) {
-  const double fb = freg3_of(c, a, b, cc);
-  const int ket[3] = {i, j, k};
-  double2 r = make_double2(0.0, 0.0);
-#pragma unroll 1
-  for (int p = 0; p < 6; ++p) {
-    // (k,l,q) +, (l,k,q) -, (q,l,k) -, (k,q,l) -, (l,q,k) +, (q,k,l) +
-    const int x = p == 0 || p == 3 ? 0 : (p == 1 || p == 4 ? 1 : 2);
-    const int y = p == 1 || p == 5 ? 0 : (p == 0 || p == 2 ? 1 : 2);
-    const int z = 3 - x - y;
-    const double2 v = chiral3_direct(c, fb, a, b, cc, ket[x], ket[y], ket[z]);
-    if (p == 0 || p >= 4) {
-      r.x += v.x;
-      r.y += v.y;
-    } else {
-      r.x -= v.x;
-      r.y -= v.y;
-    }
-  }
-  return r;
-}
-
 // Table mode, one wave per particle triple: a block takes particle pairs
 // (a,b), its four waves take c = b+1+wave, b+5+wave, ..., and the 64 lanes of
 // a wave stride over the hole triples of that (K3,Tz3) channel.  Every lane of
@@ -354,7 +330,7 @@ __device__ __forceinline__ double2 w3_element(const Chiral3Dev &c, int a, int b,
 //   MODE 2: |W3|^2 / D                CCDT-1 energy of the start T3 = W3/D
 //           (setup_t3, ccm_t3full_channels.f90:291-567)
 //   MODE 3: |W + W3|^2 / D            (T) at tnf_approx 3, et_5 (:656-722)
-template <int MODE>
+template <int MODE, bool ONE>
 __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, double volume, double2 *partial,
                                                    unsigned long long *count) {
   __shared__ double sre[256], sim[256];
@@ -375,6 +351,14 @@ __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, 
       const double fai = d.fdiag[a].y, fbi = d.fdiag[b].y, fci = d.fdiag[c].y;
       const int h0 = td.hptr[ch], h1 = td.hptr[ch + 1];
       if (lane == 0) nel += (unsigned long long)(h1 - h0);
+      Nucleon na{}, nb{}, nc{};
+      double fbra = 0.0;
+      if constexpr (MODE != 0) {
+        na = nucleon_of(td.c3w, a);
+        nb = nucleon_of(td.c3w, b);
+        nc = nucleon_of(td.c3w, c);
+        fbra = freg3(td.c3w, na.k, nb.k, nc.k);
+      }
       for (int h = h0 + lane; h < h1; h += 64) {
         const int i = td.hijk[3 * h], j = td.hijk[3 * h + 1], k = td.hijk[3 * h + 2];
         double2 w = make_double2(0.0, 0.0);
@@ -398,7 +382,8 @@ __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, 
         if constexpr (MODE == 0) {
           nre = w.x * w.x + w.y * w.y;
         } else {
-          const double2 w3 = w3_element(td.c3w, a, b, c, i, j, k);
+          const double2 w3 = chiral3_asym<ONE>(td.c3w, fbra, na, nb, nc, nucleon_of(td.c3w, i), nucleon_of(td.c3w, j),
+                                               nucleon_of(td.c3w, k));
           if constexpr (MODE == 1) {
             const double xr = w3.x + w.x, xi = w3.y + w.y;
             nre = xr * w3.x + xi * w3.y;
@@ -602,7 +587,10 @@ __global__ void k_triples_final(const double2 *partial, int n, double2 *out) {
 
 void launch_t3_tables(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *hppp, double2 *hhhp,
                       hipStream_t st) {
-  hipLaunchKernelGGL(k_t3_fill_hppp, dim3(8192), dim3(256), 0, st, d, td, volume, hppp);
+  if (td.tnf && !td.c3.one_species)
+    hipLaunchKernelGGL(k_t3_fill_hppp<false>, dim3(8192), dim3(256), 0, st, d, td, volume, hppp);
+  else
+    hipLaunchKernelGGL(k_t3_fill_hppp<true>, dim3(8192), dim3(256), 0, st, d, td, volume, hppp);
   hipLaunchKernelGGL(k_t3_fill_hhhp, dim3(1024), dim3(256), 0, st, d, td, volume, hhhp);
 }
 
@@ -616,18 +604,19 @@ void launch_t3_td(const SolveDesc &d, const TriplesDesc &td, double2 *tdt, hipSt
 void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *partial,
                     unsigned long long *count, int nblocks, double2 *out, unsigned long long *count_out,
                     hipStream_t st, int mode, const double2 *tdt, int maxnhh) {
+  const bool one = td.c3w.one_species != 0;
   const int variant = getenv("CCGPU_T3_KERNEL") ? atoi(getenv("CCGPU_T3_KERNEL")) : 1;
   if (mode == 0 && variant == 1 && tdt && td.vhppp && td.vhhhp) {
     const size_t lds = (size_t)4 * 3 * maxnhh * sizeof(double2);
     hipLaunchKernelGGL(k_triples_s, dim3(nblocks), dim3(256), lds, st, d, td, tdt, maxnhh, partial, count);
   } else if (mode == 1)
-    hipLaunchKernelGGL(k_triples_w<1>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+    hipLaunchKernelGGL((one ? k_triples_w<1, true> : k_triples_w<1, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
   else if (mode == 2)
-    hipLaunchKernelGGL(k_triples_w<2>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+    hipLaunchKernelGGL((one ? k_triples_w<2, true> : k_triples_w<2, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
   else if (mode == 3)
-    hipLaunchKernelGGL(k_triples_w<3>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+    hipLaunchKernelGGL((one ? k_triples_w<3, true> : k_triples_w<3, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
   else if (td.vhppp && td.vhhhp && (variant == 1 || variant == 3))
-    hipLaunchKernelGGL(k_triples_w<0>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+    hipLaunchKernelGGL((k_triples_w<0, true>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
   else if (td.vhppp && td.vhhhp)
     hipLaunchKernelGGL(k_triples<true>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
   else
