@@ -74,8 +74,11 @@ void launch_t3_tables(const SolveDesc &d, const TriplesDesc &td, double volume, 
                       hipStream_t st);
 void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *partial,
                     unsigned long long *count, int nblocks, double2 *out, unsigned long long *count_out,
-                    hipStream_t st, int mode, const double2 *tdt, int maxnhh);
+                    hipStream_t st, int variant, const double2 *tdt, int maxnhh);
 void launch_t3_td(const SolveDesc &d, const TriplesDesc &td, double2 *tdt, hipStream_t st);
+void launch_t3_group_v(const SolveDesc &d, const TriplesDesc &td, double volume, hipStream_t st);
+void launch_triples_group(const SolveDesc &d, const TriplesDesc &td, double2 *partial, unsigned long long *count,
+                          int nblocks, double2 *out, unsigned long long *count_out, hipStream_t st, int mode);
 // mlp.hip
 void launch_mlp_forward(const float *params, const uint16_t *feat, int64_t n, float *y, hipStream_t st);
 void launch_mlp_loss_grad(const float *params, const uint16_t *feat, const float *target, int64_t n, int64_t npad,
@@ -402,13 +405,17 @@ struct Solve {
   int64_t *d_off_vpp = nullptr, *d_off_vpp32 = nullptr;
   int *d_npp = nullptr;
   bool have_t3 = false;
+  bool t3_lattice = false;       // the lattice's lists of t3 are made
+  std::vector<void *> t3_owned;  // device memory of the current interaction's t3
+  std::vector<int> t3_orbitof;
+  double2 *t3_gE = nullptr, *t3_gD = nullptr;   // the group tables
   bool have_w3 = false;          // t3.c3w holds the W3 constants
   bool have_ccdt1 = false;       // setup_t3 done
   double2 ccdt1_e3{0.0, 0.0};    // energy of the last t3_intermediate
   double2 t3_et4{0.0, 0.0}, t3_et5{0.0, 0.0};   // parts of the last (T)
   TriplesDesc t3{};
   double2 *t3_partial = nullptr, *t3_out = nullptr;
-  double2 *t3_td = nullptr;   // t(x d, u v) of the F terms, refilled from T for every (T) sum
+  double2 *t3_td = nullptr;   // t(x d, u v) of the staged kernel's F terms
   unsigned long long *t3_count = nullptr;   // per block, then the total at [8192]
   long long t3_elements = 0;
   double t3_seconds = 0.0;
@@ -433,6 +440,7 @@ struct Solve {
   double2 *scal = nullptr;
   ~Solve() {
     for (void *p : owned) (void)hipFree(p);
+    for (void *p : t3_owned) (void)hipFree(p);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -2786,8 +2794,9 @@ int ccgpu_get_t2_labels(int handle, int *abij) {
 }  // extern "C"
 namespace {
 // (K3,Tz3) hole-triple channels, orbital lookup and particle-pair list of
-// setup_t3_channel_structures (ccm_t3full_channels.f90:4-284), built once.
-void build_triples(Solve &S) {
+// setup_t3_channel_structures (ccm_t3full_channels.f90:4-284), and the groups
+// of the group kernel, built once per handle.
+void build_triples_lattice(Solve &S) {
   const Plan &P = S.plan;
   const Orbitals &o = P.orb;
   int nh = 0;
@@ -2834,9 +2843,90 @@ void build_triples(Solve &S) {
   td.hptr = dupload(hptr, S.owned);
   td.hijk = dupload(hijk, S.owned);
   td.orbitof = dupload(orbitof, S.owned);
+  S.t3_orbitof = orbitof;
   td.pair_a = dupload(pa, S.owned);
   td.pair_b = dupload(pb, S.owned);
   td.npairs = (int64_t)pa.size();
+  // groups: particle (hole) states of one momentum and isospin, in orbital order
+  std::vector<int2> pg, hg;
+  std::vector<int4> pgn;
+  std::vector<int> og(P.nsp);
+  std::map<std::tuple<int, int, int, int>, int> at[2];
+  for (int x = 0; x < P.nsp; ++x) {
+    const int kind = x < P.A ? 0 : 1;
+    std::vector<int2> &gs = kind ? pg : hg;
+    auto ins = at[kind].emplace(std::make_tuple(o.nx[x], o.ny[x], o.nz[x], o.tz[x]), (int)gs.size());
+    if (ins.second) {
+      gs.push_back(int2{x, -1});
+      if (kind) pgn.push_back(int4{o.nx[x], o.ny[x], o.nz[x], o.tz[x]});
+      og[x] = 2 * ins.first->second;
+    } else {
+      gs[ins.first->second].y = x;
+      og[x] = 2 * ins.first->second + 1;
+    }
+  }
+  td.npg = (int)pg.size();
+  td.nhg = (int)hg.size();
+  td.nhp = td.nhg * (td.nhg + 1) / 2;
+  auto gkey = [&](int g, int q) {
+    const int x = hg[g].x;
+    return q == 0 ? o.tz[x] : q == 1 ? o.nx[x] : q == 2 ? o.ny[x] : o.nz[x];
+  };
+  std::vector<std::vector<T3Hole>> lists(ch);
+  auto hpair = [](int u, int v) { return v * (v + 1) / 2 + u; };   // u <= v
+  for (int I = 0; I < td.nhg; ++I)
+    for (int J = I; J < td.nhg; ++J)
+      for (int K = J; K < td.nhg; ++K) {
+        int mask = 0;
+        for (int c = 0; c < 8; ++c) {
+          const int si = c >> 2, sj = (c >> 1) & 1, sk = c & 1;
+          const int i = si ? hg[I].y : hg[I].x, j = sj ? hg[J].y : hg[J].x, k = sk ? hg[K].y : hg[K].x;
+          if (i >= 0 && j >= 0 && k >= 0 && (I != J || si < sj) && (J != K || sj < sk)) mask |= 1 << c;
+        }
+        if (!mask) continue;
+        int tot[4];
+        for (int q = 0; q < 4; ++q) tot[q] = gkey(I, q) + gkey(J, q) + gkey(K, q);
+        const size_t idx =
+            (((size_t)(tot[0] - td.tz0) * td.nk + (tot[1] - td.k0)) * td.nk + (tot[2] - td.k0)) * td.nk + (tot[3] - td.k0);
+        lists[chan[idx]].push_back(T3Hole{I, J, K, hpair(I, J), hpair(I, K), hpair(J, K), mask, 0});
+      }
+  std::vector<int> gptr = {0};
+  std::vector<T3Hole> gtrip;
+  for (auto &l : lists) {
+    gtrip.insert(gtrip.end(), l.begin(), l.end());
+    gptr.push_back((int)gtrip.size());
+  }
+  td.pg = dupload(pg, S.owned);
+  td.hg = dupload(hg, S.owned);
+  td.pgn = dupload(pgn, S.owned);
+  td.og = dupload(og, S.owned);
+  td.gptr = dupload(gptr, S.owned);
+  td.gtrip = dupload(gtrip, S.owned);
+  td.ngtrip = (int)gtrip.size();
+  td.gf = dalloc<double2>(8 * gtrip.size(), S.owned);
+  td.gE = td.gD = nullptr;
+  td.vhppp = td.vhhhp = nullptr;
+  S.t3_partial = dalloc<double2>(8192, S.owned);
+  S.t3_out = dalloc<double2>(1, S.owned);
+  S.t3_count = dalloc<unsigned long long>(8193, S.owned);
+  S.t3_lattice = true;
+}
+
+double t3_table_limit() {   // bytes
+  return (getenv("CCGPU_T3_TABLE_GB") ? atof(getenv("CCGPU_T3_TABLE_GB")) : 16.0) * 1e9;
+}
+
+// The element source of the current interaction and, when they fit, the group
+// tables' interaction halves.  Device memory of an earlier interaction of the
+// handle is kept (its size is the lattice's) or given back.
+void build_triples(Solve &S) {
+  if (!S.t3_lattice) build_triples_lattice(S);
+  const Plan &P = S.plan;
+  const Orbitals &o = P.orb;
+  TriplesDesc &td = S.t3;
+  const int nm = td.nmax, n = 2 * nm + 1;
+  for (void *p : S.t3_owned) (void)hipFree(p);
+  S.t3_owned.clear();
   td.vkeys = nullptr;
   td.vvals = nullptr;
   td.vmask = 0;
@@ -2869,7 +2959,7 @@ void build_triples(Solve &S) {
       for (int g = 0; g < 3; ++g)
         tab[3 * m + g] = v0[g] * std::pow(pi, 1.5) * std::exp(-q2 / (4.0 * kap[g])) / std::pow(kap[g], 1.5);
     }
-    td.mtab = dupload(tab, S.owned);
+    td.mtab = dupload(tab, S.t3_owned);
   }
   if (!S.native_v) {
     if (S.t3v.empty())
@@ -2889,8 +2979,8 @@ void build_triples(Solve &S) {
       keys[h] = kv.first;
       vals[h] = double2{kv.second.real(), kv.second.imag()};
     }
-    td.vkeys = dupload(keys, S.owned);
-    td.vvals = dupload(vals, S.owned);
+    td.vkeys = dupload(keys, S.t3_owned);
+    td.vvals = dupload(vals, S.t3_owned);
     td.vmask = cap - 1;
   }
   // parity: with no twist, n -> -n maps the lattice onto itself with k -> -k
@@ -2902,37 +2992,57 @@ void build_triples(Solve &S) {
     for (int x = 0; x < P.nsp && ok; ++x) {
       const size_t idx = (((size_t)(nm - o.nx[x]) * n + (nm - o.ny[x])) * n + (nm - o.nz[x])) * 4 +
                          ((o.sz[x] + 1) / 2) * 2 + (o.tz[x] + 1) / 2;
-      const int y = orbitof[idx];
+      const int y = S.t3_orbitof[idx];
       ok = y >= 0 && (x < P.A) == (y < P.A) && o.kx[y] == -o.kx[x] && o.ky[y] == -o.ky[x] && o.kz[y] == -o.kz[x];
     }
     td.parity = ok ? 1 : 0;
   }
-  // dense <cb||kd> and <jk||lc> tables, evaluated once per interaction, when
-  // they fit in CCGPU_T3_TABLE_GB (default 16 GB); otherwise the kernel
-  // evaluates the elements in place
+  // the group tables, when they fit in CCGPU_T3_TABLE_GB (default 16 GB; the
+  // size of one entry per (c, b, k) and per (j, k, c) for both spins, which
+  // theirs is up to the diagonals of their triangles); otherwise (T) evaluates
+  // the elements in place
   td.vhppp = nullptr;
   td.vhhhp = nullptr;
-  {
-    const double lim = (getenv("CCGPU_T3_TABLE_GB") ? atof(getenv("CCGPU_T3_TABLE_GB")) : 16.0) * 1e9;
-    const int64_t nh = (int64_t)P.np * P.np * P.A * 2, nl = (int64_t)P.A * P.A * P.np * 2;
-    if ((double)(nh + nl) * sizeof(double2) <= lim && nh > 0 && nl > 0) {
-      double2 *hppp = dalloc<double2>(nh, S.owned), *hhhp = dalloc<double2>(nl, S.owned);
-      launch_t3_tables(S.desc, td, P.orb.volume, hppp, hhhp, S.stream);
-      check_launch();
-      HIPCHK(hipStreamSynchronize(S.stream));
-      td.vhppp = hppp;
-      td.vhhhp = hhhp;
+  const int64_t ntab = (int64_t)P.np * P.np * P.A * 2 + (int64_t)P.A * P.A * P.np * 2;
+  if ((double)ntab * sizeof(double2) <= t3_table_limit() && P.np > 0) {
+    if (!S.t3_gE) {
+      S.t3_gE = dalloc<double2>((size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 4, S.owned);
+      S.t3_gD = dalloc<double2>((size_t)td.npg * 2 * td.nhp * 4 * 4, S.owned);
     }
-    if (td.tnf && !td.vhppp)
-      throw Error("(T) with the three-nucleon force needs its element tables: raise CCGPU_T3_TABLE_GB");
+    td.gE = S.t3_gE;
+    td.gD = S.t3_gD;
+    launch_t3_group_v(S.desc, td, P.orb.volume, S.stream);
+    check_launch();
+    HIPCHK(hipStreamSynchronize(S.stream));
+  } else {
+    td.gE = td.gD = nullptr;
   }
-  S.t3_partial = dalloc<double2>(8192, S.owned);
-  S.t3_out = dalloc<double2>(1, S.owned);
-  S.t3_count = dalloc<unsigned long long>(8193, S.owned);
+  if (td.tnf && !td.gE)
+    throw Error("(T) with the three-nucleon force needs its element tables: raise CCGPU_T3_TABLE_GB");
   S.have_t3 = true;
 }
 
-// One sum over the triples (modes of k_triples_w): returns it and counts the
+// The dense tables of the element-by-element kernels (CCGPU_T3_KERNEL=1, 3),
+// made on their first use for an interaction.
+bool legacy_tables(Solve &S) {
+  TriplesDesc &td = S.t3;
+  if (td.vhppp) return true;
+  const Plan &P = S.plan;
+  const int64_t nh = (int64_t)P.np * P.np * P.A * 2, nl = (int64_t)P.A * P.A * P.np * 2, nd = nl;
+  if ((double)(nh + nl + nd) * sizeof(double2) > t3_table_limit() ||
+      (size_t)4 * 3 * P.max_nhh * sizeof(double2) > 65536 || nh == 0)
+    return false;
+  double2 *hppp = dalloc<double2>(nh, S.t3_owned), *hhhp = dalloc<double2>(nl, S.t3_owned);
+  S.t3_td = dalloc<double2>(nd, S.t3_owned);
+  launch_t3_tables(S.desc, td, P.orb.volume, hppp, hhhp, S.stream);
+  check_launch();
+  HIPCHK(hipStreamSynchronize(S.stream));
+  td.vhppp = hppp;
+  td.vhhhp = hhhp;
+  return true;
+}
+
+// One sum over the triples (modes of k_triples_g): returns it and counts the
 // elements.
 double2 triples_sum(Solve &S, int mode) {
   if (!S.have_t3) build_triples(S);
@@ -2949,26 +3059,22 @@ double2 triples_sum(Solve &S, int mode) {
     S.t3.c3w = c;
     S.have_w3 = true;
   }
-  if (mode != 2 && !(S.t3.vhppp && S.t3.vhhhp) && mode != 0)
+  if (mode != 2 && mode != 0 && !S.t3.gE)
     throw Error("CCDT-1 and the three-body (T) need the element tables: raise CCGPU_T3_TABLE_GB");
-  int nb = (int)std::min<int64_t>(8192, std::max<int64_t>(1, S.t3.npairs));
-  // the staged (T) kernel: the F terms' amplitude table (np A^2 x 2 spins),
-  // made once per handle when the element tables exist and it fits with them
-  // in CCGPU_T3_TABLE_GB, refilled from the current T for every sum
   const Plan &P = S.plan;
-  if (mode == 0 && S.t3.vhppp && S.t3.vhhhp && !S.t3_td) {
-    const double lim = (getenv("CCGPU_T3_TABLE_GB") ? atof(getenv("CCGPU_T3_TABLE_GB")) : 16.0) * 1e9;
-    const int64_t ntab = (int64_t)P.np * P.np * P.A * 2 + (int64_t)P.A * P.A * P.np * 2;
-    const int64_t ntd = (int64_t)P.np * P.A * P.A * 2;
-    if ((double)(ntab + ntd) * sizeof(double2) <= lim && (size_t)4 * 3 * P.max_nhh * sizeof(double2) <= 65536)
-      S.t3_td = dalloc<double2>(ntd, S.owned);
+  int nb = (int)std::min<int64_t>(8192, std::max<int64_t>(1, S.t3.npairs));
+  // CCGPU_T3_KERNEL=1, 3 (studies and tests): (T) element by element
+  const int variant = getenv("CCGPU_T3_KERNEL") ? atoi(getenv("CCGPU_T3_KERNEL")) : 2;
+  if (mode == 0 && (variant == 1 || variant == 3) && legacy_tables(S)) {
+    if (variant == 1) launch_t3_td(S.desc, S.t3, S.t3_td, S.stream);
+    launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream,
+                   variant, S.t3_td, P.max_nhh);
+  } else if (mode == 2 || (S.t3.gE && variant != 0)) {
+    launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
+  } else {
+    launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream, 0,
+                   nullptr, P.max_nhh);
   }
-  if (mode == 0 && S.t3_td) {
-    launch_t3_td(S.desc, S.t3, S.t3_td, S.stream);
-    check_launch();
-  }
-  launch_triples(S.desc, S.t3, S.plan.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192,
-                 S.stream, mode, mode == 0 ? S.t3_td : nullptr, P.max_nhh);
   check_launch();
   double2 r;
   unsigned long long cnt = 0;

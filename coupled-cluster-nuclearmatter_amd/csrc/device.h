@@ -88,6 +88,14 @@ struct GemmTile {
   int kb, ke, pad0, pad1;  // k range of this tile
 };
 
+// A triple of hole groups I <= J <= K (a group: the up to two spin states of one
+// momentum and isospin, in orbital order) of one (K3, Tz3) channel: its pair
+// indices into the tables below and the spin combinations 4 is + 2 js + ks that
+// are distinct states in canonical order.
+struct T3Hole {
+  int I, J, K, hij, hik, hjk, mask, pad;
+};
+
 // (T) channel tables and, for handed-over interactions, the open-addressing
 // table of the <cb||kd> and <jk||lc> elements (key ((p*nsp+q)*nsp+r)*nsp+s,
 // empty slots ~0, capacity a power of two at least twice the entries).
@@ -116,6 +124,25 @@ struct TriplesDesc {
   // momentum and isospin follow from conservation); vhhhp holds <jk||lc> at
   // (j A + k) np + (c-A), times 2 for the spin of l
   const double2 *vhppp, *vhhhp;
+  // Groups (k_triples_g): the two states of every particle and hole group
+  // (orbital or -1), a particle group's momentum and isospin, and per orbital
+  // 2 group + state.  Group triples of a channel: [gptr[ch], gptr[ch + 1]), with
+  // f_i + f_j + f_k of their eight spin combinations in gf.
+  int npg, nhg, nhp, ngtrip;     // groups, hole group pairs U <= V, group triples
+  const int2 *pg, *hg;
+  const int4 *pgn;
+  const int *og;
+  const int *gptr;
+  const T3Hole *gtrip;
+  double2 *gf;
+  // Tables of the group kernel, 64-byte records of four elements:
+  //   gE[((pair(y, z) 4 + 2 ys + zs) nhg + S) 2 + ss]: conj <yz||s d> for both
+  //     spins of d, t(yz, s l) for both spins of l; pair(y, z) = y (y + 1) / 2 + z
+  //     over particle groups y >= z, S the hole group of s
+  //   gD[((x 2 + xs) nhp + pair(v, u)) 4 + 2 us + vs]: t(x d, u v), conj <uv||l x>
+  // The spin of d (l) is that of the orbital lookup; its momentum and isospin
+  // follow from conservation.  The t halves are refilled for every sum.
+  double2 *gE, *gD;
   // 1: the lattice maps onto itself under n -> -n with k -> -k exactly (no
   // twist) and holes onto holes, so <cb||kd> = <Pc Pb||Pk Pd> (the NN and 3NF
   // elements are even under parity) and the table fill evaluates one of each

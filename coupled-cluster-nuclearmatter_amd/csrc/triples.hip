@@ -232,7 +232,6 @@ __constant__ TermCode kTerms[18] = {
 
 __device__ __forceinline__ int sel3(int s, int x0, int x1, int x2) { return s == 0 ? x0 : (s == 1 ? x1 : x2); }
 
-template <bool TAB>
 __global__ __launch_bounds__(256) void k_triples(SolveDesc d, TriplesDesc td, double volume, double2 *partial,
                                                  unsigned long long *count) {
   __shared__ double sre[256], sim[256];
@@ -255,37 +254,24 @@ __global__ __launch_bounds__(256) void k_triples(SolveDesc d, TriplesDesc td, do
         const int i = td.hijk[3 * h], j = td.hijk[3 * h + 1], k = td.hijk[3 * h + 2];
         double2 w = make_double2(0.0, 0.0);
         auto add = [&](double sg, double2 v) { w.x += sg * v.x; w.y += sg * v.y; };
-        if constexpr (TAB) {
-          // the same 18 terms in the same order, one at a time (fewer live
-          // registers than the unrolled form)
-#pragma unroll 1
-          for (int t = 0; t < 18; ++t) {
-            const TermCode tc = kTerms[t];
-            const int x = sel3(tc.p0, a, b, c), y = sel3(tc.p1, a, b, c), z = sel3(tc.p2, a, b, c);
-            const int u = sel3(tc.h0, i, j, k), v = sel3(tc.h1, i, j, k), q = sel3(tc.h2, i, j, k);
-            add((double)tc.sign, tc.kind == 0 ? f_term<true>(d, td, volume, x, y, z, u, v, q)
-                                              : h_term<true>(d, td, volume, x, y, z, u, v, q));
-          }
-        } else {
-        add(1, f_term<TAB>(d, td, volume, a, b, c, i, j, k));
-        add(-1, f_term<TAB>(d, td, volume, b, a, c, i, j, k));
-        add(-1, f_term<TAB>(d, td, volume, c, b, a, i, j, k));
-        add(-1, f_term<TAB>(d, td, volume, a, b, c, k, j, i));
-        add(-1, f_term<TAB>(d, td, volume, a, b, c, i, k, j));
-        add(1, f_term<TAB>(d, td, volume, c, b, a, i, k, j));
-        add(1, f_term<TAB>(d, td, volume, c, b, a, k, j, i));
-        add(1, f_term<TAB>(d, td, volume, b, a, c, i, k, j));
-        add(1, f_term<TAB>(d, td, volume, b, a, c, k, j, i));
-        add(-1, h_term<TAB>(d, td, volume, a, b, c, i, j, k));
-        add(1, h_term<TAB>(d, td, volume, a, c, b, i, j, k));
-        add(1, h_term<TAB>(d, td, volume, c, b, a, i, j, k));
-        add(1, h_term<TAB>(d, td, volume, a, b, c, k, j, i));
-        add(1, h_term<TAB>(d, td, volume, a, b, c, j, i, k));
-        add(-1, h_term<TAB>(d, td, volume, c, b, a, j, i, k));
-        add(-1, h_term<TAB>(d, td, volume, c, b, a, k, j, i));
-        add(-1, h_term<TAB>(d, td, volume, a, c, b, j, i, k));
-        add(-1, h_term<TAB>(d, td, volume, a, c, b, k, j, i));
-        }
+        add(1, f_term<false>(d, td, volume, a, b, c, i, j, k));
+        add(-1, f_term<false>(d, td, volume, b, a, c, i, j, k));
+        add(-1, f_term<false>(d, td, volume, c, b, a, i, j, k));
+        add(-1, f_term<false>(d, td, volume, a, b, c, k, j, i));
+        add(-1, f_term<false>(d, td, volume, a, b, c, i, k, j));
+        add(1, f_term<false>(d, td, volume, c, b, a, i, k, j));
+        add(1, f_term<false>(d, td, volume, c, b, a, k, j, i));
+        add(1, f_term<false>(d, td, volume, b, a, c, i, k, j));
+        add(1, f_term<false>(d, td, volume, b, a, c, k, j, i));
+        add(-1, h_term<false>(d, td, volume, a, b, c, i, j, k));
+        add(1, h_term<false>(d, td, volume, a, c, b, i, j, k));
+        add(1, h_term<false>(d, td, volume, c, b, a, i, j, k));
+        add(1, h_term<false>(d, td, volume, a, b, c, k, j, i));
+        add(1, h_term<false>(d, td, volume, a, b, c, j, i, k));
+        add(-1, h_term<false>(d, td, volume, c, b, a, j, i, k));
+        add(-1, h_term<false>(d, td, volume, c, b, a, k, j, i));
+        add(-1, h_term<false>(d, td, volume, a, c, b, j, i, k));
+        add(-1, h_term<false>(d, td, volume, a, c, b, k, j, i));
         // conj(W) W / D with complex D
         const double dre = d.fdiag[i].x + d.fdiag[j].x + d.fdiag[k].x - fa - fb - fc;
         const double dim = d.fdiag[i].y + d.fdiag[j].y + d.fdiag[k].y - fai - fbi - fci;
@@ -319,18 +305,6 @@ __global__ __launch_bounds__(256) void k_triples(SolveDesc d, TriplesDesc td, do
 // a wave stride over the hole triples of that (K3,Tz3) channel.  Every lane of
 // a wave reads the same <c.||..> and <..||.c> table rows (cache-friendly), and
 // no lane waits for a longer hole-triple list than its wave's.
-//
-// With W the 18-term numerator (pert_triples2, ccm_triples.f90:611-700), W3 =
-// <abc||ijk> the antisymmetrized three-nucleon element (chiral_3nf_asym) and D
-// = f_i + f_j + f_k - f_a - f_b - f_c, the sum over a<b<c, i<j<k is
-//   MODE 0: |W|^2 / D                 (T), et_4
-//   MODE 1: (W3 + W) conj(W3) / D     CCDT-1 energy of T3 = (W3 + W)/D
-//           (t3_intermediate, ccm_t3_eqn.f90:1-192; t3_energy,
-//           ccm_t3full_channels.f90:570-667)
-//   MODE 2: |W3|^2 / D                CCDT-1 energy of the start T3 = W3/D
-//           (setup_t3, ccm_t3full_channels.f90:291-567)
-//   MODE 3: |W + W3|^2 / D            (T) at tnf_approx 3, et_5 (:656-722)
-template <int MODE, bool ONE>
 __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, double volume, double2 *partial,
                                                    unsigned long long *count) {
   __shared__ double sre[256], sim[256];
@@ -351,50 +325,23 @@ __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, 
       const double fai = d.fdiag[a].y, fbi = d.fdiag[b].y, fci = d.fdiag[c].y;
       const int h0 = td.hptr[ch], h1 = td.hptr[ch + 1];
       if (lane == 0) nel += (unsigned long long)(h1 - h0);
-      Nucleon na{}, nb{}, nc{};
-      double fbra = 0.0;
-      if constexpr (MODE != 0) {
-        na = nucleon_of(td.c3w, a);
-        nb = nucleon_of(td.c3w, b);
-        nc = nucleon_of(td.c3w, c);
-        fbra = freg3(td.c3w, na.k, nb.k, nc.k);
-      }
       for (int h = h0 + lane; h < h1; h += 64) {
         const int i = td.hijk[3 * h], j = td.hijk[3 * h + 1], k = td.hijk[3 * h + 2];
         double2 w = make_double2(0.0, 0.0);
-        if constexpr (MODE != 2) {
 #pragma unroll 1
-          for (int t = 0; t < 18; ++t) {
-            const TermCode tc = kTerms[t];
-            const int x = sel3(tc.p0, a, b, c), y = sel3(tc.p1, a, b, c), z = sel3(tc.p2, a, b, c);
-            const int u = sel3(tc.h0, i, j, k), v = sel3(tc.h1, i, j, k), q = sel3(tc.h2, i, j, k);
-            const double2 f = tc.kind == 0 ? f_term<true>(d, td, volume, x, y, z, u, v, q)
-                                           : h_term<true>(d, td, volume, x, y, z, u, v, q);
-            w.x += (double)tc.sign * f.x;
-            w.y += (double)tc.sign * f.y;
-          }
+        for (int t = 0; t < 18; ++t) {
+          const TermCode tc = kTerms[t];
+          const int x = sel3(tc.p0, a, b, c), y = sel3(tc.p1, a, b, c), z = sel3(tc.p2, a, b, c);
+          const int u = sel3(tc.h0, i, j, k), v = sel3(tc.h1, i, j, k), q = sel3(tc.h2, i, j, k);
+          const double2 f = tc.kind == 0 ? f_term<true>(d, td, volume, x, y, z, u, v, q)
+                                         : h_term<true>(d, td, volume, x, y, z, u, v, q);
+          w.x += (double)tc.sign * f.x;
+          w.y += (double)tc.sign * f.y;
         }
         const double dre = d.fdiag[i].x + d.fdiag[j].x + d.fdiag[k].x - fa - fb - fc;
         const double dim = d.fdiag[i].y + d.fdiag[j].y + d.fdiag[k].y - fai - fbi - fci;
         const double den = dre * dre + dim * dim;
-        // numerator n, then n / D = n conj(D) / |D|^2
-        double nre, nim = 0.0;
-        if constexpr (MODE == 0) {
-          nre = w.x * w.x + w.y * w.y;
-        } else {
-          const double2 w3 = chiral3_asym<ONE>(td.c3w, fbra, na, nb, nc, nucleon_of(td.c3w, i), nucleon_of(td.c3w, j),
-                                               nucleon_of(td.c3w, k));
-          if constexpr (MODE == 1) {
-            const double xr = w3.x + w.x, xi = w3.y + w.y;
-            nre = xr * w3.x + xi * w3.y;
-            nim = xi * w3.x - xr * w3.y;
-          } else if constexpr (MODE == 2) {
-            nre = w3.x * w3.x + w3.y * w3.y;
-          } else {
-            const double xr = w3.x + w.x, xi = w3.y + w.y;
-            nre = xr * xr + xi * xi;
-          }
-        }
+        const double nre = w.x * w.x + w.y * w.y, nim = 0.0;
         re += (nre * dre + nim * dim) / den;
         im += (nim * dre - nre * dim) / den;
       }
@@ -558,31 +505,470 @@ __global__ __launch_bounds__(256) void k_triples_s(SolveDesc d, TriplesDesc td, 
   }
 }
 
-__global__ void k_triples_count(const unsigned long long *count, int n, unsigned long long *out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  unsigned long long s = 0;
-  for (int k = 0; k < n; ++k) s += count[k];
-  out[0] = s;
+// ---------------------------------------------------------------------------
+// The group kernel: (T) and the CCDT-1 sums over spin groups.
+//
+// Momentum conservation acts on groups (the two spin states of one momentum and
+// isospin), so a particle group triple and a hole group triple that conserve
+// it are 8 x 8 elements (abc, ijk) that share every index.  With
+//   E_a[s] = (conj <cb||s d-+>, t(cb, s l-+)),  E_b, E_c likewise with the pairs
+//            (c, a) and (b, a),
+//   D_x[uv] = (t(x d-+, u v), conj <uv||l-+ x>)
+// the 18 signed F and H terms (pert_triples2, ccm_triples.f90:611-700) are
+//   W = sum over the splits (ij|k) - (ik|j) + (jk|i) of the three holes into
+//       pair uv and single s of  E_a[s].D_a[uv] - E_b[s].D_b[uv] + E_c[s].D_c[uv],
+// nine products of length four.  A lane takes one of the four components k and,
+// for one hole group triple and one (as, bs), all 16 (cs, is, js, ks): per split
+// 26 loads of 16 bytes, four lanes to a 64-byte record, for 192 FMAs, no index
+// arithmetic per element.  The four lanes then add up (each keeps four
+// elements).  One wave per particle group triple, four hole group triples at a
+// time.
+//
+// Bound: the L1 (26 KB per 256 elements and split) and FP64 issue.  The kernel
+// it replaced gathered 36 x 32 bytes per element with a lookup for each: PNM
+// A=66 |n_i|<=3 (1.62e9 elements) 181 to 66 ms.
+//
+// With W3 = <abc||ijk> the antisymmetrized three-nucleon element
+// (chiral_3nf_asym) and D = f_i + f_j + f_k - f_a - f_b - f_c, the sum over
+// a<b<c, i<j<k is
+//   MODE 0: |W|^2 / D                 (T), et_4
+//   MODE 1: (W3 + W) conj(W3) / D     CCDT-1 energy of T3 = (W3 + W)/D
+//           (t3_intermediate, ccm_t3_eqn.f90:1-192; t3_energy,
+//           ccm_t3full_channels.f90:570-667)
+//   MODE 2: |W3|^2 / D                CCDT-1 energy of the start T3 = W3/D
+//           (setup_t3, ccm_t3full_channels.f90:291-567)
+//   MODE 3: |W + W3|^2 / D            (T) at tnf_approx 3, et_5 (:656-722)
+// The four elements a lane keeps differ in js and ks only, so W3 takes its
+// geometry once for them.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int slot_of(int2 g, int s) { return s ? g.y : g.x; }
+
+// pair index t = y (y + 1) / 2 + z, z <= y
+__device__ __forceinline__ void tri_yz(int64_t t, int &y, int &z) {
+  int64_t x = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while (x * (x + 1) / 2 > t) --x;
+  while ((x + 1) * (x + 2) / 2 <= t) ++x;
+  y = (int)x;
+  z = (int)(t - x * (x + 1) / 2);
+}
+__device__ __forceinline__ int64_t tri_at(int64_t y, int64_t z) { return y * (y + 1) / 2 + z; }
+
+// an entry of gE: the orbitals of its record and the d (or l) of spin sd
+struct T3E {
+  int y, z, s, ys, zs, ss, S, d;
+  int64_t gp;
+};
+__device__ __forceinline__ T3E t3_e_entry(const SolveDesc &d, const TriplesDesc &td, int64_t rec, int sd) {
+  T3E e;
+  e.ss = (int)(rec & 1);
+  int64_t r = rec >> 1;
+  e.S = (int)(r % td.nhg);
+  r /= td.nhg;
+  e.zs = (int)(r & 1);
+  e.ys = (int)((r >> 1) & 1);
+  e.gp = r >> 2;
+  int gy, gz;
+  tri_yz(e.gp, gy, gz);
+  e.y = slot_of(td.pg[gy], e.ys);
+  e.z = slot_of(td.pg[gz], e.zs);
+  e.s = slot_of(td.hg[e.S], e.ss);
+  e.d = -1;
+  if (e.y >= 0 && e.z >= 0 && e.s >= 0 && e.y != e.z)
+    e.d = orb_lookup(td, d.nx[e.y] + d.nx[e.z] - d.nx[e.s], d.ny[e.y] + d.ny[e.z] - d.ny[e.s],
+                     d.nz[e.y] + d.nz[e.z] - d.nz[e.s], 2 * sd - 1, d.tz[e.y] + d.tz[e.z] - d.tz[e.s]);
+  return e;
 }
 
-__global__ void k_triples_final(const double2 *partial, int n, double2 *out) {
-  __shared__ double sre[256], sim[256];
+// conj <yz||s d> of every record, both spins of d: once per interaction.  The
+// element is evaluated for the ascending orbital order of (y, z) and signed.
+// With no twist one of each parity pair (n -> -n) is evaluated and written to
+// both places.  A block lists the entries of its chunk that need evaluating
+// (half or more conserve momentum with no particle d) and evaluates the list
+// with full waves.
+template <bool ONE>
+__global__ __launch_bounds__(256) void k_t3_fill_ev(SolveDesc d, TriplesDesc td, double vol, int64_t nrec) {
+  constexpr int kChunk = 4096;
+  __shared__ int list[kChunk];
+  __shared__ int cnt;
+  const int64_t n = 2 * nrec;
+  auto image = [&](const T3E &e, int64_t &rec, double &sg) {   // record of the parity image, its sign
+    auto img = [&](int x) { return td.og[orb_lookup(td, -d.nx[x], -d.ny[x], -d.nz[x], d.sz[x], d.tz[x])]; };
+    const int oy = img(e.y), oz = img(e.z), os = img(e.s);
+    const bool keep = (oy >> 1) >= (oz >> 1);
+    const int o1 = keep ? oy : oz, o2 = keep ? oz : oy;
+    sg = keep ? 1.0 : -1.0;
+    rec = ((tri_at(o1 >> 1, o2 >> 1) * 4 + 2 * (o1 & 1) + (o2 & 1)) * td.nhg + (os >> 1)) * 2 + (os & 1);
+  };
+  for (int64_t base = (int64_t)blockIdx.x * kChunk; base < n; base += (int64_t)gridDim.x * kChunk) {
+    if (threadIdx.x == 0) cnt = 0;
+    __syncthreads();
+    for (int t = threadIdx.x; t < kChunk && base + t < n; t += 256) {
+      const int64_t rec = (base + t) >> 1;
+      const int sd = t & 1;
+      const T3E e = t3_e_entry(d, td, rec, sd);
+      if (e.d < d.A) {
+        td.gE[4 * rec + sd] = make_double2(0.0, 0.0);
+        continue;
+      }
+      if (td.parity) {
+        int64_t ir;
+        double sg;
+        image(e, ir, sg);
+        const int64_t igp = ir / ((int64_t)8 * td.nhg);
+        const int iS = (int)((ir >> 1) % td.nhg);
+        if (igp < e.gp || (igp == e.gp && iS < e.S)) continue;
+      }
+      list[atomicAdd(&cnt, 1)] = t;
+    }
+    __syncthreads();
+    const int m = cnt;
+    for (int q = threadIdx.x; q < m; q += 256) {
+      const int64_t rec = (base + list[q]) >> 1;
+      const int sd = list[q] & 1;
+      const T3E e = t3_e_entry(d, td, rec, sd);
+      const int lo = min(e.y, e.z), hi = max(e.y, e.z);
+      double2 v = vas_t(d, td, vol, lo, hi, e.s, e.d);
+      if (td.tnf) {
+        const double2 w = no2b_sum<ONE>(td.c3, d.A, lo, hi, e.s, e.d);
+        v.x += w.x;
+        v.y += w.y;
+      }
+      const double s1 = e.y < e.z ? 1.0 : -1.0;
+      v = make_double2(s1 * v.x, -s1 * v.y);   // conjugated
+      td.gE[4 * rec + sd] = v;
+      if (td.parity) {
+        int64_t ir;
+        double sg;
+        image(e, ir, sg);
+        const int64_t igp = ir / ((int64_t)8 * td.nhg);
+        const int iS = (int)((ir >> 1) % td.nhg);
+        if (igp != e.gp || iS != e.S) td.gE[4 * ir + sd] = make_double2(sg * v.x, sg * v.y);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// t(yz, s l) of every record, both spins of the hole l
+__global__ __launch_bounds__(256) void k_t3_fill_et(SolveDesc d, TriplesDesc td, int64_t nrec) {
+  for (int64_t rec = (int64_t)blockIdx.x * 256 + threadIdx.x; rec < nrec; rec += (int64_t)gridDim.x * 256) {
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      const T3E e = t3_e_entry(d, td, rec, sl);
+      td.gE[4 * rec + 2 + sl] = e.d >= 0 && e.d < d.A ? t_of(d, e.y, e.z, e.s, e.d) : make_double2(0.0, 0.0);
+    }
+  }
+}
+
+// gD: T false conj <uv||l x> (once per interaction), true t(x d, u v)
+template <bool T>
+__global__ __launch_bounds__(256) void k_t3_fill_d(SolveDesc d, TriplesDesc td, double vol, int64_t nrec) {
+  for (int64_t rec = (int64_t)blockIdx.x * 256 + threadIdx.x; rec < nrec; rec += (int64_t)gridDim.x * 256) {
+    const int vs = (int)(rec & 1), us = (int)((rec >> 1) & 1);
+    const int64_t r = rec >> 2;
+    const int gx = (int)(r / td.nhp);
+    int gu, gv;
+    tri_yz(r - (int64_t)gx * td.nhp, gv, gu);
+    const int x = slot_of(td.pg[gx >> 1], gx & 1), u = slot_of(td.hg[gu], us), v = slot_of(td.hg[gv], vs);
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) {
+      double2 o = make_double2(0.0, 0.0);
+      if (x >= 0 && u >= 0 && v >= 0 && u != v) {
+        const int w = orb_lookup(td, d.nx[u] + d.nx[v] - d.nx[x], d.ny[u] + d.ny[v] - d.ny[x],
+                                 d.nz[u] + d.nz[v] - d.nz[x], 2 * sp - 1, d.tz[u] + d.tz[v] - d.tz[x]);
+        if (T && w >= d.A) o = t_of(d, x, w, u, v);
+        if (!T && w >= 0 && w < d.A) {
+          o = vas_t(d, td, vol, u, v, w, x);
+          o.y = -o.y;
+        }
+      }
+      td.gD[4 * rec + (T ? 0 : 2) + sp] = o;
+    }
+  }
+}
+
+// f_i + f_j + f_k of the hole group triples' states
+__global__ __launch_bounds__(256) void k_t3_fill_gf(SolveDesc d, TriplesDesc td) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= 8 * td.ngtrip) return;
+  const T3Hole t = td.gtrip[e >> 3];
+  double2 f = make_double2(0.0, 0.0);
+  if ((t.mask >> (e & 7)) & 1) {
+    const int i = slot_of(td.hg[t.I], (e >> 2) & 1), j = slot_of(td.hg[t.J], (e >> 1) & 1),
+              k = slot_of(td.hg[t.K], e & 1);
+    f = make_double2(d.fdiag[i].x + d.fdiag[j].x + d.fdiag[k].x, d.fdiag[i].y + d.fdiag[j].y + d.fdiag[k].y);
+  }
+  td.gf[e] = f;
+}
+
+__device__ __forceinline__ void cmac(double2 &a, const double2 &e, const double2 &x) {
+  a.x = fma(e.x, x.x, a.x);
+  a.x = fma(-e.y, x.y, a.x);
+  a.y = fma(e.x, x.y, a.y);
+  a.y = fma(e.y, x.x, a.y);
+}
+__device__ __forceinline__ void cmac_neg(double2 &a, const double2 &e, const double2 &x) {
+  a.x = fma(-e.x, x.x, a.x);
+  a.x = fma(e.y, x.y, a.x);
+  a.y = fma(-e.x, x.y, a.y);
+  a.y = fma(-e.y, x.x, a.y);
+}
+// One split of the hole triple: SP 0 (ij|k), 1 (ik|j) with the minus sign, 2
+// (jk|i).  acc[8 cs + 4 is + 2 js + ks]; pointers at the lane's component.
+template <int SP>
+__device__ __forceinline__ void t3_split(double2 (&acc)[16], const double2 *Da, const double2 *Db, const double2 *Dc0,
+                                         const double2 *Dc1, const double2 *Ea0, const double2 *Ea1,
+                                         const double2 *Eb0, const double2 *Eb1, const double2 *Ec) {
+  double2 da[4], db[4], dc[2][4], ea[2][2], eb[2][2], ec[2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    da[q] = Da[4 * q];
+    db[q] = Db[4 * q];
+    dc[0][q] = Dc0[4 * q];
+    dc[1][q] = Dc1[4 * q];
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    ea[0][s] = Ea0[4 * s];
+    ea[1][s] = Ea1[4 * s];
+    eb[0][s] = Eb0[4 * s];
+    eb[1][s] = Eb1[4 * s];
+    ec[s] = Ec[4 * s];
+  }
+#pragma unroll
+  for (int cs = 0; cs < 2; ++cs)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int o = 8 * cs + (SP == 0 ? 4 * u + 2 * v + s : SP == 1 ? 4 * u + 2 * s + v : 4 * s + 2 * u + v);
+          const int q = 2 * u + v;
+          if (SP != 1) {
+            cmac(acc[o], ea[cs][s], da[q]);
+            cmac_neg(acc[o], eb[cs][s], db[q]);
+            cmac(acc[o], ec[s], dc[cs][q]);
+          } else {
+            cmac_neg(acc[o], ea[cs][s], da[q]);
+            cmac(acc[o], eb[cs][s], db[q]);
+            cmac_neg(acc[o], ec[s], dc[cs][q]);
+          }
+        }
+}
+
+// value of the lane 1 (CTRL 0xB1) or 2 (0x4E) away within a group of four
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+template <int MODE, bool ONE>
+__global__ __launch_bounds__(256) void k_triples_g(SolveDesc d, TriplesDesc td, double2 *partial,
+                                                   unsigned long long *count) {
+  __shared__ double sre[4], sim[4];
+  __shared__ unsigned long long scnt[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int kk = lane & 3, as = (lane >> 2) & 1, bs = (lane >> 3) & 1, hq = lane >> 4;
+  const int cs_f = kk & 1, is_f = kk >> 1;   // of the four elements this lane finishes
   double re = 0.0, im = 0.0;
-  for (int p = threadIdx.x; p < n; p += blockDim.x) {
+  unsigned long long nel = 0;
+  const int64_t npair = tri_at(td.npg, 0);
+  const int64_t erow = (int64_t)td.nhg * 8, drow = (int64_t)td.nhp * 16;   // double2 per (pair, ys, zs) and per x
+  for (int64_t pr = blockIdx.x; pr < npair; pr += gridDim.x) {
+    int gb, ga;
+    tri_yz(pr, gb, ga);
+    const int a = slot_of(td.pg[ga], as), b = slot_of(td.pg[gb], bs);
+    const int4 ma = td.pgn[ga], mb_ = td.pgn[gb];
+    const bool ab_ok = a >= 0 && b >= 0 && (ga != gb || (as == 0 && bs == 1));
+    for (int gc = gb + wave; gc < td.npg; gc += 4) {
+      if (gc == ga) continue;   // three particles in two states
+      const int4 mc = td.pgn[gc];
+      const int ix = ma.x + mb_.x + mc.x - td.k0, iy = ma.y + mb_.y + mc.y - td.k0, iz = ma.z + mb_.z + mc.z - td.k0;
+      const int it = ma.w + mb_.w + mc.w - td.tz0;
+      if (ix < 0 || iy < 0 || iz < 0 || ix >= td.nk || iy >= td.nk || iz >= td.nk || it < 0 || it >= td.ntz) continue;
+      const int ch = td.chan[((it * td.nk + ix) * td.nk + iy) * td.nk + iz];
+      if (ch < 0) continue;
+      const int g0 = td.gptr[ch], g1 = td.gptr[ch + 1];
+      const int2 pc = td.pg[gc];
+      const bool v0 = ab_ok && pc.x >= 0 && gb != gc, v1 = ab_ok && pc.y >= 0 && (gb != gc || bs == 0);
+      const bool pv = cs_f ? v1 : v0;
+      const int c = slot_of(pc, cs_f);
+      double2 fabc = make_double2(0.0, 0.0);
+      if (pv) {
+        fabc.x = d.fdiag[a].x + d.fdiag[b].x + d.fdiag[c].x;
+        fabc.y = d.fdiag[a].y + d.fdiag[b].y + d.fdiag[c].y;
+      }
+      const double2 *Ea0 = nullptr, *Ea1 = nullptr, *Eb0 = nullptr, *Eb1 = nullptr, *Ec = nullptr;
+      const double2 *Da = nullptr, *Db = nullptr, *Dc0 = nullptr, *Dc1 = nullptr;
+      if constexpr (MODE != 2) {
+        Ea0 = td.gE + (tri_at(gc, gb) * 4 + bs) * erow + kk;
+        Ea1 = Ea0 + 2 * erow;
+        Eb0 = td.gE + (tri_at(gc, ga) * 4 + as) * erow + kk;
+        Eb1 = Eb0 + 2 * erow;
+        Ec = td.gE + (tri_at(gb, ga) * 4 + 2 * bs + as) * erow + kk;
+        Da = td.gD + (int64_t)(2 * ga + as) * drow + kk;
+        Db = td.gD + (int64_t)(2 * gb + bs) * drow + kk;
+        Dc0 = td.gD + (int64_t)(2 * gc) * drow + kk;
+        Dc1 = Dc0 + drow;
+      }
+      Nucleon na{}, nb{}, nc{};
+      double fbra = 0.0;
+      if constexpr (MODE != 0) {
+        auto rep = [&](int2 g) { return nucleon_of(td.c3w, g.x >= 0 ? g.x : g.y); };
+        na = rep(td.pg[ga]);
+        nb = rep(td.pg[gb]);
+        nc = rep(pc);
+        fbra = freg3(td.c3w, na.k, nb.k, nc.k);
+      }
+      for (int gg = g0; gg < g1; gg += 4) {
+        const int g = min(gg + hq, g1 - 1);
+        const T3Hole t = td.gtrip[g];
+        const bool ok = gg + hq < g1 && pv;
+        double2 w[4];
+        if constexpr (MODE != 2) {
+          double2 acc[16];
+#pragma unroll
+          for (int o = 0; o < 16; ++o) acc[o] = make_double2(0.0, 0.0);
+          t3_split<0>(acc, Da + 16 * t.hij, Db + 16 * t.hij, Dc0 + 16 * t.hij, Dc1 + 16 * t.hij, Ea0 + 8 * t.K,
+                      Ea1 + 8 * t.K, Eb0 + 8 * t.K, Eb1 + 8 * t.K, Ec + 8 * t.K);
+          t3_split<1>(acc, Da + 16 * t.hik, Db + 16 * t.hik, Dc0 + 16 * t.hik, Dc1 + 16 * t.hik, Ea0 + 8 * t.J,
+                      Ea1 + 8 * t.J, Eb0 + 8 * t.J, Eb1 + 8 * t.J, Ec + 8 * t.J);
+          t3_split<2>(acc, Da + 16 * t.hjk, Db + 16 * t.hjk, Dc0 + 16 * t.hjk, Dc1 + 16 * t.hjk, Ea0 + 8 * t.I,
+                      Ea1 + 8 * t.I, Eb0 + 8 * t.I, Eb1 + 8 * t.I, Ec + 8 * t.I);
+          // sum over the four components: lane kk keeps cs = kk & 1, then is = kk >> 1
+          double2 h[8];
+#pragma unroll
+          for (int o = 0; o < 8; ++o) {
+            const double2 x = cs_f ? acc[o] : acc[8 + o], y = cs_f ? acc[8 + o] : acc[o];
+            h[o] = make_double2(y.x + quad_swap<0xB1>(x.x), y.y + quad_swap<0xB1>(x.y));
+          }
+#pragma unroll
+          for (int o = 0; o < 4; ++o) {
+            const double2 x = is_f ? h[o] : h[4 + o], y = is_f ? h[4 + o] : h[o];
+            w[o] = make_double2(y.x + quad_swap<0x4E>(x.x), y.y + quad_swap<0x4E>(x.y));
+          }
+        }
+        const int m4 = ok ? (t.mask >> (4 * is_f)) & 15 : 0;
+        nel += (unsigned long long)__popc(m4);
+        Geo3 geo;
+        int ks0 = 0, ks1 = 0, ks2 = 0, kt0 = 0, kt1 = 0, kt2 = 0;   // hole spins per state (bit s), isospins
+        if constexpr (MODE != 0) {
+          auto rep = [&](int2 q) { return nucleon_of(td.c3w, q.x >= 0 ? q.x : q.y); };
+          const Nucleon ni = rep(td.hg[t.I]), nj = rep(td.hg[t.J]), nk = rep(td.hg[t.K]);
+          geo3_transfer<0, 0>(td.c3w, geo, na, ni);
+          geo3_transfer<0, 1>(td.c3w, geo, na, nj);
+          geo3_transfer<0, 2>(td.c3w, geo, na, nk);
+          geo3_transfer<1, 0>(td.c3w, geo, nb, ni);
+          geo3_transfer<1, 1>(td.c3w, geo, nb, nj);
+          geo3_transfer<1, 2>(td.c3w, geo, nb, nk);
+          geo3_transfer<2, 0>(td.c3w, geo, nc, ni);
+          geo3_transfer<2, 1>(td.c3w, geo, nc, nj);
+          geo3_transfer<2, 2>(td.c3w, geo, nc, nk);
+          const double f = fbra * td.c3w.scale;
+          geo.f[0] = f * freg3(td.c3w, nj.k, nk.k, ni.k);
+          geo.f[1] = f * freg3(td.c3w, ni.k, nk.k, nj.k);
+          geo.f[2] = f * freg3(td.c3w, ni.k, nj.k, nk.k);
+          auto up = [&](int2 q) {
+            return (q.x >= 0 && d.sz[q.x] > 0 ? 1 : 0) | (q.y >= 0 && d.sz[q.y] > 0 ? 2 : 0);
+          };
+          ks0 = up(td.hg[t.I]);
+          ks1 = up(td.hg[t.J]);
+          ks2 = up(td.hg[t.K]);
+          kt0 = ni.tz;
+          kt1 = nj.tz;
+          kt2 = nk.tz;
+        }
+        auto finish = [&](int o, double2 wo) {
+          const double2 fh = td.gf[8 * (int64_t)g + 4 * is_f + o];
+          const double dre = fh.x - fabc.x, dim = fh.y - fabc.y;
+          const double inv = 1.0 / (dre * dre + dim * dim);
+          double nre, nim = 0.0;
+          if constexpr (MODE == 0) {
+            nre = wo.x * wo.x + wo.y * wo.y;
+          } else {
+            auto sp = [](int bits, int s) { return (bits >> s) & 1 ? 1 : -1; };
+            const int mb[3] = {d.sz[a], d.sz[b], d.sz[c]}, tb[3] = {na.tz, nb.tz, nc.tz};
+            const int mk[3] = {sp(ks0, is_f), sp(ks1, o >> 1), sp(ks2, o & 1)}, tk[3] = {kt0, kt1, kt2};
+            const double2 w3 = asym3<ONE, false>(td.c3w, geo, mb, mk, tb, tk);
+            if constexpr (MODE == 1) {
+              const double xr = w3.x + wo.x, xi = w3.y + wo.y;
+              nre = xr * w3.x + xi * w3.y;
+              nim = xi * w3.x - xr * w3.y;
+            } else if constexpr (MODE == 2) {
+              nre = w3.x * w3.x + w3.y * w3.y;
+            } else {
+              const double xr = w3.x + wo.x, xi = w3.y + wo.y;
+              nre = xr * xr + xi * xi;
+            }
+          }
+          re += (nre * dre + nim * dim) * inv;
+          im += (nim * dre - nre * dim) * inv;
+        };
+        if constexpr (MODE == 0) {
+#pragma unroll
+          for (int o = 0; o < 4; ++o)
+            if ((m4 >> o) & 1) finish(o, w[o]);
+        } else {
+#pragma unroll 1
+          for (int o = 0; o < 4; ++o) {
+            double2 wo = make_double2(0.0, 0.0);
+            if constexpr (MODE != 2) wo = o == 0 ? w[0] : o == 1 ? w[1] : o == 2 ? w[2] : w[3];
+            if ((m4 >> o) & 1) finish(o, wo);
+          }
+        }
+      }
+    }
+  }
+  // fixed-order sums: butterfly in the wave, then the four waves
+  for (int off = 32; off > 0; off >>= 1) {
+    re += __shfl_xor(re, off);
+    im += __shfl_xor(im, off);
+    nel += __shfl_xor(nel, off);
+  }
+  if (lane == 0) {
+    sre[wave] = re;
+    sim[wave] = im;
+    scnt[wave] = nel;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = make_double2(((sre[0] + sre[1]) + sre[2]) + sre[3], ((sim[0] + sim[1]) + sim[2]) + sim[3]);
+    count[blockIdx.x] = scnt[0] + scnt[1] + scnt[2] + scnt[3];
+  }
+}
+
+// Sums of the blocks' partials and element counts
+__global__ __launch_bounds__(256) void k_triples_final(const double2 *partial, const unsigned long long *count, int n,
+                                                       double2 *out, unsigned long long *count_out) {
+  __shared__ double sre[256], sim[256];
+  __shared__ unsigned long long scnt[256];
+  double re = 0.0, im = 0.0;
+  unsigned long long c = 0;
+  for (int p = threadIdx.x; p < n; p += 256) {
     re += partial[p].x;
     im += partial[p].y;
+    c += count[p];
   }
   sre[threadIdx.x] = re;
   sim[threadIdx.x] = im;
+  scnt[threadIdx.x] = c;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) {
       sre[threadIdx.x] += sre[threadIdx.x + s];
       sim[threadIdx.x] += sim[threadIdx.x + s];
+      scnt[threadIdx.x] += scnt[threadIdx.x + s];
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = make_double2(sre[0], sim[0]);
+  if (threadIdx.x == 0) {
+    out[0] = make_double2(sre[0], sim[0]);
+    count_out[0] = scnt[0];
+  }
 }
 
 void launch_t3_tables(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *hppp, double2 *hhhp,
@@ -598,31 +984,61 @@ void launch_t3_td(const SolveDesc &d, const TriplesDesc &td, double2 *tdt, hipSt
   hipLaunchKernelGGL(k_t3_fill_td, dim3(4096), dim3(256), 0, st, d, td, tdt);
 }
 
-// CCGPU_T3_KERNEL (studies and the tests that compare the forms): 1 (default)
-// the staged kernel when its amplitude table tdt exists, else the table
-// kernel k_triples_w; 3 k_triples_w; other values the thread-per-triple form.
+static int64_t t3_e_records(const TriplesDesc &td) {
+  return (int64_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2;
+}
+static int64_t t3_d_records(const TriplesDesc &td) { return (int64_t)td.npg * 2 * td.nhp * 4; }
+static unsigned t3_grid(int64_t n, int64_t most) {
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, most));
+}
+
+// The interaction halves of the group tables
+void launch_t3_group_v(const SolveDesc &d, const TriplesDesc &td, double volume, hipStream_t st) {
+  const int64_t ne = t3_e_records(td), nd = t3_d_records(td);
+  const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>((2 * ne + 4095) / 4096, 16384));
+  if (td.tnf && !td.c3.one_species)
+    hipLaunchKernelGGL(k_t3_fill_ev<false>, dim3(g), dim3(256), 0, st, d, td, volume, ne);
+  else
+    hipLaunchKernelGGL(k_t3_fill_ev<true>, dim3(g), dim3(256), 0, st, d, td, volume, ne);
+  hipLaunchKernelGGL(k_t3_fill_d<false>, dim3(t3_grid(nd, 16384)), dim3(256), 0, st, d, td, volume, nd);
+}
+
+// Sum over the triples with the group kernel (modes above); the amplitude
+// halves of the tables are refilled from the current T first.
+void launch_triples_group(const SolveDesc &d, const TriplesDesc &td, double2 *partial, unsigned long long *count,
+                          int nblocks, double2 *out, unsigned long long *count_out, hipStream_t st, int mode) {
+  if (mode != 2) {
+    const int64_t ne = t3_e_records(td), nd = t3_d_records(td);
+    hipLaunchKernelGGL(k_t3_fill_et, dim3(t3_grid(ne, 16384)), dim3(256), 0, st, d, td, ne);
+    hipLaunchKernelGGL(k_t3_fill_d<true>, dim3(t3_grid(nd, 16384)), dim3(256), 0, st, d, td, 0.0, nd);
+  }
+  if (td.ngtrip > 0)
+    hipLaunchKernelGGL(k_t3_fill_gf, dim3((8 * td.ngtrip + 255) / 256), dim3(256), 0, st, d, td);
+  const bool one = td.c3w.one_species != 0;
+  const int64_t npair = (int64_t)td.npg * (td.npg + 1) / 2;
+  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(npair, nblocks));
+  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, st, d, td, partial, count); };
+  if (mode == 0) run(k_triples_g<0, true>);
+  else if (mode == 1) run(one ? k_triples_g<1, true> : k_triples_g<1, false>);
+  else if (mode == 2) run(one ? k_triples_g<2, true> : k_triples_g<2, false>);
+  else run(one ? k_triples_g<3, true> : k_triples_g<3, false>);
+  hipLaunchKernelGGL(k_triples_final, dim3(1), dim3(256), 0, st, partial, count, nb, out, count_out);
+}
+
+// (T) by one of the element-by-element kernels: 0 in place (no tables), 1 the
+// staged kernel, 3 the kernel that gathers every amplitude
 void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *partial,
                     unsigned long long *count, int nblocks, double2 *out, unsigned long long *count_out,
-                    hipStream_t st, int mode, const double2 *tdt, int maxnhh) {
-  const bool one = td.c3w.one_species != 0;
-  const int variant = getenv("CCGPU_T3_KERNEL") ? atoi(getenv("CCGPU_T3_KERNEL")) : 1;
-  if (mode == 0 && variant == 1 && tdt && td.vhppp && td.vhhhp) {
+                    hipStream_t st, int variant, const double2 *tdt, int maxnhh) {
+  if (variant == 1) {
     const size_t lds = (size_t)4 * 3 * maxnhh * sizeof(double2);
     hipLaunchKernelGGL(k_triples_s, dim3(nblocks), dim3(256), lds, st, d, td, tdt, maxnhh, partial, count);
-  } else if (mode == 1)
-    hipLaunchKernelGGL((one ? k_triples_w<1, true> : k_triples_w<1, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  else if (mode == 2)
-    hipLaunchKernelGGL((one ? k_triples_w<2, true> : k_triples_w<2, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  else if (mode == 3)
-    hipLaunchKernelGGL((one ? k_triples_w<3, true> : k_triples_w<3, false>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  else if (td.vhppp && td.vhhhp && (variant == 1 || variant == 3))
-    hipLaunchKernelGGL((k_triples_w<0, true>), dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  else if (td.vhppp && td.vhhhp)
-    hipLaunchKernelGGL(k_triples<true>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  else
-    hipLaunchKernelGGL(k_triples<false>, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
-  hipLaunchKernelGGL(k_triples_final, dim3(1), dim3(256), 0, st, partial, nblocks, out);
-  hipLaunchKernelGGL(k_triples_count, dim3(1), dim3(64), 0, st, count, nblocks, count_out);
+  } else if (variant == 3) {
+    hipLaunchKernelGGL(k_triples_w, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+  } else {
+    hipLaunchKernelGGL(k_triples, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+  }
+  hipLaunchKernelGGL(k_triples_final, dim3(1), dim3(256), 0, st, partial, count, nblocks, out, count_out);
 }
 
 }  // namespace ccgpu

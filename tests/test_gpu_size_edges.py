@@ -102,3 +102,55 @@ def test_mlp_training_step_takes_the_gradient_of_its_minibatch(ccnm, batch):
     # float32 powers of beta (1 - beta2 keeps 2^-24 / 1e-3 = 6e-5 relative,
     # half of it after the root) and the roundings of m, v and the step
     assert np.max(np.abs(net.params - (th - step))) <= 1e-4 * lr + 2.0 ** -23 * np.max(np.abs(th))
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist", [
+    (14, "pnm", 1, (0.0, 0.0, 0.0)), (2, "pnm", 1, (0.0, 0.0, 0.0)), (15, "pnm", 1, (0.3, 0.7, 1.1)),
+    (13, "pnm", 1, (0.0, 0.0, 0.0)), (4, "snm", 1, (0.0, 0.0, 0.0)), (9, "snm", 1, (0.4, 0.2, 0.9)),
+    (28, "snm", 1, (0.0, 0.0, 0.0)), (38, "pnm", 2, (0.5, 1.0, 1.5))])
+def test_triples_group_kernel_equals_element_kernels(ccnm, monkeypatch, A, matter, nmax, twist):
+    """(T) over spin groups against the kernel that gathers every element and
+    the one that evaluates them in place, on closed and open shells (groups
+    with one spin state, a group split between holes and particles, fewer than
+    three holes).  The same terms in another order: each of the 36 products of
+    W and the sum over the elements round by 2^-53 of their moduli; the sum has
+    one sign per element (every D is negative here), so 1e-12 leaves room for
+    cancellation inside W."""
+    s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax, twist=twist)
+    s.set_chiral(ccnm.NNLO, 450.0)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    s.setup_t_amplitudes()
+    for _ in range(2):
+        s.t2_intermediate()
+        s.diis_t1t2(1, 1)
+    out = {}
+    for variant in (None, "3", "0"):
+        if variant is None:
+            monkeypatch.delenv("CCGPU_T3_KERNEL", raising=False)
+        else:
+            monkeypatch.setenv("CCGPU_T3_KERNEL", variant)
+        out[variant] = (s.pert_triples2(), s.triples_stats()[0])
+    s.close()
+    (e, n), (e3, n3), (e0, n0) = out[None], out["3"], out["0"]
+    assert n == n3 == n0
+    assert abs(e - e3) <= 1e-12 * abs(e3), out
+    assert abs(e - e0) <= 1e-12 * abs(e0), out
+
+
+def test_triples_after_a_new_interaction_and_fock(ccnm):
+    """The tables of a handle follow its interaction: (T) after a second
+    generation equals that of a fresh handle."""
+    def fresh(order):
+        s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1)
+        s.set_chiral(order, 450.0)
+        s.generate_interaction(ccnm.INT_CHIRAL)
+        s.setup_t_amplitudes()
+        return s
+    a = fresh(ccnm.NNLO)
+    first = a.pert_triples2()
+    a.set_chiral(ccnm.LO, 450.0)
+    a.generate_interaction(ccnm.INT_CHIRAL)
+    a.setup_t_amplitudes()
+    b = fresh(ccnm.LO)
+    assert a.pert_triples2() == b.pert_triples2()
+    assert abs(first - b.pert_triples2()) > 1e-6
