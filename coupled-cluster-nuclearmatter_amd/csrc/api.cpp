@@ -2997,17 +2997,16 @@ void build_triples(Solve &S) {
     }
     td.parity = ok ? 1 : 0;
   }
-  // the group tables, when they fit in CCGPU_T3_TABLE_GB (default 16 GB; the
-  // size of one entry per (c, b, k) and per (j, k, c) for both spins, which
-  // theirs is up to the diagonals of their triangles); otherwise (T) evaluates
-  // the elements in place
+  // the group tables, when one entry per (c, b, k) and per (j, k, c) for both
+  // spins would fit in CCGPU_T3_TABLE_GB (default 16 GB; the tables take about
+  // half of that); otherwise (T) evaluates the elements in place
   td.vhppp = nullptr;
   td.vhhhp = nullptr;
   const int64_t ntab = (int64_t)P.np * P.np * P.A * 2 + (int64_t)P.A * P.A * P.np * 2;
   if ((double)ntab * sizeof(double2) <= t3_table_limit() && P.np > 0) {
     if (!S.t3_gE) {
-      S.t3_gE = dalloc<double2>((size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 4, S.owned);
-      S.t3_gD = dalloc<double2>((size_t)td.npg * 2 * td.nhp * 4 * 4, S.owned);
+      S.t3_gE = dalloc<double2>((size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 2, S.owned);
+      S.t3_gD = dalloc<double2>((size_t)td.npg * 2 * td.nhp * 4 * 2, S.owned);
     }
     td.gE = S.t3_gE;
     td.gD = S.t3_gD;

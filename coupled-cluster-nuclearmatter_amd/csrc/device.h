@@ -135,13 +135,14 @@ struct TriplesDesc {
   const int *gptr;
   const T3Hole *gtrip;
   double2 *gf;
-  // Tables of the group kernel, 64-byte records of four elements:
-  //   gE[((pair(y, z) 4 + 2 ys + zs) nhg + S) 2 + ss]: conj <yz||s d> for both
-  //     spins of d, t(yz, s l) for both spins of l; pair(y, z) = y (y + 1) / 2 + z
-  //     over particle groups y >= z, S the hole group of s
-  //   gD[((x 2 + xs) nhp + pair(v, u)) 4 + 2 us + vs]: t(x d, u v), conj <uv||l x>
-  // The spin of d (l) is that of the orbital lookup; its momentum and isospin
-  // follow from conservation.  The t halves are refilled for every sum.
+  // Tables of the group kernel, 32-byte records of two elements, one per spin
+  // state w of the group whose momentum and isospin conservation leaves:
+  //   gE[((pair(y, z) 4 + 2 ys + zs) nhg + S) 2 + ss]: conj <yz||s w> where w is a
+  //     particle, t(yz, s w) where it is a hole; pair(y, z) = y (y + 1) / 2 + z over
+  //     particle groups y >= z, S the hole group of s
+  //   gD[((x 2 + xs) nhp + pair(v, u)) 4 + 2 us + vs]: t(x w, u v) where w is a
+  //     particle, conj <uv||w x> where it is a hole
+  // The amplitude entries are refilled for every sum.
   double2 *gE, *gD;
   // 1: the lattice maps onto itself under n -> -n with k -> -k exactly (no
   // twist) and holes onto holes, so <cb||kd> = <Pc Pb||Pk Pd> (the NN and 3NF

@@ -510,23 +510,29 @@ __global__ __launch_bounds__(256) void k_triples_s(SolveDesc d, TriplesDesc td, 
 //
 // Momentum conservation acts on groups (the two spin states of one momentum and
 // isospin), so a particle group triple and a hole group triple that conserve
-// it are 8 x 8 elements (abc, ijk) that share every index.  With
-//   E_a[s] = (conj <cb||s d-+>, t(cb, s l-+)),  E_b, E_c likewise with the pairs
-//            (c, a) and (b, a),
-//   D_x[uv] = (t(x d-+, u v), conj <uv||l-+ x>)
+// it are 8 x 8 elements (abc, ijk) that share every index.  The F and the H
+// term of a particle x and a hole pair uv sum over the states d and l of the
+// same momentum n_u + n_v - n_x: w, a particle in the F term and a hole in the H
+// term.  With
+//   E_a[s](w) = conj <cb||s w> (particle) or t(cb, s w) (hole); E_b, E_c likewise
+//               with the pairs (c, a) and (b, a),
+//   D_x[uv](w) = t(x w, u v) or conj <uv||w x>
 // the 18 signed F and H terms (pert_triples2, ccm_triples.f90:611-700) are
 //   W = sum over the splits (ij|k) - (ik|j) + (jk|i) of the three holes into
 //       pair uv and single s of  E_a[s].D_a[uv] - E_b[s].D_b[uv] + E_c[s].D_c[uv],
-// nine products of length four.  A lane takes one of the four components k and,
-// for one hole group triple and one (as, bs), all 16 (cs, is, js, ks): per split
-// 26 loads of 16 bytes, four lanes to a 64-byte record, for 192 FMAs, no index
-// arithmetic per element.  The four lanes then add up (each keeps four
-// elements).  One wave per particle group triple, four hole group triples at a
-// time.
+// nine products of length two.  A lane takes one w and, for one hole group
+// triple and one (as, bs), all 16 (cs, is, js, ks): per split 26 loads of 16
+// bytes, two lanes to a record, for 192 FMAs, no index arithmetic per element.
+// The two lanes then add up (each keeps eight elements).  A block takes a pair
+// of particle groups (a, b) and lists the (c, hole group triple) items of its
+// channels in LDS, eight items to a wave at a time, so no lane idles on a short
+// channel.
 //
-// Bound: the L1 (26 KB per 256 elements and split) and FP64 issue.  The kernel
-// it replaced gathered 36 x 32 bytes per element with a lookup for each: PNM
-// A=66 |n_i|<=3 (1.62e9 elements) 181 to 66 ms.
+// Bound: the L1's request rate (275 requests per 64 elements at 0.7 a clock and
+// CU, most for 32 bytes), then FP64 issue (6 of 16.7 ms).  The kernel before
+// gathered 36 x 16 bytes per element with a lookup for each: PNM A=66 |n_i|<=3
+// (1.62e9 elements) 181 to 16.7 ms; with the d and l terms kept apart (64-byte
+// records, one wave per particle group triple) it took 66 ms.
 //
 // With W3 = <abc||ijk> the antisymmetrized three-nucleon element
 // (chiral_3nf_asym) and D = f_i + f_j + f_k - f_a - f_b - f_c, the sum over
@@ -538,7 +544,7 @@ __global__ __launch_bounds__(256) void k_triples_s(SolveDesc d, TriplesDesc td, 
 //   MODE 2: |W3|^2 / D                CCDT-1 energy of the start T3 = W3/D
 //           (setup_t3, ccm_t3full_channels.f90:291-567)
 //   MODE 3: |W + W3|^2 / D            (T) at tnf_approx 3, et_5 (:656-722)
-// The four elements a lane keeps differ in js and ks only, so W3 takes its
+// The eight elements a lane keeps differ in is, js and ks only, so W3 takes its
 // geometry once for them.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int slot_of(int2 g, int s) { return s ? g.y : g.x; }
@@ -553,7 +559,7 @@ __device__ __forceinline__ void tri_yz(int64_t t, int &y, int &z) {
 }
 __device__ __forceinline__ int64_t tri_at(int64_t y, int64_t z) { return y * (y + 1) / 2 + z; }
 
-// an entry of gE: the orbitals of its record and the d (or l) of spin sd
+// an entry of gE: the orbitals of its record and the w of spin sd
 struct T3E {
   int y, z, s, ys, zs, ss, S, d;
   int64_t gp;
@@ -579,11 +585,11 @@ __device__ __forceinline__ T3E t3_e_entry(const SolveDesc &d, const TriplesDesc 
   return e;
 }
 
-// conj <yz||s d> of every record, both spins of d: once per interaction.  The
+// conj <yz||s w> of every record and particle w: once per interaction.  The
 // element is evaluated for the ascending orbital order of (y, z) and signed.
 // With no twist one of each parity pair (n -> -n) is evaluated and written to
 // both places.  A block lists the entries of its chunk that need evaluating
-// (half or more conserve momentum with no particle d) and evaluates the list
+// (half or more conserve momentum with no particle w) and evaluates the list
 // with full waves.
 template <bool ONE>
 __global__ __launch_bounds__(256) void k_t3_fill_ev(SolveDesc d, TriplesDesc td, double vol, int64_t nrec) {
@@ -606,8 +612,8 @@ __global__ __launch_bounds__(256) void k_t3_fill_ev(SolveDesc d, TriplesDesc td,
       const int64_t rec = (base + t) >> 1;
       const int sd = t & 1;
       const T3E e = t3_e_entry(d, td, rec, sd);
-      if (e.d < d.A) {
-        td.gE[4 * rec + sd] = make_double2(0.0, 0.0);
+      if (e.d < d.A) {   // a hole's entry is the amplitude's
+        if (e.d < 0) td.gE[2 * rec + sd] = make_double2(0.0, 0.0);
         continue;
       }
       if (td.parity) {
@@ -635,32 +641,33 @@ __global__ __launch_bounds__(256) void k_t3_fill_ev(SolveDesc d, TriplesDesc td,
       }
       const double s1 = e.y < e.z ? 1.0 : -1.0;
       v = make_double2(s1 * v.x, -s1 * v.y);   // conjugated
-      td.gE[4 * rec + sd] = v;
+      td.gE[2 * rec + sd] = v;
       if (td.parity) {
         int64_t ir;
         double sg;
         image(e, ir, sg);
         const int64_t igp = ir / ((int64_t)8 * td.nhg);
         const int iS = (int)((ir >> 1) % td.nhg);
-        if (igp != e.gp || iS != e.S) td.gE[4 * ir + sd] = make_double2(sg * v.x, sg * v.y);
+        if (igp != e.gp || iS != e.S) td.gE[2 * ir + sd] = make_double2(sg * v.x, sg * v.y);
       }
     }
     __syncthreads();
   }
 }
 
-// t(yz, s l) of every record, both spins of the hole l
+// t(yz, s w) of every record and hole w
 __global__ __launch_bounds__(256) void k_t3_fill_et(SolveDesc d, TriplesDesc td, int64_t nrec) {
   for (int64_t rec = (int64_t)blockIdx.x * 256 + threadIdx.x; rec < nrec; rec += (int64_t)gridDim.x * 256) {
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
       const T3E e = t3_e_entry(d, td, rec, sl);
-      td.gE[4 * rec + 2 + sl] = e.d >= 0 && e.d < d.A ? t_of(d, e.y, e.z, e.s, e.d) : make_double2(0.0, 0.0);
+      if (e.d >= 0 && e.d < d.A) td.gE[2 * rec + sl] = t_of(d, e.y, e.z, e.s, e.d);
     }
   }
 }
 
-// gD: T false conj <uv||l x> (once per interaction), true t(x d, u v)
+// gD: T false conj <uv||w x> of the holes w (once per interaction; zero where
+// there is no w), true t(x w, u v) of the particles w
 template <bool T>
 __global__ __launch_bounds__(256) void k_t3_fill_d(SolveDesc d, TriplesDesc td, double vol, int64_t nrec) {
   for (int64_t rec = (int64_t)blockIdx.x * 256 + threadIdx.x; rec < nrec; rec += (int64_t)gridDim.x * 256) {
@@ -672,17 +679,20 @@ __global__ __launch_bounds__(256) void k_t3_fill_d(SolveDesc d, TriplesDesc td, 
     const int x = slot_of(td.pg[gx >> 1], gx & 1), u = slot_of(td.hg[gu], us), v = slot_of(td.hg[gv], vs);
 #pragma unroll
     for (int sp = 0; sp < 2; ++sp) {
-      double2 o = make_double2(0.0, 0.0);
-      if (x >= 0 && u >= 0 && v >= 0 && u != v) {
-        const int w = orb_lookup(td, d.nx[u] + d.nx[v] - d.nx[x], d.ny[u] + d.ny[v] - d.ny[x],
-                                 d.nz[u] + d.nz[v] - d.nz[x], 2 * sp - 1, d.tz[u] + d.tz[v] - d.tz[x]);
-        if (T && w >= d.A) o = t_of(d, x, w, u, v);
-        if (!T && w >= 0 && w < d.A) {
+      int w = -1;
+      if (x >= 0 && u >= 0 && v >= 0 && u != v)
+        w = orb_lookup(td, d.nx[u] + d.nx[v] - d.nx[x], d.ny[u] + d.ny[v] - d.ny[x],
+                       d.nz[u] + d.nz[v] - d.nz[x], 2 * sp - 1, d.tz[u] + d.tz[v] - d.tz[x]);
+      if (T) {
+        if (w >= d.A) td.gD[2 * rec + sp] = t_of(d, x, w, u, v);
+      } else if (w < d.A) {
+        double2 o = make_double2(0.0, 0.0);
+        if (w >= 0) {
           o = vas_t(d, td, vol, u, v, w, x);
           o.y = -o.y;
         }
+        td.gD[2 * rec + sp] = o;
       }
-      td.gD[4 * rec + (T ? 0 : 2) + sp] = o;
     }
   }
 }
@@ -722,18 +732,18 @@ __device__ __forceinline__ void t3_split(double2 (&acc)[16], const double2 *Da, 
   double2 da[4], db[4], dc[2][4], ea[2][2], eb[2][2], ec[2];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    da[q] = Da[4 * q];
-    db[q] = Db[4 * q];
-    dc[0][q] = Dc0[4 * q];
-    dc[1][q] = Dc1[4 * q];
+    da[q] = Da[2 * q];
+    db[q] = Db[2 * q];
+    dc[0][q] = Dc0[2 * q];
+    dc[1][q] = Dc1[2 * q];
   }
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    ea[0][s] = Ea0[4 * s];
-    ea[1][s] = Ea1[4 * s];
-    eb[0][s] = Eb0[4 * s];
-    eb[1][s] = Eb1[4 * s];
-    ec[s] = Ec[4 * s];
+    ea[0][s] = Ea0[2 * s];
+    ea[1][s] = Ea1[2 * s];
+    eb[0][s] = Eb0[2 * s];
+    eb[1][s] = Eb1[2 * s];
+    ec[s] = Ec[2 * s];
   }
 #pragma unroll
   for (int cs = 0; cs < 2; ++cs)
@@ -757,173 +767,205 @@ __device__ __forceinline__ void t3_split(double2 (&acc)[16], const double2 *Da, 
         }
 }
 
-// value of the lane 1 (CTRL 0xB1) or 2 (0x4E) away within a group of four
-template <int CTRL>
-__device__ __forceinline__ double quad_swap(double x) {
+// value of the neighbouring lane (lane ^ 1)
+__device__ __forceinline__ double pair_swap(double x) {
   const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+constexpr int kT3Items = 2048;
+
+// Order of the pairs (a, b) of particle groups, a <= b: tiles of 2 a by 4 b, a
+// tile at a time to the blocks that an XCD runs together (workgroup i runs on
+// XCD i mod 8), so that they share rows of the tables: (T) of PNM A=66
+// |n_i|<=3 25.6 to 16.7 ms (tiles of 4 x 8 the same, 8 x 16 18.0 ms and slower on
+// smaller lattices).  Tile t holds b in [4 tb, 4 tb + 4) and a in [2 ta, 2 ta +
+// 2), t = tb (tb + 1) + ta.
+constexpr int kTileA = 2, kTileB = 4, kTile = kTileA * kTileB;
+__host__ __device__ inline int64_t t3_tile_ids(int npg) {   // virtual block indices, a multiple of 8
+  const int64_t nb = (npg + kTileB - 1) / kTileB;
+  return (nb * (nb + 1) + 7) / 8 * 8 * kTile;
+}
+__device__ __forceinline__ bool t3_tile_pair(int64_t v, int npg, int &ga, int &gb) {
+  const int64_t s = v >> 3;
+  const int64_t t = s / kTile * 8 + (v & 7);
+  const int p = (int)(s % kTile);
+  int64_t tb = (int64_t)((sqrt(4.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while (tb * (tb + 1) > t) --tb;
+  while ((tb + 1) * (tb + 2) <= t) ++tb;
+  gb = (int)tb * kTileB + p / kTileA;
+  ga = (int)(t - tb * (tb + 1)) * kTileA + p % kTileA;
+  return gb < npg && ga <= gb;
+}
+constexpr int t3_threads(int mode) { return mode == 0 ? 512 : 256; }   // W3 takes twice the registers
+
 template <int MODE, bool ONE>
-__global__ __launch_bounds__(256) void k_triples_g(SolveDesc d, TriplesDesc td, double2 *partial,
-                                                   unsigned long long *count) {
-  __shared__ double sre[4], sim[4];
-  __shared__ unsigned long long scnt[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kk = lane & 3, as = (lane >> 2) & 1, bs = (lane >> 3) & 1, hq = lane >> 4;
-  const int cs_f = kk & 1, is_f = kk >> 1;   // of the four elements this lane finishes
+__global__ __launch_bounds__(t3_threads(MODE), 2) void k_triples_g(SolveDesc d, TriplesDesc td, double2 *partial,
+                                                          unsigned long long *count) {
+  constexpr int kT3Threads = t3_threads(MODE), kT3Waves = kT3Threads / 64;
+  __shared__ int ic[kT3Items], ig[kT3Items];   // items: particle group c, hole group triple
+  __shared__ int wsum[kT3Waves];
+  __shared__ double sre[kT3Waves], sim[kT3Waves];
+  __shared__ unsigned long long scnt[kT3Waves];
+  __shared__ double2 stash[MODE == 0 || MODE == 2 ? 1 : 8][MODE == 0 || MODE == 2 ? 1 : kT3Threads];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kk = lane & 1, as = (lane >> 1) & 1, bs = (lane >> 2) & 1, hq = lane >> 3;
   double re = 0.0, im = 0.0;
   unsigned long long nel = 0;
-  const int64_t npair = tri_at(td.npg, 0);
-  const int64_t erow = (int64_t)td.nhg * 8, drow = (int64_t)td.nhp * 16;   // double2 per (pair, ys, zs) and per x
-  for (int64_t pr = blockIdx.x; pr < npair; pr += gridDim.x) {
+  const int64_t nid = t3_tile_ids(td.npg);
+  const int64_t erow = (int64_t)td.nhg * 4, drow = (int64_t)td.nhp * 8;   // double2 per (pair, ys, zs) and per x
+  for (int64_t id = blockIdx.x; id < nid; id += gridDim.x) {
     int gb, ga;
-    tri_yz(pr, gb, ga);
+    if (!t3_tile_pair(id, td.npg, ga, gb)) continue;
     const int a = slot_of(td.pg[ga], as), b = slot_of(td.pg[gb], bs);
     const int4 ma = td.pgn[ga], mb_ = td.pgn[gb];
     const bool ab_ok = a >= 0 && b >= 0 && (ga != gb || (as == 0 && bs == 1));
-    for (int gc = gb + wave; gc < td.npg; gc += 4) {
-      if (gc == ga) continue;   // three particles in two states
-      const int4 mc = td.pgn[gc];
-      const int ix = ma.x + mb_.x + mc.x - td.k0, iy = ma.y + mb_.y + mc.y - td.k0, iz = ma.z + mb_.z + mc.z - td.k0;
-      const int it = ma.w + mb_.w + mc.w - td.tz0;
-      if (ix < 0 || iy < 0 || iz < 0 || ix >= td.nk || iy >= td.nk || iz >= td.nk || it < 0 || it >= td.ntz) continue;
-      const int ch = td.chan[((it * td.nk + ix) * td.nk + iy) * td.nk + iz];
-      if (ch < 0) continue;
-      const int g0 = td.gptr[ch], g1 = td.gptr[ch + 1];
-      const int2 pc = td.pg[gc];
-      const bool v0 = ab_ok && pc.x >= 0 && gb != gc, v1 = ab_ok && pc.y >= 0 && (gb != gc || bs == 0);
-      const bool pv = cs_f ? v1 : v0;
-      const int c = slot_of(pc, cs_f);
-      double2 fabc = make_double2(0.0, 0.0);
-      if (pv) {
-        fabc.x = d.fdiag[a].x + d.fdiag[b].x + d.fdiag[c].x;
-        fabc.y = d.fdiag[a].y + d.fdiag[b].y + d.fdiag[c].y;
-      }
-      const double2 *Ea0 = nullptr, *Ea1 = nullptr, *Eb0 = nullptr, *Eb1 = nullptr, *Ec = nullptr;
-      const double2 *Da = nullptr, *Db = nullptr, *Dc0 = nullptr, *Dc1 = nullptr;
-      if constexpr (MODE != 2) {
-        Ea0 = td.gE + (tri_at(gc, gb) * 4 + bs) * erow + kk;
-        Ea1 = Ea0 + 2 * erow;
-        Eb0 = td.gE + (tri_at(gc, ga) * 4 + as) * erow + kk;
-        Eb1 = Eb0 + 2 * erow;
-        Ec = td.gE + (tri_at(gb, ga) * 4 + 2 * bs + as) * erow + kk;
-        Da = td.gD + (int64_t)(2 * ga + as) * drow + kk;
-        Db = td.gD + (int64_t)(2 * gb + bs) * drow + kk;
-        Dc0 = td.gD + (int64_t)(2 * gc) * drow + kk;
-        Dc1 = Dc0 + drow;
-      }
-      Nucleon na{}, nb{}, nc{};
-      double fbra = 0.0;
-      if constexpr (MODE != 0) {
-        auto rep = [&](int2 g) { return nucleon_of(td.c3w, g.x >= 0 ? g.x : g.y); };
-        na = rep(td.pg[ga]);
-        nb = rep(td.pg[gb]);
-        nc = rep(pc);
-        fbra = freg3(td.c3w, na.k, nb.k, nc.k);
-      }
-      for (int gg = g0; gg < g1; gg += 4) {
-        const int g = min(gg + hq, g1 - 1);
-        const T3Hole t = td.gtrip[g];
-        const bool ok = gg + hq < g1 && pv;
-        double2 w[4];
-        if constexpr (MODE != 2) {
-          double2 acc[16];
-#pragma unroll
-          for (int o = 0; o < 16; ++o) acc[o] = make_double2(0.0, 0.0);
-          t3_split<0>(acc, Da + 16 * t.hij, Db + 16 * t.hij, Dc0 + 16 * t.hij, Dc1 + 16 * t.hij, Ea0 + 8 * t.K,
-                      Ea1 + 8 * t.K, Eb0 + 8 * t.K, Eb1 + 8 * t.K, Ec + 8 * t.K);
-          t3_split<1>(acc, Da + 16 * t.hik, Db + 16 * t.hik, Dc0 + 16 * t.hik, Dc1 + 16 * t.hik, Ea0 + 8 * t.J,
-                      Ea1 + 8 * t.J, Eb0 + 8 * t.J, Eb1 + 8 * t.J, Ec + 8 * t.J);
-          t3_split<2>(acc, Da + 16 * t.hjk, Db + 16 * t.hjk, Dc0 + 16 * t.hjk, Dc1 + 16 * t.hjk, Ea0 + 8 * t.I,
-                      Ea1 + 8 * t.I, Eb0 + 8 * t.I, Eb1 + 8 * t.I, Ec + 8 * t.I);
-          // sum over the four components: lane kk keeps cs = kk & 1, then is = kk >> 1
-          double2 h[8];
-#pragma unroll
-          for (int o = 0; o < 8; ++o) {
-            const double2 x = cs_f ? acc[o] : acc[8 + o], y = cs_f ? acc[8 + o] : acc[o];
-            h[o] = make_double2(y.x + quad_swap<0xB1>(x.x), y.y + quad_swap<0xB1>(x.y));
-          }
-#pragma unroll
-          for (int o = 0; o < 4; ++o) {
-            const double2 x = is_f ? h[o] : h[4 + o], y = is_f ? h[4 + o] : h[o];
-            w[o] = make_double2(y.x + quad_swap<0x4E>(x.x), y.y + quad_swap<0x4E>(x.y));
+    const double2 *Ec = nullptr, *Da = nullptr, *Db = nullptr;
+    if constexpr (MODE != 2) {
+      Ec = td.gE + (tri_at(gb, ga) * 4 + 2 * bs + as) * erow + kk;
+      Da = td.gD + (int64_t)(2 * ga + as) * drow + kk;
+      Db = td.gD + (int64_t)(2 * gb + bs) * drow + kk;
+    }
+    for (int c0 = gb; c0 < td.npg; c0 += kT3Threads) {
+      // items of this thread's c: the hole group triples of its channel
+      int n = 0, g0 = 0;
+      const int myc = c0 + tid;
+      if (myc < td.npg && myc != ga) {   // three particles do not fit in two states
+        const int4 mc = td.pgn[myc];
+        const int ix = ma.x + mb_.x + mc.x - td.k0, iy = ma.y + mb_.y + mc.y - td.k0, iz = ma.z + mb_.z + mc.z - td.k0;
+        const int it = ma.w + mb_.w + mc.w - td.tz0;
+        if (ix >= 0 && iy >= 0 && iz >= 0 && ix < td.nk && iy < td.nk && iz < td.nk && it >= 0 && it < td.ntz) {
+          const int ch = td.chan[((it * td.nk + ix) * td.nk + iy) * td.nk + iz];
+          if (ch >= 0) {
+            g0 = td.gptr[ch];
+            n = td.gptr[ch + 1] - g0;
           }
         }
-        const int m4 = ok ? (t.mask >> (4 * is_f)) & 15 : 0;
-        nel += (unsigned long long)__popc(m4);
-        Geo3 geo;
-        int ks0 = 0, ks1 = 0, ks2 = 0, kt0 = 0, kt1 = 0, kt2 = 0;   // hole spins per state (bit s), isospins
-        if constexpr (MODE != 0) {
-          auto rep = [&](int2 q) { return nucleon_of(td.c3w, q.x >= 0 ? q.x : q.y); };
-          const Nucleon ni = rep(td.hg[t.I]), nj = rep(td.hg[t.J]), nk = rep(td.hg[t.K]);
-          geo3_transfer<0, 0>(td.c3w, geo, na, ni);
-          geo3_transfer<0, 1>(td.c3w, geo, na, nj);
-          geo3_transfer<0, 2>(td.c3w, geo, na, nk);
-          geo3_transfer<1, 0>(td.c3w, geo, nb, ni);
-          geo3_transfer<1, 1>(td.c3w, geo, nb, nj);
-          geo3_transfer<1, 2>(td.c3w, geo, nb, nk);
-          geo3_transfer<2, 0>(td.c3w, geo, nc, ni);
-          geo3_transfer<2, 1>(td.c3w, geo, nc, nj);
-          geo3_transfer<2, 2>(td.c3w, geo, nc, nk);
-          const double f = fbra * td.c3w.scale;
-          geo.f[0] = f * freg3(td.c3w, nj.k, nk.k, ni.k);
-          geo.f[1] = f * freg3(td.c3w, ni.k, nk.k, nj.k);
-          geo.f[2] = f * freg3(td.c3w, ni.k, nj.k, nk.k);
-          auto up = [&](int2 q) {
-            return (q.x >= 0 && d.sz[q.x] > 0 ? 1 : 0) | (q.y >= 0 && d.sz[q.y] > 0 ? 2 : 0);
-          };
-          ks0 = up(td.hg[t.I]);
-          ks1 = up(td.hg[t.J]);
-          ks2 = up(td.hg[t.K]);
-          kt0 = ni.tz;
-          kt1 = nj.tz;
-          kt2 = nk.tz;
+      }
+      int pos = n;   // inclusive scan over the block
+      for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(pos, off);
+        if (lane >= off) pos += x;
+      }
+      if (lane == 63) wsum[wave] = pos;
+      __syncthreads();
+      int total = 0;
+      for (int w = 0; w < kT3Waves; ++w) {
+        if (w < wave) pos += wsum[w];
+        total += wsum[w];
+      }
+      pos -= n;
+      for (int i0 = 0; i0 < total; i0 += kT3Items) {
+        __syncthreads();   // the items before are done
+        for (int q = max(0, i0 - pos); q < n && pos + q < i0 + kT3Items; ++q) {
+          ic[pos + q - i0] = myc;
+          ig[pos + q - i0] = g0 + q;
         }
-        auto finish = [&](int o, double2 wo) {
-          const double2 fh = td.gf[8 * (int64_t)g + 4 * is_f + o];
-          const double dre = fh.x - fabc.x, dim = fh.y - fabc.y;
-          const double inv = 1.0 / (dre * dre + dim * dim);
-          double nre, nim = 0.0;
-          if constexpr (MODE == 0) {
-            nre = wo.x * wo.x + wo.y * wo.y;
-          } else {
-            auto sp = [](int bits, int s) { return (bits >> s) & 1 ? 1 : -1; };
-            const int mb[3] = {d.sz[a], d.sz[b], d.sz[c]}, tb[3] = {na.tz, nb.tz, nc.tz};
-            const int mk[3] = {sp(ks0, is_f), sp(ks1, o >> 1), sp(ks2, o & 1)}, tk[3] = {kt0, kt1, kt2};
-            const double2 w3 = asym3<ONE, false>(td.c3w, geo, mb, mk, tb, tk);
-            if constexpr (MODE == 1) {
-              const double xr = w3.x + wo.x, xi = w3.y + wo.y;
-              nre = xr * w3.x + xi * w3.y;
-              nim = xi * w3.x - xr * w3.y;
-            } else if constexpr (MODE == 2) {
-              nre = w3.x * w3.x + w3.y * w3.y;
-            } else {
-              const double xr = w3.x + wo.x, xi = w3.y + wo.y;
-              nre = xr * xr + xi * xi;
+        __syncthreads();
+        const int m = min(kT3Items, total - i0);
+        for (int q0 = 8 * wave; q0 < m; q0 += 8 * kT3Waves) {
+          const int q = min(q0 + hq, m - 1);
+          const int gc = ic[q], g = ig[q];
+          const T3Hole t = td.gtrip[g];
+          const int2 pc = td.pg[gc];
+          // this lane finishes cs = kk
+          const int c = kk ? pc.y : pc.x;
+          const bool ok = q0 + hq < m && ab_ok && c >= 0 && (gb != gc || (kk == 1 && bs == 0));
+          double2 w[8];
+          if constexpr (MODE != 2) {
+            const double2 *Ea0 = td.gE + (tri_at(gc, gb) * 4 + bs) * erow + kk, *Ea1 = Ea0 + 2 * erow;
+            const double2 *Eb0 = td.gE + (tri_at(gc, ga) * 4 + as) * erow + kk, *Eb1 = Eb0 + 2 * erow;
+            const double2 *Dc0 = td.gD + (int64_t)(2 * gc) * drow + kk, *Dc1 = Dc0 + drow;
+            double2 acc[16];
+#pragma unroll
+            for (int o = 0; o < 16; ++o) acc[o] = make_double2(0.0, 0.0);
+            t3_split<0>(acc, Da + 8 * t.hij, Db + 8 * t.hij, Dc0 + 8 * t.hij, Dc1 + 8 * t.hij, Ea0 + 4 * t.K,
+                        Ea1 + 4 * t.K, Eb0 + 4 * t.K, Eb1 + 4 * t.K, Ec + 4 * t.K);
+            t3_split<1>(acc, Da + 8 * t.hik, Db + 8 * t.hik, Dc0 + 8 * t.hik, Dc1 + 8 * t.hik, Ea0 + 4 * t.J,
+                        Ea1 + 4 * t.J, Eb0 + 4 * t.J, Eb1 + 4 * t.J, Ec + 4 * t.J);
+            t3_split<2>(acc, Da + 8 * t.hjk, Db + 8 * t.hjk, Dc0 + 8 * t.hjk, Dc1 + 8 * t.hjk, Ea0 + 4 * t.I,
+                        Ea1 + 4 * t.I, Eb0 + 4 * t.I, Eb1 + 4 * t.I, Ec + 4 * t.I);
+            // sum over the two w: lane kk keeps cs = kk
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+              const double2 x = kk ? acc[o] : acc[8 + o], y = kk ? acc[8 + o] : acc[o];
+              w[o] = make_double2(y.x + pair_swap(x.x), y.y + pair_swap(x.y));
+              if constexpr (MODE != 0) stash[o][tid] = w[o];
             }
           }
-          re += (nre * dre + nim * dim) * inv;
-          im += (nim * dre - nre * dim) * inv;
-        };
-        if constexpr (MODE == 0) {
+          if (!ok) continue;
+          nel += (unsigned long long)__popc(t.mask);
+          const double2 fabc = make_double2(d.fdiag[a].x + d.fdiag[b].x + d.fdiag[c].x,
+                                            d.fdiag[a].y + d.fdiag[b].y + d.fdiag[c].y);
+          auto finish = [&](int o, double nre, double nim) {
+            const double2 fh = td.gf[8 * (int64_t)g + o];
+            const double dre = fh.x - fabc.x, dim = fh.y - fabc.y;
+            const double inv = 1.0 / (dre * dre + dim * dim);
+            re += (nre * dre + nim * dim) * inv;
+            im += (nim * dre - nre * dim) * inv;
+          };
+          if constexpr (MODE == 0) {
 #pragma unroll
-          for (int o = 0; o < 4; ++o)
-            if ((m4 >> o) & 1) finish(o, w[o]);
-        } else {
+            for (int o = 0; o < 8; ++o)
+              if ((t.mask >> o) & 1) finish(o, w[o].x * w[o].x + w[o].y * w[o].y, 0.0);
+          } else {
+            auto rep = [&](int2 s) { return nucleon_of(td.c3w, s.x >= 0 ? s.x : s.y); };
+            const int2 hi = td.hg[t.I], hj = td.hg[t.J], hk = td.hg[t.K];
+            const Nucleon ni = rep(hi), nj = rep(hj), nk = rep(hk);
+            const Nucleon na = nucleon_of(td.c3w, a), nb = nucleon_of(td.c3w, b), nc = nucleon_of(td.c3w, c);
+            Geo3 geo;
+            geo3_transfer<0, 0>(td.c3w, geo, na, ni);
+            geo3_transfer<0, 1>(td.c3w, geo, na, nj);
+            geo3_transfer<0, 2>(td.c3w, geo, na, nk);
+            geo3_transfer<1, 0>(td.c3w, geo, nb, ni);
+            geo3_transfer<1, 1>(td.c3w, geo, nb, nj);
+            geo3_transfer<1, 2>(td.c3w, geo, nb, nk);
+            geo3_transfer<2, 0>(td.c3w, geo, nc, ni);
+            geo3_transfer<2, 1>(td.c3w, geo, nc, nj);
+            geo3_transfer<2, 2>(td.c3w, geo, nc, nk);
+            const double f = freg3(td.c3w, na.k, nb.k, nc.k) * td.c3w.scale;
+            geo.f[0] = f * freg3(td.c3w, nj.k, nk.k, ni.k);
+            geo.f[1] = f * freg3(td.c3w, ni.k, nk.k, nj.k);
+            geo.f[2] = f * freg3(td.c3w, ni.k, nj.k, nk.k);
+            auto up = [&](int2 s) {   // bit s: the state's spin is up
+              return (s.x >= 0 && d.sz[s.x] > 0 ? 1 : 0) | (s.y >= 0 && d.sz[s.y] > 0 ? 2 : 0);
+            };
+            const int ui = up(hi), uj = up(hj), uk = up(hk);
+            const int mb[3] = {na.sz, nb.sz, nc.sz}, tb[3] = {na.tz, nb.tz, nc.tz}, tk[3] = {ni.tz, nj.tz, nk.tz};
 #pragma unroll 1
-          for (int o = 0; o < 4; ++o) {
-            double2 wo = make_double2(0.0, 0.0);
-            if constexpr (MODE != 2) wo = o == 0 ? w[0] : o == 1 ? w[1] : o == 2 ? w[2] : w[3];
-            if ((m4 >> o) & 1) finish(o, wo);
+            for (int o = 0; o < 8; ++o) {
+              if (!((t.mask >> o) & 1)) continue;
+              // the geometry changes for all the compiler knows: what asym3
+              // derives from it stays inside the loop (hoisted, it spills)
+#pragma unroll
+              for (int x = 0; x < 3; ++x)
+#pragma unroll
+                for (int y = 0; y < 3; ++y) {
+                  asm volatile("" : "+v"(geo.w[x][y]));
+#pragma unroll
+                  for (int z = 0; z < 3; ++z) asm volatile("" : "+v"(geo.q[x][y][z]));
+                }
+              const int mk[3] = {2 * ((ui >> (o >> 2)) & 1) - 1, 2 * ((uj >> ((o >> 1) & 1)) & 1) - 1,
+                                 2 * ((uk >> (o & 1)) & 1) - 1};
+              const double2 w3 = asym3<ONE, false>(td.c3w, geo, mb, mk, tb, tk);
+              if constexpr (MODE == 2) {
+                finish(o, w3.x * w3.x + w3.y * w3.y, 0.0);
+              } else {
+                const double2 wo = stash[o][tid];
+                const double xr = w3.x + wo.x, xi = w3.y + wo.y;
+                if constexpr (MODE == 1) finish(o, xr * w3.x + xi * w3.y, xi * w3.x - xr * w3.y);
+                else finish(o, xr * xr + xi * xi, 0.0);
+              }
+            }
           }
         }
       }
+      __syncthreads();   // wsum and the items
     }
   }
-  // fixed-order sums: butterfly in the wave, then the four waves
+  // fixed-order sums: butterfly in the wave, then the waves
   for (int off = 32; off > 0; off >>= 1) {
     re += __shfl_xor(re, off);
     im += __shfl_xor(im, off);
@@ -935,9 +977,14 @@ __global__ __launch_bounds__(256) void k_triples_g(SolveDesc d, TriplesDesc td, 
     scnt[wave] = nel;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    partial[blockIdx.x] = make_double2(((sre[0] + sre[1]) + sre[2]) + sre[3], ((sim[0] + sim[1]) + sim[2]) + sim[3]);
-    count[blockIdx.x] = scnt[0] + scnt[1] + scnt[2] + scnt[3];
+  if (tid == 0) {
+    for (int w = 1; w < kT3Waves; ++w) {
+      sre[0] += sre[w];
+      sim[0] += sim[w];
+      scnt[0] += scnt[w];
+    }
+    partial[blockIdx.x] = make_double2(sre[0], sim[0]);
+    count[blockIdx.x] = scnt[0];
   }
 }
 
@@ -1015,9 +1062,11 @@ void launch_triples_group(const SolveDesc &d, const TriplesDesc &td, double2 *pa
   if (td.ngtrip > 0)
     hipLaunchKernelGGL(k_t3_fill_gf, dim3((8 * td.ngtrip + 255) / 256), dim3(256), 0, st, d, td);
   const bool one = td.c3w.one_species != 0;
-  const int64_t npair = (int64_t)td.npg * (td.npg + 1) / 2;
-  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(npair, nblocks));
-  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, st, d, td, partial, count); };
+  // nblocks is a multiple of 8: a block's later pairs stay on its XCD
+  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(t3_tile_ids(td.npg), nblocks));
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(t3_threads(mode)), 0, st, d, td, partial, count);
+  };
   if (mode == 0) run(k_triples_g<0, true>);
   else if (mode == 1) run(one ? k_triples_g<1, true> : k_triples_g<1, false>);
   else if (mode == 2) run(one ? k_triples_g<2, true> : k_triples_g<2, false>);
