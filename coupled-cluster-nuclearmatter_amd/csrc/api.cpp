@@ -66,6 +66,11 @@ void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *
                       int nvec, hipStream_t st);
 void launch_gemm_shape(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const SolveDesc *dd,
                        const int *gsolve, int kind, int mb, int nb, int lb, hipStream_t st);
+int ring64_class(int nph, int nhp);
+int ring64_columns(int cls);
+void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *dd, hipStream_t st);
+void launch_x64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
+void launch_hh64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
 void launch_gemm_valu(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const SolveDesc *dd,
                       const int *gsolve, hipStream_t st);
 void launch_splitk_reduce(const GemmGroup *groups, const int *gidx, int n, int64_t maxmn, const SolveDesc *dd,
@@ -148,15 +153,19 @@ T *dupload(const std::vector<T> &v, std::vector<void *> &owned) {
 // Tiles reordered so that each channel's tiles go to one XCD (workgroup i runs
 // on XCD i mod 8, which keeps the channel's B operand in that XCD's L2) and the
 // XCDs get equal tile counts.
-void xcd_order_list(std::vector<GemmTile> &tiles, size_t ngroups) {
+double tile_cost(const GemmTile &t) { return (double)(t.ke - t.kb); }   // a tile's time goes with its k range
+double tile_cost(const ZTile &t) { return t.cost; }
+double tile_cost(const RingTile &t) { return t.cost; }
+template <typename Tile>
+void xcd_order_list(std::vector<Tile> &tiles, size_t ngroups) {
   const int nx = 8;
-  std::vector<std::vector<GemmTile>> bins(nx);
+  std::vector<std::vector<Tile>> bins(nx);
   std::vector<double> load(nx, 0.0);
-  std::vector<std::vector<GemmTile>> per(ngroups);
+  std::vector<std::vector<Tile>> per(ngroups);
   std::vector<double> cost(ngroups, 0.0);
   for (auto &t : tiles) {
     per[t.g].push_back(t);
-    cost[t.g] += (double)(t.ke - t.kb);   // a tile's time goes with its k range
+    cost[t.g] += tile_cost(t);
   }
   // groups largest first onto the least-loaded XCD: the longest tiles start
   // first and the tail of the launch is made of short ones
@@ -169,7 +178,7 @@ void xcd_order_list(std::vector<GemmTile> &tiles, size_t ngroups) {
     for (auto &t : per[g]) bins[best].push_back(t);
     load[best] += cost[g];
   }
-  std::vector<GemmTile> out;
+  std::vector<Tile> out;
   size_t maxlen = 0;
   for (auto &b : bins) maxlen = std::max(maxlen, b.size());
   for (size_t r = 0; r < maxlen; ++r)
@@ -673,6 +682,16 @@ struct Batch {
   GemmList g_xb, g_hhb, g_i4b, g_rtb;   // the same groups for the BF16x3 kernel
   GemmList g_i4f, g_rtf;   // BF16x3 ring GEMMs on the FP32 ring blocks (when every solve has them)
   bool ring32 = false;
+  // FP64 tiles of the X, hh and ring contractions (contract.hip); channels too
+  // large for the fused ring keep the list kernels (g_i4big, g_rtbig)
+  struct Fp64 {
+    bool ready = false;
+    int nx = 0, nhh = 0, nring[3] = {0, 0, 0};
+    ZTile *x = nullptr, *hh = nullptr;
+    RingTile *ring[3] = {nullptr, nullptr, nullptr};
+  } f64;
+  GemmList g_i4big, g_rtbig;
+  bool i4_in_lds = false;   // the last ring was the fused one, which keeps I4 in LDS
   GemmList g_ppbf;         // BF16x3 pp ladder reading the split copy of T (when every solve has one)
   bool ppbf = false;
   // Shared pp ladder of a batch of twists of one lattice and interaction: the
@@ -920,6 +939,7 @@ void autotune(GemmList &L, int kind, const SolveDesc *d_descs, hipStream_t st) {
   g_tune_report += rep;
 }
 
+int tail_low_mask();
 bool share_enabled();
 bool share_eligible(const std::vector<Solve *> &ss);
 void build_shared(Batch &B);
@@ -1030,6 +1050,17 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
     to32(B->g_i4f);
     to32(B->g_rtf);
   }
+  // ring groups of the channels the fused FP64 kernel does not take
+  for (size_t g = 0; g < B->g_i4.groups.size(); ++g) {
+    const GemmGroup &q = B->g_i4.groups[g];
+    if (ring64_class(q.K, q.M) >= 0) continue;
+    B->g_i4big.groups.push_back(q);
+    B->g_i4big.gsolve.push_back(B->g_i4.gsolve[g]);
+    B->g_rtbig.groups.push_back(B->g_rt.groups[g]);
+    B->g_rtbig.gsolve.push_back(B->g_rt.gsolve[g]);
+  }
+  B->g_i4big.fam = 3;
+  B->g_rtbig.fam = 4;
   const int fams[13] = {0, 1, 2, 3, 4, 1, 0, 2, 3, 4, 3, 4, 1};
   GemmList *lists[13] = {&B->g_x, &B->g_pp, &B->g_hh, &B->g_i4, &B->g_rt, &B->g_pp32,
                          &B->g_xb, &B->g_hhb, &B->g_i4b, &B->g_rtb, &B->g_i4f, &B->g_rtf, &B->g_ppbf};
@@ -1276,13 +1307,76 @@ void refresh_shared(Batch &B) {
 // prec needs, made on first use (outside any graph capture): lists a batch
 // never contracts (a single-solve batch used only for its MBPT2 start or
 // energy, the FP32 ladder of an FP64 solve) are never tuned.
+// The FP64 contractions run on the tiles of contract.hip unless a study or test
+// asks for forms of the list kernels.
+bool fp64_tiles() {
+  return !getenv("CCGPU_SHAPES") && gemm_variant_override() < 0 && !getenv("CCGPU_SPLIT_TILES") &&
+         !getenv("CCGPU_SPLIT_K");
+}
+
+void prepare_fp64(Batch &B) {
+  Batch::Fp64 &F = B.f64;
+  if (F.ready) return;
+  std::vector<ZTile> x, hh;
+  std::vector<RingTile> ring[3];
+  int gx = 0, gr = 0;
+  for (size_t s = 0; s < B.solves.size(); ++s) {
+    const Plan &P = B.solves[s]->plan;
+    const SolveDesc &d = B.h_descs[s];
+    for (int c = 0; c < P.nch; ++c, ++gx) {
+      const int np_ = P.npp[c], nh = P.nhh[c];
+      double2 *X = d.X + P.off_vhh[c], *I9 = d.X + P.nVhh + P.off_vhh[c];
+      for (int n0 = 0; n0 < nh; n0 += 32) {
+        const int nb = std::min(2, (nh - n0 + 15) / 16);
+        for (int m0 = 0; m0 < nh; m0 += 16)
+          x.push_back(ZTile{d.Vhhpp + P.off_t[c], d.T + P.off_t[c], d.Vhhhh + P.off_vhh[c], X, I9, nh, nh, np_, m0, n0,
+                            nb, (int)s, gx, (float)np_ * nb});
+        for (int m0 = 0; m0 < np_; m0 += 64)
+          hh.push_back(ZTile{d.T + P.off_t[c], I9, nullptr, d.Rh + P.off_t[c], nullptr, np_, nh, nh, m0, n0, nb, (int)s,
+                             gx, (float)nh * nb});
+      }
+    }
+    for (int K = 0; K < P.nphc; ++K, ++gr) {
+      const int nph = P.nph[K], nhp = P.nhp[K], cls = ring64_class(nph, nhp);
+      if (cls < 0 || nph <= 0 || nhp <= 0) continue;
+      for (int n0 = 0; n0 < nhp; n0 += ring64_columns(cls))
+        ring[cls].push_back(RingTile{d.Vt + P.off_vt[K], d.Tt + P.off_rt[K], d.W0 + P.off_i4[K], d.Rt + P.off_rt[K],
+                                     nhp, nph, n0, (int)s, gr, (float)nph + nhp});
+    }
+  }
+  xcd_order_list(x, gx);
+  xcd_order_list(hh, gx);
+  F.nx = (int)x.size();
+  F.nhh = (int)hh.size();
+  F.x = dupload(x, B.owned);
+  F.hh = dupload(hh, B.owned);
+  for (int c = 0; c < 3; ++c) {
+    xcd_order_list(ring[c], gr);
+    F.nring[c] = (int)ring[c].size();
+    F.ring[c] = dupload(ring[c], B.owned);
+  }
+  for (GemmList *L : {&B.g_i4big, &B.g_rtbig}) {
+    if (L->groups.empty()) continue;
+    autotune(*L, 0, B.d_descs, B.stream);
+    L->build_tiles();
+    L->upload(B.owned);
+    L->ready = true;
+  }
+  F.ready = true;
+}
+
 void prepare_lists(Batch &B, int prec) {
   const int kinds[13] = {0, 3, 0, 0, 0, 4, 6, 6, 6, 6, 8, 8, 10};   // the kernel kind each list is tuned for
   GemmList *lists[13] = {&B.g_x, &B.g_pp, &B.g_hh, &B.g_i4, &B.g_rt, &B.g_pp32, &B.g_xb, &B.g_hhb, &B.g_i4b, &B.g_rtb,
                          &B.g_i4f, &B.g_rtf, &B.g_ppbf};
+  // families in FP64 that the tiles of contract.hip contract
+  const bool tiles64 = fp64_tiles() && tail_low_mask() == 0;
+  const bool all64 = prec == CCGPU_PREC_FP64 || prec == CCGPU_PREC_V32;
+  if (tiles64) prepare_fp64(B);
   for (int k = 0; k < 13; ++k) {
     GemmList &L = *lists[k];
     if (L.ready) continue;
+    if (tiles64 && all64 && k < 5 && k != 1) continue;
     if (k == 5 && (prec == CCGPU_PREC_FP64 || !B.has_f32)) continue;
     if (k >= 6 && prec != CCGPU_PREC_BF16X3) continue;
     if (k >= 10 && k < 12 && !B.ring32) continue;
@@ -1403,6 +1497,9 @@ void residual_launches(Batch &B, int prec, bool timing) {
   auto list = [&](GemmList &L64, GemmList &Lbf, int bit) -> const GemmList & {
     return pf(bit) == CCGPU_PREC_BF16X3 ? Lbf : L64;
   };
+  // the families in FP64 run the tiles of contract.hip
+  const bool tiles64 = B.f64.ready && fp64_tiles();
+  auto t64 = [&](int bit) { return tiles64 && pf(bit) == CCGPU_PREC_FP64; };
   // Three streams outside the timing mode (fork/join through events, also
   // inside a captured graph).  The ring chain (T -> T~, I4, R~) reads only T
   // and the ring blocks and touches R only in the final scatter: a second
@@ -1437,12 +1534,13 @@ void residual_launches(Batch &B, int prec, bool timing) {
   if (fork6) HIPCHK(hipEventRecord(B.ev_join3, s6));
   {
     Timer t(timing, st, "gemm_x_vhhpp_t");
-    run_gemm(list(B.g_x, B.g_xb, 0), B, pf(0), false, st);
+    if (t64(0)) launch_x64(B.f64.x, B.f64.nx, B.d_descs, st);
+    else run_gemm(list(B.g_x, B.g_xb, 0), B, pf(0), false, st);
   }
   {
     Timer t(timing, st, "i7_i9");
     launch_i7(B.d_descs, n, B.maxA, st);
-    launch_i9(B.d_descs, n, B.maxVhh, st);
+    if (!t64(0)) launch_i9(B.d_descs, n, B.maxVhh, st);   // the X tiles write I9 too
   }
   if (terms & 4) {
     if (fork6) {
@@ -1450,7 +1548,8 @@ void residual_launches(Batch &B, int prec, bool timing) {
       HIPCHK(hipStreamWaitEvent(s6, B.ev_x, 0));
     }
     Timer t(timing, s6, "gemm_hh_ladder");
-    run_gemm(list(B.g_hh, B.g_hhb, 2), B, pf(2), false, s6);
+    if (t64(2)) launch_hh64(B.f64.hh, B.f64.nhh, B.d_descs, s6);
+    else run_gemm(list(B.g_hh, B.g_hhb, 2), B, pf(2), false, s6);
   }
   if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
   if (terms & 8) {
@@ -1458,12 +1557,20 @@ void residual_launches(Batch &B, int prec, bool timing) {
       Timer t(timing, sr, "ring_gather");
       launch_ring_gather(B.d_descs, n, B.maxT, ring32, sr);
     }
-    {
+    B.i4_in_lds = t64(3);
+    if (t64(3)) {
+      Timer t(timing, sr, "gemm_ring");
+      for (int c = 2; c >= 0; --c) launch_ring64(B.f64.ring[c], B.f64.nring[c], c, B.d_descs, sr);
+      if (!B.g_i4big.groups.empty()) {
+        run_gemm(B.g_i4big, B, CCGPU_PREC_FP64, false, sr);
+        run_gemm(B.g_rtbig, B, CCGPU_PREC_FP64, false, sr);
+      }
+    } else {
       Timer t(timing, sr, "gemm_ring_i4");
       if (ring32) run_gemm(B.g_i4f, B, pf(3), true, sr, false, 8);
       else run_gemm(list(B.g_i4, B.g_i4b, 3), B, pf(3), false, sr);
     }
-    {
+    if (!t64(3)) {
       Timer t(timing, sr, "gemm_ring_rt");
       if (ring32) run_gemm(B.g_rtf, B, pf(3), true, sr, false, 8);
       else run_gemm(list(B.g_rt, B.g_rtb, 3), B, pf(3), false, sr);
@@ -3160,6 +3267,16 @@ int ccgpu_debug_fetch(int handle, int what, double *out, long long n) {
                {d.fpart, P.nsp}, {d.W0, P.nI4}, {d.Vt, P.nRt}};
     if (what < 0 || what >= (int)(sizeof a / sizeof a[0])) throw Error(fmt("unknown debug array %d", what));
     if (n != a[what].n) throw Error(fmt("debug array %d has %lld elements, caller asked %lld", what, a[what].n, n));
+    if (what == 8 && single(handle).i4_in_lds) {   // formed here from the last T~
+      Batch &B = single(handle);
+      if (!B.g_i4.ready) {
+        B.g_i4.build_tiles();
+        B.g_i4.upload(B.owned);
+        B.g_i4.ready = true;
+      }
+      run_gemm(B.g_i4, B, CCGPU_PREC_FP64, false, B.stream);
+      check_launch();
+    }
     HIPCHK(hipDeviceSynchronize());
     HIPCHK(hipMemcpy(out, a[what].p, n * sizeof(double2), hipMemcpyDeviceToHost));
   });

@@ -1,0 +1,336 @@
+// FP64 contractions of the CCD residual outside the pp ladder, one launch each
+// (the ring one per channel size class), every channel and solve of a batch in
+// it: X = V_hhpp T with I9 = V_hhhh + X (ccm_t2_eqn.f90:431-464, 558-560), the
+// hh ladder T I9 (:614-647), and the ring I4 = W0 + 1/2 V~ T~, R~ = T~ I4
+// (:657-780, 995-1026).
+//
+// Complex products take three real MFMAs (Gauss: ar br, ai bi, (ar+ai)(br+bi)).
+// A 16-wide k chunk is four 16x16x4 steps; lane group g = lane / 16 of step q
+// takes k0 + 4 q + g, so each operand load reads 64 contiguous bytes of a row.
+// Operands that one wave alone needs go straight to its registers: a 16x16x4
+// FP64 MFMA takes 64 clocks of its SIMD, so even 16 columns per row need
+// only 21 bytes a clock and CU.
+#include "device.h"
+
+#include <algorithm>
+
+namespace ccgpu {
+
+typedef double cd4 __attribute__((ext_vector_type(4)));
+typedef double cd2 __attribute__((ext_vector_type(2)));
+
+// element e of a block whose base is the same for the whole wave (a scalar
+// base and a 32-bit offset per lane; a channel's block is far below 4 GB)
+__device__ __forceinline__ double2 gl(const double2 *base, unsigned e) {
+  const __attribute__((address_space(1))) char *p = (const __attribute__((address_space(1))) char *)base;
+  const cd2 v = *(const __attribute__((address_space(1))) cd2 *)(p + (e << 4));
+  return make_double2(v.x, v.y);
+}
+// The elements of a lane for the Q steps from k0 of a row of length K that
+// starts at element `row`, clamped to the row (the other operand, or zero_past,
+// is zero past it).
+template <int Q>
+__device__ __forceinline__ void row_chunk(double2 (&a)[Q], const double2 *base, unsigned row, int K, int k0, int lg) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q) a[q] = gl(base, row + min(k0 + 4 * q + lg, K - 1));
+}
+__device__ __forceinline__ void zero_past(double2 (&a)[4], int K, int k0, int lg) {
+  if (k0 + 16 > K)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (k0 + 4 * q + lg >= K) a[q] = make_double2(0.0, 0.0);
+}
+// The same k of one column: row length N, column c < N
+__device__ __forceinline__ void column_chunk(double2 (&b)[4], const double2 *base, unsigned c, int N, int K, int k0,
+                                             int lg) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) b[q] = gl(base, (unsigned)min(k0 + 4 * q + lg, K - 1) * N + c);
+}
+__device__ __forceinline__ double2 zero_unless(bool ok, double2 v) {
+  return make_double2(ok ? v.x : 0.0, ok ? v.y : 0.0);
+}
+
+// accumulators of one 16 x 16 block, and its value in register r
+struct CAcc {
+  cd4 re, im, s;
+  __device__ __forceinline__ void clear() { re = im = s = (cd4){0.0, 0.0, 0.0, 0.0}; }
+  __device__ __forceinline__ void mac(double2 a, double2 b) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, im, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x + a.y, b.x + b.y, s, 0, 0, 0);
+  }
+  __device__ __forceinline__ double2 at(int r) const { return make_double2(re[r] - im[r], s[r] - re[r] - im[r]); }
+};
+
+// ---------------------------------------------------------------------------
+// X and I9.  K is the long side (particle pairs, up to thousands) and M = N the
+// short one (hole pairs of a channel): a tile is 16 rows by up to 32 columns, its
+// four waves take every fourth 16-wide chunk of k and add their partials in
+// LDS in wave order.  Bound by the k chain of a tile; one block per 64 x 16
+// tile over the whole k range, in a launch per width class, took 128 us of an
+// iteration of PNM A=66 |n_i|<=4 (seven launches), this one 27 us, I9 included.
+// ---------------------------------------------------------------------------
+template <int NB>
+__device__ __forceinline__ void x64_tile(const ZTile &t, double2 *red) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  CAcc acc[NB];
+#pragma unroll
+  for (int y = 0; y < NB; ++y) acc[y].clear();
+  // rows and columns past the matrix are copies of the last one and never stored
+  const unsigned row = (unsigned)min(t.m0 + li, t.M - 1) * t.K;
+  unsigned col[NB];
+#pragma unroll
+  for (int y = 0; y < NB; ++y) col[y] = min(t.n0 + 16 * y + li, t.N - 1);
+  double2 a0[4], b0[NB][4], a1[4], b1[NB][4];
+  auto load = [&](double2 (&a)[4], double2 (&b)[NB][4], int k0) {
+    row_chunk(a, t.A, row, t.K, k0, lg);
+#pragma unroll
+    for (int y = 0; y < NB; ++y) column_chunk(b[y], t.B, col[y], t.N, t.K, k0, lg);
+    zero_past(a, t.K, k0, lg);
+  };
+  auto compute = [&](const double2 (&a)[4], const double2 (&b)[NB][4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int y = 0; y < NB; ++y) acc[y].mac(a[q], b[y][q]);
+  };
+  int k0 = 16 * w;
+  if (k0 < t.K) {
+    load(a0, b0, k0);
+    for (; k0 < t.K; k0 += 128) {
+      if (k0 + 64 < t.K) load(a1, b1, k0 + 64);
+      compute(a0, b0);
+      if (k0 + 64 >= t.K) break;
+      if (k0 + 128 < t.K) load(a0, b0, k0 + 128);
+      compute(a1, b1);
+    }
+  }
+#pragma unroll
+  for (int y = 0; y < NB; ++y)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[((w * NB + y) * 4 + r) * 64 + lane] = acc[y].at(r);
+  __syncthreads();
+  // register r of lane l: row (l >> 4) + 4 r, column l & 15 of its block
+  for (int i = w; i < 4 * NB; i += 4) {
+    const int y = i >> 2, r = i & 3;
+    double2 v = red[i * 64 + lane];
+#pragma unroll
+    for (int p = 1; p < 4; ++p) {
+      const double2 x = red[(p * 4 * NB + i) * 64 + lane];
+      v.x += x.x;
+      v.y += x.y;
+    }
+    const int mm = t.m0 + lg + 4 * r, n = t.n0 + 16 * y + li;
+    if (mm < t.M && n < t.N) {
+      const int64_t e = (int64_t)mm * t.N + n;
+      const double2 c = t.C0[e];
+      t.C[e] = v;
+      t.C2[e] = make_double2(v.x + c.x, v.y + c.y);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void k_x64(const ZTile *__restrict__ tiles, const SolveDesc *__restrict__ descs) {
+  __shared__ double2 red[4 * 2 * 4 * 64];
+  const ZTile t = tiles[blockIdx.x];
+  if (!descs[t.solve].active) return;
+  if (t.nb == 1) x64_tile<1>(t, red);
+  else x64_tile<2>(t, red);
+}
+
+// ---------------------------------------------------------------------------
+// hh ladder: M = particle pairs, N = K = hole pairs.  64 rows by up to 32
+// columns, a wave per 16 rows; I9 comes through the L1.  24 us on the same
+// lattice; a launch per width class took 68 us in four.
+// ---------------------------------------------------------------------------
+template <int NB>
+__device__ __forceinline__ void hh64_tile(const ZTile &t) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  const int mw = t.m0 + 16 * w;
+  if (mw >= t.M) return;
+  CAcc acc[NB];
+#pragma unroll
+  for (int y = 0; y < NB; ++y) acc[y].clear();
+  const unsigned row = (unsigned)min(mw + li, t.M - 1) * t.K;
+  unsigned col[NB];
+#pragma unroll
+  for (int y = 0; y < NB; ++y) col[y] = min(t.n0 + 16 * y + li, t.N - 1);
+  double2 a0[4], b0[NB][4], a1[4], b1[NB][4];
+  auto load = [&](double2 (&a)[4], double2 (&b)[NB][4], int k0) {
+    row_chunk(a, t.A, row, t.K, k0, lg);
+#pragma unroll
+    for (int y = 0; y < NB; ++y) column_chunk(b[y], t.B, col[y], t.N, t.K, k0, lg);
+    zero_past(a, t.K, k0, lg);
+  };
+  auto compute = [&](const double2 (&a)[4], const double2 (&b)[NB][4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int y = 0; y < NB; ++y) acc[y].mac(a[q], b[y][q]);
+  };
+  load(a0, b0, 0);
+  for (int k0 = 0; k0 < t.K; k0 += 32) {
+    if (k0 + 16 < t.K) load(a1, b1, k0 + 16);
+    compute(a0, b0);
+    if (k0 + 16 >= t.K) break;
+    if (k0 + 32 < t.K) load(a0, b0, k0 + 32);
+    compute(a1, b1);
+  }
+#pragma unroll
+  for (int y = 0; y < NB; ++y)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int mm = mw + lg + 4 * r, n = t.n0 + 16 * y + li;
+      if (mm < t.M && n < t.N) t.C[(int64_t)mm * t.N + n] = acc[y].at(r);
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_hh64(const ZTile *__restrict__ tiles, const SolveDesc *__restrict__ descs) {
+  const ZTile t = tiles[blockIdx.x];
+  if (!descs[t.solve].active) return;
+  if (t.nb == 1) hh64_tile<1>(t);
+  else hh64_tile<2>(t);
+}
+
+// ---------------------------------------------------------------------------
+// Ring: column block n0 of I4 needs V~ and column block n0 of T~ only, and the
+// same column block of R~ = T~ I4 needs T~ and that block of I4 only: one block
+// does both, with the T~ columns and then the I4 columns in LDS (I4 never goes
+// to memory), W waves of RB 16-row blocks each, 16 NB columns.  V~ and T~ rows
+// go straight to the wave that owns them.  Column blocks of a channel run on
+// one XCD, whose L2 holds V~ and T~ for them.
+//
+// W RB 16 covers the channel's larger side: 64 (W 4) and 128 (W 8) with 32
+// columns, 256 (W 8, RB 2) with 16; 64 KB of LDS at most, two workgroups per CU
+// (one with RB 2).
+// Bound by FP64 MFMA: PNM A=66 |n_i|<=4 takes 238 + 34 us (classes 128 and 64,
+// alone on the device; MFMA alone 137 + 15).  I4 and R~ as two launches per width class
+// with I4 in memory took 486 us in twelve.  16 columns 258, 48 columns 286, one workgroup
+// per CU 244.
+// ---------------------------------------------------------------------------
+template <int W, int RB, int NB>
+__global__ __launch_bounds__(64 * W, W == 8 && RB == 1 ? 4 : 2) void k_ring64(const RingTile *__restrict__ tiles,
+                                                                   const SolveDesc *__restrict__ descs) {
+  constexpr int BC = 16 * NB, NT = 64 * W;
+  __shared__ double2 Bs[16 * W * RB * BC];
+  const RingTile t = tiles[blockIdx.x];
+  if (!descs[t.solve].active) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  CAcc acc[RB][NB];
+  // two MFMA steps (8 k) ahead: with four waves on a SIMD the loads have the
+  // other waves' 3 x 768 clocks, and 16 registers less keep 128 without spills
+  double2 a0[RB][2], a1[RB][2];
+  // steps from k0 of this wave's rows (blocks w and w + W) of A, M x K.  Rows
+  // past M are copies of the last and never used; k past K meets zeros in LDS.
+  auto load = [&](double2 (&a)[RB][2], const double2 *A, int M, int K, int k0) {
+#pragma unroll
+    for (int x = 0; x < RB; ++x) row_chunk(a[x], A, (unsigned)min(16 * (w + W * x) + li, M - 1) * K, K, k0, lg);
+  };
+  auto compute = [&](const double2 (&a)[RB][2], int k0) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const double2 *b = Bs + (k0 + 4 * q + lg) * BC + li;
+#pragma unroll
+      for (int y = 0; y < NB; ++y) {
+        const double2 bv = b[16 * y];
+#pragma unroll
+        for (int x = 0; x < RB; ++x) acc[x][y].mac(a[x][q], bv);
+      }
+    }
+  };
+  // the rows times the columns in LDS; the first two steps are in a0 already
+  auto product = [&](const double2 *A, int M, int K) {
+#pragma unroll
+    for (int x = 0; x < RB; ++x)
+#pragma unroll
+      for (int y = 0; y < NB; ++y) acc[x][y].clear();
+    if (16 * w >= M) return;
+    for (int k0 = 0; k0 < K; k0 += 16) {   // whole chunks of 16: LDS is zero past K
+      load(a1, A, M, K, k0 + 8);
+      compute(a0, k0);
+      load(a0, A, M, K, k0 + 16);
+      compute(a1, k0 + 8);
+    }
+  };
+  load(a0, t.Vt, t.nhp, t.nph, 0);
+  // T~ columns, zero past the matrix (up to the last whole chunk of k); eight
+  // loads per thread in flight
+  {
+    const int n = ((t.nph + 15) & ~15) * BC;
+    for (int e0 = threadIdx.x; e0 < n; e0 += 8 * NT) {
+      double2 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int e = e0 + j * NT, k = e / BC, c = t.n0 + e % BC;
+        v[j] = zero_unless(k < t.nph && c < t.nhp, gl(t.Tt, (unsigned)min(k, t.nph - 1) * t.nhp + min(c, t.nhp - 1)));
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (e0 + j * NT < n) Bs[e0 + j * NT] = v[j];
+    }
+  }
+  __syncthreads();
+  product(t.Vt, t.nhp, t.nph);
+  // I4 = W0 + 1/2 V~ T~ in the place of the T~ columns; rows past nhp in a
+  // wave's block are zero
+#pragma unroll
+  for (int x = 0; x < RB; ++x)
+#pragma unroll
+    for (int y = 0; y < NB; ++y) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = 16 * (w + W * x) + lg + 4 * r, c = t.n0 + 16 * y + li;
+        const double2 s = acc[x][y].at(r);
+        const double2 c0 = gl(t.W0, (unsigned)min(m, t.nhp - 1) * t.nhp + min(c, t.nhp - 1));
+        const bool ok = m < t.nhp && c < t.nhp;
+        acc[x][y].re[r] = ok ? 0.5 * s.x + c0.x : 0.0;
+        acc[x][y].im[r] = ok ? 0.5 * s.y + c0.y : 0.0;
+      }
+    }
+  load(a0, t.Tt, t.nph, t.nhp, 0);
+  __syncthreads();   // every wave has read the T~ columns
+#pragma unroll
+  for (int x = 0; x < RB; ++x) {
+    if (16 * (w + W * x) >= t.nhp) continue;
+#pragma unroll
+    for (int y = 0; y < NB; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Bs[(16 * (w + W * x) + lg + 4 * r) * BC + 16 * y + li] = make_double2(acc[x][y].re[r], acc[x][y].im[r]);
+  }
+  __syncthreads();
+  product(t.Tt, t.nph, t.nhp);
+#pragma unroll
+  for (int x = 0; x < RB; ++x) {
+    const int mw = 16 * (w + W * x);
+    if (mw >= t.nph) continue;
+#pragma unroll
+    for (int y = 0; y < NB; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = mw + lg + 4 * r, c = t.n0 + 16 * y + li;
+        if (m < t.nph && c < t.nhp) t.Rt[(int64_t)m * t.nhp + c] = acc[x][y].at(r);
+      }
+  }
+}
+
+int ring64_class(int nph, int nhp) {   // tile class of a channel, -1: too large for the fused kernel
+  const int d = std::max(nph, nhp);
+  return d <= 64 ? 0 : d <= 128 ? 1 : d <= 256 ? 2 : -1;
+}
+int ring64_columns(int cls) { return cls == 2 ? 16 : 32; }
+
+void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *dd, hipStream_t st) {
+  if (ntiles <= 0) return;
+  if (cls == 0) hipLaunchKernelGGL((k_ring64<4, 1, 2>), dim3(ntiles), dim3(256), 0, st, tiles, dd);
+  else if (cls == 1) hipLaunchKernelGGL((k_ring64<8, 1, 2>), dim3(ntiles), dim3(512), 0, st, tiles, dd);
+  else hipLaunchKernelGGL((k_ring64<8, 2, 1>), dim3(ntiles), dim3(512), 0, st, tiles, dd);
+}
+void launch_x64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st) {
+  if (ntiles > 0) hipLaunchKernelGGL(k_x64, dim3(ntiles), dim3(256), 0, st, tiles, dd);
+}
+void launch_hh64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st) {
+  if (ntiles > 0) hipLaunchKernelGGL(k_hh64, dim3(ntiles), dim3(256), 0, st, tiles, dd);
+}
+
+}  // namespace ccgpu

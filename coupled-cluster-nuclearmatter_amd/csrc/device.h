@@ -88,6 +88,24 @@ struct GemmTile {
   int kb, ke, pad0, pad1;  // k range of this tile
 };
 
+// One tile of the FP64 X or hh-ladder contraction (contract.hip): 16 (X) or 64
+// (hh) rows from m0 by nb <= 2 blocks of 16 columns from n0 of C = A B.  X also
+// writes C2 = C + C0 (I9).
+struct ZTile {
+  const double2 *A, *B, *C0;
+  double2 *C, *C2;
+  int M, N, K, m0, n0, nb, solve, g;
+  float cost;
+};
+
+// Columns n0 .. of one Pandya channel's two ring contractions (contract.hip)
+struct RingTile {
+  const double2 *Vt, *Tt, *W0;
+  double2 *Rt;
+  int nhp, nph, n0, solve, g;
+  float cost;
+};
+
 // A triple of hole groups I <= J <= K (a group: the up to two spin states of one
 // momentum and isospin, in orbital order) of one (K3, Tz3) channel: its pair
 // indices into the tables below and the spin combinations 4 is + 2 js + ks that

@@ -154,3 +154,34 @@ def test_triples_after_a_new_interaction_and_fock(ccnm):
     b = fresh(ccnm.LO)
     assert a.pert_triples2() == b.pert_triples2()
     assert abs(first - b.pert_triples2()) > 1e-6
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist", [
+    (2, "pnm", 2, (0.0, 0.0, 0.0)), (14, "pnm", 1, (0.0, 0.0, 0.0)), (15, "pnm", 1, (0.3, 0.6, 0.9)),
+    (38, "pnm", 2, (0.5, 1.0, 1.5)), (54, "pnm", 2, (0.0, 0.0, 0.0)), (66, "pnm", 4, (0.0, 0.0, 0.0)),
+    (162, "pnm", 3, (0.0, 0.0, 0.0)), (246, "pnm", 3, (0.2, 0.4, 0.6)), (28, "snm", 2, (0.0, 0.0, 0.0)),
+    (228, "snm", 3, (0.0, 0.0, 0.0))])
+def test_fp64_contraction_tiles_equal_list_kernels(ccnm, monkeypatch, A, matter, nmax, twist):
+    """X, I9, the hh ladder and the fused ring against the grouped list kernels
+    over the classes of their tiles: ring sides 4, 16, 18, 60 (sides that
+    differ by up to 16), 76, 128, 172, 212 (differing by up to 40) and 296, past
+    the fused kernel; 1 to 245 hole pairs.  Both sum the same products, k in
+    another order: each contraction rounds by at most 2^-53 (K + 8) times four
+    (three-product complex terms) of its sum of moduli, K at most 1144, so
+    6e-13 of it; the amplitudes after two steps without extrapolation are such
+    sums over denominators above 1, and a lost k would be 1e-3 of one."""
+    out = []
+    for lists in (False, True):
+        if lists:
+            monkeypatch.setenv("CCGPU_SPLIT_K", "256")   # the lists' own default; they run as soon as one is asked for
+        s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax, twist=twist)
+        s.generate_interaction(ccnm.INT_MINNESOTA)
+        s.setup_t_amplitudes()
+        for _ in range(2):
+            s.t2_intermediate()
+            s.diis_t1t2(1, 1)
+        out.append(s.t2_unique())
+        s.close()
+    t, ref = out
+    assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0
+    assert np.abs(t - ref).max() <= 1e-12 * np.abs(ref).max()
