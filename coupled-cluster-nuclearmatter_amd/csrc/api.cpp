@@ -42,26 +42,18 @@ void launch_to_f32(const double2 *src, float2 *dst, int64_t n, hipStream_t st);
 void launch_to_f32_rows(const double2 *src, float2 *dst, const int64_t *off, const int64_t *off32, const int *npp,
                         int nch, int max_npp, hipStream_t st);
 void launch_mbpt2(const SolveDesc *dd, int nsolve, int64_t maxT, hipStream_t st);
-void launch_energy(const SolveDesc *dd, int nsolve, int slot, hipStream_t st);
+void launch_energy(const SolveDesc *dd, int nsolve, double2 *out, hipStream_t st);
 void launch_i7(const SolveDesc *dd, int nsolve, int maxA, hipStream_t st);
 void launch_i6(const SolveDesc *dd, int nsolve, int maxnp, int64_t maxrows, hipStream_t st);
 void launch_i9(const SolveDesc *dd, int nsolve, int64_t maxvhh, hipStream_t st);
-void launch_resid_init(const SolveDesc *dd, int nsolve, int64_t maxT, bool onebody, hipStream_t st);
-void launch_ring_gather(const SolveDesc *dd, int nsolve, int64_t maxT, bool f32, hipStream_t st);
-void launch_t_split(const SolveDesc *dd, int nsolve, int64_t maxT, hipStream_t st);
-void launch_ring_scatter(const SolveDesc *dd, int nsolve, int64_t maxT, bool f32, bool ring, bool hh,
-                         hipStream_t st);
-void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slot, hipStream_t st);
-void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, hipStream_t st);
-void launch_aa_update(const SolveDesc *dd, int nsolve, const int *slots, double beta, hipStream_t st);
+void launch_t_begin(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64_t maxT, int ring, bool form, bool split,
+                    const uint32_t *const *maps, double2 *Tu, hipStream_t st);
+void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, bool f32, int mode, int terms,
+                  const uint32_t *const *maps, const double2 *Ru, double2 *out, hipStream_t st);
+void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const IterCtrl *ctrl, hipStream_t st);
+void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, double2 *out, hipStream_t st);
 void launch_scatter_values(double2 *dst, const int64_t *idx, const double2 *val, int64_t n, hipStream_t st);
 void launch_fill_vpppp(const SolveDesc &d, double volume, const ChiralDev *c, int nch, int max_npp, hipStream_t st);
-void launch_share_gather(const SolveDesc *dd, int nsolve, int64_t maxT, const uint32_t *const *maps, double2 *Tu,
-                         hipStream_t st);
-void launch_share_scatter(const SolveDesc *dd, int nsolve, int64_t maxT, const uint32_t *const *maps,
-                          const double2 *Ru, hipStream_t st);
-void launch_aa_combine(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slots, const double *coef,
-                       hipStream_t st);
 void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slots, const double2 *coef,
                       int nvec, hipStream_t st);
 void launch_gemm_shape(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const SolveDesc *dd,
@@ -440,13 +432,9 @@ struct Solve {
   int depth_f = 0;         // columns of desc.histf (Anderson residual vectors)
   std::vector<int> ring;  // logical column -> physical slot
   int nstep = 0, count = 0;
-  int *d_slot = nullptr;   // [1] physical slot for k_update
-  int *d_slots = nullptr;  // [16] physical slots in logical order
-  double2 *d_coef = nullptr;
   // work lists for the five GEMM families
   GemmList g_x, g_pp, g_hh, g_i4, g_rt;
   bool vpppp32 = false;
-  double2 *scal = nullptr;
   ~Solve() {
     for (void *p : owned) (void)hipFree(p);
     for (void *p : t3_owned) (void)hipFree(p);
@@ -578,10 +566,8 @@ void build_device(Solve &S) {
   d.dp = dalloc<double2>(P.np, o);
   d.I6off = dalloc<double2>(P.np, o);
   d.e0 = dalloc<double2>(1, o);
-  d.red = dalloc<double2>(1024 * 36, o);
-  d.scal = dalloc<double2>(64, o);
+  d.red = dalloc<double2>(2048 * 36, o);
   d.hist = nullptr;
-  S.scal = d.scal;
   HIPCHK(hipMemset(d.Tt, 0, P.nRt * sizeof(double2)));  // entries with a=b or i=j stay zero
   HIPCHK(hipMemset(d.Rh, 0, P.nT * sizeof(double2)));
   HIPCHK(hipMemset(d.T, 0, P.nT * sizeof(double2)));
@@ -590,9 +576,6 @@ void build_device(Solve &S) {
   HIPCHK(hipMemset(d.Vhhhh, 0, P.nVhh * sizeof(double2)));
   HIPCHK(hipMemset(d.W0, 0, P.nI4 * sizeof(double2)));
   S.d_desc = dalloc<SolveDesc>(1, o);
-  S.d_slot = dalloc<int>(1, o);
-  S.d_slots = dalloc<int>(16, o);
-  S.d_coef = dalloc<double2>(16, o);
   HIPCHK(hipMemcpy(S.d_desc, &d, sizeof(SolveDesc), hipMemcpyHostToDevice));
 
   // GEMM work lists
@@ -600,10 +583,9 @@ void build_device(Solve &S) {
     int np_ = P.npp[c], nh = P.nhh[c];
     // X = Vhhpp T
     S.g_x.add(mkgroup(d.Vhhpp + P.off_t[c], d.T + P.off_t[c], d.X + P.off_vhh[c], nullptr, nh, nh, np_, np_, nh, nh, 0, 1.0, 0.0), 0);
-    // R += Vpppp T   (pp ladder, ccm_t2_eqn.f90:574-607)
-    S.g_pp.add(mkgroup(d.Vpppp + P.off_vpp[c], d.T + P.off_t[c], d.R + P.off_t[c], d.R + P.off_t[c], np_, nh, np_, np_, nh, nh, nh, 1.0, 1.0), 0);
-    // R += T I9      (hh ladder, ccm_t2_eqn.f90:614-647)
-    // the hh ladder into Rh (beta 0), beside the pp ladder; the ring scatter adds it to R
+    // Vpppp T into R (pp ladder, ccm_t2_eqn.f90:574-607); the closing pass adds the rest
+    S.g_pp.add(mkgroup(d.Vpppp + P.off_vpp[c], d.T + P.off_t[c], d.R + P.off_t[c], nullptr, np_, nh, np_, np_, nh, nh, 0, 1.0, 0.0), 0);
+    // T I9 into Rh (hh ladder, ccm_t2_eqn.f90:614-647), beside the pp ladder
     S.g_hh.add(mkgroup(d.T + P.off_t[c], d.X + P.nVhh + P.off_vhh[c], d.Rh + P.off_t[c], nullptr, np_, nh, nh, nh, nh, nh, nh, 1.0, 0.0), 0);
   }
   for (int K = 0; K < P.nphc; ++K) {
@@ -720,34 +702,33 @@ struct Batch {
   bool has_f32 = true;   // every solve has the FP32 copy of its pppp blocks
   int64_t maxT = 0, maxVhh = 0, maxRows = 0;
   int maxA = 0, maxNp = 0;
-  int *d_slot = nullptr, *d_slots = nullptr;
+  IterCtrl *d_ctrl = nullptr;   // one per solve
+  std::vector<IterCtrl> ctrl;
+  double2 *results = nullptr;   // pinned, 64 per solve: the reductions write it
+  int *d_slots = nullptr;
   double2 *d_coef = nullptr;
-  double2 *d_scal = nullptr;  // nsolve * 64
-  std::vector<int> h_slot, h_slots;       // host staging of control arrays
-  std::vector<double2> h_coef, h_scal;
+  std::vector<int> h_slots;               // host staging of control arrays
+  std::vector<double2> h_coef;
   std::vector<int> status;                // CCGPU_STATUS_* per solve of the current run
   bool forced_done = false;               // CCGPU_FORCE_SINGULAR fired in this run
   // Anderson update: per solve the held vectors (physical history slots,
   // oldest first), their Gram matrix Re<f_j, f_k> and the energies of the
-  // mixed iterates y_j; device copies of the slots and coefficients
+  // mixed iterates y_j
   struct AA {
     std::vector<int> slot;
     std::vector<double> gram;   // kAAHeld x kAAHeld, logical order
     std::vector<std::complex<double>> ey;
   };
   std::vector<AA> aa;
-  int *d_aaslots = nullptr;
-  double *d_aacoef = nullptr;
-  std::vector<int> h_aaslots;
-  std::vector<double> h_aacoef;
   std::vector<void *> owned;
   hipStream_t stream = nullptr;
   // second stream (default priority) for the ring branch of the residual, and
   // the fork/join events
   hipStream_t stream2 = nullptr, stream3 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_join3 = nullptr, ev_x = nullptr, ev_hh = nullptr;
-  hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};        // per precision mode
-  hipGraphExec_t gexec[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_x = nullptr, ev_hh = nullptr;
+  // a residual with its update, per precision mode and accelerator
+  hipGraph_t graph[8] = {};
+  hipGraphExec_t gexec[8] = {};
   // pinned staging of the small copies of every iteration, one buffer per
   // call site; each site's copy is followed by a stream synchronisation
   // before the host writes its buffer again
@@ -766,13 +747,12 @@ struct Batch {
   ~Batch() {
     for (void *p : pin)
       if (p) (void)hipHostFree(p);
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < 8; ++q) {
       if (gexec[q]) (void)hipGraphExecDestroy(gexec[q]);
       if (graph[q]) (void)hipGraphDestroy(graph[q]);
     }
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
-    if (ev_join3) (void)hipEventDestroy(ev_join3);
     if (ev_x) (void)hipEventDestroy(ev_x);
     if (ev_hh) (void)hipEventDestroy(ev_hh);
     if (stream2) (void)hipStreamDestroy(stream2);
@@ -945,19 +925,15 @@ bool share_eligible(const std::vector<Solve *> &ss);
 void build_shared(Batch &B);
 void check_launch();
 
-// Copies of the solve loop through the batch's pinned buffers (site: one per
-// call site): host to device without a pageable staging copy; device to host
-// completes with the stream
+// Copies of the solve loop to the device through the batch's pinned buffers
+// (site: one per call site), without a pageable staging copy
 void h2d_pinned(Batch &B, int site, void *dst, const void *src, size_t bytes, hipStream_t st) {
   void *p = B.pinned(site, bytes);
   memcpy(p, src, bytes);
   HIPCHK(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, st));
 }
-void d2h_pinned_sync(Batch &B, int site, void *dst, const void *src, size_t bytes, hipStream_t st) {
-  void *p = B.pinned(site, bytes);
-  HIPCHK(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  memcpy(dst, p, bytes);
+void upload_ctrl(Batch &B) {
+  h2d_pinned(B, 0, B.d_ctrl, B.ctrl.data(), B.ctrl.size() * sizeof(IterCtrl), B.stream);
 }
 
 std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st) {
@@ -965,12 +941,11 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
   B->solves = ss;
   B->stream = st;
   int n = (int)ss.size();
-  B->d_scal = dalloc<double2>((size_t)n * 64, B->owned);
+  B->results = (double2 *)B->pinned(3, (size_t)n * 64 * sizeof(double2));
   for (int s = 0; s < n; ++s) {
     Solve &S = *ss[s];
     SolveDesc d = S.desc;
     d.active = 1;
-    d.scal = B->d_scal + (size_t)s * 64;
     B->h_descs.push_back(d);
     merge(B->g_x, S.g_x, s);
     merge(B->g_pp, S.g_pp, s);
@@ -1099,14 +1074,12 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
   HIPCHK(hipStreamCreateWithFlags(&B->stream3, hipStreamNonBlocking));
   HIPCHK(hipEventCreateWithFlags(&B->ev_fork, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&B->ev_join, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&B->ev_join3, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&B->ev_x, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&B->ev_hh, hipEventDisableTiming));
-  B->d_slot = dalloc<int>(n, B->owned);
+  B->d_ctrl = dalloc<IterCtrl>(n, B->owned);
+  B->ctrl.assign(n, IterCtrl{});
   B->d_slots = dalloc<int>((size_t)n * 16, B->owned);
   B->d_coef = dalloc<double2>((size_t)n * 16, B->owned);
-  B->d_aaslots = dalloc<int>((size_t)n * 16, B->owned);
-  B->d_aacoef = dalloc<double>((size_t)n * 16, B->owned);
   B->status.assign(n, 0);
   if (share_enabled() && share_eligible(ss)) build_shared(*B);
   return B;
@@ -1480,7 +1453,11 @@ bool fork_enabled() {
   return !(e && atoi(e) == 0);
 }
 
-void residual_launches(Batch &B, int prec, bool timing) {
+// One residual of every active solve.  mode 0: R alone, from T as it is; 1 and 2:
+// an iteration of the solve loop under d_ctrl, T formed first where the last
+// update left it to that, the reference's or the Anderson update in the closing
+// pass, and its sums in B.results once the stream is done.
+void residual_launches(Batch &B, int prec, int mode, bool timing) {
   const int n = (int)B.solves.size();
   hipStream_t st = B.stream;
   const int terms = term_mask();
@@ -1501,24 +1478,30 @@ void residual_launches(Batch &B, int prec, bool timing) {
   const bool tiles64 = B.f64.ready && fp64_tiles();
   auto t64 = [&](int bit) { return tiles64 && pf(bit) == CCGPU_PREC_FP64; };
   // Three streams outside the timing mode (fork/join through events, also
-  // inside a captured graph).  The ring chain (T -> T~, I4, R~) reads only T
-  // and the ring blocks and touches R only in the final scatter: a second
-  // stream from the start of the residual, beside the one-body intermediates,
-  // whose small launches leave most of the chip idle, and beside the ladders,
-  // which stream V_pppp from HBM while the ring GEMMs keep the matrix cores
-  // busy.  A third stream takes I6 (rows of V* against rows of T) and the split
-  // copy of T for the BF16x3 pp ladder, both joined before the residual start,
-  // then the hh ladder into Rh once X is done, joined before the scatter that
-  // adds it: R = (Rh + R) + ring, the order of the single-stream sums.
+  // inside a captured graph), from the opening pass on.  The ring contractions
+  // read only T and the ring blocks and touch R only in the closing pass: a
+  // second stream, beside the one-body intermediates, whose small launches leave
+  // most of the chip idle, and beside the ladders, which stream V_pppp from HBM
+  // while the ring keeps the matrix cores busy.  A third stream takes I6 (rows
+  // of V* against rows of T), then the hh ladder into Rh once X is done.  All
+  // three meet in the closing pass.
   const bool fork = !timing && (terms & 8) && fork_enabled();
   const bool fork6 = !timing && fork_enabled();
   hipStream_t sr = fork ? B.stream2 : st;
   hipStream_t s6 = fork6 ? B.stream3 : st;
   // BF16x3 ring on the FP32 ring blocks when every solve has them
   const bool ring32 = pf(3) == CCGPU_PREC_BF16X3 && B.ring32;
-  // BF16x3 reads T split once (k_t_split) rather than per wave and row tile;
+  // BF16x3 reads T split once (in the opening pass) rather than per wave and row tile;
   // CCGPU_PPL_TSPLIT=0 keeps the in-kernel split (same bits)
   const bool tsplit = (terms & 2) && !B.share.on && pp_prec == CCGPU_PREC_BF16X3 && B.ppbf && tsplit_enabled();
+  const bool shared = (terms & 2) && B.share.on;
+  {
+    Timer t(timing, st, shared ? "pp_share_gather" : "ring_gather");
+    const int ring = !(terms & 8) ? 0 : ring32 ? 2 : 1;
+    if (ring || tsplit || shared || mode)
+      launch_t_begin(B.d_descs, B.d_ctrl, n, B.maxT, ring, mode != 0, tsplit, shared ? B.share.d_maps : nullptr,
+                     B.share.Tu, st);
+  }
   if (fork || fork6) HIPCHK(hipEventRecord(B.ev_fork, st));
   if (fork) HIPCHK(hipStreamWaitEvent(sr, B.ev_fork, 0));
   if (fork6) HIPCHK(hipStreamWaitEvent(s6, B.ev_fork, 0));
@@ -1527,11 +1510,6 @@ void residual_launches(Batch &B, int prec, bool timing) {
     Timer t(timing, s6, "i6");
     launch_i6(B.d_descs, n, B.maxNp, B.maxRows, s6);
   }
-  if (tsplit) {
-    Timer t(timing, s6, "pp_t_split");
-    launch_t_split(B.d_descs, n, B.maxT, s6);
-  }
-  if (fork6) HIPCHK(hipEventRecord(B.ev_join3, s6));
   {
     Timer t(timing, st, "gemm_x_vhhpp_t");
     if (t64(0)) launch_x64(B.f64.x, B.f64.nx, B.d_descs, st);
@@ -1553,10 +1531,6 @@ void residual_launches(Batch &B, int prec, bool timing) {
   }
   if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
   if (terms & 8) {
-    {
-      Timer t(timing, sr, "ring_gather");
-      launch_ring_gather(B.d_descs, n, B.maxT, ring32, sr);
-    }
     B.i4_in_lds = t64(3);
     if (t64(3)) {
       Timer t(timing, sr, "gemm_ring");
@@ -1576,41 +1550,28 @@ void residual_launches(Batch &B, int prec, bool timing) {
       else run_gemm(list(B.g_rt, B.g_rtb, 3), B, pf(3), false, sr);
     }
   }
-  if (fork6) HIPCHK(hipStreamWaitEvent(st, B.ev_join3, 0));
-  {
-    Timer t(timing, st, "resid_init_onebody");
-    launch_resid_init(B.d_descs, n, B.maxT, (terms & 1) != 0, st);
-  }
-  if ((terms & 2) && B.share.on) {
-    // shared pp ladder: FP64 GEMMs on V_u, or BF16x3 on its FP32 copy in every
-    // low-precision mode
-    {
-      Timer t(timing, st, "pp_share_gather");
-      launch_share_gather(B.d_descs, n, B.maxT, B.share.d_maps, B.share.Tu, st);
-    }
-    {
-      Timer t(timing, st, "gemm_pp_ladder");
+  if (terms & 2) {
+    Timer t(timing, st, "gemm_pp_ladder");
+    if (shared) {
+      // FP64 GEMMs on V_u, or BF16x3 on its FP32 copy in every low-precision mode
       if (pp_prec == CCGPU_PREC_FP64) run_gemm(B.share.g64, B, CCGPU_PREC_FP64, false, st, false, 0);
       else run_gemm(B.share.gbf, B, CCGPU_PREC_BF16X3, true, st, false, 7);
+    } else if (tsplit) {
+      run_gemm(B.g_ppbf, B, pp_prec, true, st, true, 10);
+    } else if (pp_prec != CCGPU_PREC_FP64) {
+      run_gemm(B.g_pp32, B, pp_prec, true, st, true);
+    } else {
+      run_gemm(B.g_pp, B, pp_prec, false, st, true);
     }
-    {
-      Timer t(timing, st, "pp_share_scatter");
-      launch_share_scatter(B.d_descs, n, B.maxT, B.share.d_maps, B.share.Ru, st);
-    }
-  } else if (terms & 2) {
-    Timer t(timing, st, "gemm_pp_ladder");
-    if (tsplit) run_gemm(B.g_ppbf, B, pp_prec, true, st, true, 10);
-    else if (pp_prec != CCGPU_PREC_FP64) run_gemm(B.g_pp32, B, pp_prec, true, st, true);
-    else run_gemm(B.g_pp, B, pp_prec, false, st, true);
   }
   if (fork) {
     HIPCHK(hipEventRecord(B.ev_join, sr));
     HIPCHK(hipStreamWaitEvent(st, B.ev_join, 0));
   }
   if (fork6) HIPCHK(hipStreamWaitEvent(st, B.ev_hh, 0));
-  if (terms & 12) {
-    Timer t(timing, st, "ring_scatter");
-    launch_ring_scatter(B.d_descs, n, B.maxT, ring32, (terms & 8) != 0, (terms & 4) != 0, st);
+  {
+    Timer t(timing, st, mode == 0 ? "residual_sum" : mode == 1 ? "residual_sum_update" : "residual_sum_anderson");
+    launch_t_end(B.d_descs, B.d_ctrl, n, ring32, mode, terms, shared ? B.share.d_maps : nullptr, B.share.Ru, B.results, st);
   }
 }
 
@@ -1627,42 +1588,36 @@ int forced_singular() {
   return e ? atoi(e) : -1;
 }
 
-// Update of every active solve (diis_t1t2, ccm_diis.f90:74-249); all active solves
-// of a batch share count/nstep because they start together.
-void update_launches(Batch &B, int &count, int &nstep, int subspace, int diis_step, bool timing) {
-  const int n = (int)B.solves.size();
-  hipStream_t st = B.stream;
-  // history column handling: shift when full (ring buffer)
-  std::vector<int> &slot = B.h_slot, &slots = B.h_slots;
-  slot.assign(n, 0);
-  slots.assign((size_t)n * 16, 0);
-  for (int s = 0; s < n; ++s) {
+// History column of the next update of every solve (diis_t1t2,
+// ccm_diis.f90:74-249): a ring buffer that drops its oldest column when full.
+// All active solves of a batch share count/nstep because they start together.
+void next_column(Batch &B, int &nstep, int subspace) {
+  for (size_t s = 0; s < B.solves.size(); ++s) {
     Solve &S = *B.solves[s];
-    if (nstep > subspace) {
-      // drop the oldest column
-      std::rotate(S.ring.begin(), S.ring.begin() + 1, S.ring.begin() + subspace);
-    }
-    slot[s] = S.ring[std::min(nstep, subspace) - 1];
+    if (nstep > subspace) std::rotate(S.ring.begin(), S.ring.begin() + 1, S.ring.begin() + subspace);
+    B.ctrl[s].fresh = S.ring[std::min(nstep, subspace) - 1];
   }
   if (nstep > subspace) nstep = subspace;
-  HIPCHK(hipMemcpyAsync(B.d_slot, slot.data(), n * sizeof(int), hipMemcpyHostToDevice, st));
-  {
-    Timer t(timing, st, "update");
-    launch_update(B.d_descs, n, B.maxT, B.d_slot, st);
-  }
-  if (count != diis_step) return;
+}
+
+// The extrapolation due every diis_step updates.  True: it formed T.
+bool extrapolate(Batch &B, int &count, int nstep, int diis_step, bool timing) {
+  const int n = (int)B.solves.size();
+  hipStream_t st = B.stream;
+  std::vector<int> &slots = B.h_slots;
+  slots.assign((size_t)n * 16, 0);
+  if (count != diis_step) return false;
   count = 0;
-  if (nstep < 2) return;
+  if (nstep < 2) return false;
   for (int s = 0; s < n; ++s)
     for (int k = 0; k < nstep; ++k) slots[(size_t)s * 16 + k] = B.solves[s]->ring[k];
   h2d_pinned(B, 4, B.d_slots, slots.data(), slots.size() * sizeof(int), st);
-  std::vector<double2> &sc = B.h_scal;
-  sc.assign((size_t)n * 64, double2{0, 0});
+  const double2 *sc = B.results;
   {
     Timer t(timing, st, "diis_gram");
-    launch_gram(B.d_descs, n, B.d_slots, nstep, st);
+    launch_gram(B.d_descs, n, B.d_slots, nstep, B.results, st);
     check_launch();
-    d2h_pinned_sync(B, 3, sc.data(), B.d_scal, sc.size() * sizeof(double2), st);
+    HIPCHK(hipStreamSynchronize(st));
   }
   std::vector<double2> &coef = B.h_coef;
   coef.assign((size_t)n * 16, double2{0, 0});
@@ -1701,24 +1656,26 @@ void update_launches(Batch &B, int &count, int &nstep, int subspace, int diis_st
     Timer t(timing, st, "diis_axpy");
     launch_diis_axpy(B.d_descs, n, B.maxT, B.d_slots, B.d_coef, ne, st);
   }
+  return true;
 }
 
 // one sum over the triples, defined with the (T) entry points below
 double2 triples_sum(Solve &S, int mode);
 
+// the energies a reduction left in results 0, once the stream is done
+std::vector<std::complex<double>> energy_results(Batch &B) {
+  HIPCHK(hipStreamSynchronize(B.stream));
+  std::vector<std::complex<double>> e;
+  for (size_t s = 0; s < B.solves.size(); ++s) e.emplace_back(B.results[s * 64].x, B.results[s * 64].y);
+  return e;
+}
 std::vector<std::complex<double>> energies(Batch &B, bool timing) {
-  const int n = (int)B.solves.size();
   {
     Timer t(timing, B.stream, "energy");
-    launch_energy(B.d_descs, n, 0, B.stream);
+    launch_energy(B.d_descs, (int)B.solves.size(), B.results, B.stream);
   }
   check_launch();
-  std::vector<double2> &sc = B.h_scal;
-  sc.assign((size_t)n * 64, double2{0, 0});
-  d2h_pinned_sync(B, 3, sc.data(), B.d_scal, sc.size() * sizeof(double2), B.stream);
-  std::vector<std::complex<double>> e(n);
-  for (int s = 0; s < n; ++s) e[s] = std::complex<double>(sc[(size_t)s * 64].x, sc[(size_t)s * 64].y);
-  return e;
+  return energy_results(B);
 }
 
 // Solution of min |sum_j c_j f_j|^2 subject to sum_j c_j = 1 for the Gram
@@ -1768,17 +1725,15 @@ bool anderson_coefficients(const std::vector<double> &G, int m, std::vector<doub
   return true;
 }
 
-// One Anderson step of every active solve after its residual: k_aa_update
-// forms f, y and the new Gram row; the host appends the row, solves for the
-// coefficients (dropping the oldest vectors while the scaled system is near
-// singular) and uploads them for k_aa_combine, which forms the next iterate at
-// the start of the next iteration.  Returns the correlation energy of the next
-// iterate, sum_j c_j E(y_j) (the energy is linear in T).
-std::vector<std::complex<double>> anderson_step(Batch &B, int depth, double beta, bool timing) {
-  const int n = (int)B.solves.size();
-  hipStream_t st = B.stream;
-  B.h_aaslots.assign((size_t)n * 16, 0);
-  for (int s = 0; s < n; ++s) {
+// One Anderson step of every active solve.  Before its residual the held
+// vectors and the column of the new pair are fixed (anderson_columns); the
+// residual's closing pass forms f, y and the new Gram row; then the host appends
+// the row and solves for the coefficients (dropping the oldest vectors while the
+// scaled system is near singular), with which the next residual's opening pass
+// forms the next iterate (anderson_step).
+void anderson_columns(Batch &B, int depth, double beta) {
+  for (size_t s = 0; s < B.solves.size(); ++s) {
+    if (!B.h_descs[s].active) continue;
     Batch::AA &q = B.aa[s];
     int m = (int)q.slot.size();
     int fresh = -1;
@@ -1795,33 +1750,32 @@ std::vector<std::complex<double>> anderson_step(Batch &B, int depth, double beta
       for (int c = 0; c < depth && fresh < 0; ++c)
         if (std::find(q.slot.begin(), q.slot.end(), c) == q.slot.end()) fresh = c;
     }
-    for (int j = 0; j < m; ++j) B.h_aaslots[(size_t)s * 16 + j] = q.slot[j];
-    B.h_aaslots[(size_t)s * 16 + 14] = fresh;
-    B.h_aaslots[(size_t)s * 16 + 15] = m;
+    IterCtrl &t = B.ctrl[s];
+    for (int j = 0; j < m; ++j) t.held[j] = q.slot[j];
+    t.m = m;
+    t.fresh = fresh;
+    t.beta = beta;
   }
-  h2d_pinned(B, 0, B.d_aaslots, B.h_aaslots.data(), B.h_aaslots.size() * sizeof(int), st);
-  {
-    Timer t(timing, st, "anderson_update");
-    launch_aa_update(B.d_descs, n, B.d_aaslots, beta, st);
-  }
-  check_launch();
-  std::vector<double2> &sc = B.h_scal;
-  sc.assign((size_t)n * 64, double2{0, 0});
-  d2h_pinned_sync(B, 3, sc.data(), B.d_scal, sc.size() * sizeof(double2), st);
+}
+
+// Returns the correlation energy of the next iterate, sum_j c_j E(y_j) (the
+// energy is linear in T).
+std::vector<std::complex<double>> anderson_step(Batch &B) {
+  const int n = (int)B.solves.size();
+  HIPCHK(hipStreamSynchronize(B.stream));
   std::vector<std::complex<double>> e(n, 0.0);
-  B.h_aacoef.assign((size_t)n * 16, 0.0);
   for (int s = 0; s < n; ++s) {
     if (!B.h_descs[s].active) continue;
     Batch::AA &q = B.aa[s];
     const int m = (int)q.slot.size();
-    const double2 *v = &sc[(size_t)s * 64 + 24];
+    const double2 *v = &B.results[(size_t)s * 64 + 24];
     std::vector<double> g((size_t)(m + 1) * (m + 1));
     for (int j = 0; j < m; ++j)
       for (int k = 0; k < m; ++k) g[(size_t)j * (m + 1) + k] = q.gram[(size_t)j * m + k];
     for (int j = 0; j < m; ++j) g[(size_t)j * (m + 1) + m] = g[(size_t)m * (m + 1) + j] = v[j].x;
     g[(size_t)m * (m + 1) + m] = v[m].x;
     q.gram.swap(g);
-    q.slot.push_back(B.h_aaslots[(size_t)s * 16 + 14]);
+    q.slot.push_back(B.ctrl[s].fresh);
     q.ey.emplace_back(v[16].x, v[16].y);
     std::vector<double> c;
     const bool forced = s == forced_singular() && !B.forced_done && q.slot.size() >= 2;
@@ -1848,15 +1802,14 @@ std::vector<std::complex<double>> anderson_step(Batch &B, int depth, double beta
       q.ey.erase(q.ey.begin());
     }
     const int mm = (int)q.slot.size();
+    IterCtrl &t = B.ctrl[s];
     for (int j = 0; j < mm; ++j) {
-      B.h_aaslots[(size_t)s * 16 + j] = q.slot[j];
-      B.h_aacoef[(size_t)s * 16 + j] = c[j];
+      t.from[j] = q.slot[j];
+      t.c[j] = c[j];
       e[s] += c[j] * q.ey[j];
     }
-    B.h_aaslots[(size_t)s * 16 + 15] = mm;
+    t.np = mm;
   }
-  h2d_pinned(B, 1, B.d_aaslots, B.h_aaslots.data(), B.h_aaslots.size() * sizeof(int), st);
-  h2d_pinned(B, 2, B.d_aacoef, B.h_aacoef.data(), B.h_aacoef.size() * sizeof(double), st);
   return e;
 }
 
@@ -1942,14 +1895,18 @@ void run_batch(Batch &B, const ccgpu_solve_opts &op, std::vector<ccgpu_solve_res
   // fall between two larger ones before the iterate has settled
   const int need = op.confirm > 0 ? op.confirm : (aa ? 2 : 1);
   std::vector<int> small(n, 0);
-  bool pending = false;   // Anderson: coefficients uploaded, next iterate not yet formed
+  // The update leaves the next iterate to the next residual's opening pass, as a
+  // combination of history columns (one column for the reference's update), also
+  // for a solve that has just met its test.
+  B.ctrl.assign(n, IterCtrl{});
+  // the iterate alone, where something else needs it first
+  auto form_t = [&] {
+    upload_ctrl(B);
+    Timer t(timing, B.stream, "form_t");
+    launch_t_begin(B.d_descs, B.d_ctrl, n, B.maxT, 0, true, false, nullptr, nullptr, B.stream);
+    check_launch();
+  };
   for (int it = 1; it <= op.maxit; ++it) {
-    if (pending) {
-      Timer t(timing, B.stream, "anderson_combine");
-      launch_aa_combine(B.d_descs, n, B.maxT, B.d_aaslots, B.d_aacoef, B.stream);
-      check_launch();
-      pending = false;
-    }
     bool any = false;
     for (int s = 0; s < n; ++s) {
       bool act = !failed[s] && (fp32_phase ? B.h_descs[s].active != 0 : small[s] < need);
@@ -1971,39 +1928,56 @@ void run_batch(Batch &B, const ccgpu_solve_opts &op, std::vector<ccgpu_solve_res
         low = false;
       }
     }
-    if (ccdt1)
+    ++count;
+    ++nstep;
+    if (aa) anderson_columns(B, op.subspace, beta);
+    else next_column(B, nstep, op.subspace);
+    if (ccdt1) {
+      form_t();
       for (int s = 0; s < n; ++s) {
+        B.ctrl[s].np = 0;
         if (!B.h_descs[s].active) continue;
         Solve &S = *B.solves[s];
         S.ccdt1_e3 = triples_sum(S, 1);
         e3[s] = std::complex<double>(S.ccdt1_e3.x, S.ccdt1_e3.y);
       }
+    }
+    upload_ctrl(B);
+    const int mode = aa ? 2 : 1;
     if (graph_ok) {
-      const int q = prec;
+      const int q = prec + (aa ? 4 : 0);
       if (!B.gexec[q]) {
         HIPCHK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
-        residual_launches(B, prec, false);
+        residual_launches(B, prec, mode, false);
         HIPCHK(hipStreamEndCapture(B.stream, &B.graph[q]));
         HIPCHK(hipGraphInstantiate(&B.gexec[q], B.graph[q], nullptr, nullptr, 0));
       }
       HIPCHK(hipGraphLaunch(B.gexec[q], B.stream));
     } else {
-      residual_launches(B, prec, timing);
+      residual_launches(B, prec, mode, timing);
     }
     check_launch();
-    ++count;
-    ++nstep;
+    for (IterCtrl &t : B.ctrl) t.np = 0;
     std::vector<std::complex<double>> e2;
     bool extrapolated;
     if (aa) {
-      e2 = anderson_step(B, op.subspace, beta, timing);
-      pending = true;
+      e2 = anderson_step(B);
       extrapolated = true;
     } else {
-      update_launches(B, count, nstep, op.subspace, op.diis_step, timing);
+      const bool formed = extrapolate(B, count, nstep, op.diis_step, timing);
       check_launch();
       extrapolated = count == 0;
-      e2 = energies(B, timing);
+      if (formed) {
+        e2 = energies(B, timing);
+      } else {
+        e2 = energy_results(B);
+        for (int s = 0; s < n; ++s)
+          if (B.h_descs[s].active) {
+            B.ctrl[s].np = 1;
+            B.ctrl[s].from[0] = B.ctrl[s].fresh;
+            B.ctrl[s].c[0] = 1.0;
+          }
+      }
     }
     double maxd = 0;
     for (int s = 0; s < n; ++s) {
@@ -2048,10 +2022,7 @@ void run_batch(Batch &B, const ccgpu_solve_opts &op, std::vector<ccgpu_solve_res
     }
     if (!extrapolated || aa) prev_maxd = maxd;
   }
-  if (pending) {   // the iterate of the last Anderson step (iteration cap)
-    launch_aa_combine(B.d_descs, n, B.maxT, B.d_aaslots, B.d_aacoef, B.stream);
-    check_launch();
-  }
+  form_t();   // the iterate of the last update
   HIPCHK(hipStreamSynchronize(B.stream));
   double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   for (int s = 0; s < n; ++s) {
@@ -2748,7 +2719,7 @@ int ccgpu_residual(int handle, int precision) {
     if (precision != CCGPU_PREC_FP64) ensure_f32(S, handle);
     Batch &B = single(handle);
     prepare_lists(B, precision);
-    residual_launches(B, precision, false);
+    residual_launches(B, precision, 0, false);
     check_launch();
     HIPCHK(hipStreamSynchronize(B.stream));
   });
@@ -2769,7 +2740,10 @@ int ccgpu_update(int handle, int *count, int *nstep, int subspace, int diis_step
       for (int k = 0; k < subspace; ++k) S.ring[k] = k;
     }
     int c = *count, n = *nstep;
-    update_launches(B, c, n, subspace, diis_step, false);
+    next_column(B, n, subspace);
+    upload_ctrl(B);
+    launch_update(B.d_descs, 1, B.maxT, B.d_ctrl, B.stream);
+    extrapolate(B, c, n, diis_step, false);
     check_launch();
     HIPCHK(hipStreamSynchronize(B.stream));
     *count = c;

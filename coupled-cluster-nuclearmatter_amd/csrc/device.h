@@ -46,7 +46,7 @@ struct SolveDesc {
   const int *ring4;   // four Pandya positions per unique amplitude (every ring block below 2^31 elements)
   // amplitudes and blocks
   double2 *T, *R, *R0, *Vhhpp, *Vhhhh, *X, *Vpppp;
-  double2 *Rh;   // hh ladder T I9 of the residual, added to R by the ring scatter
+  double2 *Rh;   // hh ladder T I9 of the residual, added to R by its closing pass
   float2 *Vpppp32;
   double2 *Tt, *Rt, *I4, *W0, *Vt;
   // FP32 ring blocks of the BF16x3 residual (null until the FP32 copies are
@@ -65,7 +65,16 @@ struct SolveDesc {
   double2 *hist;
   float2 *histf;
   double2 *red;             // reduction partials
-  double2 *scal;            // small scalar outputs (energy, Gram)
+};
+
+// What one iteration of the solve loop tells the kernels about one solve,
+// uploaded once per iteration.
+struct IterCtrl {
+  // T = sum_j c[j] hist[from[j]] over np columns opens the iteration; np = 0: T as it is
+  int np, from[8];
+  int fresh;          // the history column the update writes
+  int m, held[8];     // Anderson: columns of the held vectors, oldest first
+  double c[8], beta;
 };
 
 // One member of a grouped complex GEMM: C = alpha * A * B + beta * C0.

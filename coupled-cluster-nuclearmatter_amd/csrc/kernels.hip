@@ -421,51 +421,9 @@ __device__ __forceinline__ double2 amp_denominator(const SolveDesc &d, int64_t u
   const double2 hi = d.dh[i], hj = d.dh[j], pa = d.dp[a - d.A], pb = d.dp[b - d.A];
   return make_double2(hi.x + hj.x - pa.x - pb.x, hi.y + hj.y - pa.y - pb.y);
 }
-__device__ __forceinline__ void unique_labels(const SolveDesc &d, int64_t u, int &c, int &r, int &s) {
-  c = d.t_ch[u];
-  int64_t loc = u - d.off_t[c];
-  int nh = d.nhh[c];
-  r = (int)(loc / nh);
-  s = (int)(loc % nh);
-}
 
 // MBPT2 start t(ab,ij) = conj(<ij||ab>)/(f_ii+f_jj-f_aa-f_bb), zero denominators
 // skipped (setup_t_amplitudes, ccm_iter.f90:2351-2367).
-// Shared pp ladder of a batch of twists of one lattice (one V_pppp over the
-// union of their particle pairs, per (K, Tz) channel one GEMM whose columns
-// are the hole pairs of every twist side by side).  maps[s][u] = 2 p + (sign
-// < 0): the position p of solve s's unique amplitude u in the union block
-// (row: the pair's union row, column: the solve's column range), with the
-// orientation sign of the pair there.  Positions no solve owns stay zero.
-__global__ void k_share_gather(const SolveDesc *descs, const uint32_t *const *maps, double2 *Tu) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  const uint32_t *m = maps[blockIdx.y];
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t w = m[u];
-    const double2 t = d.T[u];
-    Tu[w >> 1] = (w & 1) ? make_double2(-t.x, -t.y) : t;
-  }
-}
-// R += the union product at each amplitude's position (active solves only)
-__global__ void k_share_scatter(const SolveDesc *descs, const uint32_t *const *maps, const double2 *Ru) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  const uint32_t *m = maps[blockIdx.y];
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t w = m[u];
-    const double2 r = Ru[w >> 1];
-    double2 x = d.R[u];
-    if (w & 1) {
-      x.x -= r.x;
-      x.y -= r.y;
-    } else {
-      x.x += r.x;
-      x.y += r.y;
-    }
-    d.R[u] = x;
-  }
-}
-
 __global__ void k_mbpt2(const SolveDesc *descs) {
   const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
   for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
@@ -503,15 +461,17 @@ __global__ void k_energy_partial(const SolveDesc *descs) {
   if (threadIdx.x == 0) d.red[blockIdx.x] = s;
 }
 
-// Pass 2: fixed-order sum of nparts partials into scal[slot].
-__global__ void k_reduce_final(const SolveDesc *descs, int nparts, int stride, int nvals, int slot) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  for (int v = 0; v < nvals; ++v) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int p = threadIdx.x; p < nparts; p += blockDim.x) acc = cadd(acc, d.red[(int64_t)p * stride + v]);
-    double2 s = block_sum(acc);
-    if (threadIdx.x == 0) d.scal[slot + v] = s;
-  }
+// Pass 2: fixed-order sum of nparts partials per value, one block per value,
+// straight into the host's pinned results (64 per solve).  One block for the 17
+// values of an Anderson step took 32 us, a chain of 17 x (4 loads, 9 barriers);
+// 5 us this.
+__global__ void k_reduce_final(const SolveDesc *descs, int nparts, int stride, int slot, double2 *out) {
+  const int v = blockIdx.x;
+  const double2 *red = descs[blockIdx.y].red;
+  double2 acc = make_double2(0.0, 0.0);
+  for (int p = threadIdx.x; p < nparts; p += blockDim.x) acc = cadd(acc, red[(int64_t)p * stride + v]);
+  const double2 s = block_sum(acc);
+  if (threadIdx.x == 0) out[blockIdx.y * 64 + slot + v] = s;
 }
 
 // I7(k,i) = f_ki + 1/2 sum_l sum_cd <kl||cd> t(cd,il) for k in {i, partner(i)}, read
@@ -631,112 +591,240 @@ __global__ void k_i9(const SolveDesc *descs) {
     d.X[n + e] = cadd(d.X[e], d.Vhhhh[e]);
 }
 
-// Residual start: R = conj(<ij||ab>) + P(ab) sum_c I6(b,c) t(ac,ij)
-//                 - P(ij) sum_k I7(k,j) t(ab,ik), diagonals removed
-// (ccm_t2_eqn.f90:81-211).  Owner-computes over unique elements.
-__global__ void k_resid_init(const SolveDesc *descs, int onebody) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    int c, r, s;
-    unique_labels(d, u, c, r, s);
-    const int64_t o = d.off_t[c];
-    const int nh = d.nhh[c];
-    const int64_t pr = d.off_pp[c] + r, hs = d.off_hh[c] + s;
-    int a = d.pp_a[pr], b = d.pp_b[pr], i = d.hh_i[hs], j = d.hh_j[hs];
-    double2 acc = d.R0[u];
-    if (!onebody) { d.R[u] = acc; continue; }
-    int vB = d.ob_rowB[pr];   // (a, partner(b))
-    if (vB >= 0) {
-      double2 tv = d.T[o + (int64_t)(vB >> 2) * nh + s];
-      acc = cadd(acc, cscale((double)((vB & 3) - 1), cmul(d.I6off[b - d.A], tv)));
-    }
-    int vA = d.ob_rowA[pr];   // (b, partner(a))
-    if (vA >= 0) {
-      double2 tv = d.T[o + (int64_t)(vA >> 2) * nh + s];
-      acc = csub(acc, cscale((double)((vA & 3) - 1), cmul(d.I6off[a - d.A], tv)));
-    }
-    int vJ = d.ob_colJ[hs];   // (i, partner(j))
-    if (vJ >= 0) {
-      double2 tv = d.T[o + (int64_t)r * nh + (vJ >> 2)];
-      acc = csub(acc, cscale((double)((vJ & 3) - 1), cmul(d.I7off[j], tv)));
-    }
-    int vI = d.ob_colI[hs];   // (j, partner(i))
-    if (vI >= 0) {
-      double2 tv = d.T[o + (int64_t)r * nh + (vI >> 2)];
-      acc = cadd(acc, cscale((double)((vI & 3) - 1), cmul(d.I7off[i], tv)));
-    }
-    d.R[u] = acc;
-  }
-}
+// T split for the BF16x3 pp ladder (its B operand (br, -bi)): the bits the
+// ladder's in-kernel split gives, computed once per amplitude instead of once
+// per wave and row tile
+__device__ __forceinline__ uint4 t_split(double2 b);
 
-// Pandya gather T~((a,i),(j,b)) = t(ab,ij) (ccm_t2_eqn.f90:37-62); F32: into
-// the FP32 blocks of the BF16x3 residual.  The four positions of an amplitude
-// are one 16-byte load.
-template <bool F32>
-__global__ void k_ring_gather(const SolveDesc *descs) {
+// The pass over the amplitudes that opens a residual: the next iterate
+// T = sum_j c_j hist_j where the last update left one (the Anderson
+// combination, or the one column of a plain step: c = 1 copies it), the Pandya
+// gather T~((a,i),(j,b)) = t(ab,ij) (ccm_t2_eqn.f90:37-62; the four positions
+// of an amplitude are one 16-byte load), and the operand of the pp ladder: T
+// split for BF16x3, or the columns of the shared union blocks.
+//
+// Shared pp ladder of a batch of twists of one lattice (one V_pppp over the
+// union of their particle pairs, per (K, Tz) channel one GEMM whose columns
+// are the hole pairs of every twist side by side).  maps[s][u] = 2 p + (sign
+// < 0): the position p of solve s's unique amplitude u in the union block
+// (row: the pair's union row, column: the solve's column range), with the
+// orientation sign of the pair there.  Positions no solve owns stay zero.
+//
+// Bound by the requests of the four scattered stores (PNM A=66 |n_i|<=4: 8 M
+// stores in 4.6 M requests, 250 MB to memory for 159 MB of T and T~): 70 us there, 346 us for eight
+// Anderson twists of |n_i|<=3.  As passes of their own, combination, gather and
+// shared gather took 390 us for the twists.
+template <int RING>   // 0 no ring, 1 FP64 blocks, 2 FP32 blocks of the BF16x3 residual
+__global__ __launch_bounds__(256) void k_t_begin(const SolveDesc *descs, const IterCtrl *ctrl, int form, int split,
+                                                 const uint32_t *const *maps, double2 *Tu) {
   const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const double2 t = d.T[u];
-    const int4 p = *(const int4 *)(d.ring4 + 4 * u);
-    if constexpr (F32) {
-      const float2 tf = make_float2((float)t.x, (float)t.y), mf = make_float2(-tf.x, -tf.y);
-      d.Tt32[p.x] = tf;
-      d.Tt32[p.y] = mf;
-      d.Tt32[p.z] = mf;
-      d.Tt32[p.w] = tf;
+  const IterCtrl q = ctrl[blockIdx.y];
+  const int np = form ? q.np : 0;
+  if (!np && (!d.active || (RING == 0 && !split && !maps))) return;
+  const uint32_t *m = maps ? maps[blockIdx.y] : nullptr;
+  const unsigned n = (unsigned)d.nT;
+  for (unsigned u = blockIdx.x * 256 + threadIdx.x; u < n; u += gridDim.x * 256) {
+    double2 t;
+    if (np) {
+      double2 h[8];   // every column's load in flight
+#pragma unroll
+      for (int p = 0; p < 8; ++p)
+        if (p < np) h[p] = d.hist[(int64_t)q.from[p] * d.nT + u];
+      t = cscale(q.c[0], h[0]);
+#pragma unroll
+      for (int p = 1; p < 8; ++p)
+        if (p < np) t = cadd(t, cscale(q.c[p], h[p]));
+      d.T[u] = t;
+      if (!d.active) continue;
     } else {
-      const double2 m = make_double2(-t.x, -t.y);
-      d.Tt[p.x] = t;
-      d.Tt[p.y] = m;
-      d.Tt[p.z] = m;
-      d.Tt[p.w] = t;
+      t = d.T[u];
+    }
+    const double2 mt = make_double2(-t.x, -t.y);
+    if constexpr (RING != 0) {
+      const int4 p = *(const int4 *)(d.ring4 + 4 * (int64_t)u);
+      if constexpr (RING == 2) {
+        const float2 tf = make_float2((float)t.x, (float)t.y), mf = make_float2(-tf.x, -tf.y);
+        d.Tt32[p.x] = tf;
+        d.Tt32[p.y] = mf;
+        d.Tt32[p.z] = mf;
+        d.Tt32[p.w] = tf;
+      } else {
+        d.Tt[p.x] = t;
+        d.Tt[p.y] = mt;
+        d.Tt[p.z] = mt;
+        d.Tt[p.w] = t;
+      }
+    }
+    if (split) d.Tbf[u] = t_split(t);
+    if (m) {
+      const uint32_t w = m[u];
+      Tu[w >> 1] = (w & 1) ? mt : t;
     }
   }
 }
 
-// Ring scatter with P(ab)P(ij) (ccm_t2_eqn.f90:1133-1185), owner-computes;
-// F32: from the FP32 R~ of the BF16x3 residual (summed in FP64).  With hh it
-// also adds the hh ladder's Rh first, R = (Rh + R) + ring: the order in which
-// the single-stream residual summed them.
-template <bool F32>
-__global__ void k_ring_scatter(const SolveDesc *descs, int ring, int hh) {
+// Jacobi step with mixing, t <- 0.75 t + 0.25 R/(dh_i+dh_j-dp_a-dp_b)
+// (diis_t1t2, ccm_diis.f90:106-126)
+__device__ __forceinline__ double2 jacobi_step(double2 t, double2 r, double2 den) {
+  return cadd(cscale(0.75, t), cscale(0.25, cdiv(r, den)));
+}
+
+// The pass over the amplitudes that closes a residual, and the update of the
+// solve loop.  Owner-computes per unique amplitude:
+//   R = conj(<ij||ab>) + P(ab) sum_c I6(b,c) t(ac,ij) - P(ij) sum_k I7(k,j) t(ab,ik),
+//       diagonals removed (ccm_t2_eqn.f90:81-211)
+//     + pp ladder (R itself, or the shared union product) + hh ladder
+//     + P(ab) P(ij) of the ring R~ (ccm_t2_eqn.f90:1133-1185; F32: from the FP32
+//       R~ of the BF16x3 residual, summed in FP64),
+// summed as (hh + (one-body + pp)) + ring.
+// MODE 0 stops there (the residual of the step-by-step interface).
+// MODE 1, the reference's update: the Jacobi step into history column q.fresh,
+//   and block partials of its energy sum t conj(R0) to red[block].
+// MODE 2, Anderson (Pulay) update of the fixed-point map g(T) = R(T)/D(T) with
+//   the dynamic denominators D = dh_i + dh_j - dp_a - dp_b: f = g(T) - T,
+//   y = T + beta f.  y goes to history column q.fresh (FP64), f to histf (FP32),
+//   and each block writes to red[36 block] its partial sums of Re<f_j, f> over
+//   the q.m held vectors j (oldest first) and of <f, f> (values 0..m, real part
+//   in .x), and of the energy of y (value 16).  The coefficients of the next
+//   iterate come from the host's solve of the bordered Gram system.  No
+//   counterpart in the reference, whose diis_t1t2 (ccm_diis.f90:74-249) mixes
+//   0.75/0.25 every iteration and extrapolates every diis_step iterations.
+// T itself is left alone: other threads read rows of it, and the next residual's
+// opening pass forms it from the history.
+//
+// Bound by the latency of the scattered R~ loads and by HBM.  One-body start, ring
+// scatter, update and energy as passes of their own took 130 us (PNM A=66
+// |n_i|<=4), 87 us this; with the shared scatter 585 us for eight Anderson twists
+// of |n_i|<=3, 338 us this.
+constexpr int kAAMax = 9;   // held vectors + the new one
+template <bool F32, int MODE>
+__global__ __launch_bounds__(256) void k_t_end(const SolveDesc *descs, const IterCtrl *ctrl, int terms,
+                                               const uint32_t *const *maps, const double2 *Ru) {
   const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
   if (!d.active) return;
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    double2 r = d.R[u];
-    if (hh) r = cadd(d.Rh[u], r);
-    if (ring) {
-      const int4 p = *(const int4 *)(d.ring4 + 4 * u);
-      double2 r0, r1, r2, r3;
-      if constexpr (F32) {
-        const float2 a = d.Rt32[p.x], b = d.Rt32[p.y], c = d.Rt32[p.z], e = d.Rt32[p.w];
-        r0 = make_double2(a.x, a.y);
-        r1 = make_double2(b.x, b.y);
-        r2 = make_double2(c.x, c.y);
-        r3 = make_double2(e.x, e.y);
+  const IterCtrl q = ctrl[blockIdx.y];
+  const uint32_t *map = maps ? maps[blockIdx.y] : nullptr;
+  double2 *y = nullptr;
+  float2 *fn = nullptr;
+  if constexpr (MODE != 0) y = d.hist + (int64_t)q.fresh * d.nT;
+  if constexpr (MODE == 2) fn = d.histf + (int64_t)q.fresh * d.nT;
+  double acc[MODE == 2 ? kAAMax : 1];
+  double2 e = make_double2(0.0, 0.0);
+#pragma unroll
+  for (double &a : acc) a = 0.0;
+  const unsigned n = (unsigned)d.nT;
+  for (unsigned u = blockIdx.x * 256 + threadIdx.x; u < n; u += gridDim.x * 256) {
+    const int c = d.t_ch[u];
+    const uint64_t lab = d.lab[u];
+    const double2 r0 = d.R0[u];
+    double2 r = r0, t = make_double2(0.0, 0.0);
+    if (MODE != 0) t = d.T[u];
+    float2 g[kAAMax - 1];
+    if constexpr (MODE == 2)
+#pragma unroll
+      for (int v = 0; v < kAAMax - 1; ++v)
+        if (v < q.m) g[v] = d.histf[(int64_t)q.held[v] * d.nT + u];
+    const int a = (int)(lab & 0xffff), b = (int)((lab >> 16) & 0xffff);
+    const int i = (int)((lab >> 32) & 0xffff), j = (int)(lab >> 48);
+    if (terms & 1) {
+      const int64_t o = d.off_t[c];
+      const unsigned nh = (unsigned)d.nhh[c], loc = u - (unsigned)o, row = loc / nh, s = loc - row * nh;
+      const int64_t pr = d.off_pp[c] + row, hs = d.off_hh[c] + s;
+      const double2 *T = d.T + o;
+      const int vB = d.ob_rowB[pr], vA = d.ob_rowA[pr];   // (a, partner(b)), (b, partner(a))
+      const int vJ = d.ob_colJ[hs], vI = d.ob_colI[hs];   // (i, partner(j)), (j, partner(i))
+      if (vB >= 0)
+        r = cadd(r, cscale((double)((vB & 3) - 1), cmul(d.I6off[b - d.A], T[(unsigned)(vB >> 2) * nh + s])));
+      if (vA >= 0)
+        r = csub(r, cscale((double)((vA & 3) - 1), cmul(d.I6off[a - d.A], T[(unsigned)(vA >> 2) * nh + s])));
+      if (vJ >= 0) r = csub(r, cscale((double)((vJ & 3) - 1), cmul(d.I7off[j], T[row * nh + (vJ >> 2)])));
+      if (vI >= 0) r = cadd(r, cscale((double)((vI & 3) - 1), cmul(d.I7off[i], T[row * nh + (vI >> 2)])));
+    }
+    if (terms & 2) {
+      if (map) {
+        const uint32_t w = map[u];
+        const double2 v = Ru[w >> 1];
+        r = (w & 1) ? csub(r, v) : cadd(r, v);
       } else {
-        r0 = d.Rt[p.x];
-        r1 = d.Rt[p.y];
-        r2 = d.Rt[p.z];
-        r3 = d.Rt[p.w];
+        r = cadd(r, d.R[u]);
       }
-      r = cadd(r, csub(csub(cadd(r0, r3), r1), r2));
+    }
+    if (terms & 4) r = cadd(d.Rh[u], r);
+    if (terms & 8) {
+      const int4 p = *(const int4 *)(d.ring4 + 4 * (int64_t)u);
+      double2 v0, v1, v2, v3;
+      if constexpr (F32) {
+        const float2 f0 = d.Rt32[p.x], f1 = d.Rt32[p.y], f2 = d.Rt32[p.z], f3 = d.Rt32[p.w];
+        v0 = make_double2(f0.x, f0.y);
+        v1 = make_double2(f1.x, f1.y);
+        v2 = make_double2(f2.x, f2.y);
+        v3 = make_double2(f3.x, f3.y);
+      } else {
+        v0 = d.Rt[p.x];
+        v1 = d.Rt[p.y];
+        v2 = d.Rt[p.z];
+        v3 = d.Rt[p.w];
+      }
+      r = cadd(r, csub(csub(cadd(v0, v3), v1), v2));
     }
     d.R[u] = r;
+    if constexpr (MODE != 0) {
+      const double2 hi = d.dh[i], hj = d.dh[j], pa = d.dp[a - d.A], pb = d.dp[b - d.A];
+      const double2 den = make_double2(hi.x + hj.x - pa.x - pb.x, hi.y + hj.y - pa.y - pb.y);
+      double2 yv;
+      if constexpr (MODE == 1) {
+        yv = jacobi_step(t, r, den);
+      } else {
+        const double2 f = csub(cdiv(r, den), t);
+        yv = cadd(t, cscale(q.beta, f));
+        const float2 f32 = make_float2((float)f.x, (float)f.y);
+        fn[u] = f32;
+        const double fr = f32.x, fi = f32.y;
+#pragma unroll
+        for (int v = 0; v < kAAMax - 1; ++v)
+          if (v < q.m) acc[v] += (double)g[v].x * fr + (double)g[v].y * fi;
+        acc[kAAMax - 1] += fr * fr + fi * fi;
+      }
+      y[u] = yv;
+      e = cadd(e, cmul(yv, cconj(r0)));
+    }
+  }
+  if constexpr (MODE == 1) {
+    const double2 s = block_sum(e);
+    if (threadIdx.x == 0) d.red[blockIdx.x] = s;
+  }
+  if constexpr (MODE == 2) {
+    // fixed-order block sums (pairwise tree over the 256 threads)
+    __shared__ double sv[kAAMax + 2][256];
+    const int x = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kAAMax; ++k) sv[k][x] = acc[k];
+    sv[kAAMax][x] = e.x;
+    sv[kAAMax + 1][x] = e.y;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (x < w)
+#pragma unroll
+        for (int k = 0; k < kAAMax + 2; ++k) sv[k][x] += sv[k][x + w];
+      __syncthreads();
+    }
+    if (x < 17) {
+      double2 v = make_double2(0.0, 0.0);
+      if (x < q.m) v.x = sv[x][0];
+      else if (x == q.m) v.x = sv[kAAMax - 1][0];
+      else if (x == 16) v = make_double2(sv[kAAMax][0], sv[kAAMax + 1][0]);
+      d.red[(int64_t)blockIdx.x * 36 + x] = v;
+    }
   }
 }
 
-// Jacobi step with mixing, t <- 0.75 t + 0.25 R/(dh_i+dh_j-dp_a-dp_b), and the
-// history write of diis_t1t2 (ccm_diis.f90:106-126).
-__global__ void k_update(const SolveDesc *descs, const int *slot) {
+// The update of the step-by-step interface, and its history write.
+__global__ void k_update(const SolveDesc *descs, const IterCtrl *ctrl) {
   const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
   if (!d.active) return;
-  double2 *h = d.hist + (int64_t)slot[blockIdx.y] * d.nT;
+  double2 *h = d.hist + (int64_t)ctrl[blockIdx.y].fresh * d.nT;
   for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const double2 den = amp_denominator(d, u);
-    double2 t = cadd(cscale(0.75, d.T[u]), cscale(0.25, cdiv(d.R[u], den)));
+    const double2 t = jacobi_step(d.T[u], d.R[u], amp_denominator(d, u));
     d.T[u] = t;
     h[u] = t;
   }
@@ -817,84 +905,6 @@ __global__ __launch_bounds__(256) void k_gram_partial(const SolveDesc *descs, co
       if ((x & 7) == 0 && q < NP) d.red[(int64_t)blockIdx.x * 36 + q] = v[0];
     }
     __syncthreads();   // sv is rewritten by the next pass
-  }
-}
-
-// Anderson (Pulay) update of the fixed-point map g(T) = R(T)/D(T) with the
-// dynamic denominators D = dh_i + dh_j - dp_a - dp_b of the residual:
-// f = g(T) - T, y = T + beta f.  y goes to history slot sl[14] (FP64), f to
-// histf (FP32), and each block writes its partial sums of Re<f_j, f> over
-// the m = sl[15] held vectors j (slots sl[0..m-1], oldest first) and of
-// <f, f> (values 0..m, real part in .x), and of the correlation energy of y,
-// sum y conj(R0) (value 16).  The coefficients of the next iterate come from
-// the host's solve of the bordered Gram system.  No counterpart in the
-// reference, whose diis_t1t2 (ccm_diis.f90:74-249) mixes 0.75/0.25 every
-// iteration and extrapolates every diis_step iterations.
-constexpr int kAAMax = 9;   // held vectors + the new one
-__global__ __launch_bounds__(256) void k_aa_update(const SolveDesc *descs, const int *slots, double beta) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  const int *sl = slots + blockIdx.y * 16;
-  const int m = sl[15];
-  double2 *y = d.hist + (int64_t)sl[14] * d.nT;
-  float2 *fn = d.histf + (int64_t)sl[14] * d.nT;
-  double acc[kAAMax];
-#pragma unroll
-  for (int q = 0; q < kAAMax; ++q) acc[q] = 0.0;
-  double2 ey = make_double2(0.0, 0.0);
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const double2 den = amp_denominator(d, u);
-    const double2 t = d.T[u];
-    const double2 f = csub(cdiv(d.R[u], den), t);
-    const double2 yv = cadd(t, cscale(beta, f));
-    y[u] = yv;
-    const float2 f32 = make_float2((float)f.x, (float)f.y);
-    fn[u] = f32;
-    const double fr = f32.x, fi = f32.y;
-#pragma unroll
-    for (int q = 0; q < kAAMax - 1; ++q)
-      if (q < m) {
-        const float2 g = d.histf[(int64_t)sl[q] * d.nT + u];
-        acc[q] += (double)g.x * fr + (double)g.y * fi;
-      }
-    acc[kAAMax - 1] += fr * fr + fi * fi;
-    ey = cadd(ey, cmul(yv, cconj(d.R0[u])));
-  }
-  // fixed-order block sums (pairwise tree over the 256 threads)
-  __shared__ double sv[kAAMax + 2][256];
-  const int x = threadIdx.x;
-#pragma unroll
-  for (int q = 0; q < kAAMax; ++q) sv[q][x] = acc[q];
-  sv[kAAMax][x] = ey.x;
-  sv[kAAMax + 1][x] = ey.y;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (x < w)
-#pragma unroll
-      for (int q = 0; q < kAAMax + 2; ++q) sv[q][x] += sv[q][x + w];
-    __syncthreads();
-  }
-  if (x < 17) {
-    double2 v = make_double2(0.0, 0.0);
-    if (x < m) v.x = sv[x][0];
-    else if (x == m) v.x = sv[kAAMax - 1][0];
-    else if (x == 16) v = make_double2(sv[kAAMax][0], sv[kAAMax + 1][0]);
-    d.red[(int64_t)blockIdx.x * 36 + x] = v;
-  }
-}
-
-// Next iterate of the Anderson update: T = sum_j c_j y_j over the m = sl[15]
-// held vectors (slots sl[0..m-1]); real coefficients coef[16 s + j].
-__global__ void k_aa_combine(const SolveDesc *descs, const int *slots, const double *coef) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  const int *sl = slots + blockIdx.y * 16;
-  const double *cf = coef + blockIdx.y * 16;
-  const int m = sl[15];
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    double2 acc = cscale(cf[0], d.hist[(int64_t)sl[0] * d.nT + u]);
-    for (int p = 1; p < m; ++p) acc = cadd(acc, cscale(cf[p], d.hist[(int64_t)sl[p] * d.nT + u]));
-    d.T[u] = acc;
   }
 }
 
@@ -1487,19 +1497,11 @@ __device__ __forceinline__ u32x4 bf3_im_pairs(u32x4 v) {
   for (int q = 0; q < 4; ++q) r[q] = ((v[q] >> 16) | (v[q] << 16)) ^ 0x8000u;
   return r;
 }
-// T split once per residual for the BF16x3 pp ladder (B operand (br, -bi)):
-// the bits the ladder's in-kernel split gives, computed once per amplitude
-// instead of once per wave and row tile
-__global__ void k_t_split(const SolveDesc *descs) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < d.nT; u += (int64_t)gridDim.x * blockDim.x) {
-    const double2 b = d.T[u];
-    unsigned h, l;
-    bf3_split((float)b.x, -(float)b.y, h, l);
-    const u32x4 im = bf3_im_pairs(u32x4{h, l, 0u, 0u});
-    d.Tbf[u] = make_uint4(h, l, im[0], im[1]);
-  }
+__device__ __forceinline__ uint4 t_split(double2 b) {
+  unsigned h, l;
+  bf3_split((float)b.x, -(float)b.y, h, l);
+  const u32x4 im = bf3_im_pairs(u32x4{h, l, 0u, 0u});
+  return make_uint4(h, l, im[0], im[1]);
 }
 
 __device__ __forceinline__ void bf3_lds_sync() {
@@ -1938,11 +1940,12 @@ void launch_mbpt2(const SolveDesc *dd, int nsolve, int64_t maxT, hipStream_t st)
   hipLaunchKernelGGL(k_mbpt2, egrid(maxT, nsolve), dim3(256), 0, st, dd);
 }
 
-// energy into scal[slot]; uses red[0..ENERGY_BLOCKS)
+// energies into results 0; partials in red[0 .. kRedBlocks)
 constexpr int kRedBlocks = 512;
-void launch_energy(const SolveDesc *dd, int nsolve, int slot, hipStream_t st) {
+constexpr int kEndBlocks = 2048;   // of the closing pass: SolveDesc::red holds 2048 x 36 partials
+void launch_energy(const SolveDesc *dd, int nsolve, double2 *out, hipStream_t st) {
   hipLaunchKernelGGL(k_energy_partial, dim3(kRedBlocks, nsolve), dim3(256), 0, st, dd);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kRedBlocks, 1, 1, slot);
+  hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kRedBlocks, 1, 0, out);
 }
 
 void launch_i7(const SolveDesc *dd, int nsolve, int maxA, hipStream_t st) {
@@ -1956,25 +1959,28 @@ void launch_i6(const SolveDesc *dd, int nsolve, int maxnp, int64_t maxrows, hipS
 void launch_i9(const SolveDesc *dd, int nsolve, int64_t maxvhh, hipStream_t st) {
   hipLaunchKernelGGL(k_i9, egrid(maxvhh, nsolve), dim3(256), 0, st, dd);
 }
-void launch_resid_init(const SolveDesc *dd, int nsolve, int64_t maxT, bool onebody, hipStream_t st) {
-  hipLaunchKernelGGL(k_resid_init, egrid(maxT, nsolve), dim3(256), 0, st, dd, onebody ? 1 : 0);
+// ring: 0 none, 1 FP64 blocks, 2 FP32 blocks
+void launch_t_begin(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64_t maxT, int ring, bool form, bool split,
+                    const uint32_t *const *maps, double2 *Tu, hipStream_t st) {
+  auto k = ring == 2 ? k_t_begin<2> : ring == 1 ? k_t_begin<1> : k_t_begin<0>;
+  hipLaunchKernelGGL(k, egrid(maxT, nsolve), dim3(256), 0, st, dd, ctrl, (int)form, (int)split, maps, Tu);
 }
-void launch_t_split(const SolveDesc *dd, int nsolve, int64_t maxT, hipStream_t st) {
-  hipLaunchKernelGGL(k_t_split, egrid(maxT, nsolve), dim3(256), 0, st, dd);
+// mode 0 residual only, 1 reference update (energies into results 0), 2 Anderson
+// update (17 values into results 24 .. 40)
+void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, bool f32, int mode, int terms,
+                  const uint32_t *const *maps, const double2 *Ru, double2 *out, hipStream_t st) {
+  auto k = mode == 2 ? (f32 ? k_t_end<true, 2> : k_t_end<false, 2>)
+         : mode == 1 ? (f32 ? k_t_end<true, 1> : k_t_end<false, 1>)
+                     : (f32 ? k_t_end<true, 0> : k_t_end<false, 0>);
+  hipLaunchKernelGGL(k, dim3(kEndBlocks, nsolve), dim3(256), 0, st, dd, ctrl, terms, maps, Ru);
+  if (mode == 1) hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kEndBlocks, 1, 0, out);
+  if (mode == 2) hipLaunchKernelGGL(k_reduce_final, dim3(17, nsolve), dim3(256), 0, st, dd, kEndBlocks, 36, 24, out);
 }
-void launch_ring_gather(const SolveDesc *dd, int nsolve, int64_t maxT, bool f32, hipStream_t st) {
-  if (f32) hipLaunchKernelGGL(k_ring_gather<true>, egrid(maxT, nsolve), dim3(256), 0, st, dd);
-  else hipLaunchKernelGGL(k_ring_gather<false>, egrid(maxT, nsolve), dim3(256), 0, st, dd);
+void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const IterCtrl *ctrl, hipStream_t st) {
+  hipLaunchKernelGGL(k_update, egrid(maxT, nsolve), dim3(256), 0, st, dd, ctrl);
 }
-void launch_ring_scatter(const SolveDesc *dd, int nsolve, int64_t maxT, bool f32, bool ring, bool hh,
-                         hipStream_t st) {
-  if (f32) hipLaunchKernelGGL(k_ring_scatter<true>, egrid(maxT, nsolve), dim3(256), 0, st, dd, (int)ring, (int)hh);
-  else hipLaunchKernelGGL(k_ring_scatter<false>, egrid(maxT, nsolve), dim3(256), 0, st, dd, (int)ring, (int)hh);
-}
-void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slot, hipStream_t st) {
-  hipLaunchKernelGGL(k_update, egrid(maxT, nsolve), dim3(256), 0, st, dd, slot);
-}
-void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, hipStream_t st) {
+// the Gram matrix's upper triangle into results 4 ..
+void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, double2 *out, hipStream_t st) {
   int ne = nstep - 1;
   dim3 gr(kRedBlocks, nsolve);
   switch (ne) {
@@ -1989,15 +1995,7 @@ void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, h
     default: return;
   }
   int nv = ne * (ne + 1) / 2;
-  hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kRedBlocks, 36, nv, 4);
-}
-void launch_share_gather(const SolveDesc *dd, int nsolve, int64_t maxT, const uint32_t *const *maps, double2 *Tu,
-                         hipStream_t st) {
-  hipLaunchKernelGGL(k_share_gather, egrid(maxT, nsolve), dim3(256), 0, st, dd, maps, Tu);
-}
-void launch_share_scatter(const SolveDesc *dd, int nsolve, int64_t maxT, const uint32_t *const *maps,
-                          const double2 *Ru, hipStream_t st) {
-  hipLaunchKernelGGL(k_share_scatter, egrid(maxT, nsolve), dim3(256), 0, st, dd, maps, Ru);
+  hipLaunchKernelGGL(k_reduce_final, dim3(nv, nsolve), dim3(256), 0, st, dd, kRedBlocks, 36, 4, out);
 }
 void launch_scatter_values(double2 *dst, const int64_t *idx, const double2 *val, int64_t n, hipStream_t st) {
   if (n <= 0) return;
@@ -2022,16 +2020,6 @@ void launch_read_probe(const double2 *a, int64_t n, double *out, int nblocks, hi
   hipLaunchKernelGGL(k_read_probe, dim3(nblocks), dim3(256), 0, st, a, n, per, out);
 }
 
-void launch_aa_update(const SolveDesc *dd, int nsolve, const int *slots, double beta, hipStream_t st) {
-  constexpr int kAABlocks = 1024;   // partials: SolveDesc::red holds 1024 x 36
-  hipLaunchKernelGGL(k_aa_update, dim3(kAABlocks, nsolve), dim3(256), 0, st, dd, slots, beta);
-  // 17 values per solve into scal[24 .. 40]
-  hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kAABlocks, 36, 17, 24);
-}
-void launch_aa_combine(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slots, const double *coef,
-                       hipStream_t st) {
-  hipLaunchKernelGGL(k_aa_combine, egrid(maxT, nsolve), dim3(256), 0, st, dd, slots, coef);
-}
 void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *slots, const double2 *coef,
                       int nvec, hipStream_t st) {
   hipLaunchKernelGGL(k_diis_axpy, egrid(maxT, nsolve), dim3(256), 0, st, dd, slots, coef, nvec);
@@ -2040,7 +2028,7 @@ void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *
 // Kernel kinds: 0 FP64, 1 FP32 (A double), 2 FP32 (A float), 3 FP64 pp ladder,
 // 4 FP32 pp ladder (A float), 5 pp ladder with A float and FP64 arithmetic,
 // 9 pp ladder on BF16x3 split products (A float), 10 the same with B the
-// split copy of T (k_t_split);
+// split copy of T (k_t_begin);
 // 6 BF16x3 split products (A double; the thin N <= 4 class stays FP64), tile
 // shapes (1,1..6), (1,8), (2,1..4), (4,1); 7 the same with A float; 8 with A,
 // B, C and C0 float (the FP32 ring blocks).
@@ -2077,7 +2065,7 @@ static void launch_shape_lb(const GemmGroup *groups, const GemmTile *tiles, int 
 //   VK 1: FP32-stored V, FP64 MFMA
 //   VK 2: FP32-stored V, FP32 MFMA (4 real products)
 //   VK 3: FP32-stored V, BF16x3 split products on bf16 MFMA (FP32 sums)
-//   VK 4: as 3, with T read already split (k_t_split; same bits)
+//   VK 4: as 3, with T read already split (k_t_begin; same bits)
 // Waits are explicit: s_waitcnt vmcnt(n) for the chunk about to be read and
 // lgkmcnt(0) for this wave's LDS reads of the stage about to be refilled, then
 // a bare s_barrier (a workgroup fence would force vmcnt(0) and drain the

@@ -185,3 +185,36 @@ def test_fp64_contraction_tiles_equal_list_kernels(ccnm, monkeypatch, A, matter,
     t, ref = out
     assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0
     assert np.abs(t - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("A,nmax,precision,graph", [
+    (2, 2, 0, 0), (14, 1, 0, 1), (14, 1, 3, 0), (66, 2, 3, 1), (66, 3, 0, 0), (66, 3, 3, 0)])
+def test_solve_loop_forms_the_iterates_of_the_step_interface(ccnm, A, nmax, precision, graph):
+    """The solve loop leaves each iterate to the next residual's opening pass and
+    updates inside the closing one; the step interface runs residual and update
+    apart, on T in place.  248 to 720540 amplitudes: fewer than a block, less
+    and more than one trip of the grids (524288).  Both add the same terms in
+    the same order; 1e-13 of the largest amplitude leaves three iterations of
+    contracted or separate roundings (2^-53 each) a factor of hundreds."""
+    out = []
+    for steps in (False, True):
+        s = ccnm.Solver(A=A, matter=ccnm.PNM, rho=0.16, nmax=nmax)
+        s.generate_interaction(ccnm.INT_MINNESOTA)
+        s.setup_t_amplitudes()
+        if steps:
+            count = nstep = 0
+            for _ in range(3):
+                s.t2_intermediate(precision)
+                count, nstep = s.diis_t1t2(count + 1, nstep + 1, 6, 6)
+            e = s.ccd_energy_save()
+        else:
+            r = s.ccd_iter(subspace=6, diis_step=6, tol=0.0, maxit=3, precision=precision, fp32_switch=0.0,
+                           use_graph=graph)
+            assert r["iterations"] == 3
+            e = r["ecorr"]
+        out.append((s.t2_unique(), e))
+        s.close()
+    (t, e), (t0, e0) = out
+    assert np.all(np.isfinite(t0)) and np.abs(t0).max() > 0
+    assert np.abs(t - t0).max() <= 1e-13 * np.abs(t0).max()
+    assert abs(e - e0) <= 1e-12 * abs(e0)
