@@ -1485,8 +1485,14 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   // while the ring keeps the matrix cores busy.  A third stream takes I6 (rows
   // of V* against rows of T), then the hh ladder into Rh once X is done.  All
   // three meet in the closing pass.
-  const bool fork = !timing && (terms & 8) && fork_enabled();
-  const bool fork6 = !timing && fork_enabled();
+  // A fork and its join cost some 10 us each on the host and the queues, which
+  // small batches do not win back: an iteration of SNM A=28 |n_i|<=2 (92 k
+  // amplitudes) takes 145 us on three streams and 124 on one, SNM A=76 |n_i|<=2
+  // (411 k) 206 on either, PNM A=66 |n_i|<=3 (721 k) 302 and 326.
+  int64_t amplitudes = 0;
+  for (const Solve *S : B.solves) amplitudes += S->plan.nT;
+  const bool fork6 = !timing && amplitudes >= 400000 && fork_enabled();
+  const bool fork = fork6 && (terms & 8);
   hipStream_t sr = fork ? B.stream2 : st;
   hipStream_t s6 = fork6 ? B.stream3 : st;
   // BF16x3 ring on the FP32 ring blocks when every solve has them
