@@ -59,7 +59,7 @@ void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *
 void launch_gemm_shape(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const SolveDesc *dd,
                        const int *gsolve, int kind, int mb, int nb, int lb, hipStream_t st);
 int ring64_class(int nph, int nhp);
-int ring64_columns(int cls);
+int ring64_columns(int nph, int nhp);
 void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *dd, hipStream_t st);
 void launch_x64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
 void launch_hh64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
@@ -498,7 +498,7 @@ void build_device(Solve &S) {
   SolveDesc &d = S.desc;
   HIPCHK(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
   d.A = P.A; d.nsp = P.nsp; d.np = P.np; d.nch = P.nch; d.nphc = P.nphc;
-  d.nT = P.nT; d.nRt = P.nRt; d.nI4 = P.nI4; d.active = 1;
+  d.nT = P.nT; d.active = 1;
   d.kx = dupload(P.orb.kx, o); d.ky = dupload(P.orb.ky, o); d.kz = dupload(P.orb.kz, o);
   d.e = dupload(P.orb.e, o);
   d.nx = dupload(P.orb.nx, o); d.ny = dupload(P.orb.ny, o); d.nz = dupload(P.orb.nz, o);
@@ -537,14 +537,11 @@ void build_device(Solve &S) {
   d.hhref = dupload(hr, o);
   d.nph = dupload(P.nph, o); d.nhp = dupload(P.nhp, o);
   d.off_ph = dupload(P.off_ph, o); d.off_hp = dupload(P.off_hp, o);
-  d.off_rt = dupload(P.off_rt, o); d.off_i4 = dupload(P.off_i4, o); d.off_vt = dupload(P.off_vt, o);
+  d.off_i4 = dupload(P.off_i4, o); d.off_vt = dupload(P.off_vt, o); d.off_w1 = dupload(P.off_w1, o);
   d.ph_a = dupload(P.ph_a, o); d.ph_i = dupload(P.ph_i, o);
   d.hp_j = dupload(P.hp_j, o); d.hp_b = dupload(P.hp_b, o);
-  {
-    if (P.nRt >= ((int64_t)1 << 31)) throw Error("ring blocks above 2^31 elements");
-    std::vector<int> r4(P.ring4.begin(), P.ring4.end());
-    d.ring4 = dupload(r4, o);
-  }
+  d.ring2 = dupload(P.ring2, o);
+  d.ring2b = P.ring2b.empty() ? nullptr : dupload(P.ring2b, o);
   d.T = dalloc<double2>(P.nT, o);
   d.R = dalloc<double2>(P.nT, o);
   d.R0 = dalloc<double2>(P.nT, o);
@@ -559,6 +556,7 @@ void build_device(Solve &S) {
   d.Vt = dalloc<double2>(P.nRt, o);
   d.I4 = dalloc<double2>(P.nI4, o);
   d.W0 = dalloc<double2>(P.nI4, o);
+  d.W1 = dalloc<double2>(P.nW1, o);
   d.fdiag = dalloc<double2>(P.nsp, o);
   d.fpart = dalloc<double2>(P.nsp, o);
   d.dh = dalloc<double2>(P.A, o);
@@ -575,6 +573,7 @@ void build_device(Solve &S) {
   HIPCHK(hipMemset(d.Vhhpp, 0, P.nT * sizeof(double2)));
   HIPCHK(hipMemset(d.Vhhhh, 0, P.nVhh * sizeof(double2)));
   HIPCHK(hipMemset(d.W0, 0, P.nI4 * sizeof(double2)));
+  HIPCHK(hipMemset(d.W1, 0, P.nW1 * sizeof(double2)));
   S.d_desc = dalloc<SolveDesc>(1, o);
   HIPCHK(hipMemcpy(S.d_desc, &d, sizeof(SolveDesc), hipMemcpyHostToDevice));
 
@@ -589,11 +588,14 @@ void build_device(Solve &S) {
     S.g_hh.add(mkgroup(d.T + P.off_t[c], d.X + P.nVhh + P.off_vhh[c], d.Rh + P.off_t[c], nullptr, np_, nh, nh, nh, nh, nh, nh, 1.0, 0.0), 0);
   }
   for (int K = 0; K < P.nphc; ++K) {
-    int nph = P.nph[K], nhp = P.nhp[K];
-    // I4 = W0 + 1/2 Vt Tt (ccm_t2_eqn.f90:657-780)
-    S.g_i4.add(mkgroup(d.Vt + P.off_vt[K], d.Tt + P.off_rt[K], d.I4 + P.off_i4[K], d.W0 + P.off_i4[K], nhp, nhp, nph, nph, nhp, nhp, nhp, 0.5, 1.0), 0);
-    // Rt = Tt I4 (ccm_t2_eqn.f90:995-1026)
-    S.g_rt.add(mkgroup(d.Tt + P.off_rt[K], d.I4 + P.off_i4[K], d.Rt + P.off_rt[K], nullptr, nph, nhp, nhp, nhp, nhp, nhp, 0, 1.0, 0.0), 0);
+    if (!P.ring_first(K)) continue;
+    const int nph = P.nph[K], nhp = P.nhp[K];
+    double2 *Tt = d.Tt + P.off_rt[K], *Rt = d.Rt + P.off_rt[K], *I4 = d.I4 + P.off_i4[K];
+    // the channel and its pair as one (Plan::ph_pair): I4 = W0 + Vt Tt (ccm_t2_eqn.f90:657-780),
+    // Rt = W1 Tt + Tt I4 (ccm_t2_eqn.f90:995-1026)
+    S.g_i4.add(mkgroup(d.Vt + P.off_vt[K], Tt, I4, d.W0 + P.off_i4[K], nhp, nhp, nph, nph, nhp, nhp, nhp, 1.0, 1.0), 0);
+    S.g_i4.add(mkgroup(d.W1 + P.off_w1[K], Tt, Rt, nullptr, nph, nhp, nph, nph, nhp, nhp, 0, 1.0, 0.0), 0);
+    S.g_rt.add(mkgroup(Tt, I4, Rt, Rt, nph, nhp, nhp, nhp, nhp, nhp, nhp, 1.0, 1.0), 0);
   }
   // tiles are made per batch (make_batch), for the batch's own class sizes
   S.g_pp.bytes = 16.0 * (double)P.nVpp;
@@ -668,12 +670,11 @@ struct Batch {
   // large for the fused ring keep the list kernels (g_i4big, g_rtbig)
   struct Fp64 {
     bool ready = false;
-    int nx = 0, nhh = 0, nring[3] = {0, 0, 0};
+    int nx = 0, nhh = 0, nring[kRingClasses] = {};
     ZTile *x = nullptr, *hh = nullptr;
-    RingTile *ring[3] = {nullptr, nullptr, nullptr};
+    RingTile *ring[kRingClasses] = {};
   } f64;
   GemmList g_i4big, g_rtbig;
-  bool i4_in_lds = false;   // the last ring was the fused one, which keeps I4 in LDS
   GemmList g_ppbf;         // BF16x3 pp ladder reading the split copy of T (when every solve has one)
   bool ppbf = false;
   // Shared pp ladder of a batch of twists of one lattice and interaction: the
@@ -1014,6 +1015,7 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
           if (q >= d.Rt && q < d.Rt + ss[L.gsolve[g]]->plan.nRt) return d.Rt32 + (q - d.Rt);
           if (q >= d.I4 && q < d.I4 + ss[L.gsolve[g]]->plan.nI4) return d.I4_32 + (q - d.I4);
           if (q >= d.W0 && q < d.W0 + ss[L.gsolve[g]]->plan.nI4) return d.W0_32 + (q - d.W0);
+          if (q >= d.W1 && q < d.W1 + ss[L.gsolve[g]]->plan.nW1) return d.W1_32 + (q - d.W1);
           throw Error("ring GEMM operand outside the ring blocks");
         };
         G.A = mv(G.A);
@@ -1026,12 +1028,14 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
     to32(B->g_rtf);
   }
   // ring groups of the channels the fused FP64 kernel does not take
-  for (size_t g = 0; g < B->g_i4.groups.size(); ++g) {
-    const GemmGroup &q = B->g_i4.groups[g];
-    if (ring64_class(q.K, q.M) >= 0) continue;
-    B->g_i4big.groups.push_back(q);
-    B->g_i4big.gsolve.push_back(B->g_i4.gsolve[g]);
-    B->g_rtbig.groups.push_back(B->g_rt.groups[g]);
+  for (size_t g = 0; g < B->g_rt.groups.size(); ++g) {
+    const GemmGroup &q = B->g_rt.groups[g];
+    if (ring64_class(q.M, q.K) >= 0) continue;
+    for (size_t k = 2 * g; k < 2 * g + 2; ++k) {
+      B->g_i4big.groups.push_back(B->g_i4.groups[k]);
+      B->g_i4big.gsolve.push_back(B->g_i4.gsolve[k]);
+    }
+    B->g_rtbig.groups.push_back(q);
     B->g_rtbig.gsolve.push_back(B->g_rt.gsolve[g]);
   }
   B->g_i4big.fam = 3;
@@ -1291,7 +1295,7 @@ void prepare_fp64(Batch &B) {
   Batch::Fp64 &F = B.f64;
   if (F.ready) return;
   std::vector<ZTile> x, hh;
-  std::vector<RingTile> ring[3];
+  std::vector<RingTile> ring[kRingClasses];
   int gx = 0, gr = 0;
   for (size_t s = 0; s < B.solves.size(); ++s) {
     const Plan &P = B.solves[s]->plan;
@@ -1311,10 +1315,10 @@ void prepare_fp64(Batch &B) {
     }
     for (int K = 0; K < P.nphc; ++K, ++gr) {
       const int nph = P.nph[K], nhp = P.nhp[K], cls = ring64_class(nph, nhp);
-      if (cls < 0 || nph <= 0 || nhp <= 0) continue;
-      for (int n0 = 0; n0 < nhp; n0 += ring64_columns(cls))
-        ring[cls].push_back(RingTile{d.Vt + P.off_vt[K], d.Tt + P.off_rt[K], d.W0 + P.off_i4[K], d.Rt + P.off_rt[K],
-                                     nhp, nph, n0, (int)s, gr, (float)nph + nhp});
+      if (cls < 0 || !P.ring_first(K)) continue;
+      for (int n0 = 0; n0 < nhp; n0 += ring64_columns(nph, nhp))
+        ring[cls].push_back(RingTile{d.Vt + P.off_vt[K], d.Tt + P.off_rt[K], d.W0 + P.off_i4[K], d.W1 + P.off_w1[K],
+                                     d.Rt + P.off_rt[K], nhp, nph, n0, (int)s, gr, 2.0f * nph + nhp});
     }
   }
   xcd_order_list(x, gx);
@@ -1323,7 +1327,7 @@ void prepare_fp64(Batch &B) {
   F.nhh = (int)hh.size();
   F.x = dupload(x, B.owned);
   F.hh = dupload(hh, B.owned);
-  for (int c = 0; c < 3; ++c) {
+  for (int c = 0; c < kRingClasses; ++c) {
     xcd_order_list(ring[c], gr);
     F.nring[c] = (int)ring[c].size();
     F.ring[c] = dupload(ring[c], B.owned);
@@ -1537,10 +1541,9 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   }
   if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
   if (terms & 8) {
-    B.i4_in_lds = t64(3);
     if (t64(3)) {
       Timer t(timing, sr, "gemm_ring");
-      for (int c = 2; c >= 0; --c) launch_ring64(B.f64.ring[c], B.f64.nring[c], c, B.d_descs, sr);
+      for (int c = kRingClasses - 1; c >= 0; --c) launch_ring64(B.f64.ring[c], B.f64.nring[c], c, B.d_descs, sr);
       if (!B.g_i4big.groups.empty()) {
         run_gemm(B.g_i4big, B, CCGPU_PREC_FP64, false, sr);
         run_gemm(B.g_rtbig, B, CCGPU_PREC_FP64, false, sr);
@@ -2084,6 +2087,7 @@ void fill_f32(Solve &S) {
   if (S.desc.Vt32) {
     launch_to_f32(S.desc.Vt, S.desc.Vt32, P.nRt, S.stream);
     launch_to_f32(S.desc.W0, S.desc.W0_32, P.nI4, S.stream);
+    launch_to_f32(S.desc.W1, S.desc.W1_32, P.nW1, S.stream);
     check_launch();
   }
   HIPCHK(hipStreamSynchronize(S.stream));
@@ -2110,6 +2114,7 @@ void ensure_f32(Solve &S, int handle) {
   S.desc.Vt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), S.owned);
   S.desc.I4_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
   S.desc.W0_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
+  S.desc.W1_32 = dalloc<float2>(std::max<int64_t>(P.nW1, 1), S.owned);
   S.desc.Tbf = dalloc<uint4>(std::max<int64_t>(P.nT, 1), S.owned);
   HIPCHK(hipMemset(S.desc.Tt32, 0, std::max<int64_t>(P.nRt, 1) * sizeof(float2)));
   fill_f32(S);
@@ -2137,7 +2142,7 @@ void fill_dims(const Plan &P, ccgpu_dims *d) {
   d->nchannels = P.nch; d->nph_channels = P.nphc;
   d->max_npp = P.max_npp; d->max_nhh = P.max_nhh;
   d->t2_unique = P.nT; d->t2_ordered = P.t2_ordered; d->vpppp_unique = P.nVpp;
-  d->ring_elems = P.nRt;
+  d->ring_elems = P.ring_elems;
   d->box = P.orb.box; d->volume = P.orb.volume; d->kf = P.orb.kf;
   double fpp = 0, fhh = 0, fr = 0;
   for (int c = 0; c < P.nch; ++c) {
@@ -2660,20 +2665,25 @@ int ccgpu_finalize_setup(int handle) {
     Solve &S = get(handle);
     const Plan &P = S.plan;
     if (!S.have_v || !S.have_fock) throw Error("set V blocks and the Fock matrix first");
-    // W0 from the staged hphp records: W0((i,a),(j,b)) = -<ib||ja>
+    // W0((i,a),(j,b)) = -<ib||ja> and W1((b,j),(a,i)) = W0((i,a),(j,b)) of -K' from the
+    // staged hphp records
     if (!S.hphp.empty()) {
-      std::vector<double2> w(P.nI4);
-      for (int K = 0; K < P.nphc; ++K)
+      std::vector<double2> w(P.nI4), w1(P.nW1);
+      auto w0 = [&](int i, int a, int j, int b) {
+        auto it = S.hphp.find((((uint64_t)i * P.nsp + b) * P.nsp + j) * P.nsp + a);
+        return it == S.hphp.end() ? double2{0.0, 0.0} : double2{-it->second.real(), -it->second.imag()};
+      };
+      for (int K = 0; K < P.nphc; ++K) {
+        if (!P.ring_first(K)) continue;
+        const int *hj = &P.hp_j[P.off_hp[K]], *hb = &P.hp_b[P.off_hp[K]];
+        const int *pa = &P.ph_a[P.off_ph[K]], *pi = &P.ph_i[P.off_ph[K]];
         for (int r = 0; r < P.nhp[K]; ++r)
-          for (int s = 0; s < P.nhp[K]; ++s) {
-            int i = P.hp_j[P.off_hp[K] + r], a = P.hp_b[P.off_hp[K] + r];
-            int j = P.hp_j[P.off_hp[K] + s], b = P.hp_b[P.off_hp[K] + s];
-            uint64_t key = (((uint64_t)i * P.nsp + b) * P.nsp + j) * P.nsp + a;
-            auto it = S.hphp.find(key);
-            std::complex<double> v = it == S.hphp.end() ? 0.0 : it->second;
-            w[P.off_i4[K] + (int64_t)r * P.nhp[K] + s] = double2{-v.real(), -v.imag()};
-          }
+          for (int s = 0; s < P.nhp[K]; ++s) w[P.off_i4[K] + (int64_t)r * P.nhp[K] + s] = w0(hj[r], hb[r], hj[s], hb[s]);
+        for (int r = 0; r < P.nph[K]; ++r)
+          for (int s = 0; s < P.nph[K]; ++s) w1[P.off_w1[K] + (int64_t)r * P.nph[K] + s] = w0(pi[s], pa[s], pi[r], pa[r]);
+      }
       HIPCHK(hipMemcpy(S.desc.W0, w.data(), P.nI4 * sizeof(double2), hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(S.desc.W1, w1.data(), P.nW1 * sizeof(double2), hipMemcpyHostToDevice));
     }
     int max_nph = 0, max_nhp = 0;
     for (int K = 0; K < P.nphc; ++K) { max_nph = std::max(max_nph, P.nph[K]); max_nhp = std::max(max_nhp, P.nhp[K]); }
@@ -3236,6 +3246,61 @@ int ccgpu_triples_stats(int handle, long long *elements, double *seconds) {
   });
 }
 
+// The ring blocks of every Pandya channel: the device holds those of the first channel
+// of each pair, and I4 and the two channels' R~ = T~ I4 not at all, so these are
+// formed here from the last T~.
+static void debug_ring(const Solve &S, int what, std::complex<double> *out) {
+  typedef std::complex<double> C;
+  const Plan &P = S.plan;
+  std::vector<C> t(P.nRt), v(P.nRt), w(P.nI4), w1(P.nW1);
+  HIPCHK(hipMemcpy(t.data(), S.desc.Tt, P.nRt * sizeof(C), hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(v.data(), S.desc.Vt, P.nRt * sizeof(C), hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(w.data(), S.desc.W0, P.nI4 * sizeof(C), hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(w1.data(), S.desc.W1, P.nW1 * sizeof(C), hipMemcpyDeviceToHost));
+  std::vector<int> pat((size_t)P.np * P.A, -1), hat((size_t)P.np * P.A, -1);   // (a,i): index in its ph, hp list
+  for (int K = 0; K < P.nphc; ++K) {
+    for (int r = 0; r < P.nph[K]; ++r)
+      pat[(size_t)(P.ph_a[P.off_ph[K] + r] - P.A) * P.A + P.ph_i[P.off_ph[K] + r]] = r;
+    for (int s = 0; s < P.nhp[K]; ++s)
+      hat[(size_t)(P.hp_b[P.off_hp[K] + s] - P.A) * P.A + P.hp_j[P.off_hp[K] + s]] = s;
+  }
+  for (int K = 0; K < P.nphc; ++K) {
+    const int64_t np_ = P.nph[K], nh = P.nhp[K];
+    const int L = P.ph_pair[K];
+    // hp pairs by hole and then particle: x[s] is the s-th; second channels: it is ph pair
+    // q[s] of the first, and ph pair r its hp pair p[r]
+    std::vector<int64_t> p(np_), q(nh), x(nh);
+    for (int64_t s = 0; s < nh; ++s) x[s] = s;
+    std::stable_sort(x.begin(), x.end(),
+                     [&](int64_t a, int64_t b) { return P.hp_j[P.off_hp[K] + a] < P.hp_j[P.off_hp[K] + b]; });
+    for (int64_t r = 0; r < np_; ++r) p[r] = hat[(size_t)(P.ph_a[P.off_ph[K] + r] - P.A) * P.A + P.ph_i[P.off_ph[K] + r]];
+    for (int64_t s = 0; s < nh; ++s)
+      q[s] = pat[(size_t)(P.hp_b[P.off_hp[K] + x[s]] - P.A) * P.A + P.hp_j[P.off_hp[K] + x[s]]];
+    std::vector<C> T(np_ * nh), V(nh * np_), W(nh * nh);
+    for (int64_t s = 0; s < nh; ++s) {
+      for (int64_t r = 0; r < np_; ++r) {
+        T[r * nh + s] = P.ring_first(K) ? t[P.off_rt[K] + r * nh + x[s]] : t[P.off_rt[L] + q[s] * np_ + p[r]];
+        V[s * np_ + r] = P.ring_first(K) ? v[P.off_vt[K] + x[s] * np_ + r] : v[P.off_vt[L] + p[r] * nh + q[s]];
+      }
+      for (int64_t r = 0; r < nh; ++r)
+        W[r * nh + s] = P.ring_first(K) ? w[P.off_i4[K] + x[r] * nh + x[s]] : w1[P.off_w1[L] + q[s] * nh + q[r]];
+    }
+    auto add = [](std::vector<C> &c, const std::vector<C> &a, const std::vector<C> &b, int64_t m, int64_t k,
+                  int64_t n, double f) {
+      for (int64_t i = 0; i < m; ++i)
+        for (int64_t x = 0; x < k; ++x) {
+          const C q = f * a[i * k + x];
+          for (int64_t j = 0; j < n; ++j) c[i * n + j] += q * b[x * n + j];
+        }
+    };
+    std::vector<C> R(np_ * nh);
+    if (what == 6 || what == 8) add(W, V, T, nh, np_, nh, 0.5);
+    if (what == 6) add(R, T, W, np_, nh, nh, 1.0);
+    const std::vector<C> &a = what == 6 ? R : what == 7 ? T : what == 14 ? V : W;
+    out = std::copy(a.begin(), a.end(), out);
+  }
+}
+
 int ccgpu_debug_fetch(int handle, int what, double *out, long long n) {
   return guarded([&] {
     Solve &S = get(handle);
@@ -3243,21 +3308,12 @@ int ccgpu_debug_fetch(int handle, int what, double *out, long long n) {
     const SolveDesc &d = S.desc;
     struct Arr { const void *p; long long n; };
     Arr a[] = {{d.R, P.nT}, {d.dh, P.A}, {d.I7off, P.A}, {d.dp, P.np}, {d.I6off, P.np}, {d.X, 2 * P.nVhh},
-               {d.Rt, P.nRt}, {d.Tt, P.nRt}, {d.I4, P.nI4}, {d.T, P.nT}, {d.R0, P.nT}, {d.fdiag, P.nsp},
-               {d.fpart, P.nsp}, {d.W0, P.nI4}, {d.Vt, P.nRt}};
+               {nullptr, P.ring_elems}, {nullptr, P.ring_elems}, {nullptr, P.w0_elems}, {d.T, P.nT}, {d.R0, P.nT},
+               {d.fdiag, P.nsp}, {d.fpart, P.nsp}, {nullptr, P.w0_elems}, {nullptr, P.ring_elems}};
     if (what < 0 || what >= (int)(sizeof a / sizeof a[0])) throw Error(fmt("unknown debug array %d", what));
     if (n != a[what].n) throw Error(fmt("debug array %d has %lld elements, caller asked %lld", what, a[what].n, n));
-    if (what == 8 && single(handle).i4_in_lds) {   // formed here from the last T~
-      Batch &B = single(handle);
-      if (!B.g_i4.ready) {
-        B.g_i4.build_tiles();
-        B.g_i4.upload(B.owned);
-        B.g_i4.ready = true;
-      }
-      run_gemm(B.g_i4, B, CCGPU_PREC_FP64, false, B.stream);
-      check_launch();
-    }
     HIPCHK(hipDeviceSynchronize());
+    if (!a[what].p) return debug_ring(S, what, (std::complex<double> *)out);
     HIPCHK(hipMemcpy(out, a[what].p, n * sizeof(double2), hipMemcpyDeviceToHost));
   });
 }

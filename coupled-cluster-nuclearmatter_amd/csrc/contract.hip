@@ -1,8 +1,8 @@
 // FP64 contractions of the CCD residual outside the pp ladder, one launch each
 // (the ring one per channel size class), every channel and solve of a batch in
 // it: X = V_hhpp T with I9 = V_hhhh + X (ccm_t2_eqn.f90:431-464, 558-560), the
-// hh ladder T I9 (:614-647), and the ring I4 = W0 + 1/2 V~ T~, R~ = T~ I4
-// (:657-780, 995-1026).
+// hh ladder T I9 (:614-647), and the ring of a channel pair, R~ = T~ (W0 + V~ T~) +
+// W1 T~ (:657-780, 995-1026; Plan::ph_pair).
 //
 // Complex products take three real MFMAs (Gauss: ar br, ai bi, (ar+ai)(br+bi)).
 // A 16-wide k chunk is four 16x16x4 steps; lane group g = lane / 16 of step q
@@ -59,7 +59,7 @@ struct CAcc {
     im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, im, 0, 0, 0);
     s = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x + a.y, b.x + b.y, s, 0, 0, 0);
   }
-  __device__ __forceinline__ double2 at(int r) const { return make_double2(re[r] - im[r], s[r] - re[r] - im[r]); }
+  __device__ __forceinline__ double2 at(int r) const { return make_double2(re[r] - im[r], s[r] - (re[r] + im[r])); }
 };
 
 // ---------------------------------------------------------------------------
@@ -193,58 +193,51 @@ __global__ __launch_bounds__(256, 2) void k_hh64(const ZTile *__restrict__ tiles
 }
 
 // ---------------------------------------------------------------------------
-// Ring: column block n0 of I4 needs V~ and column block n0 of T~ only, and the
-// same column block of R~ = T~ I4 needs T~ and that block of I4 only: one block
-// does both, with the T~ columns and then the I4 columns in LDS (I4 never goes
-// to memory), W waves of RB 16-row blocks each, 16 NB columns.  V~ and T~ rows
-// go straight to the wave that owns them.  Column blocks of a channel run on
-// one XCD, whose L2 holds V~ and T~ for them.
+// Ring of a channel pair: column block n0 of R~ = W1 T~ + T~ (W0 + V~ T~)
+// needs the T~ columns n0 and that block of I4 = W0 + V~ T~ only, so one block does all
+// three products, with the T~ columns and then the I4 columns in LDS (I4 never goes
+// to memory).  Eight waves: WR along the rows, RB 16-row blocks each, by WC of 16
+// columns.  V~, W1 and T~ rows go straight to the wave that owns them.  Column
+// blocks of a channel run on one XCD, whose L2 holds the operands for them.
 //
-// W RB 16 covers the channel's larger side: 64 (W 4) and 128 (W 8) with 32
-// columns, 256 (W 8, RB 2) with 16; 64 KB of LDS at most, two workgroups per CU
-// (one with RB 2).
-// Bound by FP64 MFMA: PNM A=66 |n_i|<=4 takes 238 + 34 us (classes 128 and 64,
-// alone on the device; MFMA alone 137 + 15).  I4 and R~ as two launches per width class
-// with I4 in memory took 486 us in twelve.  16 columns 258, 48 columns 286, one workgroup
-// per CU 244.
+// 16 WR RB covers the channel's larger side: 64 (WR 4, WC 2) and 128 (WR 8) in one
+// launch, 32 KB of LDS and two workgroups per CU, 256 (WR 8, RB 2) in another.
+// Bound by FP64 MFMA: PNM A=66 |n_i|<=4 takes 190 us alone on the device, MFMA alone
+// 114.  Both channels of a pair contracted on their own (four products instead of
+// three, T~ and R~ of both) took 272 us; launches of their own for up to 64, 96 (six
+// waves) and 128 rows 224, 32 columns per wave 216.
 // ---------------------------------------------------------------------------
-template <int W, int RB, int NB>
-__global__ __launch_bounds__(64 * W, W == 8 && RB == 1 ? 4 : 2) void k_ring64(const RingTile *__restrict__ tiles,
-                                                                   const SolveDesc *__restrict__ descs) {
-  constexpr int BC = 16 * NB, NT = 64 * W;
-  __shared__ double2 Bs[16 * W * RB * BC];
-  const RingTile t = tiles[blockIdx.x];
-  if (!descs[t.solve].active) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
-  CAcc acc[RB][NB];
+template <int WR, int WC, int RB>
+__device__ __forceinline__ void ring64_tile(const RingTile &t, double2 *Bs) {
+  constexpr int BC = 16 * WC, NT = 512;
+  const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) % WR, li = lane & 15, lg = lane >> 4;
+  const int cw = 16 * ((threadIdx.x >> 6) / WR);   // first column of the wave in LDS
+  const int c = t.n0 + cw + li;
+  CAcc acc[RB];
   // two MFMA steps (8 k) ahead: with four waves on a SIMD the loads have the
   // other waves' 3 x 768 clocks, and 16 registers less keep 128 without spills
   double2 a0[RB][2], a1[RB][2];
-  // steps from k0 of this wave's rows (blocks w and w + W) of A, M x K.  Rows
+  // steps from k0 of this wave's rows (blocks w and w + WR) of A, M x K.  Rows
   // past M are copies of the last and never used; k past K meets zeros in LDS.
   auto load = [&](double2 (&a)[RB][2], const double2 *A, int M, int K, int k0) {
 #pragma unroll
-    for (int x = 0; x < RB; ++x) row_chunk(a[x], A, (unsigned)min(16 * (w + W * x) + li, M - 1) * K, K, k0, lg);
+    for (int x = 0; x < RB; ++x) row_chunk(a[x], A, (unsigned)min(16 * (w + WR * x) + li, M - 1) * K, K, k0, lg);
   };
   auto compute = [&](const double2 (&a)[RB][2], int k0) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const double2 *b = Bs + (k0 + 4 * q + lg) * BC + li;
+      const double2 bv = Bs[(k0 + 4 * q + lg) * BC + cw + li];
 #pragma unroll
-      for (int y = 0; y < NB; ++y) {
-        const double2 bv = b[16 * y];
-#pragma unroll
-        for (int x = 0; x < RB; ++x) acc[x][y].mac(a[x][q], bv);
-      }
+      for (int x = 0; x < RB; ++x) acc[x].mac(a[x][q], bv);
     }
   };
-  // the rows times the columns in LDS; the first two steps are in a0 already
+  auto clear = [&] {
+#pragma unroll
+    for (int x = 0; x < RB; ++x) acc[x].clear();
+  };
+  // plus the rows times the columns in LDS; the first two steps are in a0 already
   auto product = [&](const double2 *A, int M, int K) {
-#pragma unroll
-    for (int x = 0; x < RB; ++x)
-#pragma unroll
-      for (int y = 0; y < NB; ++y) acc[x][y].clear();
-    if (16 * w >= M) return;
+    if (16 * w >= M || t.n0 + cw >= t.nhp) return;
     for (int k0 = 0; k0 < K; k0 += 16) {   // whole chunks of 16: LDS is zero past K
       load(a1, A, M, K, k0 + 8);
       compute(a0, k0);
@@ -261,8 +254,8 @@ __global__ __launch_bounds__(64 * W, W == 8 && RB == 1 ? 4 : 2) void k_ring64(co
       double2 v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int e = e0 + j * NT, k = e / BC, c = t.n0 + e % BC;
-        v[j] = zero_unless(k < t.nph && c < t.nhp, gl(t.Tt, (unsigned)min(k, t.nph - 1) * t.nhp + min(c, t.nhp - 1)));
+        const int e = e0 + j * NT, k = e / BC, x = t.n0 + e % BC;
+        v[j] = zero_unless(k < t.nph && x < t.nhp, gl(t.Tt, (unsigned)min(k, t.nph - 1) * t.nhp + min(x, t.nhp - 1)));
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -270,61 +263,62 @@ __global__ __launch_bounds__(64 * W, W == 8 && RB == 1 ? 4 : 2) void k_ring64(co
     }
   }
   __syncthreads();
+  clear();
   product(t.Vt, t.nhp, t.nph);
-  // I4 = W0 + 1/2 V~ T~ in the place of the T~ columns; rows past nhp in a
-  // wave's block are zero
+  load(a0, t.W1, t.nph, t.nph, 0);
+  // I4 = W0 + V~ T~ in registers; rows past nhp in a wave's block are zero
+  double2 i4[RB][4];
 #pragma unroll
   for (int x = 0; x < RB; ++x)
 #pragma unroll
-    for (int y = 0; y < NB; ++y) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 16 * (w + W * x) + lg + 4 * r, c = t.n0 + 16 * y + li;
-        const double2 s = acc[x][y].at(r);
-        const double2 c0 = gl(t.W0, (unsigned)min(m, t.nhp - 1) * t.nhp + min(c, t.nhp - 1));
-        const bool ok = m < t.nhp && c < t.nhp;
-        acc[x][y].re[r] = ok ? 0.5 * s.x + c0.x : 0.0;
-        acc[x][y].im[r] = ok ? 0.5 * s.y + c0.y : 0.0;
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * (w + WR * x) + lg + 4 * r;
+      const double2 s = acc[x].at(r);
+      const double2 c0 = gl(t.W0, (unsigned)min(m, t.nhp - 1) * t.nhp + min(c, t.nhp - 1));
+      i4[x][r] = zero_unless(m < t.nhp && c < t.nhp, make_double2(s.x + c0.x, s.y + c0.y));
     }
+  clear();
+  product(t.W1, t.nph, t.nph);
   load(a0, t.Tt, t.nph, t.nhp, 0);
   __syncthreads();   // every wave has read the T~ columns
 #pragma unroll
   for (int x = 0; x < RB; ++x) {
-    if (16 * (w + W * x) >= t.nhp) continue;
+    if (16 * (w + WR * x) >= t.nhp) continue;
 #pragma unroll
-    for (int y = 0; y < NB; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        Bs[(16 * (w + W * x) + lg + 4 * r) * BC + 16 * y + li] = make_double2(acc[x][y].re[r], acc[x][y].im[r]);
+    for (int r = 0; r < 4; ++r) Bs[(16 * (w + WR * x) + lg + 4 * r) * BC + cw + li] = i4[x][r];
   }
   __syncthreads();
   product(t.Tt, t.nph, t.nhp);
 #pragma unroll
-  for (int x = 0; x < RB; ++x) {
-    const int mw = 16 * (w + W * x);
-    if (mw >= t.nph) continue;
+  for (int x = 0; x < RB; ++x)
 #pragma unroll
-    for (int y = 0; y < NB; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = mw + lg + 4 * r, c = t.n0 + 16 * y + li;
-        if (m < t.nph && c < t.nhp) t.Rt[(int64_t)m * t.nhp + c] = acc[x][y].at(r);
-      }
-  }
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * (w + WR * x) + lg + 4 * r;
+      if (m < t.nph && c < t.nhp) t.Rt[(int64_t)m * t.nhp + c] = acc[x].at(r);
+    }
 }
 
-int ring64_class(int nph, int nhp) {   // tile class of a channel, -1: too large for the fused kernel
-  const int d = std::max(nph, nhp);
-  return d <= 64 ? 0 : d <= 128 ? 1 : d <= 256 ? 2 : -1;
+// channels of up to 128 (RB 1) or 256 (RB 2) rows
+template <int RB>
+__global__ __launch_bounds__(512, RB == 1 ? 4 : 2) void k_ring64(const RingTile *__restrict__ tiles,
+                                                                 const SolveDesc *__restrict__ descs) {
+  __shared__ double2 Bs[128 * RB * 16];
+  const RingTile t = tiles[blockIdx.x];
+  if (!descs[t.solve].active) return;
+  if (RB == 1 && max(t.nph, t.nhp) <= 64) ring64_tile<4, 2, 1>(t, Bs);
+  else ring64_tile<8, 1, RB>(t, Bs);
 }
-int ring64_columns(int cls) { return cls == 2 ? 16 : 32; }
+
+int ring64_class(int nph, int nhp) {   // launch of a channel, -1: too large for the fused kernel
+  const int d = std::max(nph, nhp);
+  return d <= 128 ? 0 : d <= 256 ? 1 : -1;
+}
+int ring64_columns(int nph, int nhp) { return std::max(nph, nhp) <= 64 ? 32 : 16; }
 
 void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *dd, hipStream_t st) {
   if (ntiles <= 0) return;
-  if (cls == 0) hipLaunchKernelGGL((k_ring64<4, 1, 2>), dim3(ntiles), dim3(256), 0, st, tiles, dd);
-  else if (cls == 1) hipLaunchKernelGGL((k_ring64<8, 1, 2>), dim3(ntiles), dim3(512), 0, st, tiles, dd);
-  else hipLaunchKernelGGL((k_ring64<8, 2, 1>), dim3(ntiles), dim3(512), 0, st, tiles, dd);
+  if (cls == 0) hipLaunchKernelGGL(k_ring64<1>, dim3(ntiles), dim3(512), 0, st, tiles, dd);
+  else hipLaunchKernelGGL(k_ring64<2>, dim3(ntiles), dim3(512), 0, st, tiles, dd);
 }
 void launch_x64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st) {
   if (ntiles > 0) hipLaunchKernelGGL(k_x64, dim3(ntiles), dim3(256), 0, st, tiles, dd);

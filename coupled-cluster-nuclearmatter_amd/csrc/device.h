@@ -17,7 +17,7 @@ struct DPair {
 // pointers; arrays indexed by unique amplitude u have length nT.
 struct SolveDesc {
   int A, nsp, np, nch, nphc;
-  int64_t nT, nRt, nI4;
+  int64_t nT;
   int active;  // 0: converged, kernels skip this solve
   // orbitals
   const double *kx, *ky, *kz, *e;
@@ -41,17 +41,19 @@ struct SolveDesc {
   const int *pimg;
   // Pandya
   const int *nph, *nhp;
-  const int64_t *off_ph, *off_hp, *off_rt, *off_i4, *off_vt;
+  const int64_t *off_ph, *off_hp, *off_i4, *off_vt, *off_w1;
   const int *ph_a, *ph_i, *hp_j, *hp_b;
-  const int *ring4;   // four Pandya positions per unique amplitude (every ring block below 2^31 elements)
+  // two ring positions per unique amplitude, and their second ones in channels that
+  // pair with themselves (-1 elsewhere; null: no such channel)
+  const int *ring2, *ring2b;
   // amplitudes and blocks
   double2 *T, *R, *R0, *Vhhpp, *Vhhhh, *X, *Vpppp;
   double2 *Rh;   // hh ladder T I9 of the residual, added to R by its closing pass
   float2 *Vpppp32;
-  double2 *Tt, *Rt, *I4, *W0, *Vt;
+  double2 *Tt, *Rt, *I4, *W0, *W1, *Vt;
   // FP32 ring blocks of the BF16x3 residual (null until the FP32 copies are
-  // made): T~, R~, I4 per iteration, V~ and W0 copied from the FP64 blocks
-  float2 *Tt32, *Rt32, *I4_32, *W0_32, *Vt32;
+  // made): T~, R~, I4 per iteration, V~, W0 and W1 copied from the FP64 blocks
+  float2 *Tt32, *Rt32, *I4_32, *W0_32, *W1_32, *Vt32;
   // T as the BF16x3 pp ladder's B operand, split once per residual: per
   // amplitude the bf16 hi and lo pairs of (re, -im) and of (im, re)
   uint4 *Tbf;
@@ -107,9 +109,11 @@ struct ZTile {
   float cost;
 };
 
-// Columns n0 .. of one Pandya channel's two ring contractions (contract.hip)
+constexpr int kRingClasses = 2;   // launches of the fused ring (ring64_class)
+
+// Columns n0 .. of one Pandya channel pair's ring contractions (contract.hip)
 struct RingTile {
-  const double2 *Vt, *Tt, *W0;
+  const double2 *Vt, *Tt, *W0, *W1;
   double2 *Rt;
   int nhp, nph, n0, solve, g;
   float cost;

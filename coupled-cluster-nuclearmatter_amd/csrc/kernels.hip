@@ -5,6 +5,7 @@
 //   Vpppp    : Npp x Npp per channel       Vhhpp : Nhh x Npp per channel
 //   Vhhhh, X : Nhh x Nhh per channel       (X = Vhhpp T, I9 = X + Vhhhh)
 //   Tt, Rt   : Pandya blocks Nph x Nhp     I4, W0 : Nhp x Nhp    Vt : Nhp x Nph
+//              and W1 : Nph x Nph, of one channel of each pair K', -K' (Plan::ph_pair)
 // Reference routines restated here are cited per kernel (paths relative to
 // deltafull-CCMkspace/ of the reference).
 #include "device.h"
@@ -88,18 +89,23 @@ __global__ void k_fill_vhhhh(SolveDesc d, V vas) {
   }
 }
 
-// W0((i,a),(j,b)) = -<ib||ja> (the recoupled hphp term of I4, ccm_t2_eqn.f90:740-780).
+// W0((i,a),(j,b)) = -<ib||ja> (the recoupled hphp term of I4, ccm_t2_eqn.f90:740-780)
+// and, blockIdx.z 1, W1((b,j),(a,i)), the same element of -K' (Plan::ph_pair).
 template <class V>
 __global__ void k_fill_w0(SolveDesc d, V vas) {
   const int K = blockIdx.y;
-  const int n = d.nhp[K];
+  if (d.off_i4[K] < 0) return;
+  const bool w1 = blockIdx.z != 0;
+  const int n = w1 ? d.nph[K] : d.nhp[K];
   const int64_t ne = (int64_t)n * n;
-  const int *hj = d.hp_j + d.off_hp[K], *hb = d.hp_b + d.off_hp[K];
+  const int *hj = w1 ? d.ph_i + d.off_ph[K] : d.hp_j + d.off_hp[K];
+  const int *hb = w1 ? d.ph_a + d.off_ph[K] : d.hp_b + d.off_hp[K];
+  double2 *W = w1 ? d.W1 + d.off_w1[K] : d.W0 + d.off_i4[K];
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x) {
-    int r = (int)(e / n), s = (int)(e % n);
+    const int x = (int)(e / n), y = (int)(e % n), r = w1 ? y : x, s = w1 ? x : y;
     int i = hj[r], a = hb[r], j = hj[s], b = hb[s];
     double2 v = vas(i, b, j, a);
-    d.W0[d.off_i4[K] + e] = make_double2(-v.x, -v.y);
+    W[e] = make_double2(-v.x, -v.y);
   }
 }
 
@@ -254,19 +260,24 @@ __global__ __launch_bounds__(256) void k_no2b_vhhpp(SolveDesc d, Chiral3Dev c) {
   }
 }
 
-// W0((i,a),(j,b)) = -<ib||ja>
+// W0 and, blockIdx.z 1, W1, as k_fill_w0
 template <bool ONE>
 __global__ __launch_bounds__(256) void k_no2b_w0(SolveDesc d, Chiral3Dev c) {
   const int K = blockIdx.y;
-  const int n = d.nhp[K];
+  if (d.off_i4[K] < 0) return;
+  const bool w1 = blockIdx.z != 0;
+  const int n = w1 ? d.nph[K] : d.nhp[K];
   const int64_t ne = (int64_t)n * (n + 1) / 2;
-  const int *hj = d.hp_j + d.off_hp[K], *hb = d.hp_b + d.off_hp[K];
+  const int *hj = w1 ? d.ph_i + d.off_ph[K] : d.hp_j + d.off_hp[K];
+  const int *hb = w1 ? d.ph_a + d.off_ph[K] : d.hp_b + d.off_hp[K];
+  double2 *W = w1 ? d.W1 + d.off_w1[K] : d.W0 + d.off_i4[K];
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x) {
-    int r, s;
-    tri_rs(e, r, s);
+    int x, y;
+    tri_rs(e, x, y);
+    const int r = w1 ? y : x, s = w1 ? x : y;
     const int i = hj[r], a = hb[r], j = hj[s], b = hb[s];
     const double2 v = herm_no2b<ONE>(c, d.A, i, b, j, a);
-    add_herm_pair(d.W0 + d.off_i4[K], n, r, s, v, -1.0);
+    add_herm_pair(W, n, x, y, v, -1.0);
   }
 }
 
@@ -373,10 +384,12 @@ __global__ void k_derive_r0(SolveDesc d) {
 __device__ __forceinline__ int pref_idx(DPair p) { return p.v >> 1; }
 __device__ __forceinline__ double pref_sign(DPair p) { return (p.v & 1) ? -1.0 : 1.0; }
 
-// Vt((i,a),(b,j)) = <ij||ab> gathered from Vhhpp (the amat gather, ccm_t2_eqn.f90:694-716).
+// Vt((i,a),(b,j)) = <ij||ab> gathered from Vhhpp (the amat gather, ccm_t2_eqn.f90:694-716),
+// in the first channel of each pair.
 __global__ void k_derive_vt(SolveDesc d) {
   const int K = blockIdx.y;
   const int nhp = d.nhp[K], nph = d.nph[K];
+  if (d.off_vt[K] < 0) return;
   const int64_t ne = (int64_t)nhp * nph;
   const int *hj = d.hp_j + d.off_hp[K], *hb = d.hp_b + d.off_hp[K];
   const int *pa = d.ph_a + d.off_ph[K], *pi = d.ph_i + d.off_ph[K];
@@ -599,8 +612,8 @@ __device__ __forceinline__ uint4 t_split(double2 b);
 // The pass over the amplitudes that opens a residual: the next iterate
 // T = sum_j c_j hist_j where the last update left one (the Anderson
 // combination, or the one column of a plain step: c = 1 copies it), the Pandya
-// gather T~((a,i),(j,b)) = t(ab,ij) (ccm_t2_eqn.f90:37-62; the four positions
-// of an amplitude are one 16-byte load), and the operand of the pp ladder: T
+// gather T~((a,i),(j,b)) = t(ab,ij) (ccm_t2_eqn.f90:37-62; the two positions of an
+// amplitude are one 8-byte load), and the operand of the pp ladder: T
 // split for BF16x3, or the columns of the shared union blocks.
 //
 // Shared pp ladder of a batch of twists of one lattice (one V_pppp over the
@@ -610,10 +623,10 @@ __device__ __forceinline__ uint4 t_split(double2 b);
 // (row: the pair's union row, column: the solve's column range), with the
 // orientation sign of the pair there.  Positions no solve owns stay zero.
 //
-// Bound by the requests of the four scattered stores (PNM A=66 |n_i|<=4: 8 M
-// stores in 4.6 M requests, 250 MB to memory for 159 MB of T and T~): 70 us there, 346 us for eight
-// Anderson twists of |n_i|<=3.  As passes of their own, combination, gather and
-// shared gather took 390 us for the twists.
+// Bound by the requests of the scattered stores: PNM A=66 |n_i|<=4 51 us, 250 us for
+// eight Anderson twists of |n_i|<=3.  With the positions of both channels of each pair
+// (four stores an amplitude) 70 and 346 us; as passes of their own, combination, gather
+// and shared gather took 390 us for the twists.
 template <int RING>   // 0 no ring, 1 FP64 blocks, 2 FP32 blocks of the BF16x3 residual
 __global__ __launch_bounds__(256) void k_t_begin(const SolveDesc *descs, const IterCtrl *ctrl, int form, int split,
                                                  const uint32_t *const *maps, double2 *Tu) {
@@ -641,19 +654,18 @@ __global__ __launch_bounds__(256) void k_t_begin(const SolveDesc *descs, const I
     }
     const double2 mt = make_double2(-t.x, -t.y);
     if constexpr (RING != 0) {
-      const int4 p = *(const int4 *)(d.ring4 + 4 * (int64_t)u);
-      if constexpr (RING == 2) {
-        const float2 tf = make_float2((float)t.x, (float)t.y), mf = make_float2(-tf.x, -tf.y);
-        d.Tt32[p.x] = tf;
-        d.Tt32[p.y] = mf;
-        d.Tt32[p.z] = mf;
-        d.Tt32[p.w] = tf;
-      } else {
-        d.Tt[p.x] = t;
-        d.Tt[p.y] = mt;
-        d.Tt[p.z] = mt;
-        d.Tt[p.w] = t;
-      }
+      auto put = [&](int2 p) {
+        if constexpr (RING == 2) {
+          const float2 tf = make_float2((float)t.x, (float)t.y), mf = make_float2(-tf.x, -tf.y);
+          if (p.x >= 0) d.Tt32[p.x] = tf;
+          if (p.y >= 0) d.Tt32[p.y] = mf;
+        } else {
+          if (p.x >= 0) d.Tt[p.x] = t;
+          if (p.y >= 0) d.Tt[p.y] = mt;
+        }
+      };
+      put(((const int2 *)d.ring2)[u]);
+      if (d.ring2b) put(((const int2 *)d.ring2b)[u]);
     }
     if (split) d.Tbf[u] = t_split(t);
     if (m) {
@@ -674,9 +686,10 @@ __device__ __forceinline__ double2 jacobi_step(double2 t, double2 r, double2 den
 //   R = conj(<ij||ab>) + P(ab) sum_c I6(b,c) t(ac,ij) - P(ij) sum_k I7(k,j) t(ab,ik),
 //       diagonals removed (ccm_t2_eqn.f90:81-211)
 //     + pp ladder (R itself, or the shared union product) + hh ladder
-//     + P(ab) P(ij) of the ring R~ (ccm_t2_eqn.f90:1133-1185; F32: from the FP32
-//       R~ of the BF16x3 residual, summed in FP64),
-// summed as (hh + (one-body + pp)) + ring.
+//     + P(ab) P(ij) of the ring R~ (ccm_t2_eqn.f90:1133-1185; two loads, Plan::ph_pair;
+//       F32: from the FP32 R~ of the BF16x3 residual, summed in FP64),
+// summed as conj V + ((hh + (one-body + pp)) + ring): conj V is the largest, so the others
+// round at their own size.
 // MODE 0 stops there (the residual of the step-by-step interface).
 // MODE 1, the reference's update: the Jacobi step into history column q.fresh,
 //   and block partials of its energy sum t conj(R0) to red[block].
@@ -692,10 +705,10 @@ __device__ __forceinline__ double2 jacobi_step(double2 t, double2 r, double2 den
 // T itself is left alone: other threads read rows of it, and the next residual's
 // opening pass forms it from the history.
 //
-// Bound by the latency of the scattered R~ loads and by HBM.  One-body start, ring
-// scatter, update and energy as passes of their own took 130 us (PNM A=66
-// |n_i|<=4), 87 us this; with the shared scatter 585 us for eight Anderson twists
-// of |n_i|<=3, 338 us this.
+// Bound by the latency of the scattered R~ loads and by HBM.  PNM A=66 |n_i|<=4
+// takes 65 us, eight Anderson twists of |n_i|<=3 with the shared scatter 268 us; with
+// four R~ loads an amplitude 87 and 338, one-body start, ring scatter, update and
+// energy as passes of their own 130 and 585.
 constexpr int kAAMax = 9;   // held vectors + the new one
 template <bool F32, int MODE>
 __global__ __launch_bounds__(256) void k_t_end(const SolveDesc *descs, const IterCtrl *ctrl, int terms,
@@ -717,7 +730,7 @@ __global__ __launch_bounds__(256) void k_t_end(const SolveDesc *descs, const Ite
     const int c = d.t_ch[u];
     const uint64_t lab = d.lab[u];
     const double2 r0 = d.R0[u];
-    double2 r = r0, t = make_double2(0.0, 0.0);
+    double2 r = make_double2(0.0, 0.0), t = r;
     if (MODE != 0) t = d.T[u];
     float2 g[kAAMax - 1];
     if constexpr (MODE == 2)
@@ -751,22 +764,19 @@ __global__ __launch_bounds__(256) void k_t_end(const SolveDesc *descs, const Ite
     }
     if (terms & 4) r = cadd(d.Rh[u], r);
     if (terms & 8) {
-      const int4 p = *(const int4 *)(d.ring4 + 4 * (int64_t)u);
-      double2 v0, v1, v2, v3;
+      const int2 p = ((const int2 *)d.ring2)[u];
+      double2 v0, v1;
       if constexpr (F32) {
-        const float2 f0 = d.Rt32[p.x], f1 = d.Rt32[p.y], f2 = d.Rt32[p.z], f3 = d.Rt32[p.w];
+        const float2 f0 = d.Rt32[p.x], f1 = d.Rt32[p.y];
         v0 = make_double2(f0.x, f0.y);
         v1 = make_double2(f1.x, f1.y);
-        v2 = make_double2(f2.x, f2.y);
-        v3 = make_double2(f3.x, f3.y);
       } else {
         v0 = d.Rt[p.x];
         v1 = d.Rt[p.y];
-        v2 = d.Rt[p.z];
-        v3 = d.Rt[p.w];
       }
-      r = cadd(r, csub(csub(cadd(v0, v3), v1), v2));
+      r = cadd(r, csub(v0, v1));
     }
+    r = cadd(r0, r);
     d.R[u] = r;
     if constexpr (MODE != 0) {
       const double2 hi = d.dh[i], hj = d.dh[j], pa = d.dp[a - d.A], pb = d.dp[b - d.A];
@@ -1818,7 +1828,7 @@ static void fill_blocks(const SolveDesc &d, const V &vas, int nch, int nphc, int
   hipLaunchKernelGGL(k_fill_vpppp<V>, dim3(gx((int64_t)max_npp * max_npp), nch), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_fill_vhhpp<V>, dim3(gx((int64_t)max_npp * max_nhh), nch), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_fill_vhhhh<V>, dim3(gx((int64_t)max_nhh * max_nhh), nch), dim3(256), 0, st, d, vas);
-  hipLaunchKernelGGL(k_fill_w0<V>, dim3(gx((int64_t)max_nhp * max_nhp), nphc), dim3(256), 0, st, d, vas);
+  hipLaunchKernelGGL(k_fill_w0<V>, dim3(gx((int64_t)max_nhp * max_nhp), nphc, 2), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_fock<V>, dim3((d.nsp + 255) / 256), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_e0<V>, dim3(1), dim3(256), 0, st, d, vas);
 }
@@ -1882,7 +1892,7 @@ static void launch_3nf_t(const SolveDesc &d, const Chiral3Dev &c, int approx, in
   hipLaunchKernelGGL(k_no2b_vpppp<ONE>, dim3(gx((int64_t)max_npp * (max_npp + 1) / 2), nch), dim3(256), 0, st, d, c);
   hipLaunchKernelGGL(k_no2b_vhhpp<ONE>, dim3(gx((int64_t)max_npp * max_nhh), nch), dim3(256), 0, st, d, c);
   hipLaunchKernelGGL(k_no2b_vhhhh<ONE>, dim3(gx((int64_t)max_nhh * (max_nhh + 1) / 2), nch), dim3(256), 0, st, d, c);
-  hipLaunchKernelGGL(k_no2b_w0<ONE>, dim3(gx((int64_t)max_nhp * (max_nhp + 1) / 2), nphc), dim3(256), 0, st, d, c);
+  hipLaunchKernelGGL(k_no2b_w0<ONE>, dim3(gx((int64_t)max_nhp * (max_nhp + 1) / 2), nphc, 2), dim3(256), 0, st, d, c);
 }
 
 void launch_3nf(const SolveDesc &d, const Chiral3Dev &c, int approx, int nch, int nphc, int max_npp, int max_nhh,

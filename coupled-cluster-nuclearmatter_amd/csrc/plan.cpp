@@ -286,11 +286,12 @@ void build_plan(const Orbitals &orb, Plan &P) {
   std::map<Key, std::vector<std::pair<int, int>>> phm, hpm;
   for (int a = A; a < nsp; ++a)
     for (int i = 0; i < A; ++i) phm[keyd(a, i)].push_back({a, i});
-  for (int j = 0; j < A; ++j)
-    for (int b = A; b < nsp; ++b) hpm[keyd(j, b)].push_back({j, b});
+  for (int b = A; b < nsp; ++b)   // both spin states of j side by side
+    for (int j = 0; j < A; ++j) hpm[keyd(j, b)].push_back({j, b});
   std::vector<int> phrow((size_t)np * A, -1), phch((size_t)np * A, -1);
   std::vector<int> hpcol((size_t)A * np, -1);
-  P.off_ph = {0}; P.off_hp = {0}; P.off_rt = {0}; P.off_i4 = {0}; P.off_vt = {0};
+  P.off_ph = {0}; P.off_hp = {0};
+  std::map<Key, int> chof;
   int K = 0;
   for (auto &kv : phm) {
     auto hit = hpm.find(kv.first);
@@ -310,14 +311,34 @@ void build_plan(const Orbitals &orb, Plan &P) {
     P.nph.push_back(nphk); P.nhp.push_back(nhpk);
     P.off_ph.push_back(P.off_ph.back() + nphk);
     P.off_hp.push_back(P.off_hp.back() + nhpk);
-    P.off_rt.push_back(P.off_rt.back() + (int64_t)nphk * nhpk);
-    P.off_i4.push_back(P.off_i4.back() + (int64_t)nhpk * nhpk);
-    P.off_vt.push_back(P.off_vt.back() + (int64_t)nhpk * nphk);
+    P.ring_elems += (int64_t)nphk * nhpk;
+    P.w0_elems += (int64_t)nhpk * nhpk;
+    chof[kv.first] = K;
     ++K;
   }
   P.nphc = K;
-  P.nRt = P.off_rt.back();
-  P.nI4 = P.off_i4.back();
+  P.ph_pair.resize(K);
+  for (auto &kv : chof) {
+    const Key &k = kv.first;
+    auto it = chof.find(Key{-k.tz, -k.x, -k.y, -k.z});
+    if (it == chof.end()) throw std::runtime_error("internal: Pandya channel without its pair");
+    P.ph_pair[kv.second] = it->second;
+  }
+  P.off_rt.assign(K, -1);
+  P.off_vt.assign(K, -1);
+  P.off_i4.assign(K, -1);
+  P.off_w1.assign(K, -1);
+  bool self = false;
+  for (int k = 0; k < K; ++k) {
+    if (!P.ring_first(k)) continue;
+    P.off_rt[k] = P.off_vt[k] = P.nRt;
+    P.nRt += (int64_t)P.nph[k] * P.nhp[k];
+    P.off_i4[k] = P.nI4;
+    P.nI4 += (int64_t)P.nhp[k] * P.nhp[k];
+    P.off_w1[k] = P.nW1;
+    P.nW1 += (int64_t)P.nph[k] * P.nph[k];
+    self = self || P.ph_pair[k] == k;
+  }
 
   auto pos = [&](int a, int i, int j, int b) -> int64_t {
     size_t pa = (size_t)(a - A) * A + i;
@@ -325,22 +346,25 @@ void build_plan(const Orbitals &orb, Plan &P) {
     if (k < 0) return -1;
     int r = phrow[pa];
     int s = hpcol[(size_t)j * np + (b - A)];
-    if (s < 0) return -1;
+    if (s < 0 || P.off_rt[k] < 0) return -1;
     return P.off_rt[k] + (int64_t)r * P.nhp[k] + s;
   };
-  P.ring4.resize((size_t)P.nT * 4);
+  if (P.nRt >= ((int64_t)1 << 31)) throw std::runtime_error("ring blocks above 2^31 elements");
+  P.ring2.resize((size_t)P.nT * 2);
+  if (self) P.ring2b.assign((size_t)P.nT * 2, -1);
   for (int ch = 0; ch < P.nch; ++ch) {
     for (int r = 0; r < P.npp[ch]; ++r) {
       int a = P.pp_a[P.off_pp[ch] + r], b = P.pp_b[P.off_pp[ch] + r];
       for (int s = 0; s < P.nhh[ch]; ++s) {
         int i = P.hh_i[P.off_hh[ch] + s], j = P.hh_j[P.off_hh[ch] + s];
         int64_t u = P.off_t[ch] + (int64_t)r * P.nhh[ch] + s;
-        P.ring4[u * 4 + 0] = pos(a, i, j, b);
-        P.ring4[u * 4 + 1] = pos(b, i, j, a);
-        P.ring4[u * 4 + 2] = pos(a, j, i, b);
-        P.ring4[u * 4 + 3] = pos(b, j, i, a);
-        for (int q = 0; q < 4; ++q)
-          if (P.ring4[u * 4 + q] < 0) throw std::runtime_error("internal: Pandya position missing");
+        const int64_t at[2][2] = {{pos(a, i, j, b), pos(b, j, i, a)}, {pos(b, i, j, a), pos(a, j, i, b)}};
+        for (int q = 0; q < 2; ++q) {
+          const int64_t x = at[q][0], y = at[q][1];
+          if (x < 0 && y < 0) throw std::runtime_error("internal: Pandya position missing");
+          P.ring2[u * 2 + q] = (int)(x < 0 ? y : x);
+          if (x >= 0 && y >= 0) P.ring2b[u * 2 + q] = (int)y;
+        }
       }
     }
   }

@@ -64,14 +64,26 @@ struct Plan {
   int nphc = 0;
   std::vector<int> nph, nhp;
   std::vector<int64_t> off_ph, off_hp;    // pair lists
-  std::vector<int64_t> off_rt;            // T~/R~ / V~^T blocks: nph x nhp
-  std::vector<int64_t> off_i4;            // I4/W0 blocks: nhp x nhp
-  std::vector<int64_t> off_vt;            // V~ blocks: nhp x nph
+  // Channels -K' and K' hold the same elements: (a,i) of one is (i,a) of the other,
+  // and T~(-K') is the transpose of T~(K'), since t(ab,ij) = t(ba,ji) (V~ likewise).
+  // The ring is contracted in the first channel of each pair only, where
+  // R~((a,i),(j,b)) is the sum of its two positions:
+  //   R~(K') = T~ (W0 + V~ T~) + W1 T~,  W1 = W0(-K')^T
+  // K' = -K' (a particle and a hole of one momentum: an open shell) pairs with itself.
+  // Blocks exist for first channels only (offset -1 elsewhere).
+  std::vector<int> ph_pair;               // the channel -K'
+  bool ring_first(int K) const { return K >= ph_pair[K]; }
+  std::vector<int64_t> off_rt;            // T~/R~: nph x nhp
+  std::vector<int64_t> off_vt;            // V~: nhp x nph
+  std::vector<int64_t> off_i4;            // I4/W0: nhp x nhp
+  std::vector<int64_t> off_w1;            // W1: nph x nph
   std::vector<int> ph_a, ph_i, hp_j, hp_b;
-  int64_t nRt = 0, nI4 = 0;
-  // four Pandya positions of every unique T element (a<b,i<j):
-  //   ((a,i),(j,b)) +,  ((b,i),(j,a)) -,  ((a,j),(i,b)) -,  ((b,j),(i,a)) +
-  std::vector<int64_t> ring4;   // nT * 4, -1 if absent
+  int64_t nRt = 0, nI4 = 0, nW1 = 0;
+  int64_t ring_elems = 0, w0_elems = 0;   // T~ and W0 elements of all channels
+  // positions in T~ and R~ of every unique T element (a<b,i<j): of ((a,i),(j,b)) or
+  // ((b,j),(i,a)) (+), and of ((b,i),(j,a)) or ((a,j),(i,b)) (-)
+  std::vector<int> ring2;    // nT * 2
+  std::vector<int> ring2b;   // the other position where the channel is its own pair, else -1; empty: none
 
   int64_t t2_ordered = 0;
 };

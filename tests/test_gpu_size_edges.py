@@ -218,3 +218,46 @@ def test_solve_loop_forms_the_iterates_of_the_step_interface(ccnm, A, nmax, prec
     assert np.all(np.isfinite(t0)) and np.abs(t0).max() > 0
     assert np.abs(t - t0).max() <= 1e-13 * np.abs(t0).max()
     assert abs(e - e0) <= 1e-12 * abs(e0)
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist", [
+    (3, "pnm", 1, (0.0, 0.0, 0.0)), (15, "pnm", 1, (0.5, 1.0, 1.5)), (6, "snm", 1, (0.0, 0.0, 0.0)),
+    (14, "pnm", 1, (0.5, 1.0, 1.5)), (38, "pnm", 2, (0.0, 0.0, 0.0))])
+@pytest.mark.parametrize("lists", [False, True])
+def test_ring_of_channel_pairs_equals_oracle(ccnm, monkeypatch, A, matter, nmax, twist, lists):
+    """The ring is contracted in one of the channels K', -K' of each pair.  A = 3, 6
+    and 15 leave a momentum half filled, so K' = 0 is its own pair.  The oracle
+    contracts every channel in 64 bits; 1e-12 of the largest element as in
+    test_residual_terms_elementwise_nmax2.  T~, W0 and R~ of all channels come back
+    through the debug arrays: R~ as T~ (W0 + 1/2 V~ T~) channel by channel."""
+    import ccd_oracle as co
+    import chiral_oracle as ch
+    lat = co.Lattice.build(A, matter, 0.16, nmax, twist)
+    cc = co.CCD(lat, ch.ChiralInteraction(lat, ch.NNLO, 450.0))
+    s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax, twist=twist)
+    s.set_chiral(ccnm.NNLO, 450.0)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    s.setup_t_amplitudes()
+    s.t2_intermediate()
+    s.diis_t1t2(1, 1)
+    t, lab = s.t2_unique(), s.t2_labels()
+    a, b, i, j = lab.T
+    x = np.zeros(cc.ch.size, np.complex128)
+    for (p, q, r_, u), sg in (((a, b, i, j), 1.0), ((b, a, i, j), -1.0), ((a, b, j, i), -1.0), ((b, a, j, i), 1.0)):
+        x[cc.ch.flat_index(p, q, r_, u)] = sg * t
+    R = cc.flat(cc.residual(cc.unflat(x), 8)[0])[cc.ch.flat_index(a, b, i, j)]
+    monkeypatch.setenv("CCGPU_TERMS", "8")
+    if lists:
+        monkeypatch.setenv("CCGPU_SPLIT_K", "256")
+    s.t2_intermediate()
+    got = s.debug_fetch("R", len(t))
+    assert np.abs(got - R).max() <= 1e-12 * np.abs(R).max()
+    n = s.dims["ring_elems"]
+    tt, rt = s.debug_fetch("Tt", n), s.debug_fetch("Rt", n)
+    r0 = s.debug_fetch("R0", len(t))
+    # every amplitude stands in four places of T~
+    assert abs(np.sum(np.abs(tt) ** 2) - 4 * np.sum(np.abs(t) ** 2)) <= 1e-12 * np.sum(np.abs(tt) ** 2)
+    # sum over the ordered amplitudes of conj(t) (R - conj V) = sum of conj(T~) R~
+    want = 4 * np.sum(np.conj(t) * (R - r0))
+    assert abs(4 * np.sum(np.conj(tt) * rt) - want) <= 1e-11 * np.sum(np.abs(tt) * np.abs(rt))
+    s.close()
