@@ -726,7 +726,7 @@ struct Batch {
   // second stream (default priority) for the ring branch of the residual, and
   // the fork/join events
   hipStream_t stream2 = nullptr, stream3 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_x = nullptr, ev_hh = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_hh = nullptr;
   // a residual with its update, per precision mode and accelerator
   hipGraph_t graph[8] = {};
   hipGraphExec_t gexec[8] = {};
@@ -754,7 +754,6 @@ struct Batch {
     }
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
-    if (ev_x) (void)hipEventDestroy(ev_x);
     if (ev_hh) (void)hipEventDestroy(ev_hh);
     if (stream2) (void)hipStreamDestroy(stream2);
     if (stream3) (void)hipStreamDestroy(stream3);
@@ -1078,7 +1077,6 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
   HIPCHK(hipStreamCreateWithFlags(&B->stream3, hipStreamNonBlocking));
   HIPCHK(hipEventCreateWithFlags(&B->ev_fork, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&B->ev_join, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&B->ev_x, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&B->ev_hh, hipEventDisableTiming));
   B->d_ctrl = dalloc<IterCtrl>(n, B->owned);
   B->ctrl.assign(n, IterCtrl{});
@@ -1481,14 +1479,14 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   // the families in FP64 run the tiles of contract.hip
   const bool tiles64 = B.f64.ready && fp64_tiles();
   auto t64 = [&](int bit) { return tiles64 && pf(bit) == CCGPU_PREC_FP64; };
-  // Three streams outside the timing mode (fork/join through events, also
-  // inside a captured graph), from the opening pass on.  The ring contractions
-  // read only T and the ring blocks and touch R only in the closing pass: a
-  // second stream, beside the one-body intermediates, whose small launches leave
-  // most of the chip idle, and beside the ladders, which stream V_pppp from HBM
-  // while the ring keeps the matrix cores busy.  A third stream takes I6 (rows
-  // of V* against rows of T), then the hh ladder into Rh once X is done.  All
-  // three meet in the closing pass.
+  // Three streams outside the timing mode (fork/join through events, also inside a
+  // captured graph) between the opening and the closing pass: the pp ladder, which
+  // streams V_pppp from HBM, on this one; X, I7, I9 and the hh ladder on the third; I6
+  // and the ring on the second.  Each writes its own arrays and reads none of the
+  // others'.  As plain chains from the fork to the join each has a queue of its own
+  // in a graph too: with the ladder after X, and the hh ladder after I6 and X, the ring
+  // shared the ladder's queue and ran after it.  PNM A=66 |n_i|<=4 in FP64 17.0 to 16.1
+  // ms, |n_i|<=3 mixed 5.70 to 5.04, four densities 19.4 to 18.6.
   // A fork and its join cost some 10 us each on the host and the queues, which
   // small batches do not win back: an iteration of SNM A=28 |n_i|<=2 (92 k
   // amplitudes) takes 145 us on three streams and 124 on one, SNM A=76 |n_i|<=2
@@ -1515,64 +1513,67 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   if (fork || fork6) HIPCHK(hipEventRecord(B.ev_fork, st));
   if (fork) HIPCHK(hipStreamWaitEvent(sr, B.ev_fork, 0));
   if (fork6) HIPCHK(hipStreamWaitEvent(s6, B.ev_fork, 0));
-  // launch (and graph node) order: the one-body chain first, the ring after it
-  {
-    Timer t(timing, s6, "i6");
-    launch_i6(B.d_descs, n, B.maxNp, B.maxRows, s6);
-  }
-  {
-    Timer t(timing, st, "gemm_x_vhhpp_t");
-    if (t64(0)) launch_x64(B.f64.x, B.f64.nx, B.d_descs, st);
-    else run_gemm(list(B.g_x, B.g_xb, 0), B, pf(0), false, st);
-  }
-  {
-    Timer t(timing, st, "i7_i9");
-    launch_i7(B.d_descs, n, B.maxA, st);
-    if (!t64(0)) launch_i9(B.d_descs, n, B.maxVhh, st);   // the X tiles write I9 too
-  }
-  if (terms & 4) {
-    if (fork6) {
-      HIPCHK(hipEventRecord(B.ev_x, st));
-      HIPCHK(hipStreamWaitEvent(s6, B.ev_x, 0));
+  auto x_chain = [&](hipStream_t q) {   // X, I7, I9, the hh ladder
+    {
+      Timer t(timing, q, "gemm_x_vhhpp_t");
+      if (t64(0)) launch_x64(B.f64.x, B.f64.nx, B.d_descs, q);
+      else run_gemm(list(B.g_x, B.g_xb, 0), B, pf(0), false, q);
     }
-    Timer t(timing, s6, "gemm_hh_ladder");
-    if (t64(2)) launch_hh64(B.f64.hh, B.f64.nhh, B.d_descs, s6);
-    else run_gemm(list(B.g_hh, B.g_hhb, 2), B, pf(2), false, s6);
-  }
-  if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
-  if (terms & 8) {
+    {
+      Timer t(timing, q, "i7_i9");
+      launch_i7(B.d_descs, n, B.maxA, q);
+      if (!t64(0)) launch_i9(B.d_descs, n, B.maxVhh, q);   // the X tiles write I9 too
+    }
+    if (terms & 4) {
+      Timer t(timing, q, "gemm_hh_ladder");
+      if (t64(2)) launch_hh64(B.f64.hh, B.f64.nhh, B.d_descs, q);
+      else run_gemm(list(B.g_hh, B.g_hhb, 2), B, pf(2), false, q);
+    }
+  };
+  auto i6 = [&](hipStream_t q) {
+    Timer t(timing, q, "i6");
+    launch_i6(B.d_descs, n, B.maxNp, B.maxRows, q);
+  };
+  auto ring = [&](hipStream_t q) {
+    if (!(terms & 8)) return;
     if (t64(3)) {
-      Timer t(timing, sr, "gemm_ring");
-      for (int c = kRingClasses - 1; c >= 0; --c) launch_ring64(B.f64.ring[c], B.f64.nring[c], c, B.d_descs, sr);
+      Timer t(timing, q, "gemm_ring");
+      for (int c = kRingClasses - 1; c >= 0; --c) launch_ring64(B.f64.ring[c], B.f64.nring[c], c, B.d_descs, q);
       if (!B.g_i4big.groups.empty()) {
-        run_gemm(B.g_i4big, B, CCGPU_PREC_FP64, false, sr);
-        run_gemm(B.g_rtbig, B, CCGPU_PREC_FP64, false, sr);
+        run_gemm(B.g_i4big, B, CCGPU_PREC_FP64, false, q);
+        run_gemm(B.g_rtbig, B, CCGPU_PREC_FP64, false, q);
       }
-    } else {
-      Timer t(timing, sr, "gemm_ring_i4");
-      if (ring32) run_gemm(B.g_i4f, B, pf(3), true, sr, false, 8);
-      else run_gemm(list(B.g_i4, B.g_i4b, 3), B, pf(3), false, sr);
+      return;
     }
-    if (!t64(3)) {
-      Timer t(timing, sr, "gemm_ring_rt");
-      if (ring32) run_gemm(B.g_rtf, B, pf(3), true, sr, false, 8);
-      else run_gemm(list(B.g_rt, B.g_rtb, 3), B, pf(3), false, sr);
+    {
+      Timer t(timing, q, "gemm_ring_i4");
+      if (ring32) run_gemm(B.g_i4f, B, pf(3), true, q, false, 8);
+      else run_gemm(list(B.g_i4, B.g_i4b, 3), B, pf(3), false, q);
     }
-  }
-  if (terms & 2) {
-    Timer t(timing, st, "gemm_pp_ladder");
+    Timer t(timing, q, "gemm_ring_rt");
+    if (ring32) run_gemm(B.g_rtf, B, pf(3), true, q, false, 8);
+    else run_gemm(list(B.g_rt, B.g_rtb, 3), B, pf(3), false, q);
+  };
+  auto pp_ladder = [&](hipStream_t q) {
+    if (!(terms & 2)) return;
+    Timer t(timing, q, "gemm_pp_ladder");
     if (shared) {
       // FP64 GEMMs on V_u, or BF16x3 on its FP32 copy in every low-precision mode
-      if (pp_prec == CCGPU_PREC_FP64) run_gemm(B.share.g64, B, CCGPU_PREC_FP64, false, st, false, 0);
-      else run_gemm(B.share.gbf, B, CCGPU_PREC_BF16X3, true, st, false, 7);
+      if (pp_prec == CCGPU_PREC_FP64) run_gemm(B.share.g64, B, CCGPU_PREC_FP64, false, q, false, 0);
+      else run_gemm(B.share.gbf, B, CCGPU_PREC_BF16X3, true, q, false, 7);
     } else if (tsplit) {
-      run_gemm(B.g_ppbf, B, pp_prec, true, st, true, 10);
+      run_gemm(B.g_ppbf, B, pp_prec, true, q, true, 10);
     } else if (pp_prec != CCGPU_PREC_FP64) {
-      run_gemm(B.g_pp32, B, pp_prec, true, st, true);
+      run_gemm(B.g_pp32, B, pp_prec, true, q, true);
     } else {
-      run_gemm(B.g_pp, B, pp_prec, false, st, true);
+      run_gemm(B.g_pp, B, pp_prec, false, q, true);
     }
-  }
+  };
+  pp_ladder(st);
+  x_chain(s6);
+  i6(sr);
+  ring(sr);
+  if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
   if (fork) {
     HIPCHK(hipEventRecord(B.ev_join, sr));
     HIPCHK(hipStreamWaitEvent(st, B.ev_join, 0));
