@@ -60,6 +60,8 @@ void launch_gemm_shape(const GemmGroup *groups, const GemmTile *tiles, int ntile
                        const int *gsolve, int kind, int mb, int nb, int lb, hipStream_t st);
 int ring64_class(int nph, int nhp);
 int ring64_columns(int nph, int nhp);
+int ringbf_columns(int nph, int nhp);
+void launch_ringbf(const RingTile32 *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
 void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *dd, hipStream_t st);
 void launch_x64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
 void launch_hh64(const ZTile *tiles, int ntiles, const SolveDesc *dd, hipStream_t st);
@@ -147,7 +149,8 @@ T *dupload(const std::vector<T> &v, std::vector<void *> &owned) {
 // XCDs get equal tile counts.
 double tile_cost(const GemmTile &t) { return (double)(t.ke - t.kb); }   // a tile's time goes with its k range
 double tile_cost(const ZTile &t) { return t.cost; }
-double tile_cost(const RingTile &t) { return t.cost; }
+template <class T>
+double tile_cost(const RingTileOf<T> &t) { return t.cost; }
 template <typename Tile>
 void xcd_order_list(std::vector<Tile> &tiles, size_t ngroups) {
   const int nx = 8;
@@ -675,6 +678,13 @@ struct Batch {
     RingTile *ring[kRingClasses] = {};
   } f64;
   GemmList g_i4big, g_rtbig;
+  // the BF16x3 ring on the FP32 blocks, fused likewise
+  struct RingBf {
+    bool ready = false;
+    int n = 0;
+    RingTile32 *tiles = nullptr;
+  } rbf;
+  GemmList g_i4fbig, g_rtfbig;
   GemmList g_ppbf;         // BF16x3 pp ladder reading the split copy of T (when every solve has one)
   bool ppbf = false;
   // Shared pp ladder of a batch of twists of one lattice and interaction: the
@@ -1026,23 +1036,33 @@ std::unique_ptr<Batch> make_batch(const std::vector<Solve *> &ss, hipStream_t st
     to32(B->g_i4f);
     to32(B->g_rtf);
   }
-  // ring groups of the channels the fused FP64 kernel does not take
-  for (size_t g = 0; g < B->g_rt.groups.size(); ++g) {
-    const GemmGroup &q = B->g_rt.groups[g];
-    if (ring64_class(q.M, q.K) >= 0) continue;
-    for (size_t k = 2 * g; k < 2 * g + 2; ++k) {
-      B->g_i4big.groups.push_back(B->g_i4.groups[k]);
-      B->g_i4big.gsolve.push_back(B->g_i4.gsolve[k]);
+  // ring groups of the channels the fused kernels do not take
+  auto large = [](const GemmList &i4, const GemmList &rt, GemmList &i4big, GemmList &rtbig, auto fused) {
+    for (size_t g = 0; g < rt.groups.size(); ++g) {
+      const GemmGroup &q = rt.groups[g];
+      if (fused(q.M, q.K)) continue;
+      for (size_t k = 2 * g; k < 2 * g + 2; ++k) {
+        i4big.groups.push_back(i4.groups[k]);
+        i4big.gsolve.push_back(i4.gsolve[k]);
+      }
+      rtbig.groups.push_back(q);
+      rtbig.gsolve.push_back(rt.gsolve[g]);
     }
-    B->g_rtbig.groups.push_back(q);
-    B->g_rtbig.gsolve.push_back(B->g_rt.gsolve[g]);
-  }
-  B->g_i4big.fam = 3;
-  B->g_rtbig.fam = 4;
+    i4big.fam = 3;
+    rtbig.fam = 4;
+  };
+  large(B->g_i4, B->g_rt, B->g_i4big, B->g_rtbig, [](int nph, int nhp) { return ring64_class(nph, nhp) >= 0; });
+  if (B->ring32)
+    large(B->g_i4f, B->g_rtf, B->g_i4fbig, B->g_rtfbig, [](int nph, int nhp) { return ringbf_columns(nph, nhp) > 0; });
   const int fams[13] = {0, 1, 2, 3, 4, 1, 0, 2, 3, 4, 3, 4, 1};
   GemmList *lists[13] = {&B->g_x, &B->g_pp, &B->g_hh, &B->g_i4, &B->g_rt, &B->g_pp32,
                          &B->g_xb, &B->g_hhb, &B->g_i4b, &B->g_rtb, &B->g_i4f, &B->g_rtf, &B->g_ppbf};
   B->d_descs = dupload(B->h_descs, B->owned);
+  for (GemmList *L : {&B->g_i4fbig, &B->g_rtfbig}) {
+    L->bf3 = L->xcd = L->nosplit = true;
+    const GemmShape def[GemmList::NCLS] = {{1, 1}, {1, 2}, {1, 4}, {1, 8}, {1, 6}, {0, 4}};
+    for (int c = 0; c < GemmList::NCLS; ++c) L->shape[c] = def[c];
+  }
   for (int k = 0; k < 13; ++k) {
     lists[k]->fam = fams[k];
     lists[k]->bf3 = k >= 6 && k < 12;
@@ -1340,6 +1360,34 @@ void prepare_fp64(Batch &B) {
   F.ready = true;
 }
 
+void prepare_ringbf(Batch &B) {
+  if (B.rbf.ready) return;
+  std::vector<RingTile32> tiles;
+  int g = 0;
+  for (size_t s = 0; s < B.solves.size(); ++s) {
+    const Plan &P = B.solves[s]->plan;
+    const SolveDesc &d = B.h_descs[s];
+    for (int K = 0; K < P.nphc; ++K, ++g) {
+      const int nph = P.nph[K], nhp = P.nhp[K], bc = ringbf_columns(nph, nhp);
+      if (!bc || !P.ring_first(K)) continue;
+      for (int n0 = 0; n0 < nhp; n0 += bc)
+        tiles.push_back(RingTile32{d.Vt32 + P.off_vt[K], d.Tt32 + P.off_rt[K], d.W0_32 + P.off_i4[K],
+                                   d.W1_32 + P.off_w1[K], d.Rt32 + P.off_rt[K], nhp, nph, n0, (int)s, g,
+                                   2.0f * nph + nhp});
+    }
+  }
+  xcd_order_list(tiles, g);
+  B.rbf.n = (int)tiles.size();
+  B.rbf.tiles = dupload(tiles, B.owned);
+  for (GemmList *L : {&B.g_i4fbig, &B.g_rtfbig}) {
+    if (L->groups.empty()) continue;
+    autotune(*L, 8, B.d_descs, B.stream);
+    L->build_tiles();
+    L->upload(B.owned);
+  }
+  B.rbf.ready = true;
+}
+
 void prepare_lists(Batch &B, int prec) {
   const int kinds[13] = {0, 3, 0, 0, 0, 4, 6, 6, 6, 6, 8, 8, 10};   // the kernel kind each list is tuned for
   GemmList *lists[13] = {&B.g_x, &B.g_pp, &B.g_hh, &B.g_i4, &B.g_rt, &B.g_pp32, &B.g_xb, &B.g_hhb, &B.g_i4b, &B.g_rtb,
@@ -1348,13 +1396,15 @@ void prepare_lists(Batch &B, int prec) {
   const bool tiles64 = fp64_tiles() && tail_low_mask() == 0;
   const bool all64 = prec == CCGPU_PREC_FP64 || prec == CCGPU_PREC_V32;
   if (tiles64) prepare_fp64(B);
+  const bool fused32 = fp64_tiles() && B.ring32;
+  if (fused32 && prec == CCGPU_PREC_BF16X3) prepare_ringbf(B);
   for (int k = 0; k < 13; ++k) {
     GemmList &L = *lists[k];
     if (L.ready) continue;
     if (tiles64 && all64 && k < 5 && k != 1) continue;
     if (k == 5 && (prec == CCGPU_PREC_FP64 || !B.has_f32)) continue;
     if (k >= 6 && prec != CCGPU_PREC_BF16X3) continue;
-    if (k >= 10 && k < 12 && !B.ring32) continue;
+    if (k >= 10 && k < 12 && (!B.ring32 || fused32)) continue;
     if (k == 12 && !B.ppbf) continue;
     autotune(L, kinds[k], B.d_descs, B.stream);
     L.build_tiles();
@@ -1542,6 +1592,15 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
       if (!B.g_i4big.groups.empty()) {
         run_gemm(B.g_i4big, B, CCGPU_PREC_FP64, false, q);
         run_gemm(B.g_rtbig, B, CCGPU_PREC_FP64, false, q);
+      }
+      return;
+    }
+    if (ring32 && B.rbf.ready && fp64_tiles()) {
+      Timer t(timing, q, "gemm_ring");
+      launch_ringbf(B.rbf.tiles, B.rbf.n, B.d_descs, q);
+      if (!B.g_i4fbig.groups.empty()) {
+        run_gemm(B.g_i4fbig, B, pf(3), true, q, false, 8);
+        run_gemm(B.g_rtfbig, B, pf(3), true, q, false, 8);
       }
       return;
     }
@@ -2109,15 +2168,17 @@ void ensure_f32(Solve &S, int handle) {
   S.d_off_vpp32 = dupload(S.off_vpp32, S.owned);
   S.d_npp = dupload(P.npp, S.owned);
   S.desc.Vpppp32 = dalloc<float2>(S.nVpp32, S.owned);
-  // FP32 ring blocks of the BF16x3 residual; T~ entries with a=b or i=j stay zero
-  S.desc.Tt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), S.owned);
+  // FP32 ring blocks of the BF16x3 residual; T~ entries with a=b or i=j stay zero, and
+  // k_ringbf reads rows in words of four elements
+  constexpr int kRing32Pad = 4;
+  S.desc.Tt32 = dalloc<float2>(P.nRt + kRing32Pad, S.owned);
   S.desc.Rt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), S.owned);
-  S.desc.Vt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), S.owned);
+  S.desc.Vt32 = dalloc<float2>(P.nRt + kRing32Pad, S.owned);
   S.desc.I4_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
   S.desc.W0_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
-  S.desc.W1_32 = dalloc<float2>(std::max<int64_t>(P.nW1, 1), S.owned);
+  S.desc.W1_32 = dalloc<float2>(P.nW1 + kRing32Pad, S.owned);
   S.desc.Tbf = dalloc<uint4>(std::max<int64_t>(P.nT, 1), S.owned);
-  HIPCHK(hipMemset(S.desc.Tt32, 0, std::max<int64_t>(P.nRt, 1) * sizeof(float2)));
+  HIPCHK(hipMemset(S.desc.Tt32, 0, (P.nRt + kRing32Pad) * sizeof(float2)));
   fill_f32(S);
   HIPCHK(hipMemcpy(S.d_desc, &S.desc, sizeof(SolveDesc), hipMemcpyHostToDevice));
   drop_single(handle);

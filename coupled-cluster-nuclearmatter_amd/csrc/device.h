@@ -112,12 +112,15 @@ struct ZTile {
 constexpr int kRingClasses = 2;   // launches of the fused ring (ring64_class)
 
 // Columns n0 .. of one Pandya channel pair's ring contractions (contract.hip)
-struct RingTile {
-  const double2 *Vt, *Tt, *W0, *W1;
-  double2 *Rt;
+template <class T>   // double2, or float2 for the FP32 blocks
+struct RingTileOf {
+  const T *Vt, *Tt, *W0, *W1;
+  T *Rt;
   int nhp, nph, n0, solve, g;
   float cost;
 };
+typedef RingTileOf<double2> RingTile;
+typedef RingTileOf<float2> RingTile32;
 
 // A triple of hole groups I <= J <= K (a group: the up to two spin states of one
 // momentum and isospin, in orbital order) of one (K3, Tz3) channel: its pair

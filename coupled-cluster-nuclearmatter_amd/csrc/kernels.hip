@@ -8,6 +8,7 @@
 //              and W1 : Nph x Nph, of one channel of each pair K', -K' (Plan::ph_pair)
 // Reference routines restated here are cited per kernel (paths relative to
 // deltafull-CCMkspace/ of the reference).
+#include "bf3.h"
 #include "device.h"
 #include "interaction.h"
 
@@ -17,7 +18,6 @@
 namespace ccgpu {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -1490,23 +1490,6 @@ __global__ __launch_bounds__(256) void k_zgemm_la(const GemmGroup *__restrict__ 
 // the count of loads in flight is the same on every path, and the barriers
 // wait for LDS only (a workgroup fence would drain the loads in flight).
 // The k order is fixed by the tile, so repeated runs give the same bits.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ void bf3_split(float x, float y, unsigned &hi, unsigned &lo) {
-  const __bf16 xh = (__bf16)x, yh = (__bf16)y;
-  const __bf16 xl = (__bf16)(x - (float)xh), yl = (__bf16)(y - (float)yh);
-  hi = __builtin_bit_cast(unsigned, (bf16x2){xh, yh});
-  lo = __builtin_bit_cast(unsigned, (bf16x2){xl, yl});
-}
-// (br, -bi) -> (bi, br): swap the halves, then flip the sign of the new low half
-__device__ __forceinline__ u32x4 bf3_im_pairs(u32x4 v) {
-  u32x4 r;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) r[q] = ((v[q] >> 16) | (v[q] << 16)) ^ 0x8000u;
-  return r;
-}
 __device__ __forceinline__ uint4 t_split(double2 b) {
   unsigned h, l;
   bf3_split((float)b.x, -(float)b.y, h, l);

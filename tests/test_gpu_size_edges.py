@@ -261,3 +261,32 @@ def test_ring_of_channel_pairs_equals_oracle(ccnm, monkeypatch, A, matter, nmax,
     want = 4 * np.sum(np.conj(t) * (R - r0))
     assert abs(4 * np.sum(np.conj(tt) * rt) - want) <= 1e-11 * np.sum(np.abs(tt) * np.abs(rt))
     s.close()
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist", [
+    (3, "pnm", 1, (0.0, 0.0, 0.0)), (15, "pnm", 1, (0.3, 0.6, 0.9)), (28, "snm", 2, (0.0, 0.0, 0.0)),
+    (66, "pnm", 3, (0.9, 1.35, 1.8)), (108, "snm", 2, (0.0, 0.0, 0.0)), (246, "pnm", 3, (0.2, 0.4, 0.6))])
+def test_bf16x3_fused_ring_equals_list_kernels(ccnm, monkeypatch, A, matter, nmax, twist):
+    """The BF16x3 ring in one launch against the list kernels: channels of 1 to
+    above 256 rows, at most 4 hp pairs, odd counts, one that is its own pair.  Both sum
+    the same split products in FP32, k at most some 500 a contraction and two of
+    them nested: 2 (2 K + 4) 2^-24 = 1.2e-4 of the sum of moduli, which the largest
+    element of the ring bounds within a factor of ten on these amplitudes, and
+    rounding errors of that many terms add up to a thirtieth of their bound: 4e-5 of
+    the largest element.  A lost k would be 1/256 and more of an element."""
+    monkeypatch.setenv("CCGPU_TERMS", "8")
+    out = []
+    for lists in (False, True):
+        if lists:
+            monkeypatch.setenv("CCGPU_SPLIT_K", "256")
+        s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax, twist=twist)
+        s.set_chiral(ccnm.NNLO, 450.0)
+        s.generate_interaction(ccnm.INT_CHIRAL)
+        s.setup_t_amplitudes()
+        s.t2_intermediate(ccnm.PREC_BF16X3)
+        n = s.dims["t2_unique"]
+        out.append(s.debug_fetch("R", n) - s.debug_fetch("R0", n))
+        s.close()
+    r, ref = out
+    assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0
+    assert np.abs(r - ref).max() <= 4e-5 * np.abs(ref).max()
