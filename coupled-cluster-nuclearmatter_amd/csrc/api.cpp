@@ -30,8 +30,7 @@ namespace ccgpu {
 // kernels.hip
 void launch_fill_blocks(const SolveDesc &d, double volume, int nch, int nphc, int max_npp, int max_nhh,
                         int max_nhp, hipStream_t st);
-void launch_fill_blocks_chiral(const SolveDesc &d, const ChiralDev &c, int nch, int nphc, int max_npp,
-                               int max_nhh, int max_nhp, hipStream_t st);
+void launch_fill_blocks_chiral(const SolveDesc &d, const ChiralDev &c, int nch, int nphc, hipStream_t st);
 void launch_elements(const SolveDesc &d, double volume, const ChiralDev *c, const int4 *pqrs, int n, double2 *out,
                      hipStream_t st);
 void launch_3nf(const SolveDesc &d, const Chiral3Dev &c, int approx, int nch, int nphc, int max_npp, int max_nhh,
@@ -495,6 +494,34 @@ struct Timer {
   }
 };
 
+// Pair groups of the pairs (a[x], b[x]), channel c at [off[c], off[c + 1]).  In a channel
+// conservation gives a group of a one group of b.
+PairGroups pair_groups(const Orbitals &o, const std::vector<int> &a, const std::vector<int> &b,
+                       const std::vector<int64_t> &off, std::vector<void *> &owned) {
+  std::map<std::array<int, 4>, int> ids;
+  std::vector<int> id(o.nsp);
+  for (int x = 0; x < o.nsp; ++x)
+    id[x] = ids.emplace(std::array<int, 4>{o.nx[x], o.ny[x], o.nz[x], o.tz[x]}, (int)ids.size()).first->second;
+  std::vector<PairGroup> g;
+  std::vector<int64_t> goff{0};
+  std::vector<int> last(ids.size(), -1);   // last group with this group of a
+  int most = 0;
+  for (size_t c = 0; c + 1 < off.size(); ++c) {
+    const int start = (int)g.size();
+    for (int64_t x = off[c]; x < off[c + 1]; ++x) {
+      int &at = last[id[a[x]]];
+      if (at < start || id[g[at].b] != id[b[x]]) {
+        at = (int)g.size();
+        g.push_back(PairGroup{a[x], b[x], {-1, -1, -1, -1}});
+      }
+      g[at].at[(o.sz[a[x]] > 0 ? 2 : 0) + (o.sz[b[x]] > 0 ? 1 : 0)] = (int)(x - off[c]);
+    }
+    goff.push_back((int64_t)g.size());
+    most = std::max(most, (int)g.size() - start);
+  }
+  return PairGroups{dupload(g, owned), dupload(goff, owned), most};
+}
+
 void build_device(Solve &S) {
   Plan &P = S.plan;
   auto &o = S.owned;
@@ -545,6 +572,10 @@ void build_device(Solve &S) {
   d.hp_j = dupload(P.hp_j, o); d.hp_b = dupload(P.hp_b, o);
   d.ring2 = dupload(P.ring2, o);
   d.ring2b = P.ring2b.empty() ? nullptr : dupload(P.ring2b, o);
+  d.gpp = pair_groups(P.orb, P.pp_a, P.pp_b, P.off_pp, o);
+  d.ghh = pair_groups(P.orb, P.hh_i, P.hh_j, P.off_hh, o);
+  d.ghp = pair_groups(P.orb, P.hp_j, P.hp_b, P.off_hp, o);
+  d.gph = pair_groups(P.orb, P.ph_i, P.ph_a, P.off_ph, o);
   d.T = dalloc<double2>(P.nT, o);
   d.R = dalloc<double2>(P.nT, o);
   d.R0 = dalloc<double2>(P.nT, o);
@@ -706,6 +737,7 @@ struct Batch {
     double2 *V = nullptr, *Tu = nullptr, *Ru = nullptr;
     float2 *V32 = nullptr;
     int *d_npp = nullptr, *d_pa = nullptr, *d_pb = nullptr;
+    PairGroups gpp{};
     int64_t *d_off_pp = nullptr, *d_off_v = nullptr;
     uint32_t **d_maps = nullptr;   // per solve: unique amplitude -> 2 * position + (sign < 0)
     GemmList g64, gbf;             // FP64 GEMMs on V_u, BF16x3 GEMMs on its FP32 copy
@@ -1242,6 +1274,7 @@ void build_shared(Batch &B) {
   }
   X.d_maps = dupload(maps, B.owned);
   X.d_npp = dupload(X.npp, B.owned);
+  X.gpp = pair_groups(B.solves[0]->plan.orb, X.pa, X.pb, X.off_pp, B.owned);
   X.d_pa = dupload(X.pa, B.owned);
   X.d_pb = dupload(X.pb, B.owned);
   X.d_off_pp = dupload(X.off_pp, B.owned);
@@ -1287,6 +1320,7 @@ void refresh_shared(Batch &B) {
   dv.off_pp = X.d_off_pp;
   dv.pp_a = X.d_pa;
   dv.pp_b = X.d_pb;
+  dv.gpp = X.gpp;
   dv.off_vpp = X.d_off_v;
   dv.Vpppp = X.V;
   launch_fill_vpppp(dv, S0.plan.orb.volume, S0.vkind == CCGPU_INT_CHIRAL ? &S0.chiral_dev : nullptr, X.nu,
@@ -2495,7 +2529,7 @@ int ccgpu_generate_interaction(int handle, int kind) {
       throw Error("the three-nucleon force belongs to the chiral interaction (CCGPU_INT_CHIRAL)");
     if (kind == CCGPU_INT_CHIRAL) {
       make_chiral_tables(S);
-      launch_fill_blocks_chiral(S.desc, S.chiral_dev, P.nch, P.nphc, P.max_npp, P.max_nhh, max_nhp, S.stream);
+      launch_fill_blocks_chiral(S.desc, S.chiral_dev, P.nch, P.nphc, S.stream);
       if (S.tnf >= 0) {
         Chiral3Dev &c = S.chiral3;
         c = chiral3_constants(S.chiral, S.tnf_ce, S.tnf_cd, S.tnf_cutoff, S.tnf_nexp);

@@ -13,6 +13,18 @@ struct DPair {
   int v;
 };
 
+// Up to four pairs of one list whose states differ in spin only: a state of each, and
+// the places at[2 s + t] of the pairs with spins s, t (0 down, 1 up), -1 absent.
+struct PairGroup {
+  int a, b, at[4];
+};
+// the pair groups of a list, channel by channel
+struct PairGroups {
+  const PairGroup *g;
+  const int64_t *off;   // channels + 1
+  int max;              // most groups of a channel
+};
+
 // Everything one solve's kernels read or write.  All pointers are device
 // pointers; arrays indexed by unique amplitude u have length nT.
 struct SolveDesc {
@@ -26,6 +38,7 @@ struct SolveDesc {
   const int *t_ch, *npp, *nhh;
   const int64_t *off_t, *off_pp, *off_hh, *off_vpp, *off_vhh;
   const int *pp_a, *pp_b, *hh_i, *hh_j;
+  PairGroups gpp, ghh, ghp, gph;   // of the lists above and below, (hole, particle) in the last two
   // per unique amplitude its orbitals a | b << 16 | i << 32 | j << 48
   const uint64_t *lab;
   const int *ob_rowB, *ob_rowA, *ob_colJ, *ob_colI;

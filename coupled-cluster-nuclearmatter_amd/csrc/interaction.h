@@ -183,6 +183,89 @@ static __device__ __forceinline__ double2 chiral_direct(const ChiralDev &c, cons
   return make_double2(g * v.x, g * v.y);
 }
 
+// What chiral_direct takes from the momenta and isospins of its four states alone, shared
+// by the sixteen spin combinations (dt: isospins unchanged).
+struct ChiralGeo {
+  double asq, a1, ass, g;
+  double qx, qy, qz, kx, ky, kz, wx, wy, wz;
+  bool spin_orbit;
+};
+
+// a = n_p - n_q, b = n_r - n_s of a combination that conserves momentum and isospin
+static __device__ __forceinline__ ChiralGeo chiral_geo(const ChiralDev &c, int ax, int ay, int az, int bx, int by,
+                                                       int bz, int t1, int t2, int t3, int t4) {
+  ChiralGeo o;
+  const int dx = ax - bx, dy = ay - by, dz = az - bz;
+  const double *R = c.rad + kChiralRad * (dx * dx + dy * dy + dz * dz);
+  const int ch = (t1 + t2) / 2 + 1;
+  const double f = c.side[ch * (c.jmax + 1) + ax * ax + ay * ay + az * az] *
+                   c.side[ch * (c.jmax + 1) + bx * bx + by * by + bz * bz];
+  const double dt = (t1 == t3 && t2 == t4) ? 1.0 : 0.0;
+  const double tt = sig_dot_sig(t1, t2, t3, t4);
+  const double u = c.qunit;
+  o.qx = u * dx; o.qy = u * dy; o.qz = u * dz;
+  o.g = c.scale * f;
+  o.spin_orbit = false;
+  o.kx = o.ky = o.kz = o.wx = o.wy = o.wz = 0.0;
+  if (c.order == 0) {
+    o.asq = R[kOpe2] * tt;
+    o.a1 = c.cs[1] * dt;
+    o.ass = c.ct[1] * dt;
+    return o;
+  }
+  double wt1;
+  if (t1 + t2 == 0) {
+    const double a = c.cg0[(1 - t1) / 2] * c.cg0[(1 - t3) / 2], b = c.cg1[(1 - t1) / 2] * c.cg1[(1 - t3) / 2];
+    wt1 = a * (-R[kOpe0] - 2.0 * R[kOpe1]) + b * (-R[kOpe0] + 2.0 * R[kOpe1]);
+  } else {
+    wt1 = R[kOpe0];
+  }
+  const double q2 = R[kQ2];
+  o.kx = 0.5 * u * (ax + bx); o.ky = 0.5 * u * (ay + by); o.kz = 0.5 * u * (az + bz);
+  const double k2 = o.kx * o.kx + o.ky * o.ky + o.kz * o.kz;
+  o.asq = wt1 + R[kVt] * dt + R[kWt] * tt + c.cnlo[5] * dt + R[kWt3] * tt;
+  o.a1 = c.cs[ch] * dt + R[kVc] * dt + R[kWc] * tt + (c.cnlo[0] * q2 + c.cnlo[1] * k2) * dt + R[kVc3] * dt;
+  o.ass = (c.ct[ch] + R[kVs] + c.cnlo[2] * q2 + c.cnlo[3] * k2) * dt + (R[kWs] + R[kWs3]) * tt;
+  o.spin_orbit = dt != 0.0;
+  o.wx = o.qy * o.kz - o.qz * o.ky; o.wy = o.qz * o.kx - o.qx * o.kz; o.wz = o.qx * o.ky - o.qy * o.kx;
+  return o;
+}
+
+// (sigma1.v)(sigma2.v) between spins that are constants after unrolling: the diagonal
+// elements of sigma.v are real
+static __device__ __forceinline__ double2 pauli_pair(int m1, int m2, int m3, int m4, double x, double y, double z) {
+  const double2 a = pauli_dot(m1, m3, x, y, z), b = pauli_dot(m2, m4, x, y, z);
+  if (m1 == m3 && m2 == m4) return make_double2(a.x * b.x, 0.0);
+  if (m1 == m3) return make_double2(a.x * b.x, a.x * b.y);
+  if (m2 == m4) return make_double2(a.x * b.x, a.y * b.x);
+  return cmul_i(a, b);
+}
+
+// chiral_direct for spins m1 m2 | m3 m4
+static __device__ __forceinline__ double2 chiral_spin(const ChiralDev &c, const ChiralGeo &o, int m1, int m2, int m3,
+                                                      int m4) {
+  const double2 sq = pauli_pair(m1, m2, m3, m4, o.qx, o.qy, o.qz);
+  const double a1 = (m1 == m3 && m2 == m4) ? o.a1 : 0.0;
+  double2 v = make_double2(o.asq * sq.x + a1 + o.ass * sig_dot_sig(m1, m2, m3, m4), o.asq * sq.y);
+  if (o.spin_orbit) {
+    double2 so = make_double2(0.0, 0.0);
+    if (m2 == m4) {
+      const double2 e = pauli_dot(m1, m3, o.wx, o.wy, o.wz);
+      so.x += e.x; so.y += e.y;
+    }
+    if (m1 == m3) {
+      const double2 e = pauli_dot(m2, m4, o.wx, o.wy, o.wz);
+      so.x += e.x; so.y += e.y;
+    }
+    v.x += c.cnlo[4] * 0.5 * so.y;
+    v.y -= c.cnlo[4] * 0.5 * so.x;
+    const double2 kk = pauli_pair(m1, m2, m3, m4, o.kx, o.ky, o.kz);
+    v.x += c.cnlo[6] * kk.x;
+    v.y += c.cnlo[6] * kk.y;
+  }
+  return make_double2(o.g * v.x, o.g * v.y);
+}
+
 // ---------------------------------------------------------------------------
 // The NNLO three-nucleon force, chiral_3nf_with_delta
 // (chiral_module_andreas_with_delta.f90:6670-6902): cD and cE contacts,

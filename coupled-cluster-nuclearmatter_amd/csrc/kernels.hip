@@ -109,20 +109,69 @@ __global__ void k_fill_w0(SolveDesc d, V vas) {
   }
 }
 
-// Fock matrix f_pq = t_p delta_pq + sum_h <ph||qh> for q in {p, partner(p)}
-// (normal_ordered_hamiltonian, ccm_main.f90:1586-1657).
-template <class V>
-__global__ void k_fock(SolveDesc d, V vas) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= d.nsp) return;
-  double2 fd = make_double2(d.e[p], 0.0), fp = make_double2(0.0, 0.0);
-  int pp = d.partner[p];
-  for (int h = 0; h < d.A; ++h) {
-    fd = cadd(fd, vas(p, h, p, h));
-    if (pp >= 0) fp = cadd(fp, vas(p, h, pp, h));
+// The chiral V blocks over pair groups: a thread takes the sixteen spin combinations of
+// a row and a column group, which share two transfers, their radial functions and
+// regulators; element by element the fill was bound by that arithmetic.  V_pppp of PNM
+// A=66 |n_i|<=4 (121 M elements, 1.93 GB) takes 0.66 ms, element by element 2.23; W0 and
+// W1 93 us, 335.
+// WHAT 0 <row||col> of pairs; 1 W0 and 2 W1, -<ib||ja> as in k_fill_w0 (rows (i,a) of W0,
+// (b,j) of W1).
+enum { kFillPairs, kFillW0, kFillW1 };
+template <int WHAT>
+__global__ __launch_bounds__(256) void k_fill_chiral(SolveDesc d, ChiralDev c, PairGroups rows, PairGroups cols,
+                                                     const int *ncol, const int64_t *off, double2 *out) {
+  const int ch = blockIdx.y;
+  if (off[ch] < 0) return;
+  const int nr = (int)(rows.off[ch + 1] - rows.off[ch]), nc = (int)(cols.off[ch + 1] - cols.off[ch]), n = ncol[ch];
+  double2 *blk = out + off[ch];
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < nr * nc; e += gridDim.x * 256) {
+    const PairGroup R = rows.g[rows.off[ch] + e / nc], C = cols.g[cols.off[ch] + e % nc];
+    const int p = WHAT == kFillW1 ? C.a : R.a, q = WHAT == kFillW0 ? C.b : R.b;
+    const int r = WHAT == kFillW1 ? R.a : C.a, s = WHAT == kFillW0 ? R.b : C.b;
+    const int ax = d.nx[p] - d.nx[q], ay = d.ny[p] - d.ny[q], az = d.nz[p] - d.nz[q];
+    const int bx = d.nx[r] - d.nx[s], by = d.ny[r] - d.ny[s], bz = d.nz[r] - d.nz[s];
+    const int t1 = d.tz[p], t2 = d.tz[q], t3 = d.tz[r], t4 = d.tz[s];
+    const ChiralGeo gd = chiral_geo(c, ax, ay, az, bx, by, bz, t1, t2, t3, t4);
+    const ChiralGeo gx = chiral_geo(c, ax, ay, az, -bx, -by, -bz, t1, t2, t4, t3);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      if (R.at[x] < 0) continue;
+      double2 *row = blk + (int64_t)R.at[x] * n;
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        if (C.at[y] < 0) continue;
+        const int ra = x & 2 ? 1 : -1, rb = x & 1 ? 1 : -1, ca = y & 2 ? 1 : -1, cb = y & 1 ? 1 : -1;
+        const int m1 = WHAT == kFillW1 ? ca : ra, m2 = WHAT == kFillW0 ? cb : rb;
+        const int m3 = WHAT == kFillW1 ? ra : ca, m4 = WHAT == kFillW0 ? rb : cb;
+        const double2 v = csub(chiral_spin(c, gd, m1, m2, m3, m4), chiral_spin(c, gx, m1, m2, m4, m3));
+        row[C.at[y]] = WHAT == kFillPairs ? v : make_double2(-v.x, -v.y);
+      }
+    }
   }
-  d.fdiag[p] = fd;
-  d.fpart[p] = fp;
+}
+
+// Fock matrix f_pq = t_p delta_pq + sum_h <ph||qh> for q in {p, partner(p)}
+// (normal_ordered_hamiltonian, ccm_main.f90:1586-1657).  A block per p, a thread per
+// hole, the terms added in hole order by one thread each; one thread per p for all
+// holes took 134 us (PNM A=66 |n_i|<=4), 9 us this.
+template <class V>
+__global__ __launch_bounds__(128) void k_fock(SolveDesc d, V vas) {
+  __shared__ double2 term[2][128];
+  const int p = blockIdx.x, pp = d.partner[p], x = threadIdx.x;
+  double2 f = make_double2(x == 0 ? d.e[p] : 0.0, 0.0);
+  for (int h0 = 0; h0 < d.A; h0 += 128) {
+    const int h = h0 + x;
+    if (h < d.A) {
+      term[0][x] = vas(p, h, p, h);
+      if (pp >= 0) term[1][x] = vas(p, h, pp, h);
+    }
+    __syncthreads();
+    if (x == 0 || (x == 64 && pp >= 0))
+      for (int k = 0; k < min(128, d.A - h0); ++k) f = cadd(f, term[x >> 6][k]);
+    __syncthreads();
+  }
+  if (x == 0) d.fdiag[p] = f;
+  if (x == 64) d.fpart[p] = f;
 }
 
 // E0 = sum_i t_ii + 1/2 sum_ij <ij||ij> (ccm_main.f90:1661-1684).  One block.
@@ -1805,6 +1854,20 @@ __global__ void k_to_f32(const double2 *src, float2 *dst, int64_t n) {
 // launch wrappers (host side)
 // ---------------------------------------------------------------------------
 template <class V>
+static void fill_fock(const SolveDesc &d, const V &vas, hipStream_t st) {
+  hipLaunchKernelGGL(k_fock<V>, dim3(d.nsp), dim3(128), 0, st, d, vas);
+  hipLaunchKernelGGL(k_e0<V>, dim3(1), dim3(256), 0, st, d, vas);
+}
+
+template <int WHAT>
+static void fill_chiral(const SolveDesc &d, const ChiralDev &c, const PairGroups &rows, const PairGroups &cols,
+                        const int *ncol, const int64_t *off, double2 *out, int nch, hipStream_t st) {
+  const int64_t n = ((int64_t)rows.max * cols.max + 255) / 256;
+  hipLaunchKernelGGL(k_fill_chiral<WHAT>, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(n, 4096)), nch),
+                     dim3(256), 0, st, d, c, rows, cols, ncol, off, out);
+}
+
+template <class V>
 static void fill_blocks(const SolveDesc &d, const V &vas, int nch, int nphc, int max_npp, int max_nhh, int max_nhp,
                         hipStream_t st) {
   auto gx = [](int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 8192)); };
@@ -1812,8 +1875,7 @@ static void fill_blocks(const SolveDesc &d, const V &vas, int nch, int nphc, int
   hipLaunchKernelGGL(k_fill_vhhpp<V>, dim3(gx((int64_t)max_npp * max_nhh), nch), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_fill_vhhhh<V>, dim3(gx((int64_t)max_nhh * max_nhh), nch), dim3(256), 0, st, d, vas);
   hipLaunchKernelGGL(k_fill_w0<V>, dim3(gx((int64_t)max_nhp * max_nhp), nphc, 2), dim3(256), 0, st, d, vas);
-  hipLaunchKernelGGL(k_fock<V>, dim3((d.nsp + 255) / 256), dim3(256), 0, st, d, vas);
-  hipLaunchKernelGGL(k_e0<V>, dim3(1), dim3(256), 0, st, d, vas);
+  fill_fock(d, vas, st);
 }
 
 void launch_fill_blocks(const SolveDesc &d, double volume, int nch, int nphc, int max_npp,
@@ -1823,22 +1885,23 @@ void launch_fill_blocks(const SolveDesc &d, double volume, int nch, int nphc, in
   fill_blocks(d, v, nch, nphc, max_npp, max_nhh, max_nhp, st);
 }
 
-void launch_fill_blocks_chiral(const SolveDesc &d, const ChiralDev &c, int nch, int nphc, int max_npp,
-                               int max_nhh, int max_nhp, hipStream_t st) {
+void launch_fill_blocks_chiral(const SolveDesc &d, const ChiralDev &c, int nch, int nphc, hipStream_t st) {
   ChiralV v;
   v.c = c;
   v.nx = d.nx; v.ny = d.ny; v.nz = d.nz; v.sz = d.sz; v.tz = d.tz;
-  fill_blocks(d, v, nch, nphc, max_npp, max_nhh, max_nhp, st);
+  fill_chiral<kFillPairs>(d, c, d.gpp, d.gpp, d.npp, d.off_vpp, d.Vpppp, nch, st);
+  fill_chiral<kFillPairs>(d, c, d.ghh, d.gpp, d.npp, d.off_t, d.Vhhpp, nch, st);
+  fill_chiral<kFillPairs>(d, c, d.ghh, d.ghh, d.nhh, d.off_vhh, d.Vhhhh, nch, st);
+  fill_chiral<kFillW0>(d, c, d.ghp, d.ghp, d.nhp, d.off_i4, d.W0, nphc, st);
+  fill_chiral<kFillW1>(d, c, d.gph, d.gph, d.nph, d.off_w1, d.W1, nphc, st);
+  fill_fock(d, v, st);
 }
 
 // V_pppp blocks only (the union blocks of a shared pp ladder)
 void launch_fill_vpppp(const SolveDesc &d, double volume, const ChiralDev *c, int nch, int max_npp, hipStream_t st) {
   const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(((int64_t)max_npp * max_npp + 255) / 256, 8192));
   if (c) {
-    ChiralV v;
-    v.c = *c;
-    v.nx = d.nx; v.ny = d.ny; v.nz = d.nz; v.sz = d.sz; v.tz = d.tz;
-    hipLaunchKernelGGL(k_fill_vpppp<ChiralV>, dim3(gx, nch), dim3(256), 0, st, d, v);
+    fill_chiral<kFillPairs>(d, *c, d.gpp, d.gpp, d.npp, d.off_vpp, d.Vpppp, nch, st);
   } else {
     MinnesotaV v;
     v.o.kx = d.kx; v.o.ky = d.ky; v.o.kz = d.kz; v.o.sz = d.sz; v.o.tz = d.tz; v.o.volume = volume;

@@ -290,3 +290,56 @@ def test_bf16x3_fused_ring_equals_list_kernels(ccnm, monkeypatch, A, matter, nma
     r, ref = out
     assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0
     assert np.abs(r - ref).max() <= 4e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist,order", [
+    (3, "pnm", 1, (0.0, 0.0, 0.0), "NNLO"), (15, "pnm", 1, (0.3, 0.6, 0.9), "NNLO"), (14, "pnm", 1, (0.0, 0.0, 0.0), "LO"),
+    (6, "snm", 1, (0.0, 0.0, 0.0), "NNLO"), (28, "snm", 1, (0.2, 0.4, 0.6), "LO"), (4, "snm", 1, (0.5, 1.0, 1.5), "NNLO")])
+def test_chiral_blocks_over_pair_groups_equal_elements(ccnm, monkeypatch, A, matter, nmax, twist, order):
+    """The V fill takes the sixteen spin combinations of two pair groups at once; single
+    elements come from the general evaluation.  Groups of one to four pairs, with and
+    without isospin exchange.  Both round the same few dozen operations: 64 * 2^-53 of
+    the largest element, 1e-14."""
+    s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax, twist=twist)
+    s.set_chiral(getattr(ccnm, order), 450.0)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    o, nt = s.orbitals(), s.dims["t2_unique"]
+    a, b, i, j = s.t2_labels().T
+    want = np.conj(s.vnn_elements(i, j, a, b))
+    got = s.debug_fetch("R0", nt)
+    scale = np.abs(want).max()
+    assert np.abs(got - want).max() <= 1e-14 * scale
+    # W0((i,a),(j,b)) = -<ib||ja>, channels by (tz, n) of j - b, hp pairs by j and then b
+    key = {}
+    for h in range(A):
+        for p in range(A, s.dims["nsp"]):
+            key.setdefault((o["tz"][h] - o["tz"][p], *(o[x][h] - o[x][p] for x in ("nx", "ny", "nz"))), []).append((h, p))
+    want = []
+    for k in sorted(key):
+        if tuple(-x for x in k) not in key:
+            continue
+        hp = np.array(key[k], np.int32)
+        r, c = np.meshgrid(np.arange(len(hp)), np.arange(len(hp)), indexing="ij")
+        r, c = r.ravel(), c.ravel()
+        want.append(-s.vnn_elements(hp[r, 0], hp[c, 1], hp[c, 0], hp[r, 1]))
+    want = np.concatenate(want)
+    got = s.debug_fetch("W0", len(want))
+    assert np.abs(got - want).max() <= 1e-14 * np.abs(want).max()
+    # V_pppp through the pp ladder of random amplitudes
+    rng = np.random.default_rng(A)
+    t = rng.standard_normal(nt) + 1j * rng.standard_normal(nt)
+    s.set_t2_unique(t)
+    monkeypatch.setenv("CCGPU_TERMS", "2")
+    s.t2_intermediate()
+    R = s.debug_fetch("R", nt) - s.debug_fetch("R0", nt)
+    at = {}
+    for u in range(nt):
+        at.setdefault((i[u], j[u]), []).append(u)
+    err = top = 0.0
+    for us in at.values():
+        us = np.array(us)
+        r, c = np.meshgrid(us, us, indexing="ij")
+        v = s.vnn_elements(a[r].ravel(), b[r].ravel(), a[c].ravel(), b[c].ravel()).reshape(r.shape)
+        err, top = max(err, np.abs(R[us] - v @ t[us]).max()), max(top, (np.abs(v) @ np.abs(t[us])).max())
+    assert err <= 1e-14 * top
+    s.close()
