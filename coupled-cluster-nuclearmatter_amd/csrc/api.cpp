@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <complex>
@@ -18,6 +19,7 @@
 #include <tuple>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -2218,6 +2220,91 @@ void ensure_f32(Solve &S, int handle) {
   drop_single(handle);
 }
 
+// Device to pageable host memory, through two pinned halves: the copy engine fills one
+// while threads empty the other.  The runtime's own pageable copy empties its staging
+// buffer with one thread, which also takes the page faults of a fresh array: 32 MB took
+// 2.25 ms, 1.26 this, 11.5 MB 742 us and 399.  One stage for the process, used
+// under the API lock and given back with the last handle.
+struct HostStage {
+  static constexpr size_t kHalf = (size_t)4 << 20, kPiece = (size_t)256 << 10;
+  char *p = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  void release() {
+    if (p) (void)hipHostFree(p);
+    for (hipEvent_t &e : ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    p = nullptr;
+  }
+  void make() {
+    if (p) return;
+    for (hipEvent_t &e : ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    HIPCHK(hipHostMalloc((void **)&p, 2 * kHalf, hipHostMallocDefault));
+  }
+} g_stage;
+
+void copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
+  constexpr size_t half = HostStage::kHalf, piece = HostStage::kPiece;
+  if (bytes < ((size_t)2 << 20)) {   // 1.5 MB: 103 us against 85, which the threads' start eats in a busy process
+    HIPCHK(hipStreamSynchronize(st));
+    HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    return;
+  }
+  g_stage.make();
+  const size_t npiece = (bytes + piece - 1) / piece, nhalf = (bytes + half - 1) / half;
+  std::atomic<size_t> next{0}, ready{0}, done{0};
+  std::atomic<bool> stop{false};
+  // empties one piece if one is there; false once all are taken
+  auto empty_one = [&](size_t k) {
+    const size_t o = k * piece;
+    memcpy((char *)dst + o, g_stage.p + (o / half % 2) * half + o % half, std::min(piece, bytes - o));
+    done.fetch_add(1, std::memory_order_release);
+  };
+  auto worker = [&] {
+    for (;;) {
+      const size_t k = next.fetch_add(1);
+      if (k >= npiece) return;
+      while (ready.load(std::memory_order_acquire) <= k) {
+        if (stop.load()) return;
+        std::this_thread::yield();
+      }
+      empty_one(k);
+    }
+  };
+  struct Threads {
+    std::vector<std::thread> t;
+    std::atomic<bool> &stop;
+    ~Threads() {
+      stop = true;
+      for (std::thread &x : t) x.join();
+    }
+  } threads{{}, stop};
+  auto fill = [&](size_t h) {
+    HIPCHK(hipMemcpyAsync(g_stage.p + h % 2 * half, (const char *)src + h * half, std::min(half, bytes - h * half),
+                          hipMemcpyDeviceToHost, st));
+    HIPCHK(hipEventRecord(g_stage.ev[h % 2], st));
+  };
+  fill(0);
+  const size_t nt = std::min<size_t>({npiece / 2, 7, std::max(2u, std::thread::hardware_concurrency()) / 2});
+  try {
+    for (size_t x = 0; x < nt; ++x) threads.t.emplace_back(worker);
+  } catch (const std::system_error &) {   // fewer threads will do, and none too
+  }
+  for (size_t h = 0; h < nhalf; ++h) {
+    if (h + 1 < nhalf) {
+      // the other half is free once the pieces of h - 1 are out
+      while (done.load(std::memory_order_acquire) < h * (half / piece)) std::this_thread::yield();
+      fill(h + 1);
+    }
+    HIPCHK(hipEventSynchronize(g_stage.ev[h % 2]));
+    ready.store(std::min(npiece, (h + 1) * (half / piece)), std::memory_order_release);
+    if (threads.t.empty())
+      for (size_t k = h * (half / piece); k < ready.load(); ++k) empty_one(k);
+  }
+  while (done.load(std::memory_order_acquire) < npiece) std::this_thread::yield();
+}
+
 template <typename F>
 int guarded(F &&f) {
   std::lock_guard<std::mutex> lk(g_mu);
@@ -2439,6 +2526,7 @@ int ccgpu_destroy(int handle) {
     get(handle);
     drop_single(handle);
     g_solves.erase(handle);
+    if (g_solves.empty()) g_stage.release();
   });
 }
 
@@ -2957,7 +3045,7 @@ int ccgpu_set_t2(int handle, int n, const int *a, const int *b, const int *i, co
 int ccgpu_get_t2_unique(int handle, double *t) {
   return guarded([&] {
     Solve &S = get(handle);
-    HIPCHK(hipMemcpy(t, S.desc.T, S.plan.nT * sizeof(double2), hipMemcpyDeviceToHost));
+    copy_to_host(t, S.desc.T, S.plan.nT * sizeof(double2), S.stream);
   });
 }
 

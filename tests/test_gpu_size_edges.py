@@ -343,3 +343,18 @@ def test_chiral_blocks_over_pair_groups_equal_elements(ccnm, monkeypatch, A, mat
         err, top = max(err, np.abs(R[us] - v @ t[us]).max()), max(top, (np.abs(v) @ np.abs(t[us])).max())
     assert err <= 1e-14 * top
     s.close()
+
+
+@pytest.mark.parametrize("A,matter,nmax", [(2, "pnm", 1), (14, "pnm", 1), (28, "snm", 2), (38, "pnm", 3), (66, "pnm", 3)])
+def test_amplitudes_come_back_whole(ccnm, A, matter, nmax):
+    """The copy to host memory goes through pinned halves of 4 MB in pieces of 256 KB: less
+    than a piece, some pieces, two and three halves with a ragged end."""
+    s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax)
+    n = s.dims["t2_unique"]
+    rng = np.random.default_rng(n)
+    for _ in range(3):
+        t = rng.standard_normal(2 * n).view(np.complex128)
+        s.set_t2_unique(t)
+        assert np.array_equal(s.t2_unique(), t)
+        assert np.array_equal(s.t2_unique(), s.debug_fetch("T", n))
+    s.close()
