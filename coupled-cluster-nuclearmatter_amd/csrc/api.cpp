@@ -59,6 +59,9 @@ void launch_diis_axpy(const SolveDesc *dd, int nsolve, int64_t maxT, const int *
                       int nvec, hipStream_t st);
 void launch_gemm_shape(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const SolveDesc *dd,
                        const int *gsolve, int kind, int mb, int nb, int lb, hipStream_t st);
+void launch_small_t(const GemmGroup *groups, const GemmTile *pp, int npp, const int *gsolve, const ZTile *x, int nx,
+                    const SolveDesc *dd, int nsolve, int64_t maxrows, hipStream_t st);
+void launch_small_x(const ZTile *hh, int nhh, const SolveDesc *dd, int nsolve, int maxA, int maxnp, hipStream_t st);
 int ring64_class(int nph, int nhp);
 int ring64_columns(int nph, int nhp);
 int ringbf_columns(int nph, int nhp);
@@ -1577,9 +1580,10 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   // small batches do not win back: an iteration of SNM A=28 |n_i|<=2 (92 k
   // amplitudes) takes 145 us on three streams and 124 on one, SNM A=76 |n_i|<=2
   // (411 k) 206 on either, PNM A=66 |n_i|<=3 (721 k) 302 and 326.
+  constexpr int64_t kForkAmplitudes = 400000;
   int64_t amplitudes = 0;
   for (const Solve *S : B.solves) amplitudes += S->plan.nT;
-  const bool fork6 = !timing && amplitudes >= 400000 && fork_enabled();
+  const bool fork6 = !timing && amplitudes >= kForkAmplitudes && fork_enabled();
   const bool fork = fork6 && (terms & 8);
   hipStream_t sr = fork ? B.stream2 : st;
   hipStream_t s6 = fork6 ? B.stream3 : st;
@@ -1664,10 +1668,22 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
       run_gemm(B.g_pp, B, pp_prec, false, q, true);
     }
   };
-  pp_ladder(st);
-  x_chain(s6);
-  i6(sr);
-  ring(sr);
+  // one stream, everything in FP64 and a ladder of one launch: merged launches
+  const GemmList &P = B.g_pp;
+  const bool one = P.ready && P.shape[0].mb == 1 && P.shape[0].nb == 1 && P.shape[0].lb == 3 && P.split.empty() &&
+                   (int)P.tiles[0].size() == P.ntiles();
+  if (!timing && amplitudes < kForkAmplitudes && terms == 15 && !shared && pp_prec == CCGPU_PREC_FP64 && t64(0) &&
+      t64(2) && one) {
+    launch_small_t(P.d_groups, P.d_tiles[0], (int)P.tiles[0].size(), P.d_gsolve, B.f64.x, B.f64.nx, B.d_descs, n,
+                   B.maxRows, st);
+    ring(st);
+    launch_small_x(B.f64.hh, B.f64.nhh, B.d_descs, n, B.maxA, B.maxNp, st);
+  } else {
+    pp_ladder(st);
+    x_chain(s6);
+    i6(sr);
+    ring(sr);
+  }
   if (fork6) HIPCHK(hipEventRecord(B.ev_hh, s6));
   if (fork) {
     HIPCHK(hipEventRecord(B.ev_join, sr));

@@ -11,6 +11,7 @@
 #include "bf3.h"
 #include "device.h"
 #include "interaction.h"
+#include "tiles64.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -541,11 +542,9 @@ __global__ void k_reduce_final(const SolveDesc *descs, int nparts, int stride, i
 // dh(i) = I7(i,i) is the dynamic hole denominator (ccm_t2_eqn.f90:81-84).
 __device__ __forceinline__ double2 wave_sum(double2 v);
 
-__global__ __launch_bounds__(256) void k_i7(const SolveDesc *descs) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
+__device__ __forceinline__ void i7_block(const SolveDesc &d, int block) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t = block * 4 + (threadIdx.x >> 6);
   if (t >= 2 * d.A) return;
   const int i = t >> 1, which = t & 1;
   const int k = which ? d.partner[i] : i;
@@ -569,6 +568,11 @@ __global__ __launch_bounds__(256) void k_i7(const SolveDesc *descs) {
   }
 }
 
+__global__ __launch_bounds__(256) void k_i7(const SolveDesc *descs) {
+  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
+  if (d.active) i7_block(d, blockIdx.x);
+}
+
 // I6(a,c) = f_ac - 1/2 sum_d sum_kl <kl||dc> t(da,kl) for c in {a, partner(a)}
 // (ccm_t2_eqn.f90:1399-1441); dp(a) = I6(a,a) (ccm_t2_eqn.f90:86-89).
 // Pass 1, one unique pp row (x<y) per 16 lanes: with V(kl,dc) = conj(R0(dc,kl))
@@ -589,12 +593,9 @@ __device__ __forceinline__ double2 cdotc(const double2 *v, const double2 *t, int
   return make_double2(re, im);
 }
 
-__global__ __launch_bounds__(256) void k_i6_rows(const SolveDesc *descs) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
+__device__ __forceinline__ void i6_rows_block(const SolveDesc &d, int block, int nblocks) {
   const int l16 = threadIdx.x & 15;
-  for (int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4; r < d.nrows;
-       r += ((int64_t)gridDim.x * blockDim.x) >> 4) {
+  for (int64_t r = ((int64_t)block * 256 + threadIdx.x) >> 4; r < d.nrows; r += (int64_t)nblocks * 16) {
     const int c = d.row_ch[r], nh = d.nhh[c];
     const int64_t base = d.off_t[c], loc = r - d.off_pp[c];
     const double2 *tr = d.T + base + loc * nh;
@@ -611,6 +612,11 @@ __global__ __launch_bounds__(256) void k_i6_rows(const SolveDesc *descs) {
   }
 }
 
+__global__ __launch_bounds__(256) void k_i6_rows(const SolveDesc *descs) {
+  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
+  if (d.active) i6_rows_block(d, blockIdx.x, gridDim.x);
+}
+
 // one wavefront per target; lanes take every 64th list entry, then a fixed
 // butterfly: deterministic for a given list
 __device__ __forceinline__ double2 wave_sum(double2 v) {
@@ -621,11 +627,9 @@ __device__ __forceinline__ double2 wave_sum(double2 v) {
   return v;
 }
 
-__global__ __launch_bounds__(256) void k_i6_reduce(const SolveDesc *descs) {
-  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
-  if (!d.active) return;
+__device__ __forceinline__ void i6_reduce_block(const SolveDesc &d, int block) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t = block * 4 + (threadIdx.x >> 6);
   if (t >= 2 * d.np) return;
   const int p = t >> 1, which = t & 1, a = d.A + p;
   if (which && d.partner[a] < d.A) {
@@ -641,6 +645,11 @@ __global__ __launch_bounds__(256) void k_i6_reduce(const SolveDesc *descs) {
     acc = cadd(acc, which ? d.fpart[a] : d.fdiag[a]);
     if (which) d.I6off[p] = acc; else d.dp[p] = acc;
   }
+}
+
+__global__ __launch_bounds__(256) void k_i6_reduce(const SolveDesc *descs) {
+  const SolveDesc d = descs[blockIdx.y];   // a copy: stores cannot change it, so no reloads
+  if (d.active) i6_reduce_block(d, blockIdx.x);
 }
 
 // I9 = Vhhhh + 1/2 Vhhpp T (ccm_t2_eqn.f90:431-464, 558-560): X[0,n) holds
@@ -2154,26 +2163,14 @@ struct PplCfg {
 };
 
 template <int NB, int VK>
-__global__ __launch_bounds__(256, 2) void k_ppl(const GemmGroup *__restrict__ groups,
-                                              const GemmTile *__restrict__ tiles,
-                                              const SolveDesc *__restrict__ descs,
-                                              const int *__restrict__ gsolve) {
+__device__ __forceinline__ void ppl_tile(const GemmGroup &g, const GemmTile &tl, char *A0, char *A1, char *A2, char *A3,
+                                         char *B0, char *B1, char *B2, char *B3) {
   typedef PplCfg<NB, VK> C;
   constexpr bool VF32 = C::VF32, MF32 = VK >= 2, BF3 = VK >= 3, TSPL = VK == 4;
   constexpr int KC = C::KC, NT = C::NT, S = C::S, IPW = C::IPW, BIW = C::BIW;
   static_assert(C::BBYTES % 4096 == 0, "T rows of a chunk in whole instructions per wave");
   typedef typename std::conditional<MF32, float, double>::type real;
   typedef typename std::conditional<MF32, f4, d4>::type acc4;
-  // one object per stage: the compiler's wait insertion then tells the
-  // stages apart and leaves the waits of the pipeline to the code below
-  __shared__ __attribute__((aligned(16))) char A0[16384], A1[16384], A2[S >= 3 ? 16384 : 16],
-      A3[S >= 4 ? 16384 : 16];
-  __shared__ __attribute__((aligned(16))) char B0[C::BBYTES], B1[C::BBYTES], B2[S >= 3 ? C::BBYTES : 16],
-      B3[S >= 4 ? C::BBYTES : 16];
-
-  const GemmTile tl = tiles[blockIdx.x];
-  if (descs && !descs[gsolve[tl.g]].active) return;
-  const GemmGroup g = groups[tl.g];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int K = g.K, nchunk = (K + KC - 1) / KC;
@@ -2379,6 +2376,83 @@ __global__ __launch_bounds__(256, 2) void k_ppl(const GemmGroup *__restrict__ gr
         g.C[(int64_t)m * g.ldc + n] = v;
       }
     }
+}
+
+template <int NB, int VK>
+__global__ __launch_bounds__(256, 2) void k_ppl(const GemmGroup *__restrict__ groups,
+                                              const GemmTile *__restrict__ tiles,
+                                              const SolveDesc *__restrict__ descs,
+                                              const int *__restrict__ gsolve) {
+  typedef PplCfg<NB, VK> C;
+  constexpr int S = C::S;
+  // one object per stage: the compiler's wait insertion then tells the
+  // stages apart and leaves the waits of the pipeline to ppl_tile
+  __shared__ __attribute__((aligned(16))) char A0[16384], A1[16384], A2[S >= 3 ? 16384 : 16],
+      A3[S >= 4 ? 16384 : 16];
+  __shared__ __attribute__((aligned(16))) char B0[C::BBYTES], B1[C::BBYTES], B2[S >= 3 ? C::BBYTES : 16],
+      B3[S >= 4 ? C::BBYTES : 16];
+  const GemmTile tl = tiles[blockIdx.x];
+  if (descs && !descs[gsolve[tl.g]].active) return;
+  const GemmGroup g = groups[tl.g];
+  ppl_tile<NB, VK>(g, tl, A0, A1, A2, A3, B0, B1, B2, B3);
+}
+
+// The FP64 residual of a small batch (one stream) in merged launches: a launch and the
+// gap before it cost as much as these kernels run.  First what reads T alone: the pp
+// ladder, X with I9, and the rows of I6; then what reads X and the rows: the hh ladder,
+// I7 and I6.  Same tiles, same bits.  A solve of SNM A=28 |n_i|<=2 3.03 to 2.37 ms (24
+// iterations), four steps of PNM A=14 |n_i|<=1 412 to 320 us.
+__global__ __launch_bounds__(256, 2) void k_small_t(const GemmGroup *__restrict__ groups,
+                                                  const GemmTile *__restrict__ pp, int npp,
+                                                  const int *__restrict__ gsolve, const ZTile *__restrict__ x, int nx,
+                                                  int rows, const SolveDesc *__restrict__ descs) {
+  typedef PplCfg<1, 0> C;
+  static_assert(C::S == 4 && C::BBYTES <= 16384, "stages of the ladder hold the sums of an X tile");
+  __shared__ __attribute__((aligned(16))) char A0[16384], A1[16384], A2[16384], A3[16384];
+  __shared__ __attribute__((aligned(16))) char B0[C::BBYTES], B1[C::BBYTES], B2[C::BBYTES], B3[C::BBYTES];
+  const int b = blockIdx.x;
+  if (b < npp) {
+    const GemmTile tl = pp[b];
+    if (!descs[gsolve[tl.g]].active) return;
+    const GemmGroup g = groups[tl.g];
+    ppl_tile<1, 0>(g, tl, A0, A1, A2, A3, B0, B1, B2, B3);
+  } else if (b < npp + nx) {
+    const ZTile t = x[b - npp];
+    if (!descs[t.solve].active) return;
+    if (t.nb == 1) x64_tile<1>(t, (double2 *)A0, (double2 *)A1);
+    else x64_tile<2>(t, (double2 *)A0, (double2 *)A1);
+  } else {
+    const SolveDesc d = descs[(b - npp - nx) / rows];
+    if (d.active) i6_rows_block(d, (b - npp - nx) % rows, rows);
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void k_small_x(const ZTile *__restrict__ hh, int nhh, int b7, int b6,
+                                                  const SolveDesc *__restrict__ descs) {
+  int b = blockIdx.x;
+  if (b < nhh) {
+    const ZTile t = hh[b];
+    if (!descs[t.solve].active) return;
+    if (t.nb == 1) hh64_tile<1>(t);
+    else hh64_tile<2>(t);
+    return;
+  }
+  b -= nhh;
+  const SolveDesc d = descs[b / (b7 + b6)];
+  if (!d.active) return;
+  b %= b7 + b6;
+  if (b < b7) i7_block(d, b);
+  else i6_reduce_block(d, b - b7);
+}
+void launch_small_t(const GemmGroup *groups, const GemmTile *pp, int npp, const int *gsolve, const ZTile *x, int nx,
+                    const SolveDesc *dd, int nsolve, int64_t maxrows, hipStream_t st) {
+  const int rows = (int)std::max<int64_t>(1, std::min<int64_t>((maxrows * 16 + 255) / 256, 4096));
+  hipLaunchKernelGGL(k_small_t, dim3(npp + nx + nsolve * rows), dim3(256), 0, st, groups, pp, npp, gsolve, x, nx, rows,
+                     dd);
+}
+void launch_small_x(const ZTile *hh, int nhh, const SolveDesc *dd, int nsolve, int maxA, int maxnp, hipStream_t st) {
+  const int b7 = (2 * maxA + 3) / 4, b6 = (2 * maxnp + 3) / 4;
+  hipLaunchKernelGGL(k_small_x, dim3(nhh + nsolve * (b7 + b6)), dim3(256), 0, st, hh, nhh, b7, b6, dd);
 }
 
 // The same pipeline with eight waves and one workgroup per CU: a tile is 64
