@@ -49,7 +49,7 @@ void launch_i6(const SolveDesc *dd, int nsolve, int maxnp, int64_t maxrows, hipS
 void launch_i9(const SolveDesc *dd, int nsolve, int64_t maxvhh, hipStream_t st);
 void launch_t_begin(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64_t maxT, int ring, bool form, bool split,
                     const uint32_t *const *maps, double2 *Tu, hipStream_t st);
-void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, bool f32, int mode, int terms,
+void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64_t maxT, bool f32, int mode, int terms,
                   const uint32_t *const *maps, const double2 *Ru, double2 *out, hipStream_t st);
 void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const IterCtrl *ctrl, hipStream_t st);
 void launch_gram(const SolveDesc *dd, int nsolve, const int *slots, int nstep, double2 *out, hipStream_t st);
@@ -1692,7 +1692,7 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   if (fork6) HIPCHK(hipStreamWaitEvent(st, B.ev_hh, 0));
   {
     Timer t(timing, st, mode == 0 ? "residual_sum" : mode == 1 ? "residual_sum_update" : "residual_sum_anderson");
-    launch_t_end(B.d_descs, B.d_ctrl, n, ring32, mode, terms, shared ? B.share.d_maps : nullptr, B.share.Ru, B.results, st);
+    launch_t_end(B.d_descs, B.d_ctrl, n, B.maxT, ring32, mode, terms, shared ? B.share.d_maps : nullptr, B.share.Ru, B.results, st);
   }
 }
 

@@ -2032,14 +2032,17 @@ void launch_t_begin(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64
 }
 // mode 0 residual only, 1 reference update (energies into results 0), 2 Anderson
 // update (17 values into results 24 .. 40)
-void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, bool f32, int mode, int terms,
+// (up to 524288 amplitudes block b takes 256 b .., and the blocks past the last one,
+// whose partials are zero, are left out: the same sums)
+void launch_t_end(const SolveDesc *dd, const IterCtrl *ctrl, int nsolve, int64_t maxT, bool f32, int mode, int terms,
                   const uint32_t *const *maps, const double2 *Ru, double2 *out, hipStream_t st) {
+  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>((maxT + 255) / 256, kEndBlocks));
   auto k = mode == 2 ? (f32 ? k_t_end<true, 2> : k_t_end<false, 2>)
          : mode == 1 ? (f32 ? k_t_end<true, 1> : k_t_end<false, 1>)
                      : (f32 ? k_t_end<true, 0> : k_t_end<false, 0>);
-  hipLaunchKernelGGL(k, dim3(kEndBlocks, nsolve), dim3(256), 0, st, dd, ctrl, terms, maps, Ru);
-  if (mode == 1) hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, kEndBlocks, 1, 0, out);
-  if (mode == 2) hipLaunchKernelGGL(k_reduce_final, dim3(17, nsolve), dim3(256), 0, st, dd, kEndBlocks, 36, 24, out);
+  hipLaunchKernelGGL(k, dim3(nb, nsolve), dim3(256), 0, st, dd, ctrl, terms, maps, Ru);
+  if (mode == 1) hipLaunchKernelGGL(k_reduce_final, dim3(1, nsolve), dim3(256), 0, st, dd, nb, 1, 0, out);
+  if (mode == 2) hipLaunchKernelGGL(k_reduce_final, dim3(17, nsolve), dim3(256), 0, st, dd, nb, 36, 24, out);
 }
 void launch_update(const SolveDesc *dd, int nsolve, int64_t maxT, const IterCtrl *ctrl, hipStream_t st) {
   hipLaunchKernelGGL(k_update, egrid(maxT, nsolve), dim3(256), 0, st, dd, ctrl);
