@@ -306,7 +306,9 @@ int ccgpu_batch_solve(int n, const int *handles, const ccgpu_solve_opts *opts,
 
 /* Copy one internal device array (what: 0 R, 1 dh, 2 I7off, 3 dp, 4 I6off,
  * 5 X|I9, 6 Rt, 7 Tt, 8 I4, 9 T, 10 R0, 11 fdiag, 12 fpart, 13 W0, 14 Vt) of
- * n complex elements to the host; for tests and diagnostics. */
+ * n complex elements to the host; for tests and diagnostics.  The ring blocks
+ * (6, 7, 8, 13, 14) come channel by channel, hp pairs by hole and then particle;
+ * 6 and 8 are formed on the host from the last 7. */
 int ccgpu_debug_fetch(int handle, int what, double *out, long long n);
 
 /* Per-kernel timings (ms, averaged over the recorded launches) of the last
