@@ -2054,7 +2054,10 @@ void run_batch(Batch &B, const ccgpu_solve_opts &op, std::vector<ccgpu_solve_res
     if (aa) anderson_columns(B, op.subspace, beta);
     else next_column(B, nstep, op.subspace);
     if (ccdt1) {
+      // the triples read T on each solve's own stream, which does not wait for the
+      // batch's, and the next upload_ctrl takes form_t's staging buffer
       form_t();
+      HIPCHK(hipStreamSynchronize(B.stream));
       for (int s = 0; s < n; ++s) {
         B.ctrl[s].np = 0;
         if (!B.h_descs[s].active) continue;

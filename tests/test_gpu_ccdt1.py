@@ -222,3 +222,28 @@ def test_three_body_force_set_after_generation_is_an_error(ccnm):
         s.setup_t3()
     with pytest.raises(RuntimeError, match="after the interaction was generated"):
         s.pert_triples2()
+
+
+def test_ccdt1_batch_whose_first_member_converges_first(ccnm):
+    """A batched CCDT-1 solve (three twists, 13, 20 and 14 iterations) against its
+    members alone: once the first is done, the triples of the others read T on
+    streams of their own, after nothing but the batch's opening pass.  The sums
+    of a member are the same in a batch, so the energies agree to rounding
+    (2^-53 of some 1e3 MeV), which the extrapolation can amplify to 1e-9; the
+    energies of two iterates of a solve differ by the tolerance, 1e-6, or more."""
+    def solver(k):
+        s = native_3nf(ccnm, 14, "pnm", 0.16, 1, tuple(golden(f"pnm14_n1_nnlo_tabc2_{k}")["twist"]), 2)
+        s.setup_t_amplitudes()
+        return s
+    opts = dict(subspace=6, diis_step=6, tol=TOL, maxit=100, ccdt1=1)
+    alone = []
+    for k in (3, 1, 2):
+        s = solver(k)
+        r = s.ccd_iter(**opts)
+        alone.append((r, s.solve_energies()))
+    assert alone[0][0]["iterations"] < max(r["iterations"] for r, _ in alone) - 1
+    batch = [solver(k) for k in (3, 1, 2)]
+    for (r, e), s, b in zip(alone, batch, ccnm.batch_solve(batch, **opts)):
+        assert b["converged"] and b["iterations"] == r["iterations"], (b["iterations"], r["iterations"])
+        got = s.solve_energies()
+        assert len(got) == len(e) and np.max(np.abs(got - e)) < 1e-8, np.abs(got - e)
