@@ -3362,17 +3362,19 @@ double2 triples_sum(Solve &S, int mode) {
     throw Error("CCDT-1 and the three-body (T) need the element tables: raise CCGPU_T3_TABLE_GB");
   const Plan &P = S.plan;
   int nb = (int)std::min<int64_t>(8192, std::max<int64_t>(1, S.t3.npairs));
-  // CCGPU_T3_KERNEL=1, 3 (studies and tests): (T) element by element
+  // CCGPU_T3_KERNEL (studies and tests): (T) element by element, 1 and 3 on tables, 0 in
+  // place, which has the two-nucleon elements alone and no W3
   const int variant = getenv("CCGPU_T3_KERNEL") ? atoi(getenv("CCGPU_T3_KERNEL")) : 2;
+  const bool in_place = mode == 0 && (!S.t3.gE || (variant == 0 && !S.t3.tnf));
   if (mode == 0 && (variant == 1 || variant == 3) && legacy_tables(S)) {
     if (variant == 1) launch_t3_td(S.desc, S.t3, S.t3_td, S.stream);
     launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream,
                    variant, S.t3_td, P.max_nhh);
-  } else if (mode == 2 || (S.t3.gE && variant != 0)) {
-    launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
-  } else {
+  } else if (in_place) {
     launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream, 0,
                    nullptr, P.max_nhh);
+  } else {
+    launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
   }
   check_launch();
   double2 r;

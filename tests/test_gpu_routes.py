@@ -1,0 +1,32 @@
+"""Calls that can take one of several kernels, tables or copies: each route
+gives what the others give, and what a route needs is made when it is taken."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_ccdt1 import native_3nf
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("A,matter,nmax,twist", [(4, "snm", 1, (0.0, 0.0, 0.0)), (14, "pnm", 1, (0.4, 0.9, 1.3))])
+def test_in_place_triples_switch_keeps_the_three_body_force(ccnm, monkeypatch, A, matter, nmax, twist):
+    """CCGPU_T3_KERNEL=0 asks for the kernel without tables, which evaluates
+    |W|^2 with the two-nucleon elements alone: (T) with the normal-ordered
+    three-nucleon force, (T) with W3 and the CCDT-1 energy are the same with
+    the switch and without it (the same terms, 1e-12 for their order)."""
+    for approx in (2, 3):
+        s = native_3nf(ccnm, A, matter, 0.16, nmax, twist, approx)
+        s.setup_t_amplitudes()
+        got = []
+        for kernel in (None, "0"):
+            if kernel is None:
+                monkeypatch.delenv("CCGPU_T3_KERNEL", raising=False)
+            else:
+                monkeypatch.setenv("CCGPU_T3_KERNEL", kernel)
+            v = [s.pert_triples2(), *s.triples_parts(), s.setup_t3()]
+            s.t3_intermediate()
+            got.append(np.array(v + [s.t3_energy()]))
+        assert np.all(got[0][[0, 1, 3, 4]] != 0)
+        assert np.max(np.abs(got[1] - got[0])) <= 1e-12 * np.max(np.abs(got[0])), got
