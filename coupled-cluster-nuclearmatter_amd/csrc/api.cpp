@@ -124,10 +124,16 @@ std::string fmt(const char *f, ...) {
   return buf;
 }
 
-#define HIPCHK(x)                                                                         \
-  do {                                                                                    \
-    hipError_t e_ = (x);                                                                  \
-    if (e_ != hipSuccess) throw Error(fmt("%s failed: %s", #x, hipGetErrorString(e_))); \
+// A call that fails.  The runtime keeps its error for the next hipGetLastError, where
+// check_launch of a later, unrelated call would find it: taken back here.
+[[noreturn]] void fail_hip(const std::string &what, hipError_t e) {
+  (void)hipGetLastError();
+  throw Error(what + " failed: " + hipGetErrorString(e));
+}
+#define HIPCHK(x)                              \
+  do {                                         \
+    hipError_t e_ = (x);                       \
+    if (e_ != hipSuccess) fail_hip(#x, e_);    \
   } while (0)
 
 template <typename T>
@@ -135,8 +141,7 @@ T *dalloc(size_t n, std::vector<void *> &owned) {
   void *p = nullptr;
   if (n == 0) n = 1;
   hipError_t e = hipMalloc(&p, n * sizeof(T));
-  if (e != hipSuccess)
-    throw Error(fmt("hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e)));
+  if (e != hipSuccess) fail_hip(fmt("hipMalloc of %zu bytes", n * sizeof(T)), e);
   owned.push_back(p);
   return (T *)p;
 }

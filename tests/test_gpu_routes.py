@@ -30,3 +30,13 @@ def test_in_place_triples_switch_keeps_the_three_body_force(ccnm, monkeypatch, A
             got.append(np.array(v + [s.t3_energy()]))
         assert np.all(got[0][[0, 1, 3, 4]] != 0)
         assert np.max(np.abs(got[1] - got[0])) <= 1e-12 * np.max(np.abs(got[0])), got
+
+
+def test_refused_allocation_leaves_the_next_call_alone(ccnm):
+    """An allocation that the card refuses is an error of that call only: the
+    runtime's record of it is not taken for one of a later launch."""
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1)
+    with pytest.raises(RuntimeError, match="hipMalloc"):
+        ccnm.hbm_read_probe(1 << 48, 1)
+    s.generate_interaction()
+    assert s.setup_t_amplitudes() != 0
