@@ -136,11 +136,18 @@ std::string fmt(const char *f, ...) {
     if (e_ != hipSuccess) fail_hip(#x, e_);    \
   } while (0)
 
+// Test hook (CCGPU_FORCE_NOMEM=bytes): allocations of at least so many bytes are
+// refused, as on a card that has no room for them.
+bool forced_nomem(size_t bytes) {
+  const char *e = getenv("CCGPU_FORCE_NOMEM");
+  return e && atof(e) > 0 && (double)bytes >= atof(e);
+}
+
 template <typename T>
 T *dalloc(size_t n, std::vector<void *> &owned) {
   void *p = nullptr;
   if (n == 0) n = 1;
-  hipError_t e = hipMalloc(&p, n * sizeof(T));
+  hipError_t e = forced_nomem(n * sizeof(T)) ? hipErrorOutOfMemory : hipMalloc(&p, n * sizeof(T));
   if (e != hipSuccess) fail_hip(fmt("hipMalloc of %zu bytes", n * sizeof(T)), e);
   owned.push_back(p);
   return (T *)p;
@@ -421,7 +428,7 @@ struct Solve {
   bool t3_lattice = false;       // the lattice's lists of t3 are made
   std::vector<void *> t3_owned;  // device memory of the current interaction's t3
   std::vector<int> t3_orbitof;
-  double2 *t3_gE = nullptr, *t3_gD = nullptr;   // the group tables
+  double2 *t3_group = nullptr;   // the group tables, gE and then gD
   bool have_w3 = false;          // t3.c3w holds the W3 constants
   bool have_ccdt1 = false;       // setup_t3 done
   double2 ccdt1_e3{0.0, 0.0};    // energy of the last t3_intermediate
@@ -3309,12 +3316,10 @@ void build_triples(Solve &S) {
   td.vhhhp = nullptr;
   const int64_t ntab = (int64_t)P.np * P.np * P.A * 2 + (int64_t)P.A * P.A * P.np * 2;
   if ((double)ntab * sizeof(double2) <= t3_table_limit() && P.np > 0) {
-    if (!S.t3_gE) {
-      S.t3_gE = dalloc<double2>((size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 2, S.owned);
-      S.t3_gD = dalloc<double2>((size_t)td.npg * 2 * td.nhp * 4 * 2, S.owned);
-    }
-    td.gE = S.t3_gE;
-    td.gD = S.t3_gD;
+    const size_t ne = (size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 2, nd = (size_t)td.npg * 2 * td.nhp * 4 * 2;
+    if (!S.t3_group) S.t3_group = dalloc<double2>(ne + nd, S.owned);   // one block: both or none
+    td.gE = S.t3_group;
+    td.gD = S.t3_group + ne;
     launch_t3_group_v(S.desc, td, P.orb.volume, S.stream);
     check_launch();
     HIPCHK(hipStreamSynchronize(S.stream));
@@ -3336,8 +3341,8 @@ bool legacy_tables(Solve &S) {
   if ((double)(nh + nl + nd) * sizeof(double2) > t3_table_limit() ||
       (size_t)4 * 3 * P.max_nhh * sizeof(double2) > 65536 || nh == 0)
     return false;
-  double2 *hppp = dalloc<double2>(nh, S.t3_owned), *hhhp = dalloc<double2>(nl, S.t3_owned);
-  S.t3_td = dalloc<double2>(nd, S.t3_owned);
+  double2 *hppp = dalloc<double2>(nh + nl + nd, S.t3_owned), *hhhp = hppp + nh;   // one block: all or none
+  S.t3_td = hhhp + nl;
   launch_t3_tables(S.desc, td, P.orb.volume, hppp, hhhp, S.stream);
   check_launch();
   HIPCHK(hipStreamSynchronize(S.stream));

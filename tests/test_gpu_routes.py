@@ -40,3 +40,25 @@ def test_refused_allocation_leaves_the_next_call_alone(ccnm):
         ccnm.hbm_read_probe(1 << 48, 1)
     s.generate_interaction()
     assert s.setup_t_amplitudes() != 0
+
+
+@pytest.mark.parametrize("kernel", [None, "1"])
+def test_triples_after_a_refused_table_allocation(ccnm, monkeypatch, kernel):
+    """A card without room for the tables of (T): the call fails, and the next
+    one, with room again, makes all of them and gives the same sum.  PNM A=38
+    |n_i|<=1 has more hole than particle groups, so the second group table
+    (390 kB) is the larger one."""
+    def solver():
+        s = native_3nf(ccnm, 38, "pnm", 0.16, 1, (0.0, 0.0, 0.0), 2)
+        s.setup_t_amplitudes()
+        return s
+    if kernel:
+        monkeypatch.setenv("CCGPU_T3_KERNEL", kernel)
+    want = solver().pert_triples2()
+    s = solver()
+    monkeypatch.setenv("CCGPU_FORCE_NOMEM", "300000")
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="hipMalloc of .* bytes failed"):
+            s.pert_triples2()
+    monkeypatch.delenv("CCGPU_FORCE_NOMEM")
+    assert want != 0 and s.pert_triples2() == want
