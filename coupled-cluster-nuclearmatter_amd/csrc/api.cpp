@@ -77,7 +77,7 @@ void launch_t3_tables(const SolveDesc &d, const TriplesDesc &td, double volume, 
                       hipStream_t st);
 void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *partial,
                     unsigned long long *count, int nblocks, double2 *out, unsigned long long *count_out,
-                    hipStream_t st, int variant, const double2 *tdt, int maxnhh);
+                    hipStream_t st, int variant, int mode, const double2 *tdt, int maxnhh);
 void launch_t3_td(const SolveDesc &d, const TriplesDesc &td, double2 *tdt, hipStream_t st);
 void launch_t3_group_v(const SolveDesc &d, const TriplesDesc &td, double volume, hipStream_t st);
 void launch_triples_group(const SolveDesc &d, const TriplesDesc &td, double2 *partial, unsigned long long *count,
@@ -429,13 +429,16 @@ struct Solve {
   std::vector<void *> t3_owned;  // device memory of the current interaction's t3
   std::vector<int> t3_orbitof;
   double2 *t3_group = nullptr;   // the group tables, gE and then gD
+  bool t3_tables = false;        // tables within CCGPU_T3_TABLE_GB: dense ones, and group tables too
+  bool t3_fit_groups = false;
+  int t3_sparse = 0;             // one state per group: hole triples per channel, else 0
   bool have_w3 = false;          // t3.c3w holds the W3 constants
   bool have_ccdt1 = false;       // setup_t3 done
   double2 ccdt1_e3{0.0, 0.0};    // energy of the last t3_intermediate
   double2 t3_et4{0.0, 0.0}, t3_et5{0.0, 0.0};   // parts of the last (T)
   TriplesDesc t3{};
   double2 *t3_partial = nullptr, *t3_out = nullptr;
-  double2 *t3_td = nullptr;   // t(x d, u v) of the staged kernel's F terms
+  double2 *t3_td = nullptr;   // t(x d, u v) of the staged kernel's F terms (null: no room)
   unsigned long long *t3_count = nullptr;   // per block, then the total at [8192]
   long long t3_elements = 0;
   double t3_seconds = 0.0;
@@ -3218,6 +3221,7 @@ void build_triples_lattice(Solve &S) {
   td.gf = dalloc<double2>(8 * gtrip.size(), S.owned);
   td.gE = td.gD = nullptr;
   td.vhppp = td.vhhhp = nullptr;
+  S.t3_sparse = ch > 0 && td.npg == P.np && td.nhg == P.A ? hptr.back() / ch : 0;
   S.t3_partial = dalloc<double2>(8192, S.owned);
   S.t3_out = dalloc<double2>(1, S.owned);
   S.t3_count = dalloc<unsigned long long>(8193, S.owned);
@@ -3227,6 +3231,8 @@ void build_triples_lattice(Solve &S) {
 double t3_table_limit() {   // bytes
   return (getenv("CCGPU_T3_TABLE_GB") ? atof(getenv("CCGPU_T3_TABLE_GB")) : 16.0) * 1e9;
 }
+size_t group_e_entries(const TriplesDesc &td) { return (size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 2; }
+size_t group_entries(const TriplesDesc &td) { return group_e_entries(td) + (size_t)td.npg * 2 * td.nhp * 4 * 2; }
 
 // The element source of the current interaction and, when they fit, the group
 // tables' interaction halves.  Device memory of an earlier interaction of the
@@ -3309,46 +3315,49 @@ void build_triples(Solve &S) {
     }
     td.parity = ok ? 1 : 0;
   }
-  // the group tables, when one entry per (c, b, k) and per (j, k, c) for both
-  // spins would fit in CCGPU_T3_TABLE_GB (default 16 GB; the tables take about
-  // half of that); otherwise (T) evaluates the elements in place
-  td.vhppp = nullptr;
-  td.vhhhp = nullptr;
+  // Tables, made by the first sum that reads them, when one entry per (c, b, k) and per
+  // (j, k, c) for both spins fits in CCGPU_T3_TABLE_GB (default 16 GB); otherwise (T)
+  // evaluates the elements in place.  The group tables take half of that with both
+  // states in every group, and up to four times it with one.
+  td.gE = td.gD = nullptr;
+  td.vhppp = td.vhhhp = nullptr;
   const int64_t ntab = (int64_t)P.np * P.np * P.A * 2 + (int64_t)P.A * P.A * P.np * 2;
-  if ((double)ntab * sizeof(double2) <= t3_table_limit() && P.np > 0) {
-    const size_t ne = (size_t)td.npg * (td.npg + 1) / 2 * 4 * td.nhg * 2 * 2, nd = (size_t)td.npg * 2 * td.nhp * 4 * 2;
-    if (!S.t3_group) S.t3_group = dalloc<double2>(ne + nd, S.owned);   // one block: both or none
-    td.gE = S.t3_group;
-    td.gD = S.t3_group + ne;
-    launch_t3_group_v(S.desc, td, P.orb.volume, S.stream);
-    check_launch();
-    HIPCHK(hipStreamSynchronize(S.stream));
-  } else {
-    td.gE = td.gD = nullptr;
-  }
-  if (td.tnf && !td.gE)
+  S.t3_tables = (double)ntab * sizeof(double2) <= t3_table_limit() && P.np > 0;
+  S.t3_fit_groups = S.t3_tables && (double)group_entries(td) * sizeof(double2) <= t3_table_limit();
+  if (td.tnf && !S.t3_tables)
     throw Error("(T) with the three-nucleon force needs its element tables: raise CCGPU_T3_TABLE_GB");
   S.have_t3 = true;
 }
 
-// The dense tables of the element-by-element kernels (CCGPU_T3_KERNEL=1, 3),
-// made on their first use for an interaction.
-bool legacy_tables(Solve &S) {
+void group_tables(Solve &S) {
   TriplesDesc &td = S.t3;
-  if (td.vhppp) return true;
+  if (td.gE) return;
+  if (!S.t3_group) S.t3_group = dalloc<double2>(group_entries(td), S.owned);   // one block: both or none
+  TriplesDesc t = td;
+  t.gE = S.t3_group;
+  t.gD = S.t3_group + group_e_entries(td);
+  launch_t3_group_v(S.desc, t, S.plan.orb.volume, S.stream);
+  check_launch();
+  HIPCHK(hipStreamSynchronize(S.stream));
+  td = t;
+}
+
+// The dense tables of the element-by-element kernels and, where it fits with them, the
+// amplitude table of the staged one.
+void element_tables(Solve &S) {
+  TriplesDesc &td = S.t3;
+  if (td.vhppp) return;
   const Plan &P = S.plan;
-  const int64_t nh = (int64_t)P.np * P.np * P.A * 2, nl = (int64_t)P.A * P.A * P.np * 2, nd = nl;
-  if ((double)(nh + nl + nd) * sizeof(double2) > t3_table_limit() ||
-      (size_t)4 * 3 * P.max_nhh * sizeof(double2) > 65536 || nh == 0)
-    return false;
-  double2 *hppp = dalloc<double2>(nh + nl + nd, S.t3_owned), *hhhp = hppp + nh;   // one block: all or none
-  S.t3_td = hhhp + nl;
+  const int64_t nh = (int64_t)P.np * P.np * P.A * 2, nl = (int64_t)P.A * P.A * P.np * 2;
+  const bool staged = (double)(nh + 2 * nl) * sizeof(double2) <= t3_table_limit() &&
+                      (size_t)4 * 3 * P.max_nhh * sizeof(double2) <= 65536;
+  double2 *hppp = dalloc<double2>(nh + (staged ? 2 : 1) * nl, S.t3_owned), *hhhp = hppp + nh;   // all or none
   launch_t3_tables(S.desc, td, P.orb.volume, hppp, hhhp, S.stream);
   check_launch();
   HIPCHK(hipStreamSynchronize(S.stream));
+  S.t3_td = staged ? hhhp + nl : nullptr;
   td.vhppp = hppp;
   td.vhhhp = hhhp;
-  return true;
 }
 
 // One sum over the triples (modes of k_triples_g): returns it and counts the
@@ -3368,23 +3377,36 @@ double2 triples_sum(Solve &S, int mode) {
     S.t3.c3w = c;
     S.have_w3 = true;
   }
-  if (mode != 2 && mode != 0 && !S.t3.gE)
+  if (mode != 2 && mode != 0 && !S.t3_tables)
     throw Error("CCDT-1 and the three-body (T) need the element tables: raise CCGPU_T3_TABLE_GB");
   const Plan &P = S.plan;
   int nb = (int)std::min<int64_t>(8192, std::max<int64_t>(1, S.t3.npairs));
-  // CCGPU_T3_KERNEL (studies and tests): (T) element by element, 1 and 3 on tables, 0 in
-  // place, which has the two-nucleon elements alone and no W3
-  const int variant = getenv("CCGPU_T3_KERNEL") ? atoi(getenv("CCGPU_T3_KERNEL")) : 2;
-  const bool in_place = mode == 0 && (!S.t3.gE || (variant == 0 && !S.t3.tnf));
-  if (mode == 0 && (variant == 1 || variant == 3) && legacy_tables(S)) {
+  // CCGPU_T3_KERNEL (studies and tests): 2 over groups, 1 and 3 element by element on
+  // dense tables, 0 (T) in place, which has the two-nucleon elements alone and no W3
+  const char *e = getenv("CCGPU_T3_KERNEL");
+  const int asked = e ? atoi(e) : -1;
+  // The group kernel does up to 64 elements per item.  With one state of every momentum
+  // and isospin (spin-polarised tables) an item is one element, and the kernels that take
+  // elements one by one win where their 64 lanes find enough hole triples per channel.  In
+  // groups and one by one, ms, (T) | W3 alone | W and W3 of neutrons: A=19 |n_i|<=3 (5 per
+  // channel) 3.1, 5.5 | 2.8, 4.2 | 2.4, 12; A=27 |n_i|<=2 (10) 0.60, 0.52 | 0.51, 0.39 |
+  // 0.9, 1.4; A=33 |n_i|<=4 (12) 77, 63 | 62, 42 | 131, 194; A=57 |n_i|<=4 (31) 347, 139 | 269,
+  // 75 | 576, 449; A=81 |n_i|<=4 (64) 936, 269 | 684, 118 | 1483, 832.  From eight elements
+  // per item groups win (holes of both spins, particles of one, A=66 |n_i|<=3: 16.5, 28.8).
+  const bool sparse = S.t3_sparse >= (mode == 1 || mode == 3 ? 24 : 8);
+  const bool groups = (asked == 2 || (asked != 1 && asked != 3 && !sparse)) && (S.t3_fit_groups || mode == 2);
+  if (mode == 0 && (!S.t3_tables || (asked == 0 && !S.t3.tnf))) {
+    launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream, 0,
+                   mode, nullptr, P.max_nhh);
+  } else if (groups) {
+    if (mode != 2) group_tables(S);
+    launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
+  } else {
+    if (mode != 2) element_tables(S);
+    const int variant = mode == 0 && asked != 3 && S.t3_td ? 1 : 3;
     if (variant == 1) launch_t3_td(S.desc, S.t3, S.t3_td, S.stream);
     launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream,
-                   variant, S.t3_td, P.max_nhh);
-  } else if (in_place) {
-    launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream, 0,
-                   nullptr, P.max_nhh);
-  } else {
-    launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
+                   variant, mode, S.t3_td, P.max_nhh);
   }
   check_launch();
   double2 r;

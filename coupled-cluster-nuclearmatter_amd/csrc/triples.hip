@@ -304,7 +304,9 @@ __global__ __launch_bounds__(256) void k_triples(SolveDesc d, TriplesDesc td, do
 // (a,b), its four waves take c = b+1+wave, b+5+wave, ..., and the 64 lanes of
 // a wave stride over the hole triples of that (K3,Tz3) channel.  Every lane of
 // a wave reads the same <c.||..> and <..||.c> table rows (cache-friendly), and
-// no lane waits for a longer hole-triple list than its wave's.
+// no lane waits for a longer hole-triple list than its wave's.  MODE as in
+// k_triples_g.
+template <int MODE, bool ONE>
 __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, double volume, double2 *partial,
                                                    unsigned long long *count) {
   __shared__ double sre[256], sim[256];
@@ -325,11 +327,19 @@ __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, 
       const double fai = d.fdiag[a].y, fbi = d.fdiag[b].y, fci = d.fdiag[c].y;
       const int h0 = td.hptr[ch], h1 = td.hptr[ch + 1];
       if (lane == 0) nel += (unsigned long long)(h1 - h0);
+      Nucleon na, nb, nc;
+      double reg = 0.0;
+      if constexpr (MODE != 0) {
+        na = nucleon_of(td.c3w, a);
+        nb = nucleon_of(td.c3w, b);
+        nc = nucleon_of(td.c3w, c);
+        reg = freg3(td.c3w, na.k, nb.k, nc.k);
+      }
       for (int h = h0 + lane; h < h1; h += 64) {
         const int i = td.hijk[3 * h], j = td.hijk[3 * h + 1], k = td.hijk[3 * h + 2];
         double2 w = make_double2(0.0, 0.0);
 #pragma unroll 1
-        for (int t = 0; t < 18; ++t) {
+        for (int t = 0; t < (MODE == 2 ? 0 : 18); ++t) {
           const TermCode tc = kTerms[t];
           const int x = sel3(tc.p0, a, b, c), y = sel3(tc.p1, a, b, c), z = sel3(tc.p2, a, b, c);
           const int u = sel3(tc.h0, i, j, k), v = sel3(tc.h1, i, j, k), q = sel3(tc.h2, i, j, k);
@@ -341,7 +351,14 @@ __global__ __launch_bounds__(256) void k_triples_w(SolveDesc d, TriplesDesc td, 
         const double dre = d.fdiag[i].x + d.fdiag[j].x + d.fdiag[k].x - fa - fb - fc;
         const double dim = d.fdiag[i].y + d.fdiag[j].y + d.fdiag[k].y - fai - fbi - fci;
         const double den = dre * dre + dim * dim;
-        const double nre = w.x * w.x + w.y * w.y, nim = 0.0;
+        double nre = w.x * w.x + w.y * w.y, nim = 0.0;
+        if constexpr (MODE != 0) {
+          const double2 w3 = chiral3_asym<ONE>(td.c3w, reg, na, nb, nc, nucleon_of(td.c3w, i), nucleon_of(td.c3w, j),
+                                               nucleon_of(td.c3w, k));
+          const double xr = w3.x + w.x, xi = w3.y + w.y;
+          nre = MODE == 3 ? xr * xr + xi * xi : xr * w3.x + xi * w3.y;
+          if constexpr (MODE == 1) nim = xi * w3.x - xr * w3.y;
+        }
         re += (nre * dre + nim * dim) / den;
         im += (nim * dre - nre * dim) / den;
       }
@@ -1074,18 +1091,28 @@ void launch_triples_group(const SolveDesc &d, const TriplesDesc &td, double2 *pa
   hipLaunchKernelGGL(k_triples_final, dim3(1), dim3(256), 0, st, partial, count, nb, out, count_out);
 }
 
-// (T) by one of the element-by-element kernels: 0 in place (no tables), 1 the
-// staged kernel, 3 the kernel that gathers every amplitude
+// The sum by one of the element-by-element kernels: 0 in place (no tables, mode 0
+// alone), 1 the staged kernel (mode 0 alone), 3 the kernel that gathers every amplitude
 void launch_triples(const SolveDesc &d, const TriplesDesc &td, double volume, double2 *partial,
                     unsigned long long *count, int nblocks, double2 *out, unsigned long long *count_out,
-                    hipStream_t st, int variant, const double2 *tdt, int maxnhh) {
+                    hipStream_t st, int variant, int mode, const double2 *tdt, int maxnhh) {
+  const bool one = td.c3w.one_species != 0;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+  };
   if (variant == 1) {
     const size_t lds = (size_t)4 * 3 * maxnhh * sizeof(double2);
     hipLaunchKernelGGL(k_triples_s, dim3(nblocks), dim3(256), lds, st, d, td, tdt, maxnhh, partial, count);
-  } else if (variant == 3) {
-    hipLaunchKernelGGL(k_triples_w, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+  } else if (variant == 0) {
+    run(k_triples);
+  } else if (mode == 0) {
+    run(k_triples_w<0, true>);
+  } else if (mode == 1) {
+    run(one ? k_triples_w<1, true> : k_triples_w<1, false>);
+  } else if (mode == 2) {
+    run(one ? k_triples_w<2, true> : k_triples_w<2, false>);
   } else {
-    hipLaunchKernelGGL(k_triples, dim3(nblocks), dim3(256), 0, st, d, td, volume, partial, count);
+    run(one ? k_triples_w<3, true> : k_triples_w<3, false>);
   }
   hipLaunchKernelGGL(k_triples_final, dim3(1), dim3(256), 0, st, partial, count, nblocks, out, count_out);
 }

@@ -62,3 +62,73 @@ def test_triples_after_a_refused_table_allocation(ccnm, monkeypatch, kernel):
             s.pert_triples2()
     monkeypatch.delenv("CCGPU_FORCE_NOMEM")
     assert want != 0 and s.pert_triples2() == want
+
+
+def device_memory_free():
+    rt = C.CDLL("libamdhip64.so.7")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert rt.hipDeviceSynchronize() == 0
+    assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def polarised(ccnm, A, nmax, both=0):
+    """Neutrons of spin up in a box at 0.16 fm^-3, the lowest `both` states with
+    their spin-down partners: a table handed over orbital by orbital."""
+    n = range(-nmax, nmax + 1)
+    up = sorted((x * x + y * y + z * z, x, y, z, 1) for x in n for y in n for z in n)
+    st = sorted(up + [(*q[:4], -1) for q in up[:both]])
+    box = (A / 0.16) ** (1 / 3)
+    f = 2 * np.pi / box
+    q = np.array(st)
+    o = dict(A=A, nx=q[:, 1], ny=q[:, 2], nz=q[:, 3], sz=q[:, 4], tz=np.ones(len(st)), kx=f * q[:, 1], ky=f * q[:, 2],
+             kz=f * q[:, 3], e=197.326968 ** 2 / (2 * 939.565) * f * f * q[:, 0], box=box, volume=box ** 3)
+    s = ccnm.Solver(orbitals=o)
+    s.set_chiral(ccnm.NNLO, 450.0)
+    s.set_3nf(3)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    s.setup_t_amplitudes()
+    return s
+
+
+@pytest.mark.parametrize("A,nmax,both", [(19, 1, 0), (27, 2, 0), (38, 2, 19), (7, 1, 0)])
+def test_triples_of_spin_polarised_tables_by_every_kernel(ccnm, monkeypatch, A, nmax, both):
+    """One spin state per momentum (few and many hole triples per channel) and
+    both for the holes alone: the sums over groups, element by element and by
+    the rule's own choice are sums of the same terms (1e-12 for their order;
+    the sums have one sign per element, W some cancellation inside)."""
+    s = polarised(ccnm, A, nmax, both)
+    got = {}
+    for kernel in (None, "2", "1", "3"):
+        if kernel is None:
+            monkeypatch.delenv("CCGPU_T3_KERNEL", raising=False)
+        else:
+            monkeypatch.setenv("CCGPU_T3_KERNEL", kernel)
+        et = s.pert_triples2()
+        n = s.triples_stats()[0]
+        v = [et, *s.triples_parts(), s.setup_t3()]
+        s.t3_intermediate()
+        got[kernel] = np.array(v + [s.t3_energy(), n])
+    assert np.all(got["2"] != 0)
+    for kernel in (None, "1", "3"):
+        assert got[kernel][-1] == got["2"][-1]
+        assert np.all(np.abs(got[kernel] - got["2"]) <= 1e-12 * np.abs(got["2"])), got
+
+
+def test_triples_tables_of_spin_polarised_matter_stay_within_their_budget(ccnm, monkeypatch):
+    """A=33 |n_i|<=3, one spin state per momentum: dense tables of 113 MB, group
+    tables of four times that.  (T) makes the dense ones, by its own choice and
+    where groups are asked for in a budget that has no room for theirs."""
+    s = polarised(ccnm, 33, 3)
+    np_ = s.dims["nparticles"]
+    dense = 32 * (np_ * np_ * 33 + 2 * 33 * 33 * np_)
+    s.set_3nf(2)   # (T) without W3
+    monkeypatch.setenv("CCGPU_T3_TABLE_GB", str(1.5 * dense / 1e9))
+    monkeypatch.setenv("CCGPU_T3_KERNEL", "2")
+    before = device_memory_free()
+    first = s.pert_triples2()
+    assert before - device_memory_free() < 1.5 * dense
+    monkeypatch.delenv("CCGPU_T3_KERNEL")
+    monkeypatch.delenv("CCGPU_T3_TABLE_GB")
+    assert s.pert_triples2() == first
+    assert before - device_memory_free() < 1.5 * dense
