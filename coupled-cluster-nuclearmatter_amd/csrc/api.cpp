@@ -265,11 +265,13 @@ struct GemmList {
   // class 5: N <= 4; 0: N <= 16; 1: <= 32; 2: <= 48; 3: <= 64 or > 80; 4: <= 80.
   // BF16x3 lists: 5: N <= 4; 0: <= 16; 1: <= 32; 2: <= 64; 4: <= 96; 3: wider
   static int cls_of(int N) {
-    return N <= 4 ? 5 : N <= 16 ? 0 : N <= 32 ? 1 : N <= 48 ? 2 : N <= 64 ? 3 : N <= 80 ? 4 : 3;
+    return N <= 16 ? 0 : N <= 32 ? 1 : N <= 48 ? 2 : N <= 64 ? 3 : N <= 80 ? 4 : 3;
   }
-  int cls(int N) const {
+  int cls(const GemmGroup &g) const {
+    const int N = g.N;
+    if (g.thin) return 5;
     if (!bf3) return cls_of(N);
-    return N <= 4 ? 5 : N <= 16 ? 0 : N <= 32 ? 1 : N <= 64 ? 2 : N <= 96 ? 4 : 3;
+    return N <= 16 ? 0 : N <= 32 ? 1 : N <= 64 ? 2 : N <= 96 ? 4 : 3;
   }
   void add(GemmGroup g, int solve) {
     if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
@@ -286,7 +288,7 @@ struct GemmList {
   }
   bool has_class(int c) const {
     for (const GemmGroup &g : groups)
-      if (cls(g.N) == c) return true;
+      if (cls(g) == c) return true;
     return false;
   }
   void apply_env_shapes() {
@@ -334,7 +336,7 @@ struct GemmList {
     maxmn = 0;
     for (size_t gi = 0; gi < groups.size(); ++gi) {
       GemmGroup &g = groups[gi];
-      const int c = cls(g.N);
+      const int c = cls(g);
       const int nsp = nosplit ? 1 : split_of(g);
       int ksz = (g.K + nsp - 1) / nsp;
       ksz = (ksz + 15) / 16 * 16;
@@ -389,6 +391,14 @@ GemmGroup mkgroup(const void *A, const double2 *B, double2 *C, const double2 *C0
   g.A = A; g.B = B; g.C = C; g.C0 = C0; g.P = nullptr;
   g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldc0 = ldc0;
   g.nsplit = 1; g.alpha = alpha; g.beta = beta;
+  g.thin = N <= 4;
+  return g;
+}
+// Group of a ring channel: thin where the channel or its pair -K' has at most four
+// columns.  The pairs were contracted as two channels, and the products of the thin one
+// were in FP64 under every precision.
+GemmGroup ring_group(GemmGroup g, int nph, int nhp) {
+  g.thin = std::min(nph, nhp) <= 4;
   return g;
 }
 
@@ -647,9 +657,10 @@ void build_device(Solve &S) {
     double2 *Tt = d.Tt + P.off_rt[K], *Rt = d.Rt + P.off_rt[K], *I4 = d.I4 + P.off_i4[K];
     // the channel and its pair as one (Plan::ph_pair): I4 = W0 + Vt Tt (ccm_t2_eqn.f90:657-780),
     // Rt = W1 Tt + Tt I4 (ccm_t2_eqn.f90:995-1026)
-    S.g_i4.add(mkgroup(d.Vt + P.off_vt[K], Tt, I4, d.W0 + P.off_i4[K], nhp, nhp, nph, nph, nhp, nhp, nhp, 1.0, 1.0), 0);
-    S.g_i4.add(mkgroup(d.W1 + P.off_w1[K], Tt, Rt, nullptr, nph, nhp, nph, nph, nhp, nhp, 0, 1.0, 0.0), 0);
-    S.g_rt.add(mkgroup(Tt, I4, Rt, Rt, nph, nhp, nhp, nhp, nhp, nhp, nhp, 1.0, 1.0), 0);
+    auto add = [&](GemmList &L, const GemmGroup &g) { L.add(ring_group(g, nph, nhp), 0); };
+    add(S.g_i4, mkgroup(d.Vt + P.off_vt[K], Tt, I4, d.W0 + P.off_i4[K], nhp, nhp, nph, nph, nhp, nhp, nhp, 1.0, 1.0));
+    add(S.g_i4, mkgroup(d.W1 + P.off_w1[K], Tt, Rt, nullptr, nph, nhp, nph, nph, nhp, nhp, 0, 1.0, 0.0));
+    add(S.g_rt, mkgroup(Tt, I4, Rt, Rt, nph, nhp, nhp, nhp, nhp, nhp, nhp, 1.0, 1.0));
   }
   // tiles are made per batch (make_batch), for the batch's own class sizes
   S.g_pp.bytes = 16.0 * (double)P.nVpp;

@@ -170,9 +170,10 @@ void launch_ring64(const RingTile *tiles, int ntiles, int cls, const SolveDesc *
 // 16-column blocks, WR along the rows by WC along the columns.
 //
 // Channels of up to 64 rows (WR 4, WC 2, NC 2), 128 (WR 8, NC 4) and 256 (RB 2, NC 1)
-// in one launch, 64 KB of LDS, two workgroups per CU.  Channels of at most 4 hp pairs
-// stay in FP64 (ringbf_thin).  Bound by the L2 reads of the rows: four densities of PNM
-// A=66 |n_i|<=4 take 313 us, as I4 and R~ with a launch per width class 561 in twelve.
+// in one launch, 64 KB of LDS, two workgroups per CU.  Channels with at most 4 pairs on
+// either side stay in FP64 (ringbf_thin, ringbf_flat).  Bound by the L2 reads of the rows:
+// four densities of PNM A=66 |n_i|<=4 take 313 us, as I4 and R~ with a launch per width
+// class 561 in twelve.
 // ---------------------------------------------------------------------------
 typedef float cf4 __attribute__((ext_vector_type(4), aligned(8)));   // two float2
 
@@ -313,14 +314,14 @@ __device__ __forceinline__ void ringbf_tile(const RingTile32 &t, unsigned *S) {
       }
 }
 
+__device__ __forceinline__ void mac(double2 &s, float2 x, float2 y) {
+  s.x += (double)x.x * y.x - (double)x.y * y.y;
+  s.y += (double)x.x * y.y + (double)x.y * y.x;
+}
 // at most 4 hp pairs: a thread per element, products and sums in FP64
 __device__ __forceinline__ void ringbf_thin(const RingTile32 &t, float2 *i4) {
   auto row = [](double2 s, const float2 *a, const float2 *b, int K, int N) {   // s + a . column of b
-    for (int k = 0; k < K; ++k) {
-      const float2 x = a[k], y = b[k * N];
-      s.x += (double)x.x * y.x - (double)x.y * y.y;
-      s.y += (double)x.x * y.y + (double)x.y * y.x;
-    }
+    for (int k = 0; k < K; ++k) mac(s, a[k], b[k * N]);
     return s;
   };
   const int N = t.nhp;
@@ -337,6 +338,36 @@ __device__ __forceinline__ void ringbf_thin(const RingTile32 &t, float2 *i4) {
   }
 }
 
+// at most 4 ph pairs: R~ = T~ W0 + (W1 + T~ V~) T~, the bracket of up to 4 x 4 elements
+// first, 32 lanes to each
+__device__ __forceinline__ void ringbf_flat(const RingTile32 &t, double2 *b) {
+  const int M = t.nph, N = t.nhp;
+  const int x = threadIdx.x >> 5, l = threadIdx.x & 31;
+  if (x < M * M) {
+    const int r = x / M, s = x % M;
+    double2 v = make_double2(0.0, 0.0);
+    for (int k = l; k < N; k += 32) mac(v, t.Tt[r * N + k], t.Vt[k * M + s]);
+    for (int off = 16; off > 0; off >>= 1) {
+      v.x += __shfl_xor(v.x, off);
+      v.y += __shfl_xor(v.y, off);
+    }
+    if (l == 0) b[x] = make_double2(v.x + t.W1[x].x, v.y + t.W1[x].y);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < M * N; e += 512) {
+    const int r = e / N, c = e % N;
+    double2 v = make_double2(0.0, 0.0);
+    for (int k = 0; k < N; ++k) mac(v, t.Tt[r * N + k], t.W0[(unsigned)k * N + c]);
+    for (int k = 0; k < M; ++k) {
+      const double2 q = b[r * M + k];
+      const float2 y = t.Tt[k * N + c];
+      v.x += q.x * y.x - q.y * y.y;
+      v.y += q.x * y.y + q.y * y.x;
+    }
+    t.Rt[e] = make_float2((float)v.x, (float)v.y);
+  }
+}
+
 __global__ __launch_bounds__(512, 4) void k_ringbf(const RingTile32 *__restrict__ tiles,
                                                    const SolveDesc *__restrict__ descs) {
   __shared__ __align__(16) unsigned S[2 * 128 * 64];
@@ -344,6 +375,7 @@ __global__ __launch_bounds__(512, 4) void k_ringbf(const RingTile32 *__restrict_
   if (!descs[t.solve].active) return;
   const int d = max(t.nph, t.nhp);
   if (t.nhp <= 4) ringbf_thin(t, (float2 *)S);
+  else if (t.nph <= 4) ringbf_flat(t, (double2 *)S);
   else if (d <= 64) ringbf_tile<4, 2, 1, 2>(t, S);
   else if (d <= 128) ringbf_tile<8, 1, 1, 4>(t, S);
   else ringbf_tile<8, 1, 2, 1>(t, S);
@@ -351,6 +383,7 @@ __global__ __launch_bounds__(512, 4) void k_ringbf(const RingTile32 *__restrict_
 
 int ringbf_columns(int nph, int nhp) {   // columns of a tile, 0: channel too large for the kernel
   const int d = std::max(nph, nhp);
+  if (nph <= 4 || nhp <= 4) return nhp;
   return d <= 128 ? 64 : d <= 256 ? 16 : 0;
 }
 void launch_ringbf(const RingTile32 *tiles, int ntiles, const SolveDesc *dd, hipStream_t st) {

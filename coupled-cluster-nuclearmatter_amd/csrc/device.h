@@ -104,6 +104,7 @@ struct GemmGroup {
   int M, N, K;
   int lda, ldb, ldc, ldc0;
   int nsplit;
+  int thin;   // runs the thin FP64 kernel in every precision
   double alpha, beta;
 };
 

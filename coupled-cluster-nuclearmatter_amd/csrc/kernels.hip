@@ -1715,7 +1715,8 @@ __global__ __launch_bounds__(256) void k_zgemm_bf3(const GemmGroup *__restrict__
 }
 
 // Thin GEMM for groups with N <= 4 columns (most pp-ladder channels with few
-// hole pairs): FP64 VALU instead of 16-column MFMA tiles, which would be 75% or
+// hole pairs), and for ring channels with at most four pairs on either side, four
+// columns a tile: FP64 VALU instead of 16-column MFMA tiles, which would be 75% or
 // more padding.  A tile is 16 rows: each wave owns 4 rows, its 64 lanes walk
 // the k range 64 consecutive elements at a time (one coalesced 1 KB read of a
 // row per instruction), each lane reuses its B row (4 columns) for the 4 rows,
@@ -1747,12 +1748,12 @@ __global__ __launch_bounds__(256) void k_zgemm_thin(const GemmGroup *__restrict_
     for (int n = 0; n < 4; ++n) {
       double2 v;
       if constexpr (F32IO) {
-        const float2 f = gload((const float2 *)g.B + (int64_t)kc * g.ldb + min(n, g.N - 1));
+        const float2 f = gload((const float2 *)g.B + (int64_t)kc * g.ldb + min(tl.n0 + n, g.N - 1));
         v = make_double2(f.x, f.y);
       } else {
-        v = gload(g.B + (int64_t)kc * g.ldb + min(n, g.N - 1));
+        v = gload(g.B + (int64_t)kc * g.ldb + min(tl.n0 + n, g.N - 1));
       }
-      const bool ok = okk && n < g.N;
+      const bool ok = okk && tl.n0 + n < g.N;
       b[n] = make_double2(ok ? v.x : 0.0, ok ? v.y : 0.0);
     }
 #pragma unroll
@@ -1799,7 +1800,7 @@ __global__ __launch_bounds__(256) void k_zgemm_thin(const GemmGroup *__restrict_
     v[0].y += __shfl_xor(v[0].y, s);
   }
   if ((lane & 3) == 0) {
-    const int r = lane >> 4, n = (lane >> 2) & 3;
+    const int r = lane >> 4, n = tl.n0 + ((lane >> 2) & 3);
     const int m = m0 + r;
     const double2 v0 = v[0];
     if (m < g.M && n < g.N) {

@@ -132,3 +132,58 @@ def test_triples_tables_of_spin_polarised_matter_stay_within_their_budget(ccnm, 
     monkeypatch.delenv("CCGPU_T3_TABLE_GB")
     assert s.pert_triples2() == first
     assert before - device_memory_free() < 1.5 * dense
+
+
+def ring_channel(o, x, y):
+    """Pandya channel of n_x - n_y, its sign dropped: the channel pair's key."""
+    k = tuple(int(o[q][x] - o[q][y]) for q in ("tz", "nx", "ny", "nz"))
+    return max(k, tuple(-v for v in k))
+
+
+@pytest.mark.parametrize("lists", [False, True])
+@pytest.mark.parametrize("prec", ["PREC_BF16X3", "PREC_FP32"])
+def test_thin_ring_channels_stay_in_fp64_arithmetic(ccnm, monkeypatch, prec, lists):
+    """Channel pairs with at most four pairs on either side are contracted in
+    FP64 arithmetic under the low precisions (BF16x3: on FP32 blocks).  With one
+    amplitude the ring of its channel pair is single products V t away from
+    the amplitude itself, so the residual equals the FP64 one to the roundings
+    of V, t and the product to FP32 (3 x 2^-24, and 2^-24 for their products), or
+    to those of FP64 where the blocks are FP64; split products are off by
+    2^-18 to 2^-16."""
+    monkeypatch.setenv("CCGPU_TERMS", "8")
+    if lists:   # the list kernels in place of the fused ring, at the default split
+        monkeypatch.setenv("CCGPU_SPLIT_TILES", "128")
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1, twist=(0.5, 1.2, 2.2))
+    s.set_chiral(ccnm.NNLO, 450.0)
+    s.generate_interaction(ccnm.INT_CHIRAL)
+    s.setup_t_amplitudes()
+    o, A = s.orbitals(), s.dims["nholes"]
+    lab = s.t2_labels()
+    size = {}   # (particle, hole) pairs of n_a - n_i = k and of -k
+    for a in range(A, s.dims["nsp"]):
+        for i in range(A):
+            k = tuple(int(o[q][a] - o[q][i]) for q in ("tz", "nx", "ny", "nz"))
+            key = max(k, tuple(-v for v in k))
+            size.setdefault(key, [0, 0])[0 if k == key else 1] += 1
+    thin = {k for k, v in size.items() if min(v) <= 4 < max(v)}
+    plus = [ring_channel(o, a, i) for a, b, i, j in lab]
+    minus = [ring_channel(o, b, i) for a, b, i, j in lab]
+    bound = 4 * 2.0 ** -24 if prec == "PREC_BF16X3" else 8 * 2.0 ** -53
+    checked = set()
+    for k in sorted(thin):
+        u = plus.index(k) if k in plus else None
+        if u is None:
+            continue
+        t = np.zeros(len(lab), np.complex128)
+        t[u] = 0.7390851332151607 + 0.5671432904097838j
+        r = []
+        for p in (ccnm.PREC_FP64, getattr(ccnm, prec)):
+            s.set_t2_unique(t)
+            s.t2_intermediate(p)
+            r.append(s.debug_fetch("R", len(lab)) - s.debug_fetch("R0", len(lab)))
+        own = (k, minus[u])
+        for v in range(len(lab)):
+            if v != u and plus[v] == k and minus[v] not in own and abs(r[0][v]) > 1e-8:
+                assert abs(r[1][v] - r[0][v]) <= bound * abs(r[0][v]) + 2.0 ** -50 * abs(t[u]), (k, v, r[0][v], r[1][v])
+                checked.add(k)
+    assert len(checked) >= 3, checked   # the channel pairs of this lattice with such elements
