@@ -3326,7 +3326,7 @@ void build_triples(Solve &S) {
     }
     td.parity = ok ? 1 : 0;
   }
-  // Tables, made by the first sum that reads them, when one entry per (c, b, k) and per
+  // Tables, made by the first sum that asks for them, when one entry per (c, b, k) and per
   // (j, k, c) for both spins fits in CCGPU_T3_TABLE_GB (default 16 GB); otherwise (T)
   // evaluates the elements in place.  The group tables take half of that with both
   // states in every group, and up to four times it with one.
@@ -3400,20 +3400,25 @@ double2 triples_sum(Solve &S, int mode) {
   // and isospin (spin-polarised tables) an item is one element, and the kernels that take
   // elements one by one win where their 64 lanes find enough hole triples per channel.  In
   // groups and one by one, ms, (T) | W3 alone | W and W3 of neutrons: A=19 |n_i|<=3 (5 per
-  // channel) 3.1, 5.5 | 2.8, 4.2 | 2.4, 12; A=27 |n_i|<=2 (10) 0.60, 0.52 | 0.51, 0.39 |
+  // channel) 3.1, 5.5 | 2.8, 4.2 | 5.2, 16; A=27 |n_i|<=2 (10) 0.60, 0.52 | 0.51, 0.39 |
   // 0.9, 1.4; A=33 |n_i|<=4 (12) 77, 63 | 62, 42 | 131, 194; A=57 |n_i|<=4 (31) 347, 139 | 269,
   // 75 | 576, 449; A=81 |n_i|<=4 (64) 936, 269 | 684, 118 | 1483, 832.  From eight elements
   // per item groups win (holes of both spins, particles of one, A=66 |n_i|<=3: 16.5, 28.8).
-  const bool sparse = S.t3_sparse >= (mode == 1 || mode == 3 ? 24 : 8);
-  const bool groups = (asked == 2 || (asked != 1 && asked != 3 && !sparse)) && (S.t3_fit_groups || mode == 2);
-  if (mode == 0 && (!S.t3_tables || (asked == 0 && !S.t3.tnf))) {
+  auto by_groups = [&](int m) {
+    const bool sparse = S.t3_sparse >= (m == 1 || m == 3 ? 24 : 8);
+    return (asked == 2 || (asked != 1 && asked != 3 && !sparse)) && (S.t3_fit_groups || m == 2);
+  };
+  const bool in_place = mode == 0 && (!S.t3_tables || (asked == 0 && !S.t3.tnf));
+  if (S.t3_tables && !in_place) {   // the start of CCDT-1 reads none, but makes those of its steps
+    if (by_groups(mode == 2 ? 1 : mode)) group_tables(S);
+    else element_tables(S);
+  }
+  if (in_place) {
     launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream, 0,
                    mode, nullptr, P.max_nhh);
-  } else if (groups) {
-    if (mode != 2) group_tables(S);
+  } else if (by_groups(mode)) {
     launch_triples_group(S.desc, S.t3, S.t3_partial, S.t3_count, 8192, S.t3_out, S.t3_count + 8192, S.stream, mode);
   } else {
-    if (mode != 2) element_tables(S);
     const int variant = mode == 0 && asked != 3 && S.t3_td ? 1 : 3;
     if (variant == 1) launch_t3_td(S.desc, S.t3, S.t3_td, S.stream);
     launch_triples(S.desc, S.t3, P.orb.volume, S.t3_partial, S.t3_count, nb, S.t3_out, S.t3_count + 8192, S.stream,
