@@ -153,6 +153,18 @@ T *dalloc(size_t n, std::vector<void *> &owned) {
   return (T *)p;
 }
 
+// Allocations that belong together: freed unless all of them were made and kept.
+struct Fresh {
+  std::vector<void *> own;
+  void keep(std::vector<void *> &owned) {
+    owned.insert(owned.end(), own.begin(), own.end());
+    own.clear();
+  }
+  ~Fresh() {
+    for (void *p : own) (void)hipFree(p);
+  }
+};
+
 template <typename T>
 T *dupload(const std::vector<T> &v, std::vector<void *> &owned) {
   T *p = dalloc<T>(v.size(), owned);
@@ -2245,21 +2257,25 @@ void ensure_f32(Solve &S, int handle) {
     S.off_vpp32.push_back(S.off_vpp32.back() + n * ((n + 1) & ~1));
   }
   S.nVpp32 = S.off_vpp32.back();
-  S.d_off_vpp = dupload(P.off_vpp, S.owned);
-  S.d_off_vpp32 = dupload(S.off_vpp32, S.owned);
-  S.d_npp = dupload(P.npp, S.owned);
-  S.desc.Vpppp32 = dalloc<float2>(S.nVpp32, S.owned);
+  Fresh f;
+  SolveDesc d = S.desc;
+  S.d_off_vpp = dupload(P.off_vpp, f.own);
+  S.d_off_vpp32 = dupload(S.off_vpp32, f.own);
+  S.d_npp = dupload(P.npp, f.own);
+  d.Vpppp32 = dalloc<float2>(S.nVpp32, f.own);
   // FP32 ring blocks of the BF16x3 residual; T~ entries with a=b or i=j stay zero, and
   // k_ringbf reads rows in words of four elements
   constexpr int kRing32Pad = 4;
-  S.desc.Tt32 = dalloc<float2>(P.nRt + kRing32Pad, S.owned);
-  S.desc.Rt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), S.owned);
-  S.desc.Vt32 = dalloc<float2>(P.nRt + kRing32Pad, S.owned);
-  S.desc.I4_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
-  S.desc.W0_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), S.owned);
-  S.desc.W1_32 = dalloc<float2>(P.nW1 + kRing32Pad, S.owned);
-  S.desc.Tbf = dalloc<uint4>(std::max<int64_t>(P.nT, 1), S.owned);
-  HIPCHK(hipMemset(S.desc.Tt32, 0, (P.nRt + kRing32Pad) * sizeof(float2)));
+  d.Tt32 = dalloc<float2>(P.nRt + kRing32Pad, f.own);
+  d.Rt32 = dalloc<float2>(std::max<int64_t>(P.nRt, 1), f.own);
+  d.Vt32 = dalloc<float2>(P.nRt + kRing32Pad, f.own);
+  d.I4_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), f.own);
+  d.W0_32 = dalloc<float2>(std::max<int64_t>(P.nI4, 1), f.own);
+  d.W1_32 = dalloc<float2>(P.nW1 + kRing32Pad, f.own);
+  d.Tbf = dalloc<uint4>(std::max<int64_t>(P.nT, 1), f.own);
+  HIPCHK(hipMemset(d.Tt32, 0, (P.nRt + kRing32Pad) * sizeof(float2)));
+  f.keep(S.owned);
+  S.desc = d;
   fill_f32(S);
   HIPCHK(hipMemcpy(S.d_desc, &S.desc, sizeof(SolveDesc), hipMemcpyHostToDevice));
   drop_single(handle);
@@ -2443,6 +2459,7 @@ struct Mlp {
     HIPCHK(hipStreamSynchronize(stream));
     for (void *p : batch_owned) (void)hipFree(p);
     batch_owned.clear();
+    bcap = 0;
     tb.x1t = dalloc<uint16_t>((size_t)16 * B, batch_owned);
     tb.h1t = dalloc<uint16_t>((size_t)64 * B, batch_owned);
     tb.h2t = dalloc<uint16_t>((size_t)64 * B, batch_owned);
@@ -2460,6 +2477,7 @@ struct Mlp {
     HIPCHK(hipStreamSynchronize(stream));
     for (void *p : scratch_owned) (void)hipFree(p);
     scratch_owned.clear();
+    scap = 0;
     sfeat = dalloc<uint16_t>((size_t)16 * n_, scratch_owned);
     sy = dalloc<float>((size_t)n_, scratch_owned);
     st = dalloc<float>((size_t)n_, scratch_owned);
@@ -2468,10 +2486,9 @@ struct Mlp {
   void grow_set(int64_t need) {
     if (need <= cap) return;
     int64_t nc = std::max<int64_t>(need, cap + cap / 2);
-    uint16_t *f2 = nullptr;
-    float *t2 = nullptr;
-    HIPCHK(hipMalloc((void **)&f2, (size_t)nc * 16 * sizeof(uint16_t)));
-    HIPCHK(hipMalloc((void **)&t2, (size_t)nc * sizeof(float)));
+    Fresh fresh;
+    uint16_t *f2 = dalloc<uint16_t>((size_t)nc * 16, fresh.own);
+    float *t2 = dalloc<float>((size_t)nc, fresh.own);
     if (n > 0) {
       HIPCHK(hipMemcpyAsync(f2, feat, (size_t)n * 16 * sizeof(uint16_t), hipMemcpyDeviceToDevice, stream));
       HIPCHK(hipMemcpyAsync(t2, target, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, stream));
@@ -2482,6 +2499,7 @@ struct Mlp {
     feat = f2;
     target = t2;
     cap = nc;
+    fresh.own.clear();
   }
 };
 

@@ -187,3 +187,55 @@ def test_thin_ring_channels_stay_in_fp64_arithmetic(ccnm, monkeypatch, prec, lis
                 assert abs(r[1][v] - r[0][v]) <= bound * abs(r[0][v]) + 2.0 ** -50 * abs(t[u]), (k, v, r[0][v], r[1][v])
                 checked.add(k)
     assert len(checked) >= 3, checked   # the channel pairs of this lattice with such elements
+
+
+def test_low_precision_after_a_refused_allocation(ccnm, monkeypatch):
+    """A card with room for the FP32 copy of V_pppp and not for what comes with
+    it: the residual fails, and the next one, with room again, equals that of a
+    handle that was never refused (no copy is taken for filled).  PNM A=38
+    |n_i|<=1 has fewer particle than hole pairs, so its split T is the larger."""
+    def solver():
+        s = ccnm.Solver(A=38, matter=ccnm.PNM, rho=0.16, nmax=1)
+        s.generate_interaction()
+        s.setup_t_amplitudes()
+        return s
+    want = solver()
+    want.t2_intermediate(ccnm.PREC_BF16X3)
+    n = want.dims["t2_unique"]
+    s = solver()
+    assert 8 * s.dims["vpppp_unique"] * 1.2 < 16 * n
+    monkeypatch.setenv("CCGPU_FORCE_NOMEM", str(16 * n))
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="hipMalloc of .* bytes failed"):
+            s.t2_intermediate(ccnm.PREC_BF16X3)
+    monkeypatch.delenv("CCGPU_FORCE_NOMEM")
+    s.t2_intermediate(ccnm.PREC_BF16X3)
+    r = want.debug_fetch("R", n)
+    assert np.all(np.isfinite(r)) and np.any(r != 0)
+    assert np.array_equal(s.debug_fetch("R", n), r)
+
+
+def test_network_after_a_refused_allocation(ccnm, monkeypatch):
+    """A minibatch and a training set that the card has no room for leave the
+    network as it was: the steps before and after are those of one that was
+    never refused."""
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=1)
+    s.generate_interaction()
+    s.setup_t_amplitudes()
+    s.ccd_iter()
+    nets = [ccnm.WarmStart(seed=3) for _ in range(2)]
+    n = s.dims["t2_unique"]
+    for net in nets:
+        net.add_solve(s)
+        net.train(2, batch=64, seed=5)
+    monkeypatch.setenv("CCGPU_FORCE_NOMEM", str(4 * n))
+    with pytest.raises(RuntimeError, match="hipMalloc of .* bytes failed"):
+        nets[1].add_solve(s)
+    with pytest.raises(RuntimeError, match="hipMalloc of .* bytes failed"):
+        nets[1].train(1, batch=1 << 20, seed=5)
+    monkeypatch.delenv("CCGPU_FORCE_NOMEM")
+    for net in nets:
+        net.train(2, batch=64, seed=6)
+        net.add_solve(s)
+        net.train(2, batch=128, seed=7)
+    assert np.array_equal(nets[0].params, nets[1].params)
