@@ -424,6 +424,7 @@ struct Solve {
   SolveDesc desc{};
   SolveDesc *d_desc = nullptr;
   hipStream_t stream = nullptr;
+  hipEvent_t ev_copy[2] = {nullptr, nullptr};   // halves of copy_to_host
   bool have_v = false, have_fock = false, derived = false, have_t = false;
   bool native_v = false;   // V from the built-in generator (needed by (T))
   uint64_t vgen = 0;       // counts changes of V (a shared pp ladder refills its union blocks)
@@ -482,6 +483,8 @@ struct Solve {
   ~Solve() {
     for (void *p : owned) (void)hipFree(p);
     for (void *p : t3_owned) (void)hipFree(p);
+    for (hipEvent_t e : ev_copy)
+      if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -569,6 +572,7 @@ void build_device(Solve &S) {
   auto &o = S.owned;
   SolveDesc &d = S.desc;
   HIPCHK(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+  for (hipEvent_t &e : S.ev_copy) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   d.A = P.A; d.nsp = P.nsp; d.np = P.np; d.nch = P.nch; d.nphc = P.nphc;
   d.nT = P.nT; d.active = 1;
   d.kx = dupload(P.orb.kx, o); d.ky = dupload(P.orb.ky, o); d.kz = dupload(P.orb.kz, o);
@@ -2285,29 +2289,36 @@ void ensure_f32(Solve &S, int handle) {
 // while threads empty the other.  The runtime's own pageable copy empties its staging
 // buffer with one thread, which also takes the page faults of a fresh array: 32 MB took
 // 2.25 ms, 1.26 this, 11.5 MB 742 us and 399.  One stage for the process, used
-// under the API lock and given back with the last handle.
+// under the API lock and given back with the last handle; the events belong to the
+// solve, on the device of its stream.
 struct HostStage {
   static constexpr size_t kHalf = (size_t)4 << 20, kPiece = (size_t)256 << 10;
   char *p = nullptr;
-  hipEvent_t ev[2] = {nullptr, nullptr};
   void release() {
     if (p) (void)hipHostFree(p);
-    for (hipEvent_t &e : ev) {
-      if (e) (void)hipEventDestroy(e);
-      e = nullptr;
-    }
     p = nullptr;
   }
   void make() {
-    if (p) return;
-    for (hipEvent_t &e : ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    HIPCHK(hipHostMalloc((void **)&p, 2 * kHalf, hipHostMallocDefault));
+    if (!p) HIPCHK(hipHostMalloc((void **)&p, 2 * kHalf, hipHostMallocPortable));
   }
 } g_stage;
 
-void copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
+// memory that only the runtime's own copies reach
+bool device_pointer(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {   // pageable memory may be an error
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeArray;
+}
+
+void copy_to_host(void *dst, const void *src, size_t bytes, const Solve &S) {
   constexpr size_t half = HostStage::kHalf, piece = HostStage::kPiece;
-  if (bytes < ((size_t)2 << 20)) {   // 1.5 MB: 103 us against 85, which the threads' start eats in a busy process
+  const hipStream_t st = S.stream;
+  if (!dst && bytes) throw Error("null pointer for the amplitudes");
+  // 1.5 MB: 103 us against 85, which the threads' start eats in a busy process
+  if (bytes < ((size_t)2 << 20) || device_pointer(dst)) {
     HIPCHK(hipStreamSynchronize(st));
     HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return;
@@ -2344,7 +2355,7 @@ void copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
   auto fill = [&](size_t h) {
     HIPCHK(hipMemcpyAsync(g_stage.p + h % 2 * half, (const char *)src + h * half, std::min(half, bytes - h * half),
                           hipMemcpyDeviceToHost, st));
-    HIPCHK(hipEventRecord(g_stage.ev[h % 2], st));
+    HIPCHK(hipEventRecord(S.ev_copy[h % 2], st));
   };
   fill(0);
   const size_t nt = std::min<size_t>({npiece / 2, 7, std::max(2u, std::thread::hardware_concurrency()) / 2});
@@ -2358,7 +2369,7 @@ void copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
       while (done.load(std::memory_order_acquire) < h * (half / piece)) std::this_thread::yield();
       fill(h + 1);
     }
-    HIPCHK(hipEventSynchronize(g_stage.ev[h % 2]));
+    HIPCHK(hipEventSynchronize(S.ev_copy[h % 2]));
     ready.store(std::min(npiece, (h + 1) * (half / piece)), std::memory_order_release);
     if (threads.t.empty())
       for (size_t k = h * (half / piece); k < ready.load(); ++k) empty_one(k);
@@ -3108,7 +3119,7 @@ int ccgpu_set_t2(int handle, int n, const int *a, const int *b, const int *i, co
 int ccgpu_get_t2_unique(int handle, double *t) {
   return guarded([&] {
     Solve &S = get(handle);
-    copy_to_host(t, S.desc.T, S.plan.nT * sizeof(double2), S.stream);
+    copy_to_host(t, S.desc.T, S.plan.nT * sizeof(double2), S);
   });
 }
 

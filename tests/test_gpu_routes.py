@@ -239,3 +239,51 @@ def test_network_after_a_refused_allocation(ccnm, monkeypatch):
         net.add_solve(s)
         net.train(2, batch=128, seed=7)
     assert np.array_equal(nets[0].params, nets[1].params)
+
+
+def pnm66_n3(ccnm):
+    s = ccnm.Solver(A=66, matter=ccnm.PNM, rho=0.16, nmax=3)   # 11.5 MB of amplitudes
+    s.generate_interaction()
+    s.setup_t_amplitudes()
+    return s
+
+
+def test_amplitudes_into_every_kind_of_memory(ccnm):
+    """ccgpu_get_t2_unique into pageable, pinned and device memory, and into
+    none, which is an error: the route through pinned halves is for host memory."""
+    rt = C.CDLL("libamdhip64.so.7")
+    s = pnm66_n3(ccnm)
+    want = s.t2_unique()
+    get = ccnm.lib().ccgpu_get_t2_unique
+    got = np.empty_like(want)
+    for alloc, free in (("hipMalloc", "hipFree"), ("hipHostMalloc", "hipHostFree")):
+        p = C.c_void_p()
+        args = (C.byref(p), C.c_size_t(want.nbytes)) + ((C.c_uint(0),) if alloc == "hipHostMalloc" else ())
+        assert getattr(rt, alloc)(*args) == 0
+        assert get(s.h, C.cast(p, C.POINTER(C.c_double))) == 0
+        assert rt.hipMemcpy(C.c_void_p(got.ctypes.data), p, C.c_size_t(want.nbytes), C.c_int(4)) == 0
+        assert getattr(rt, free)(p) == 0
+        assert np.any(want != 0) and np.array_equal(got, want), alloc
+        got[:] = 0
+    assert get(s.h, C.POINTER(C.c_double)()) != 0
+    assert np.array_equal(s.t2_unique(), want)
+
+
+def test_amplitudes_of_a_handle_on_a_second_gpu(ccnm):
+    """Large copies to host memory from handles on two devices of one process."""
+    rt = C.CDLL("libamdhip64.so.7")
+    n = C.c_int()
+    assert rt.hipGetDeviceCount(C.byref(n)) == 0
+    if n.value < 2:
+        pytest.skip("one GPU")
+    got = []
+    try:
+        for dev in (0, 1):
+            assert rt.hipSetDevice(dev) == 0
+            got.append(pnm66_n3(ccnm))
+        for dev in (1, 0):   # also with the other device current
+            assert rt.hipSetDevice(dev) == 0
+            a, b = (s.t2_unique() for s in got)
+            assert np.any(a != 0) and np.array_equal(a, b)
+    finally:
+        rt.hipSetDevice(0)
