@@ -431,6 +431,8 @@ struct Solve {
   int vkind = -1;          // CCGPU_INT_* of the generated V
   ChiralModel chiral = chiral_model(3, 450.0, nullptr);   // constants of CCGPU_INT_CHIRAL
   ChiralDev chiral_dev{};  // its device tables (set by the generator)
+  double *rad = nullptr, *side = nullptr;   // and their memory
+  int *pimg = nullptr;     // parity images of the orbitals
   // three-nucleon force of CCGPU_INT_CHIRAL: -1 off, else the normal-ordering
   // level (0 E0, 1 and Fock, 2 and 3 and the two-body blocks; 3 also puts the
   // three-body element into (T)) and its constants; tnf_set once the
@@ -2644,8 +2646,13 @@ void make_chiral_tables(Solve &S) {
   std::vector<double> rad = chiral_radial_table(c, qunit, mmax);
   std::vector<double> side = chiral_side_table(c, qunit, jmax);
   ChiralDev &d = S.chiral_dev;
-  d.rad = dupload(rad, S.owned);
-  d.side = dupload(side, S.owned);
+  // sizes are the lattice's, so another interaction takes the tables of the last
+  if (!S.rad) S.rad = dalloc<double>(rad.size(), S.owned);
+  if (!S.side) S.side = dalloc<double>(side.size(), S.owned);
+  HIPCHK(hipMemcpy(S.rad, rad.data(), rad.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(S.side, side.data(), side.size() * sizeof(double), hipMemcpyHostToDevice));
+  d.rad = S.rad;
+  d.side = S.side;
   d.jmax = jmax;
   d.order = c.order;
   d.qunit = qunit;
@@ -2719,7 +2726,8 @@ int ccgpu_generate_interaction(int handle, int kind) {
             ok = (x < P.A) == (y < P.A) && o.kx[y] == -o.kx[x] && o.ky[y] == -o.ky[x] && o.kz[y] == -o.kz[x];
             img[x] = y;
           }
-          if (ok) S.desc.pimg = dupload(img, S.owned);
+          if (ok && !S.pimg) S.pimg = dupload(img, S.owned);   // the lattice's
+          if (ok) S.desc.pimg = S.pimg;
         }
         check_launch();
         launch_3nf(S.desc, c, S.tnf, P.nch, P.nphc, P.max_npp, P.max_nhh, max_nhp, S.stream);

@@ -287,3 +287,19 @@ def test_amplitudes_of_a_handle_on_a_second_gpu(ccnm):
             assert np.any(a != 0) and np.array_equal(a, b)
     finally:
         rt.hipSetDevice(0)
+
+
+def test_generating_again_takes_no_more_device_memory(ccnm):
+    """A scan over the constants of the interaction on one handle: its tables
+    (of the lattice's size: 20 kB of radial functions at |n_i|<=2, side factors,
+    parity images of the orbitals) are written again, not added."""
+    s = ccnm.Solver(A=2, matter=ccnm.PNM, rho=0.16, nmax=2)
+    def generate(k):
+        s.set_chiral(ccnm.NNLO, 450.0, ci=(-0.74, -0.49 - 1e-3 * k, -0.65, 0.96))
+        s.set_3nf(0)
+        s.generate_interaction(ccnm.INT_CHIRAL)
+    generate(0)
+    before = device_memory_free()
+    for k in range(1, 513):
+        generate(k)
+    assert before - device_memory_free() < 4 << 20
