@@ -1467,6 +1467,7 @@ void prepare_ringbf(Batch &B) {
     autotune(*L, 8, B.d_descs, B.stream);
     L->build_tiles();
     L->upload(B.owned);
+    L->ready = true;
   }
   B.rbf.ready = true;
 }
@@ -1477,16 +1478,17 @@ void prepare_lists(Batch &B, int prec) {
                          &B.g_i4f, &B.g_rtf, &B.g_ppbf};
   // families in FP64 that the tiles of contract.hip contract
   const bool tiles64 = fp64_tiles() && tail_low_mask() == 0;
-  const bool all64 = prec == CCGPU_PREC_FP64 || prec == CCGPU_PREC_V32;
   if (tiles64) prepare_fp64(B);
   const bool fused32 = fp64_tiles() && B.ring32;
   if (fused32 && prec == CCGPU_PREC_BF16X3) prepare_ringbf(B);
   for (int k = 0; k < 13; ++k) {
     GemmList &L = *lists[k];
     if (L.ready) continue;
-    if (tiles64 && all64 && k < 5 && k != 1) continue;
+    // in FP64 these families run tiles, under BF16x3 lists of their own or the fused ring
+    if (tiles64 && prec != CCGPU_PREC_FP32 && k < 5 && k != 1) continue;
     if (k == 5 && (prec == CCGPU_PREC_FP64 || !B.has_f32)) continue;
     if (k >= 6 && prec != CCGPU_PREC_BF16X3) continue;
+    if (k >= 8 && k < 10 && B.ring32) continue;
     if (k >= 10 && k < 12 && (!B.ring32 || fused32)) continue;
     if (k == 12 && !B.ppbf) continue;
     autotune(L, kinds[k], B.d_descs, B.stream);
@@ -1537,6 +1539,7 @@ bool known_precision(int p) {
 
 void run_gemm(const GemmList &L, const Batch &B, int prec, bool a_f32, hipStream_t st, bool pp = false,
               int kind_override = -1) {
+  if (!L.ready && !L.groups.empty()) throw Error(fmt("internal: work list %d not prepared", L.id()));
   // the shared pp ladder's groups span every solve of the batch: no per-solve skip
   const SolveDesc *dd = L.fam == 5 ? nullptr : B.d_descs;
   if (gemm_variant_override() == 3) {

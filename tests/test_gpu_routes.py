@@ -303,3 +303,19 @@ def test_generating_again_takes_no_more_device_memory(ccnm):
     for k in range(1, 513):
         generate(k)
     assert before - device_memory_free() < 4 << 20
+
+
+def test_low_precision_solve_tunes_only_lists_that_it_launches(ccnm):
+    """A BF16x3 solve contracts X and the hh ladder on its own lists, the ring in
+    one launch, and its FP64 iterations outside the pp ladder on tiles that need
+    no tuning: no time goes to shapes of the lists these replace."""
+    s = ccnm.Solver(A=14, matter=ccnm.PNM, rho=0.16, nmax=2, twist=(0.31, 1.27, 2.03))
+    s.generate_interaction()
+    s.setup_t_amplitudes()
+    seen = len(ccnm.autotune_report())
+    r = s.ccd_iter(precision=ccnm.PREC_BF16X3, fp32_switch=1e-3)
+    assert r["converged"] and r["fp32_iterations"] < r["iterations"]
+    tuned = {x.split(":")[0].strip() for x in ccnm.autotune_report()[seen:].split(";") if x.strip()}
+    assert "fam10/kind6" in tuned   # X under BF16x3
+    dead = {f"fam{f}/kind0" for f in (0, 2, 3, 4)} | {f"fam{f}/kind6" for f in (13, 14)}
+    assert not tuned & dead, tuned
