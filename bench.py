@@ -392,8 +392,8 @@ def ladder_roofline(ccnm, s, precision):
     d = s.dims
     ms, n = st["gemm_pp_ladder"]   # FP32 runs stop at DEPTH iterations: all in FP32
     vbytes = 16.0 if precision == ccnm.PREC_FP64 else 8.0
-    # V read once, T read, R read and written once (complex16 each)
-    alg_bytes = vbytes * d["vpppp_unique"] + 3 * 16.0 * d["t2_unique"]
+    # V and T read once, their product written once (complex16 each)
+    alg_bytes = vbytes * d["vpppp_unique"] + 2 * 16.0 * d["t2_unique"]
     flops = d["pp_ladder_flops"]
     return ms, n, alg_bytes, flops, st
 

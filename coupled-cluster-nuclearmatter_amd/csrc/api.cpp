@@ -1623,10 +1623,12 @@ void residual_launches(Batch &B, int prec, int mode, bool timing) {
   // in a graph too: with the ladder after X, and the hh ladder after I6 and X, the ring
   // shared the ladder's queue and ran after it.  PNM A=66 |n_i|<=4 in FP64 17.0 to 16.1
   // ms, |n_i|<=3 mixed 5.70 to 5.04, four densities 19.4 to 18.6.
-  // A fork and its join cost some 10 us each on the host and the queues, which
-  // small batches do not win back: an iteration of SNM A=28 |n_i|<=2 (92 k
-  // amplitudes) takes 145 us on three streams and 124 on one, SNM A=76 |n_i|<=2
-  // (411 k) 206 on either, PNM A=66 |n_i|<=3 (721 k) 302 and 326.
+  // A fork and its join cost some 10 us each on the host and the queues, which small
+  // batches do not win back.  An iteration on one stream and on three, us, FP64 (reference
+  // update) | V32 | BF16x3 with Anderson | FP32: PNM A=66 |n_i|<=2 (123 k amplitudes) 84, 110
+  // | 93, 111 | 108, 124 | 157, 161; A=38 |n_i|<=3 (296 k) 149, 174 | 169, 184 | 179, 186 | 248,
+  // 229; SNM A=28 |n_i|<=3 (302 k) 248, 258 | 256, 247 | 248, 235 | 303, 267; PNM A=54 |n_i|<=3
+  // (528 k) 240, 231 | 246, 235 | 246, 224 | 351, 292.
   constexpr int64_t kForkAmplitudes = 400000;
   int64_t amplitudes = 0;
   for (const Solve *S : B.solves) amplitudes += S->plan.nT;
