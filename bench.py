@@ -553,8 +553,7 @@ def main():
         return
 
     # plain arm: the FP64 answer of every density and the time to it
-    plain = run_plain(ccnm, solvers)   # warm (tunes the tile shapes of the lists)
-    shapes = ccnm.autotune_report()
+    plain = run_plain(ccnm, solvers)   # warm
     plain_s, plain = timed(lambda: run_plain(ccnm, solvers), 2)
     print(f"# plain FP64: {plain_s * 1e3:.1f} ms, iterations {[r['iterations'] for r in plain]}",
           file=sys.stderr, flush=True)
@@ -628,6 +627,7 @@ def main():
     ms64, n64, bytes64, flops64, st64 = ladder_roofline(ccnm, solvers[2], ccnm.PREC_FP64)
     ms32, n32, bytes32, flops32, st32 = ladder_roofline(ccnm, solvers[2], ccnm.PREC_FP32)
     stbf = ladder_roofline(ccnm, solvers[2], ccnm.PREC_BF16X3)[4]
+    shapes = ccnm.autotune_report()   # of the bench lattice's lists and the training lattices'
     gbs64 = bytes64 / (ms64 * 1e-3) / 1e9
     tfs64 = flops64 / (ms64 * 1e-3) / 1e12
     ai64 = flops64 / bytes64
