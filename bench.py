@@ -681,7 +681,7 @@ def main():
                                "chiral NNLO(450) NN; FP64 answer: the plain arm at |dE| <= 1e-8 MeV",
                    "arms": "fast = learned warm start + the four densities in one batch + hipGraph + Anderson "
                            "update + precision plan (low precision until |dE| <= 3e-2 MeV, then FP64, stop at "
-                           "|dE/N| <= 1e-5 MeV twice in a row), must land within 1e-5 MeV/N of FP64; plain = "
+                           "|dE/N| <= 1e-5 MeV), must land within 1e-5 MeV/N of FP64; plain = "
                            "MBPT2 start, the reference's update with DIIS 8/8, FP64, one density after another, "
                            "to |dE| <= 1e-8 MeV",
                    "fast_plan": best,
