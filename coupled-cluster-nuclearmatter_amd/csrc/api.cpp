@@ -620,6 +620,10 @@ void build_device(Solve &S) {
   d.hp_j = dupload(P.hp_j, o); d.hp_b = dupload(P.hp_b, o);
   d.ring2 = dupload(P.ring2, o);
   d.ring2b = P.ring2b.empty() ? nullptr : dupload(P.ring2b, o);
+  d.gpp = pair_groups(P.orb, P.pp_a, P.pp_b, P.off_pp, o);
+  d.ghh = pair_groups(P.orb, P.hh_i, P.hh_j, P.off_hh, o);
+  d.ghp = pair_groups(P.orb, P.hp_j, P.hp_b, P.off_hp, o);
+  d.gph = pair_groups(P.orb, P.ph_i, P.ph_a, P.off_ph, o);
   d.T = dalloc<double2>(P.nT, o);
   d.R = dalloc<double2>(P.nT, o);
   d.R0 = dalloc<double2>(P.nT, o);
@@ -2634,21 +2638,6 @@ int one_species(const Orbitals &o) {
   return 1;
 }
 
-// Pair groups of the chiral fill, the lattice's: made for the first chiral interaction
-// (0.1 ms of every handle's creation otherwise: 1.14 to 1.25 ms at A=14 |n_i|<=1)
-void make_pair_groups(Solve &S) {
-  const Plan &P = S.plan;
-  SolveDesc &d = S.desc;
-  if (d.gph.g) return;
-  Fresh f;
-  d.gpp = pair_groups(P.orb, P.pp_a, P.pp_b, P.off_pp, f.own);
-  d.ghh = pair_groups(P.orb, P.hh_i, P.hh_j, P.off_hh, f.own);
-  d.ghp = pair_groups(P.orb, P.hp_j, P.hp_b, P.off_hp, f.own);
-  const PairGroups last = pair_groups(P.orb, P.ph_i, P.ph_a, P.off_ph, f.own);
-  f.keep(S.owned);
-  d.gph = last;
-}
-
 // Device tables of the chiral NN for this lattice: radial functions over
 // m = |dn|^2 <= 3 (4 nmax)^2 and the per-side factors over j <= 3 (2 nmax)^2.
 void make_chiral_tables(Solve &S) {
@@ -2714,7 +2703,6 @@ int ccgpu_generate_interaction(int handle, int kind) {
       throw Error("the three-nucleon force belongs to the chiral interaction (CCGPU_INT_CHIRAL)");
     if (kind == CCGPU_INT_CHIRAL) {
       make_chiral_tables(S);
-      make_pair_groups(S);
       launch_fill_blocks_chiral(S.desc, S.chiral_dev, P.nch, P.nphc, S.stream);
       if (S.tnf >= 0) {
         Chiral3Dev &c = S.chiral3;
