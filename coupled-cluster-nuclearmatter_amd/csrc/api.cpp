@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -541,32 +542,50 @@ struct Timer {
   }
 };
 
-// Pair groups of the pairs (a[x], b[x]), channel c at [off[c], off[c + 1]).  In a channel
-// conservation gives a group of a one group of b.
-PairGroups pair_groups(const Orbitals &o, const std::vector<int> &a, const std::vector<int> &b,
-                       const std::vector<int64_t> &off, std::vector<void *> &owned) {
+// Pair groups of lists of pairs (a[x], b[x]), channel c at [off[c], off[c + 1]).  In a
+// channel conservation gives a group of a one group of b.  The lists share one upload.
+struct PairList {
+  const std::vector<int> &a, &b;
+  const std::vector<int64_t> &off;
+  PairGroups &out;
+};
+void pair_groups(const Orbitals &o, std::initializer_list<PairList> lists, std::vector<void *> &owned) {
   std::map<std::array<int, 4>, int> ids;
   std::vector<int> id(o.nsp);
   for (int x = 0; x < o.nsp; ++x)
     id[x] = ids.emplace(std::array<int, 4>{o.nx[x], o.ny[x], o.nz[x], o.tz[x]}, (int)ids.size()).first->second;
   std::vector<PairGroup> g;
-  std::vector<int64_t> goff{0};
-  std::vector<int> last(ids.size(), -1);   // last group with this group of a
-  int most = 0;
-  for (size_t c = 0; c + 1 < off.size(); ++c) {
-    const int start = (int)g.size();
-    for (int64_t x = off[c]; x < off[c + 1]; ++x) {
-      int &at = last[id[a[x]]];
-      if (at < start || id[g[at].b] != id[b[x]]) {
-        at = (int)g.size();
-        g.push_back(PairGroup{a[x], b[x], {-1, -1, -1, -1}});
+  std::vector<int64_t> goff;
+  std::vector<std::array<size_t, 2>> at;   // where a list starts in g and goff
+  for (const PairList &l : lists) {
+    const size_t base = g.size();
+    at.push_back({base, goff.size()});
+    goff.push_back(0);
+    std::vector<int> last(ids.size(), -1);   // last group with this group of a
+    int most = 0;
+    for (size_t c = 0; c + 1 < l.off.size(); ++c) {
+      const int start = (int)(g.size() - base);
+      for (int64_t x = l.off[c]; x < l.off[c + 1]; ++x) {
+        int &k = last[id[l.a[x]]];
+        if (k < start || id[g[base + k].b] != id[l.b[x]]) {
+          k = (int)(g.size() - base);
+          g.push_back(PairGroup{l.a[x], l.b[x], {-1, -1, -1, -1}});
+        }
+        g[base + k].at[(o.sz[l.a[x]] > 0 ? 2 : 0) + (o.sz[l.b[x]] > 0 ? 1 : 0)] = (int)(x - l.off[c]);
       }
-      g[at].at[(o.sz[a[x]] > 0 ? 2 : 0) + (o.sz[b[x]] > 0 ? 1 : 0)] = (int)(x - off[c]);
+      goff.push_back((int64_t)(g.size() - base));
+      most = std::max(most, (int)(g.size() - base) - start);
     }
-    goff.push_back((int64_t)g.size());
-    most = std::max(most, (int)g.size() - start);
+    l.out.max = most;
   }
-  return PairGroups{dupload(g, owned), dupload(goff, owned), most};
+  const PairGroup *dg = dupload(g, owned);
+  const int64_t *doff = dupload(goff, owned);
+  size_t k = 0;
+  for (const PairList &l : lists) {
+    l.out.g = dg + at[k][0];
+    l.out.off = doff + at[k][1];
+    ++k;
+  }
 }
 
 void build_device(Solve &S) {
@@ -620,10 +639,8 @@ void build_device(Solve &S) {
   d.hp_j = dupload(P.hp_j, o); d.hp_b = dupload(P.hp_b, o);
   d.ring2 = dupload(P.ring2, o);
   d.ring2b = P.ring2b.empty() ? nullptr : dupload(P.ring2b, o);
-  d.gpp = pair_groups(P.orb, P.pp_a, P.pp_b, P.off_pp, o);
-  d.ghh = pair_groups(P.orb, P.hh_i, P.hh_j, P.off_hh, o);
-  d.ghp = pair_groups(P.orb, P.hp_j, P.hp_b, P.off_hp, o);
-  d.gph = pair_groups(P.orb, P.ph_i, P.ph_a, P.off_ph, o);
+  pair_groups(P.orb, {{P.pp_a, P.pp_b, P.off_pp, d.gpp}, {P.hh_i, P.hh_j, P.off_hh, d.ghh},
+                      {P.hp_j, P.hp_b, P.off_hp, d.ghp}, {P.ph_i, P.ph_a, P.off_ph, d.gph}}, o);
   d.T = dalloc<double2>(P.nT, o);
   d.R = dalloc<double2>(P.nT, o);
   d.R0 = dalloc<double2>(P.nT, o);
@@ -1323,7 +1340,7 @@ void build_shared(Batch &B) {
   }
   X.d_maps = dupload(maps, B.owned);
   X.d_npp = dupload(X.npp, B.owned);
-  X.gpp = pair_groups(B.solves[0]->plan.orb, X.pa, X.pb, X.off_pp, B.owned);
+  pair_groups(B.solves[0]->plan.orb, {{X.pa, X.pb, X.off_pp, X.gpp}}, B.owned);
   X.d_pa = dupload(X.pa, B.owned);
   X.d_pb = dupload(X.pb, B.owned);
   X.d_off_pp = dupload(X.off_pp, B.owned);
