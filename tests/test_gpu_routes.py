@@ -319,3 +319,24 @@ def test_low_precision_solve_tunes_only_lists_that_it_launches(ccnm):
     assert "fam10/kind6" in tuned   # X under BF16x3
     dead = {f"fam{f}/kind0" for f in (0, 2, 3, 4)} | {f"fam{f}/kind6" for f in (13, 14)}
     assert not tuned & dead, tuned
+
+
+@pytest.mark.parametrize("A,matter,nmax", [(28, "snm", 2), (54, "pnm", 3)])
+def test_residual_launches_give_the_same_bits(ccnm, monkeypatch, A, matter, nmax):
+    """Below 400 k amplitudes an FP64 residual runs in merged launches on one
+    stream, above it on three; CCGPU_FORK=0 keeps one stream, CCGPU_TIMING=1 one
+    launch after another: the same tiles and sums, so the same bits."""
+    s = ccnm.Solver(A=A, matter=ccnm.PNM if matter == "pnm" else ccnm.SNM, rho=0.16, nmax=nmax)
+    assert (s.dims["t2_unique"] < 400000) == (nmax == 2)
+    s.generate_interaction()
+    got = []
+    for env in (None, "CCGPU_FORK", "CCGPU_TIMING"):
+        with monkeypatch.context() as m:
+            if env:
+                m.setenv(env, "0" if env == "CCGPU_FORK" else "1")
+            s.setup_t_amplitudes()
+            s.ccd_iter(subspace=4, diis_step=4, tol=1e-30, maxit=3)
+            got.append(s.t2_unique())
+    assert np.any(got[0] != 0)
+    for t in got[1:]:
+        assert np.array_equal(t, got[0])
